@@ -69,6 +69,13 @@ int moe_topk_softmax(const float* gating_output, float* topk_weights, int32_t* t
                      int32_t* token_expert_indices, int T, int E, int K, int renormalize,
                      void* stream);
 
+/* moe_topk_softmax on logits of any MoeDtype code of 16 or 32 bits (MOE_F32, MOE_F16, MOE_BF16): the
+ * row is widened to fp32 as it is loaded, which is what the reference's `.float()` in front of the op
+ * does with a pass over memory of its own (nanovllm/layers/for_moe/fused_moe.py:408-414).
+ * `token_expert_indices` may be NULL when the caller has no use for it. */
+int moe_topk_softmax_typed(const void* gating_output, int dtype, float* topk_weights, int32_t* topk_ids,
+                           int32_t* token_expert_indices, int T, int E, int K, int renormalize, void* stream);
+
 /* Router gate fused in front of `topk_softmax`: logits = x . gate_weight^T (the
  * `ReplicatedLinear` gate of nanovllm/models/qwen3_moe.py:93-104 followed by the
  * call at :113-118; nanovllm/layers/linear.py:53-60), rounded to the activation
@@ -230,6 +237,37 @@ typedef struct MoeFusedExpertsArgs {
 int64_t moe_fused_experts_workspace_bytes(int T, int H, int I, int E, int K, int block_size,
                                           int act_dtype, int weight_dtype);
 int moe_fused_experts(const MoeFusedExpertsArgs* args);
+
+/* The layer from the router's logits (or from its weights and ids) to the combined result as one call:
+ * what FusedMoE.forward enqueues (nanovllm/layers/fused_moe.py:163-216: select_experts, then
+ * fused_experts of nanovllm/layers/for_moe/fused_moe.py:422-631, whose alignment is part of it). */
+typedef struct MoeLayerArgs {
+  const void* x;             /* [T, H]                                                */
+  void* out;                 /* [T, H], may be x                                      */
+  const void* w13;           /* as in MoeFusedExpertsArgs                             */
+  const void* w2;
+  const void* w13_bias;
+  const void* w2_bias;
+  const float* w13_scale;
+  const float* w2_scale;
+  const void* router_logits; /* [T, E] of logits_dtype; NULL: topk_weights / topk_ids are given */
+  float* topk_weights;       /* [T, K], read when router_logits is NULL               */
+  int32_t* topk_ids;         /* [T, K], likewise                                      */
+  void* workspace;           /* 256-byte aligned, one call at a time                  */
+  int64_t workspace_bytes;
+  int64_t w13_stride_e, w13_stride_n, w2_stride_e, w2_stride_n;
+  int32_t T, H, I, E, K;
+  int32_t block_size;        /* alignment block; 0: the library's choice              */
+  int32_t logits_dtype, renormalize;
+  int32_t act_dtype, weight_dtype, activation, apply_router_weight_on_input;
+  float swiglu_alpha, swiglu_limit;
+  int32_t weight_layout;
+  void* stream;
+} MoeLayerArgs;
+/* Workspace of a call with these arguments (pointers other than null / non-null do not matter, except
+ * that tensors of a 16-bit or e4m3 call that are not 16-byte aligned choose other kernels). */
+int64_t moe_layer_workspace_bytes(const MoeLayerArgs* args);
+int moe_layer(const MoeLayerArgs* args);
 
 /* No counterpart in the reference (its two Triton launches need no hand-off).  With 16-bit
  * dtypes and blocks of 256 slots moe_fused_experts enqueues both GEMM passes as one launch,

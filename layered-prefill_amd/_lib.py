@@ -32,6 +32,7 @@ EXPORTS = (
     "moe_fused_experts_status", "moe_fused_experts_set_wait_limit", "moe_align_block_size_static",
     "moe_tile_expert_weights", "moe_tile_expert_weights_supported",
     "moe_route_align_supported", "moe_route_align_block_size",
+    "moe_topk_softmax_typed", "moe_layer_workspace_bytes", "moe_layer",
 )
 
 
@@ -55,7 +56,27 @@ class MoeFusedExpertsArgs(ctypes.Structure):
     ]
 
 
+class MoeLayerArgs(ctypes.Structure):
+    _fields_ = [
+        ("x", ctypes.c_void_p), ("out", ctypes.c_void_p), ("w13", ctypes.c_void_p),
+        ("w2", ctypes.c_void_p), ("w13_bias", ctypes.c_void_p), ("w2_bias", ctypes.c_void_p),
+        ("w13_scale", ctypes.c_void_p), ("w2_scale", ctypes.c_void_p),
+        ("router_logits", ctypes.c_void_p), ("topk_weights", ctypes.c_void_p), ("topk_ids", ctypes.c_void_p),
+        ("workspace", ctypes.c_void_p), ("workspace_bytes", ctypes.c_int64),
+        ("w13_stride_e", ctypes.c_int64), ("w13_stride_n", ctypes.c_int64),
+        ("w2_stride_e", ctypes.c_int64), ("w2_stride_n", ctypes.c_int64),
+        ("T", ctypes.c_int32), ("H", ctypes.c_int32), ("I", ctypes.c_int32),
+        ("E", ctypes.c_int32), ("K", ctypes.c_int32), ("block_size", ctypes.c_int32),
+        ("logits_dtype", ctypes.c_int32), ("renormalize", ctypes.c_int32),
+        ("act_dtype", ctypes.c_int32), ("weight_dtype", ctypes.c_int32), ("activation", ctypes.c_int32),
+        ("apply_router_weight_on_input", ctypes.c_int32),
+        ("swiglu_alpha", ctypes.c_float), ("swiglu_limit", ctypes.c_float),
+        ("weight_layout", ctypes.c_int32), ("stream", ctypes.c_void_p),
+    ]
+
+
 _lib: Optional[ctypes.CDLL] = None
+_host = None
 
 
 def build_library(verbose: bool = False) -> str:
@@ -73,6 +94,12 @@ def _declare(L: ctypes.CDLL) -> None:
     L.moe_abi_version.restype = i32
     L.moe_topk_softmax.restype = i32
     L.moe_topk_softmax.argtypes = [p, p, p, p, i32, i32, i32, i32, p]
+    L.moe_topk_softmax_typed.restype = i32
+    L.moe_topk_softmax_typed.argtypes = [p, i32, p, p, p, i32, i32, i32, i32, p]
+    L.moe_layer_workspace_bytes.restype = i64
+    L.moe_layer_workspace_bytes.argtypes = [ctypes.POINTER(MoeLayerArgs)]
+    L.moe_layer.restype = i32
+    L.moe_layer.argtypes = [ctypes.POINTER(MoeLayerArgs)]
     L.moe_gate_topk_softmax.restype = i32
     L.moe_gate_topk_softmax.argtypes = [p, p, i32, p, p, p, p, i32, i32, i32, i32, i32, p]
     L.moe_align_workspace_bytes.restype = i64
@@ -134,6 +161,20 @@ def lib() -> ctypes.CDLL:
         _declare(L)
         _lib = L
     return _lib
+
+
+def host():
+    """The native host module (csrc/host.cpp).  Raises if it has not been built."""
+    global _host
+    if _host is None:
+        lib()
+        try:
+            from . import _moe_host
+        except ImportError as e:
+            raise RuntimeError(f"_moe_host.so is missing or does not load ({e}): run `make -C {CSRC_DIR}` "
+                               "(or __graft_entry__.build())") from e
+        _host = _moe_host
+    return _host
 
 
 def check(rc: int) -> None:

@@ -1,0 +1,252 @@
+// The host side of the layer's calls in native code: checks a call's tensors, allocates its result and
+// workspace from torch's allocator and enters the C ABI, in a few microseconds where the same steps in
+// Python take tens (a decode step of a few tokens is over on the GPU in less).  Every function answers
+// None when the call is anything but the plain case; the Python caller then takes its own path, which
+// names what is wrong or serves what is rare.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+
+#include <ATen/ops/empty.h>
+#include <c10/core/DeviceGuard.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include "../../include/moe_gfx950.h"
+
+namespace {
+
+PyObject* g_raw_stream = nullptr;   // torch._C._cuda_getCurrentRawStream
+
+int dtype_code(at::ScalarType t) {
+  switch (t) {
+    case at::kFloat: return MOE_F32;
+    case at::kHalf: return MOE_F16;
+    case at::kBFloat16: return MOE_BF16;
+    default: return -1;
+  }
+}
+
+const at::Tensor* tensor(PyObject* o) { return THPVariable_Check(o) ? &THPVariable_Unpack(o) : nullptr; }
+
+// A GPU tensor, or null.
+const at::Tensor* gpu_tensor(PyObject* o) {
+  const at::Tensor* t = tensor(o);
+  return t && t->is_cuda() ? t : nullptr;
+}
+
+// False when `o` is neither None nor a contiguous GPU tensor on `dev` of `type` and `shape`; else `t` is it or null.
+bool optional_tensor(PyObject* o, const at::Device& dev, at::ScalarType type, at::IntArrayRef shape, const at::Tensor** t) {
+  *t = nullptr;
+  if (o == Py_None) return true;
+  const at::Tensor* x = gpu_tensor(o);
+  if (!x || x->device() != dev || x->scalar_type() != type || !x->is_contiguous() || x->sizes() != shape) return false;
+  *t = x;
+  return true;
+}
+
+void* current_stream(const at::Device& dev) {
+  PyObject* idx = PyLong_FromLong(dev.index());
+  PyObject* r = idx ? PyObject_CallOneArg(g_raw_stream, idx) : nullptr;
+  Py_XDECREF(idx);
+  if (!r) throw python_error();
+  void* s = PyLong_AsVoidPtr(r);
+  Py_DECREF(r);
+  return s;
+}
+
+void check(int rc) {
+  if (rc == 0) return;
+  PyErr_SetString(PyExc_RuntimeError, moe_last_error());
+  throw python_error();
+}
+
+at::Tensor empty(at::IntArrayRef shape, at::ScalarType type, const at::Device& dev) {
+  return at::empty(shape, at::TensorOptions().dtype(type).device(dev));
+}
+
+PyObject* tuple_of(const at::Tensor& a, const at::Tensor& b, const at::Tensor& c) {
+  PyObject* t = PyTuple_New(3);
+  if (!t) throw python_error();
+  PyTuple_SET_ITEM(t, 0, THPVariable_Wrap(a));
+  PyTuple_SET_ITEM(t, 1, THPVariable_Wrap(b));
+  PyTuple_SET_ITEM(t, 2, THPVariable_Wrap(c));
+  return t;
+}
+
+#define MOE_NONE Py_RETURN_NONE
+
+// layer(x, router_logits | None, w13, w2, w13_bias, w2_bias, w13_scale, w2_scale, topk_weights | None,
+//       topk_ids | None, top_k, renormalize, activation, weight_on_input, weight_layout, inplace)
+// -> result tensor, or None.  Codes as in moe_gfx950.h.
+PyObject* layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 16) MOE_NONE;
+  const at::Tensor *x = gpu_tensor(a[0]), *w13 = gpu_tensor(a[2]), *w2 = gpu_tensor(a[3]);
+  if (!x || !w13 || !w2 || x->dim() != 2 || w13->dim() != 3 || w2->dim() != 3) MOE_NONE;
+  const at::Device dev = x->device();
+  if (w13->device() != dev || w2->device() != dev || !x->is_contiguous()) MOE_NONE;
+  const int64_t T = x->size(0), H = x->size(1), E = w13->size(0), N = w13->size(1), I = N / 2;
+  if (T < 1 || T > 65536 || N % 2 || I < 1 || w13->size(2) != H || w2->size(0) != E || w2->size(1) != H || w2->size(2) != I)
+    MOE_NONE;
+  if (w13->stride(2) != 1 || w2->stride(2) != 1) MOE_NONE;
+  const int act = dtype_code(x->scalar_type());
+  if (act < 0 || w2->scalar_type() != w13->scalar_type()) MOE_NONE;
+  const bool fp8 = w13->scalar_type() == at::kFloat8_e4m3fn;
+  const at::Tensor *b13, *b2, *s13, *s2;
+  const int64_t n13[2] = {E, N}, n2[2] = {E, H};
+  if (!optional_tensor(a[4], dev, x->scalar_type(), n13, &b13) || !optional_tensor(a[5], dev, x->scalar_type(), n2, &b2) ||
+      !optional_tensor(a[6], dev, at::kFloat, n13, &s13) || !optional_tensor(a[7], dev, at::kFloat, n2, &s2))
+    MOE_NONE;
+  if (fp8) {
+    if (act == MOE_F32 || !s13 || !s2 || b13 || b2 || H % 16 || I % 16) MOE_NONE;
+    for (const at::Tensor* w : {w13, w2}) {
+      if ((E > 1 && w->stride(0) % 16) || w->stride(1) % 16) MOE_NONE;
+      if (reinterpret_cast<uintptr_t>(w->data_ptr()) & 15u) MOE_NONE;
+    }
+    if (reinterpret_cast<uintptr_t>(x->data_ptr()) & 15u) MOE_NONE;
+  } else if (w13->scalar_type() != x->scalar_type() || s13 || s2) {
+    MOE_NONE;
+  }
+  MoeLayerArgs m{};
+  const int64_t K = PyLong_AsLong(a[10]);
+  if (K < 1 || K > E || T * K > INT32_MAX) MOE_NONE;
+  if (a[1] != Py_None) {
+    const at::Tensor* g = gpu_tensor(a[1]);
+    if (!g || g->device() != dev || g->dim() != 2 || g->size(0) != T || g->size(1) != E || !g->is_contiguous()) MOE_NONE;
+    m.logits_dtype = dtype_code(g->scalar_type());
+    if (m.logits_dtype < 0) MOE_NONE;
+    m.router_logits = g->data_ptr();
+    m.renormalize = PyObject_IsTrue(a[11]);
+  } else {
+    const at::Tensor *w, *ids;
+    const int64_t tk[2] = {T, K};
+    if (!optional_tensor(a[8], dev, at::kFloat, tk, &w) || !optional_tensor(a[9], dev, at::kInt, tk, &ids) || !w || !ids) MOE_NONE;
+    m.topk_weights = static_cast<float*>(w->data_ptr());
+    m.topk_ids = static_cast<int32_t*>(ids->data_ptr());
+  }
+  m.activation = static_cast<int32_t>(PyLong_AsLong(a[12]));
+  m.apply_router_weight_on_input = PyObject_IsTrue(a[13]);
+  m.weight_layout = static_cast<int32_t>(PyLong_AsLong(a[14]));
+  const bool inplace = PyObject_IsTrue(a[15]);
+  c10::OptionalDeviceGuard guard(dev);
+  const at::Tensor out = inplace ? *x : empty({T, H}, x->scalar_type(), dev);
+  m.x = x->data_ptr();
+  m.out = out.data_ptr();
+  m.w13 = w13->data_ptr();
+  m.w2 = w2->data_ptr();
+  m.w13_bias = b13 ? b13->data_ptr() : nullptr;
+  m.w2_bias = b2 ? b2->data_ptr() : nullptr;
+  m.w13_scale = s13 ? static_cast<const float*>(s13->data_ptr()) : nullptr;
+  m.w2_scale = s2 ? static_cast<const float*>(s2->data_ptr()) : nullptr;
+  m.w13_stride_e = w13->stride(0);
+  m.w13_stride_n = w13->stride(1);
+  m.w2_stride_e = w2->stride(0);
+  m.w2_stride_n = w2->stride(1);
+  m.T = static_cast<int32_t>(T);
+  m.H = static_cast<int32_t>(H);
+  m.I = static_cast<int32_t>(I);
+  m.E = static_cast<int32_t>(E);
+  m.K = static_cast<int32_t>(K);
+  m.act_dtype = act;
+  m.weight_dtype = fp8 ? static_cast<int>(MOE_E4M3) : act;
+  m.swiglu_alpha = 1.702f;
+  m.swiglu_limit = 7.0f;
+  m.stream = current_stream(dev);
+  m.workspace_bytes = moe_layer_workspace_bytes(&m);
+  if (m.workspace_bytes <= 0) MOE_NONE;
+  const at::Tensor ws = empty({m.workspace_bytes}, at::kByte, dev);
+  m.workspace = ws.data_ptr();
+  check(moe_layer(&m));
+  if (inplace) {
+    Py_INCREF(a[0]);
+    return a[0];
+  }
+  return THPVariable_Wrap(out);
+  END_HANDLE_TH_ERRORS
+}
+
+// topk(router_logits, top_k, renormalize) -> (weights, ids, token_expert_indices), or None.
+PyObject* topk(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 3) MOE_NONE;
+  const at::Tensor* g = gpu_tensor(a[0]);
+  if (!g || g->dim() != 2 || !g->is_contiguous() || g->size(0) < 1) MOE_NONE;
+  const int dtype = dtype_code(g->scalar_type());
+  const int64_t T = g->size(0), E = g->size(1), K = PyLong_AsLong(a[1]);
+  if (dtype < 0 || K < 1 || K > E || T * K > INT32_MAX) MOE_NONE;
+  const at::Device dev = g->device();
+  c10::OptionalDeviceGuard guard(dev);
+  const at::Tensor w = empty({T, K}, at::kFloat, dev), ids = empty({T, K}, at::kInt, dev), tei = empty({T, K}, at::kInt, dev);
+  check(moe_topk_softmax_typed(g->data_ptr(), dtype, static_cast<float*>(w.data_ptr()), static_cast<int32_t*>(ids.data_ptr()),
+                               static_cast<int32_t*>(tei.data_ptr()), static_cast<int>(T), static_cast<int>(E),
+                               static_cast<int>(K), PyObject_IsTrue(a[2]), current_stream(dev)));
+  return tuple_of(w, ids, tei);
+  END_HANDLE_TH_ERRORS
+}
+
+// rms_norm(x, residual | None, weight, eps) -> the normalised tensor (residual updated in place), or None.
+PyObject* rms_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 4) MOE_NONE;
+  const at::Tensor *x = gpu_tensor(a[0]), *w = gpu_tensor(a[2]);
+  const at::Tensor* res = a[1] == Py_None ? nullptr : gpu_tensor(a[1]);
+  if (!x || !w || (!res && a[1] != Py_None) || x->dim() != 2) MOE_NONE;
+  const at::Device dev = x->device();
+  const int dtype = dtype_code(x->scalar_type());
+  const int64_t T = x->size(0), H = x->size(1);
+  if (dtype < 0 || T < 1 || H < 1 || H > INT32_MAX || !x->is_contiguous()) MOE_NONE;
+  if (w->device() != dev || w->dim() != 1 || w->size(0) != H || w->scalar_type() != x->scalar_type() || !w->is_contiguous())
+    MOE_NONE;
+  if (res && (res->device() != dev || res->scalar_type() != x->scalar_type() || res->sizes() != x->sizes() || !res->is_contiguous()))
+    MOE_NONE;
+  c10::OptionalDeviceGuard guard(dev);
+  const at::Tensor out = empty({T, H}, x->scalar_type(), dev);
+  check(moe_add_rms_norm(out.data_ptr(), H, res ? res->data_ptr() : nullptr, H, x->data_ptr(), H, w->data_ptr(), dtype, T,
+                         static_cast<int>(H), static_cast<float>(PyFloat_AsDouble(a[3])), current_stream(dev)));
+  return THPVariable_Wrap(out);
+  END_HANDLE_TH_ERRORS
+}
+
+// gate_topk(x, gate_weight, top_k, renormalize) -> (weights, ids, token_expert_indices), or None.
+PyObject* gate_topk(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 4) MOE_NONE;
+  const at::Tensor *x = gpu_tensor(a[0]), *g = gpu_tensor(a[1]);
+  if (!x || !g || x->dim() != 2 || g->dim() != 2 || !x->is_contiguous() || !g->is_contiguous()) MOE_NONE;
+  const at::Device dev = x->device();
+  const int dtype = dtype_code(x->scalar_type());
+  const int64_t T = x->size(0), H = x->size(1), E = g->size(0), K = PyLong_AsLong(a[2]);
+  if (T < 1 || g->device() != dev || g->scalar_type() != x->scalar_type() || g->size(1) != H || K < 1 || K > E ||
+      T * K > INT32_MAX || T * H * 2 >= (int64_t{1} << 32))
+    MOE_NONE;
+  if ((dtype != MOE_BF16 && dtype != MOE_F16) || (E != 32 && E != 64 && E != 128) || H % 64) MOE_NONE;
+  if ((reinterpret_cast<uintptr_t>(x->data_ptr()) | reinterpret_cast<uintptr_t>(g->data_ptr())) & 15u) MOE_NONE;
+  c10::OptionalDeviceGuard guard(dev);
+  const at::Tensor w = empty({T, K}, at::kFloat, dev), ids = empty({T, K}, at::kInt, dev), tei = empty({T, K}, at::kInt, dev);
+  check(moe_gate_topk_softmax(x->data_ptr(), g->data_ptr(), dtype, nullptr, static_cast<float*>(w.data_ptr()),
+                              static_cast<int32_t*>(ids.data_ptr()), static_cast<int32_t*>(tei.data_ptr()),
+                              static_cast<int>(T), static_cast<int>(H), static_cast<int>(E), static_cast<int>(K),
+                              PyObject_IsTrue(a[3]), current_stream(dev)));
+  return tuple_of(w, ids, tei);
+  END_HANDLE_TH_ERRORS
+}
+
+PyMethodDef methods[] = {
+    {"layer", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(layer)), METH_FASTCALL, nullptr},
+    {"topk", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(topk)), METH_FASTCALL, nullptr},
+    {"rms_norm", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(rms_norm)), METH_FASTCALL, nullptr},
+    {"gate_topk", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(gate_topk)), METH_FASTCALL, nullptr},
+    {nullptr, nullptr, 0, nullptr}};
+
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_moe_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__moe_host(void) {
+  PyObject* c = PyImport_ImportModule("torch._C");
+  if (!c) return nullptr;
+  g_raw_stream = PyObject_GetAttrString(c, "_cuda_getCurrentRawStream");
+  Py_DECREF(c);
+  if (!g_raw_stream) return nullptr;
+  return PyModule_Create(&module);
+}

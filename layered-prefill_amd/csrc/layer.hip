@@ -1,0 +1,121 @@
+// The expert MLP from routing to combine as one call: moe_layer enqueues whatever kernels suit the
+// batch: the router, the alignment of the ids by expert and moe_fused_experts.
+//
+// Replaces the sequence of nanovllm/layers/fused_moe.py:163-216 (select_experts, fused_experts) and
+// nanovllm/layers/for_moe/fused_moe.py:547-631 of the reference, whose host enqueues the steps apart.
+#include "common.h"
+
+namespace {
+
+struct Carver {   // places regions of a workspace one behind the other
+  char* base;
+  int64_t at = 0;
+  void* take(int64_t bytes) {
+    void* p = base + at;
+    at += moe_align_up(bytes, 256);
+    return p;
+  }
+};
+
+// Where everything sits in the workspace of a call.
+struct Layout {
+  int block;
+  int64_t sorted_cap, expert_cap, align_bytes, fused_bytes, bytes;
+  float* topk_w;
+  int32_t *topk_ids, *sorted, *experts, *npp;
+  void *align_ws, *fused_ws;
+};
+Layout layout_of(const MoeLayerArgs* a) {
+  Layout l{};
+  Carver c{static_cast<char*>(a->workspace)};
+  const int64_t numel = static_cast<int64_t>(a->T) * a->K;
+  if (a->router_logits) {
+    l.topk_w = static_cast<float*>(c.take(numel * 4));
+    l.topk_ids = static_cast<int32_t*>(c.take(numel * 4));
+  } else {
+    l.topk_w = a->topk_weights;
+    l.topk_ids = a->topk_ids;
+  }
+  l.block = a->block_size ? a->block_size : moe_preferred_block_size(a->T, a->E, a->K, a->act_dtype, a->weight_dtype);
+  l.sorted_cap = numel + static_cast<int64_t>(a->E) * (l.block - 1);
+  l.expert_cap = (l.sorted_cap + l.block - 1) / l.block;
+  l.align_bytes = moe_align_workspace_bytes(numel, a->E);
+  l.fused_bytes = moe_fused_experts_workspace_bytes(a->T, a->H, a->I, a->E, a->K, l.block, a->act_dtype, a->weight_dtype);
+  l.sorted = static_cast<int32_t*>(c.take(l.sorted_cap * 4));
+  l.experts = static_cast<int32_t*>(c.take(l.expert_cap * 4));
+  l.npp = static_cast<int32_t*>(c.take(4));
+  l.align_ws = c.take(l.align_bytes);
+  l.fused_ws = c.take(l.fused_bytes);
+  l.bytes = c.at;
+  return l;
+}
+
+int check_layer_args(const MoeLayerArgs* a) {
+  if (!a) return moe_fail(MOE_ERR_ARG, "layer: null argument block");
+  if (a->T < 0 || a->H < 1 || a->I < 1 || a->E < 1 || a->K < 1 || a->block_size < 0)
+    return moe_fail(MOE_ERR_ARG, "layer: bad sizes T=%d H=%d I=%d E=%d K=%d block_size=%d", a->T, a->H, a->I, a->E, a->K,
+                    a->block_size);
+  if (static_cast<int64_t>(a->T) * a->K > INT32_MAX) return moe_fail(MOE_ERR_ARG, "layer: T*K overflows int32");
+  return MOE_OK;
+}
+
+}  // namespace
+
+MOE_EXPORT int64_t moe_layer_workspace_bytes(const MoeLayerArgs* a) {
+  if (check_layer_args(a)) return 0;
+  return a->T == 0 ? 0 : layout_of(a).bytes;
+}
+
+MOE_EXPORT int moe_layer(const MoeLayerArgs* a) {
+  if (int rc = check_layer_args(a)) return rc;
+  if (a->T == 0) return MOE_OK;
+  if (!a->x || !a->out || !a->w13 || !a->w2) return moe_fail(MOE_ERR_ARG, "layer: null tensor pointer");
+  if (!a->router_logits && (!a->topk_weights || !a->topk_ids))
+    return moe_fail(MOE_ERR_ARG, "layer: neither router_logits nor topk_weights and topk_ids");
+  const Layout l = layout_of(a);
+  if (!a->workspace || a->workspace_bytes < l.bytes)
+    return moe_fail(MOE_ERR_WORKSPACE, "layer: workspace %lld B, needs %lld B", static_cast<long long>(a->workspace_bytes),
+                    static_cast<long long>(l.bytes));
+  if (reinterpret_cast<uintptr_t>(a->workspace) & 255u)
+    return moe_fail(MOE_ERR_WORKSPACE, "layer: workspace must be 256-byte aligned");
+  const int64_t numel = static_cast<int64_t>(a->T) * a->K;
+  if (a->router_logits) {
+    if (int rc = moe_topk_softmax_typed(a->router_logits, a->logits_dtype, l.topk_w, l.topk_ids, nullptr, a->T, a->E, a->K,
+                                        a->renormalize, a->stream))
+      return rc;
+  }
+  // align, with the large-tile kernel's plan left in its workspace when the sizes allow
+  int64_t bounds_off = 0, done_off = 0;
+  int32_t num_done = 0, cap_mb = 0;
+  const bool plan = l.block == 256 && moe_align_can_plan(numel, a->E) &&
+                    moe_fused_experts_plan_layout(a->T, a->H, a->I, a->E, a->K, l.block, a->act_dtype, a->weight_dtype,
+                                                  &bounds_off, &done_off, &num_done, &cap_mb);
+  char* fws = static_cast<char*>(l.fused_ws);
+  int rc;
+  if (plan)
+    rc = moe_align_block_size_planned(l.topk_ids, MOE_ID_I32, numel, a->E, l.block, l.sorted, l.sorted_cap, l.experts,
+                                      l.expert_cap, l.npp, l.align_ws, l.align_bytes, a->stream,
+                                      reinterpret_cast<int32_t*>(fws + bounds_off), reinterpret_cast<int32_t*>(fws + done_off),
+                                      num_done, cap_mb);
+  else
+    rc = moe_align_block_size(l.topk_ids, MOE_ID_I32, numel, a->E, l.block, l.sorted, l.sorted_cap, l.experts, l.expert_cap,
+                              l.npp, l.align_ws, l.align_bytes, a->stream);
+  if (rc) return rc;
+  MoeFusedExpertsArgs f{};
+  f.x = a->x; f.out = a->out; f.w13 = a->w13; f.w2 = a->w2;
+  f.w13_bias = a->w13_bias; f.w2_bias = a->w2_bias; f.w13_scale = a->w13_scale; f.w2_scale = a->w2_scale;
+  f.topk_weights = l.topk_w;
+  f.sorted_token_ids = l.sorted; f.expert_ids = l.experts; f.num_tokens_post_pad = l.npp;
+  f.workspace = l.fused_ws; f.workspace_bytes = l.fused_bytes;
+  f.w13_stride_e = a->w13_stride_e; f.w13_stride_n = a->w13_stride_n;
+  f.w2_stride_e = a->w2_stride_e; f.w2_stride_n = a->w2_stride_n;
+  f.T = a->T; f.H = a->H; f.I = a->I; f.E = a->E; f.K = a->K;
+  f.block_size = l.block; f.sorted_cap = l.sorted_cap;
+  f.act_dtype = a->act_dtype; f.weight_dtype = a->weight_dtype; f.activation = a->activation;
+  f.apply_router_weight_on_input = a->apply_router_weight_on_input;
+  f.swiglu_alpha = a->swiglu_alpha; f.swiglu_limit = a->swiglu_limit;
+  f.passes = plan ? 16 : 0;
+  f.weight_layout = a->weight_layout;
+  f.stream = a->stream;
+  return moe_fused_experts(&f);
+}

@@ -14,9 +14,9 @@
 
 namespace {
 
-template <int E>
+template <int E, typename El>
 __global__ __launch_bounds__(kWave* kWavesPerBlock) void topk_softmax_pow2_kernel(
-    const float* __restrict__ gating, float* __restrict__ topk_w, int32_t* __restrict__ topk_ids,
+    const typename El::S* __restrict__ gating, float* __restrict__ topk_w, int32_t* __restrict__ topk_ids,
     int32_t* __restrict__ tok_exp_idx, int T, int K, int renormalize) {
   using G = Pow2Geom<E>;
   constexpr int VPT = G::kVpt, TPR = G::kTpr;
@@ -28,7 +28,7 @@ __global__ __launch_bounds__(kWave* kWavesPerBlock) void topk_softmax_pow2_kerne
   const int ld_row = live ? row : (T - 1);
 
   float v[VPT];
-  load_row<E>(gating, ld_row, t, v);
+  load_row<E, El>(gating, ld_row, t, v);
   route_row<E>(v, t, row, live, topk_w, topk_ids, tok_exp_idx, T, K, renormalize);
 }
 
@@ -223,13 +223,14 @@ int launch_gate_e(const void* x, const void* wg, float* logits_out, float* w, in
 // One wavefront per row; lane l holds columns l, l+64, ... (up to 16 of them).
 constexpr int kGenericMaxPerLane = 16;
 
+template <typename El>
 __global__ __launch_bounds__(kWave* kWavesPerBlock) void topk_softmax_generic_kernel(
-    const float* __restrict__ gating, float* __restrict__ topk_w, int32_t* __restrict__ topk_ids,
+    const typename El::S* __restrict__ gating, float* __restrict__ topk_w, int32_t* __restrict__ topk_ids,
     int32_t* __restrict__ tok_exp_idx, int T, int E, int K, int renormalize) {
   const int lane = threadIdx.x % kWave;
   const int row = blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
   const bool live = row < T;
-  const float* src = gating + static_cast<size_t>(live ? row : T - 1) * E;
+  const typename El::S* src = gating + static_cast<size_t>(live ? row : T - 1) * E;
   const float ninf = -__builtin_inff();
 
   float v[kGenericMaxPerLane];
@@ -237,7 +238,7 @@ __global__ __launch_bounds__(kWave* kWavesPerBlock) void topk_softmax_generic_ke
 #pragma unroll
   for (int j = 0; j < kGenericMaxPerLane; ++j) {
     const int c = lane + j * kWave;
-    v[j] = c < E ? src[c] : ninf;
+    v[j] = c < E ? El::ld(src[c]) : ninf;
     mx = fmaxf(mx, v[j]);
   }
 #pragma unroll
@@ -278,7 +279,7 @@ __global__ __launch_bounds__(kWave* kWavesPerBlock) void topk_softmax_generic_ke
       const size_t o = static_cast<size_t>(row) * K + k;
       topk_w[o] = best;
       topk_ids[o] = bidx;
-      tok_exp_idx[o] = k * T + row;
+      if (tok_exp_idx) tok_exp_idx[o] = k * T + row;
     }
     wsum += best;
 #pragma unroll
@@ -300,22 +301,23 @@ __global__ __launch_bounds__(kWave* kWavesPerBlock) void topk_softmax_generic_ke
 // no barrier appears.
 constexpr int kWideMaxExperts = 16384;  // 64 KiB of LDS per row
 
+template <typename El>
 __global__ __launch_bounds__(kWave) void topk_softmax_wide_kernel(
-    const float* __restrict__ gating, float* __restrict__ topk_w, int32_t* __restrict__ topk_ids,
+    const typename El::S* __restrict__ gating, float* __restrict__ topk_w, int32_t* __restrict__ topk_ids,
     int32_t* __restrict__ tok_exp_idx, int T, int E, int K, int renormalize) {
   extern __shared__ float prob[];
   const int lane = threadIdx.x;
   const int row = blockIdx.x;
-  const float* src = gating + static_cast<size_t>(row) * E;
+  const typename El::S* src = gating + static_cast<size_t>(row) * E;
   const float ninf = -__builtin_inff();
 
   float mx = ninf;
-  for (int c = lane; c < E; c += kWave) mx = fmaxf(mx, src[c]);
+  for (int c = lane; c < E; c += kWave) mx = fmaxf(mx, El::ld(src[c]));
 #pragma unroll
   for (int m = 32; m > 0; m /= 2) mx = fmaxf(mx, __shfl_xor(mx, m, kWave));
   float sum = 0.f;
   for (int c = lane; c < E; c += kWave) {
-    const float e = moe_expf(src[c] - mx);
+    const float e = moe_expf(El::ld(src[c]) - mx);
     prob[c] = e;
     sum += e;
   }
@@ -345,7 +347,7 @@ __global__ __launch_bounds__(kWave) void topk_softmax_wide_kernel(
       const size_t o = static_cast<size_t>(row) * K + k;
       topk_w[o] = best;
       topk_ids[o] = bidx;
-      tok_exp_idx[o] = k * T + row;
+      if (tok_exp_idx) tok_exp_idx[o] = k * T + row;
     }
     wsum += best;
     if (lane == bidx % kWave) prob[bidx] = -10000.f;
@@ -358,20 +360,46 @@ __global__ __launch_bounds__(kWave) void topk_softmax_wide_kernel(
   }
 }
 
-template <int E>
-void launch_pow2(const float* g, float* w, int32_t* ids, int32_t* tei, int T, int K, int renorm,
+template <int E, typename El>
+void launch_pow2(const typename El::S* g, float* w, int32_t* ids, int32_t* tei, int T, int K, int renorm,
                  hipStream_t s) {
   constexpr int rows_per_block = Pow2Geom<E>::kRowsPerWave * kWavesPerBlock;
   const int blocks = (T + rows_per_block - 1) / rows_per_block;
-  hipLaunchKernelGGL(topk_softmax_pow2_kernel<E>, dim3(blocks), dim3(kWave * kWavesPerBlock), 0, s,
+  hipLaunchKernelGGL((topk_softmax_pow2_kernel<E, El>), dim3(blocks), dim3(kWave * kWavesPerBlock), 0, s,
                      g, w, ids, tei, T, K, renorm);
+}
+
+template <typename El>
+int launch_topk(const void* logits, float* w, int32_t* ids, int32_t* tei, int T, int E, int K, int renorm, hipStream_t s) {
+  const typename El::S* g = static_cast<const typename El::S*>(logits);
+  switch (E) {
+    case 1: launch_pow2<1, El>(g, w, ids, tei, T, K, renorm, s); break;
+    case 2: launch_pow2<2, El>(g, w, ids, tei, T, K, renorm, s); break;
+    case 4: launch_pow2<4, El>(g, w, ids, tei, T, K, renorm, s); break;
+    case 8: launch_pow2<8, El>(g, w, ids, tei, T, K, renorm, s); break;
+    case 16: launch_pow2<16, El>(g, w, ids, tei, T, K, renorm, s); break;
+    case 32: launch_pow2<32, El>(g, w, ids, tei, T, K, renorm, s); break;
+    case 64: launch_pow2<64, El>(g, w, ids, tei, T, K, renorm, s); break;
+    case 128: launch_pow2<128, El>(g, w, ids, tei, T, K, renorm, s); break;
+    case 256: launch_pow2<256, El>(g, w, ids, tei, T, K, renorm, s); break;
+    default: {
+      if (E > kWave * kGenericMaxPerLane) {
+        hipLaunchKernelGGL(topk_softmax_wide_kernel<El>, dim3(T), dim3(kWave), sizeof(float) * E, s, g, w, ids, tei, T, E,
+                           K, renorm);
+        break;
+      }
+      const int blocks = (T + kWavesPerBlock - 1) / kWavesPerBlock;
+      hipLaunchKernelGGL(topk_softmax_generic_kernel<El>, dim3(blocks), dim3(kWave * kWavesPerBlock), 0, s, g, w, ids,
+                         tei, T, E, K, renorm);
+    }
+  }
+  return moe_check_launch("topk_softmax");
 }
 
 }  // namespace
 
-MOE_EXPORT int moe_topk_softmax(const float* gating_output, float* topk_weights, int32_t* topk_ids,
-                                int32_t* token_expert_indices, int T, int E, int K,
-                                int renormalize, void* stream) {
+MOE_EXPORT int moe_topk_softmax_typed(const void* gating_output, int dtype, float* topk_weights, int32_t* topk_ids,
+                                      int32_t* token_expert_indices, int T, int E, int K, int renormalize, void* stream) {
   if (T < 0 || E < 1 || K < 1) return moe_fail(MOE_ERR_ARG, "topk_softmax: bad sizes T=%d E=%d K=%d", T, E, K);
   if (K > E) return moe_fail(MOE_ERR_ARG, "topk_softmax: topk %d exceeds num_experts %d", K, E);
   if (E > kWideMaxExperts)
@@ -383,33 +411,22 @@ MOE_EXPORT int moe_topk_softmax(const float* gating_output, float* topk_weights,
     return moe_fail(MOE_ERR_UNSUPPORTED, "topk_softmax: %d rows of %d experts exceed the launch limit of %lld rows", T, E,
                     static_cast<long long>(UINT32_MAX / kWave));
   if (T == 0) return MOE_OK;
-  if (!gating_output || !topk_weights || !topk_ids || !token_expert_indices)
-    return moe_fail(MOE_ERR_ARG, "topk_softmax: null pointer");
+  if (!gating_output || !topk_weights || !topk_ids) return moe_fail(MOE_ERR_ARG, "topk_softmax: null pointer");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  switch (E) {
-    case 1: launch_pow2<1>(gating_output, topk_weights, topk_ids, token_expert_indices, T, K, renormalize, s); break;
-    case 2: launch_pow2<2>(gating_output, topk_weights, topk_ids, token_expert_indices, T, K, renormalize, s); break;
-    case 4: launch_pow2<4>(gating_output, topk_weights, topk_ids, token_expert_indices, T, K, renormalize, s); break;
-    case 8: launch_pow2<8>(gating_output, topk_weights, topk_ids, token_expert_indices, T, K, renormalize, s); break;
-    case 16: launch_pow2<16>(gating_output, topk_weights, topk_ids, token_expert_indices, T, K, renormalize, s); break;
-    case 32: launch_pow2<32>(gating_output, topk_weights, topk_ids, token_expert_indices, T, K, renormalize, s); break;
-    case 64: launch_pow2<64>(gating_output, topk_weights, topk_ids, token_expert_indices, T, K, renormalize, s); break;
-    case 128: launch_pow2<128>(gating_output, topk_weights, topk_ids, token_expert_indices, T, K, renormalize, s); break;
-    case 256: launch_pow2<256>(gating_output, topk_weights, topk_ids, token_expert_indices, T, K, renormalize, s); break;
-    default: {
-      if (E > kWave * kGenericMaxPerLane) {
-        hipLaunchKernelGGL(topk_softmax_wide_kernel, dim3(T), dim3(kWave), sizeof(float) * E, s,
-                           gating_output, topk_weights, topk_ids, token_expert_indices, T, E, K,
-                           renormalize);
-        break;
-      }
-      const int blocks = (T + kWavesPerBlock - 1) / kWavesPerBlock;
-      hipLaunchKernelGGL(topk_softmax_generic_kernel, dim3(blocks), dim3(kWave * kWavesPerBlock), 0,
-                         s, gating_output, topk_weights, topk_ids, token_expert_indices, T, E, K,
-                         renormalize);
-    }
+  switch (dtype) {
+    case MOE_F32: return launch_topk<ElemF32>(gating_output, topk_weights, topk_ids, token_expert_indices, T, E, K, renormalize, s);
+    case MOE_F16: return launch_topk<ElemF16>(gating_output, topk_weights, topk_ids, token_expert_indices, T, E, K, renormalize, s);
+    case MOE_BF16: return launch_topk<ElemBF16>(gating_output, topk_weights, topk_ids, token_expert_indices, T, E, K, renormalize, s);
+    default: return moe_fail(MOE_ERR_ARG, "topk_softmax: dtype code %d", dtype);
   }
-  return moe_check_launch("topk_softmax");
+}
+
+MOE_EXPORT int moe_topk_softmax(const float* gating_output, float* topk_weights, int32_t* topk_ids,
+                                int32_t* token_expert_indices, int T, int E, int K,
+                                int renormalize, void* stream) {
+  if (T > 0 && !token_expert_indices && E >= 1 && K >= 1 && K <= E && E <= kWideMaxExperts)
+    return moe_fail(MOE_ERR_ARG, "topk_softmax: null pointer");
+  return moe_topk_softmax_typed(gating_output, MOE_F32, topk_weights, topk_ids, token_expert_indices, T, E, K, renormalize, stream);
 }
 
 MOE_EXPORT int moe_gate_topk_softmax(const void* x, const void* gate_weight, int dtype,

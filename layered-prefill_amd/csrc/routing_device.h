@@ -55,25 +55,24 @@ __device__ __forceinline__ void argmax_level(float& best, int& bidx) {
   }
 }
 
-// The logits of row `row` as route_row wants them: lane t of the row loads columns
+// The logits of row `row` as route_row wants them, widened to fp32: lane t of the row loads columns
 // (i / EPL) * EPL * TPR + t * EPL + i % EPL into v[i], EPL at a time.
-template <int E>
-__device__ __forceinline__ void load_row(const float* __restrict__ gating, int row, int t,
+template <typename S, int N>
+struct alignas(sizeof(S) * N) RowVec {
+  S v[N];
+};
+template <int E, typename El = ElemF32>
+__device__ __forceinline__ void load_row(const typename El::S* __restrict__ gating, int row, int t,
                                          float (&v)[Pow2Geom<E>::kVpt]) {
   using G = Pow2Geom<E>;
   constexpr int EPL = G::kEpl, VECS = G::kVecs, TPR = G::kTpr;
-  const float* src = gating + static_cast<size_t>(row) * E + t * EPL;
+  using V = RowVec<typename El::S, EPL>;
+  const typename El::S* src = gating + static_cast<size_t>(row) * E + t * EPL;
 #pragma unroll
   for (int j = 0; j < VECS; ++j) {
-    if constexpr (EPL == 4) {
-      float4 q = *reinterpret_cast<const float4*>(src + j * EPL * TPR);
-      v[j * 4 + 0] = q.x; v[j * 4 + 1] = q.y; v[j * 4 + 2] = q.z; v[j * 4 + 3] = q.w;
-    } else if constexpr (EPL == 2) {
-      float2 q = *reinterpret_cast<const float2*>(src + j * EPL * TPR);
-      v[j * 2 + 0] = q.x; v[j * 2 + 1] = q.y;
-    } else {
-      v[j] = src[j * EPL * TPR];
-    }
+    const V q = *reinterpret_cast<const V*>(src + j * EPL * TPR);
+#pragma unroll
+    for (int i = 0; i < EPL; ++i) v[j * EPL + i] = El::ld(q.v[i]);
   }
 }
 
@@ -147,7 +146,7 @@ __device__ __forceinline__ void route_row(float (&v)[Pow2Geom<E>::kVpt], int t, 
         const size_t o = static_cast<size_t>(row) * K + t;
         topk_w[o] = renormalize ? my_w / wsum : my_w;
         topk_ids[o] = my_i;
-        tok_exp_idx[o] = t * T + row;
+        if (tok_exp_idx) tok_exp_idx[o] = t * T + row;
       }
     } else if (live && t == 0) {
 #pragma unroll
@@ -156,7 +155,7 @@ __device__ __forceinline__ void route_row(float (&v)[Pow2Geom<E>::kVpt], int t, 
           const size_t o = static_cast<size_t>(row) * K + k;
           topk_w[o] = renormalize ? bw[k] / wsum : bw[k];
           topk_ids[o] = bi[k];
-          tok_exp_idx[o] = k * T + row;
+          if (tok_exp_idx) tok_exp_idx[o] = k * T + row;
         }
     }
   } else {
@@ -168,7 +167,7 @@ __device__ __forceinline__ void route_row(float (&v)[Pow2Geom<E>::kVpt], int t, 
         const size_t o = static_cast<size_t>(row) * K + k;
         topk_w[o] = best;
         topk_ids[o] = bidx;
-        tok_exp_idx[o] = k * T + row;
+        if (tok_exp_idx) tok_exp_idx[o] = k * T + row;
       }
     }
     if (renormalize && live && t == 0) {

@@ -46,22 +46,6 @@ def _align_block_size(topk_ids: torch.Tensor, block_size: int, num_experts: int,
     return sorted_ids, expert_ids, num_tokens_post_pad
 
 
-def _route_align_block_size(gating_output: torch.Tensor, renormalize: bool, topk_weights: torch.Tensor,
-                            topk_ids: torch.Tensor, block_size: int, num_experts: int, plan
-                            ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
-    """``fused_topk`` into ``topk_weights`` / ``topk_ids`` and ``moe_align_block_size`` on the
-    ids as one launch (``ops.route_align_block_size``)."""
-    dev = topk_ids.device
-    max_num_tokens_padded = topk_ids.numel() + num_experts * (block_size - 1)
-    sorted_ids = torch.empty((max_num_tokens_padded,), dtype=torch.int32, device=dev)
-    expert_ids = torch.empty((cdiv(max_num_tokens_padded, block_size),), dtype=torch.int32, device=dev)
-    num_tokens_post_pad = torch.empty((1), dtype=torch.int32, device=dev)
-    token_expert_indicies = torch.empty_like(topk_ids)
-    ops.route_align_block_size(topk_weights, topk_ids, token_expert_indicies, gating_output, renormalize,
-                               num_experts, block_size, sorted_ids, expert_ids, num_tokens_post_pad, plan)
-    return sorted_ids, expert_ids, num_tokens_post_pad
-
-
 def _plan_in_workspace(workspace: torch.Tensor, T: int, H: int, I: int, E: int, K: int, block_size: int,
                        act_code: int, weight_code: int, numel: int):
     """Where the alignment may leave the large-tile kernel's per-XCD ranges and
@@ -96,10 +80,31 @@ def try_get_optimal_moe_config(w1_shape, w2_shape, top_k: int, dtype: Optional[s
     return {"BLOCK_SIZE_M": bm}
 
 
+_LIBRARY_CONFIG = try_get_optimal_moe_config
+
+
+def _layer_call(hidden_states, gating_output, w1, w2, w1_bias, w2_bias, w1_scale, w2_scale, topk_weights, topk_ids,
+                topk, renormalize, activation, weight_on_input, weight_layout, inplace):
+    """The call as one entry into native code (``moe_layer``), or None when it is not a plain one: tensors that
+    something is wrong with, more than a chunk of tokens, a block size of the caller's own
+    (``try_get_optimal_moe_config`` replaced) or the hand-off check switched on."""
+    if try_get_optimal_moe_config is not _LIBRARY_CONFIG or _CHECK_HANDOFF:
+        return None
+    act, layout = _lib.ACTIVATION_CODE.get(activation), _lib.WEIGHT_LAYOUT_CODE.get(weight_layout)
+    if act is None or layout is None:
+        return None
+    return _lib.host().layer(hidden_states, gating_output, w1, w2, w1_bias, w2_bias, w1_scale, w2_scale, topk_weights,
+                             topk_ids, topk, renormalize, act, weight_on_input, layout, inplace)
+
+
 def fused_topk(hidden_states: torch.Tensor, gating_output: torch.Tensor, topk: int,
                renormalize: bool):
     """nanovllm/layers/for_moe/fused_moe.py:393-419."""
     assert hidden_states.shape[0] == gating_output.shape[0], "Number of tokens mismatch"
+    if gating_output.is_cuda and hidden_states.device == gating_output.device:
+        routed = _lib.host().topk(gating_output, topk, renormalize)
+        if routed is not None:
+            return routed
     M, _ = hidden_states.shape
     topk_weights = torch.empty(M, topk, dtype=torch.float32, device=hidden_states.device)
     topk_ids = torch.empty(M, topk, dtype=torch.int32, device=hidden_states.device)
@@ -122,6 +127,10 @@ def fused_gate_topk(hidden_states: torch.Tensor, gate_weight: torch.Tensor, topk
     parallelism wins, measured 13 us against 20 us at 256 tokens, 30 us against
     28 us at 8448), else as the two steps the reference runs.  Returns what
     ``fused_topk`` returns."""
+    if hidden_states.shape[0] >= FUSED_GATE_MIN_TOKENS and hidden_states.is_cuda:
+        routed = _lib.host().gate_topk(hidden_states, gate_weight, topk, renormalize)
+        if routed is not None:
+            return routed
     if hidden_states.shape[0] >= FUSED_GATE_MIN_TOKENS and \
             ops.gate_topk_softmax_supported(hidden_states, gate_weight):
         M = hidden_states.shape[0]
@@ -160,6 +169,12 @@ def fused_experts(hidden_states: torch.Tensor,
                   weight_layout: str = "plain") -> torch.Tensor:
     """nanovllm/layers/for_moe/fused_moe.py:422-460.  ``weight_layout`` (not in the
     reference) is "tiled" when ``w1`` and ``w2`` came out of ``ops.tile_expert_weights``."""
+    if (w1_zp is None and w2_zp is None and a1_scale is None and a2_scale is None and block_shape is None
+            and expert_map is None and global_num_experts in (-1, w1.size(0)) and hidden_states.is_cuda):
+        out = _layer_call(hidden_states, None, w1, w2, w1_bias, w2_bias, w1_scale, w2_scale, topk_weights, topk_ids,
+                          topk_ids.size(-1), False, activation, apply_router_weight_on_input, weight_layout, inplace)
+        if out is not None:
+            return out
     if inplace:
         fused_experts_impl(hidden_states, w1, w2, topk_weights, topk_ids, True, activation,
                            apply_router_weight_on_input, per_channel_quant, global_num_experts,
@@ -180,24 +195,14 @@ def fused_topk_experts(hidden_states: torch.Tensor, gating_output: torch.Tensor,
                        w1_scale: Optional[torch.Tensor] = None, w2_scale: Optional[torch.Tensor] = None,
                        weight_layout: str = "plain") -> torch.Tensor:
     """``fused_topk`` followed by ``fused_experts``: the two calls of
-    ``UnquantizedFusedMoEMethod.apply`` (nanovllm/layers/fused_moe.py:163-216) as one function, so
-    that for the smallest batches (``ops.route_align_supported``: up to 32 tokens) routing and
-    alignment go out as one launch instead of two.  Same result as the two calls, bit for bit.
-    The one launch saves host time (a launch is some 9 us of it), not GPU time: replayed from a HIP
-    graph the two kernels take 13.2 us and the one 14.7 us at 32 tokens.  So a call made while the
-    stream is being captured enqueues the two kernels."""
+    ``UnquantizedFusedMoEMethod.apply`` (nanovllm/layers/fused_moe.py:163-216) as one function and, where the call
+    is a plain one, as one entry into native code.  Same result as the two calls, bit for bit."""
     assert hidden_states.shape[0] == gating_output.shape[0], "Number of tokens mismatch"
-    M, E = gating_output.shape
-    if (hidden_states.is_cuda and M > 0 and w1.size(0) == E and ops.route_align_supported(M, E, topk)
-            and not torch.cuda.is_current_stream_capturing()):
-        gating = gating_output if gating_output.dtype == torch.float32 else gating_output.float()
-        topk_weights = torch.empty(M, topk, dtype=torch.float32, device=hidden_states.device)
-        topk_ids = torch.empty(M, topk, dtype=torch.int32, device=hidden_states.device)
-        out = fused_experts_impl(hidden_states, w1, w2, topk_weights, topk_ids, inplace, activation,
-                                 apply_router_weight_on_input, w1_scale is not None, -1, None, w1_scale, w2_scale,
-                                 None, None, None, None, None, w1_bias, w2_bias, weight_layout,
-                                 _route=(gating.contiguous(), renormalize))
-        return hidden_states if inplace else out
+    if hidden_states.is_cuda:
+        out = _layer_call(hidden_states, gating_output, w1, w2, w1_bias, w2_bias, w1_scale, w2_scale, None, None, topk,
+                          renormalize, activation, apply_router_weight_on_input, weight_layout, inplace)
+        if out is not None:
+            return out
     topk_weights, topk_ids, _ = fused_topk(hidden_states, gating_output, topk, renormalize)
     return fused_experts(hidden_states, w1, w2, w1_bias, w2_bias, topk_weights, topk_ids, inplace=inplace,
                          activation=activation, apply_router_weight_on_input=apply_router_weight_on_input,
@@ -316,7 +321,7 @@ def fused_experts_impl(hidden_states: torch.Tensor,
                        block_shape: Optional[list] = None,
                        w1_bias: Optional[torch.Tensor] = None,
                        w2_bias: Optional[torch.Tensor] = None,
-                       weight_layout: str = "plain", _route=None) -> torch.Tensor:
+                       weight_layout: str = "plain") -> torch.Tensor:
     """nanovllm/layers/for_moe/fused_moe.py:461-633: align -> gate-up GEMM with
     the gated activation -> down GEMM times the routed weight -> top-k sum, in
     chunks of 64K tokens."""
@@ -414,14 +419,8 @@ def fused_experts_impl(hidden_states: torch.Tensor,
         if global_num_experts == E:
             plan = _plan_in_workspace(workspace, tokens_in_chunk, w1.size(2), N // 2, E, top_k_num, bm,
                                       act_code, weight_code, curr_ids.numel())
-        if _route is not None:
-            # routing and alignment as one launch (fused_topk_experts): topk_weights / topk_ids
-            # are this call's own buffers and are filled here, in front of their first use
-            sorted_token_ids, expert_ids, num_tokens_post_padded = _route_align_block_size(
-                _route[0], _route[1], curr_w, curr_ids, bm, global_num_experts, plan)
-        else:
-            sorted_token_ids, expert_ids, num_tokens_post_padded = _align_block_size(
-                curr_ids, bm, global_num_experts, plan)
+        sorted_token_ids, expert_ids, num_tokens_post_padded = _align_block_size(
+            curr_ids, bm, global_num_experts, plan)
         args = launch_fused_experts(hidden_states[begin:end], out_hidden_states[begin:end], w1, w2,
                                     w1_bias, w2_bias, w1_scale, w2_scale, curr_w, sorted_token_ids,
                                     expert_ids, num_tokens_post_padded, bm, activation,

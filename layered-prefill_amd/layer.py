@@ -15,7 +15,7 @@ from typing import Callable, Optional
 import torch
 import torch.distributed as dist
 
-from . import ops
+from . import _lib, ops
 from .fused_moe import fused_experts, fused_gate_topk, fused_topk, fused_topk_experts
 
 
@@ -96,12 +96,11 @@ class UnquantizedFusedMoEMethod:
         if (custom_routing_function is None and not use_grouped_topk and scoring_func == "softmax"
                 and e_score_correction_bias is None and expert_map is None
                 and self.topk_indices_dtype is None and self.fused_experts is fused_experts):
-            # plain softmax routing: select_experts + fused_experts as one function, which
-            # enqueues routing and alignment of a batch of up to 32 tokens as one launch
+            # plain softmax routing: select_experts + fused_experts as one function
+            params = layer._parameters   # (the module's own attribute lookup costs a microsecond per name)
             return fused_topk_experts(
-                x, router_logits, layer.w13_weight, layer.w2_weight, top_k, renormalize,
-                w1_bias=layer.w13_bias if hasattr(layer, "w13_bias") else None,
-                w2_bias=layer.w2_bias if hasattr(layer, "w2_bias") else None,
+                x, router_logits, params["w13_weight"], params["w2_weight"], top_k, renormalize,
+                w1_bias=params.get("w13_bias"), w2_bias=params.get("w2_bias"),
                 inplace=True, activation=activation,
                 apply_router_weight_on_input=apply_router_weight_on_input, weight_layout=layout)
         topk_weights, topk_ids = FusedMoE.select_experts(
@@ -162,8 +161,16 @@ class Fp8E4M3FusedMoEMethod(UnquantizedFusedMoEMethod):
               apply_router_weight_on_input: bool = False, global_num_experts: int = -1,
               expert_map: Optional[torch.Tensor] = None,
               custom_routing_function: Optional[Callable] = None, **unused) -> torch.Tensor:
-        if not hasattr(layer, "w13_weight_scale"):
+        params = layer._parameters
+        if "w13_weight_scale" not in params:
             raise RuntimeError("Fp8E4M3FusedMoEMethod.apply before process_weights_after_loading")
+        if (custom_routing_function is None and expert_map is None and self.topk_indices_dtype is None
+                and self.fused_experts is fused_experts):
+            return fused_topk_experts(
+                x, router_logits, params["w13_weight"], params["w2_weight"], top_k, renormalize,
+                w1_bias=params.get("w13_bias"), w2_bias=params.get("w2_bias"), inplace=True, activation=activation,
+                apply_router_weight_on_input=apply_router_weight_on_input,
+                w1_scale=params["w13_weight_scale"], w2_scale=params["w2_weight_scale"])
         topk_weights, topk_ids = FusedMoE.select_experts(
             hidden_states=x, router_logits=router_logits, use_grouped_topk=False, top_k=top_k,
             renormalize=renormalize, custom_routing_function=custom_routing_function,
@@ -487,6 +494,10 @@ class RMSNorm(torch.nn.Module):
     def forward(self, x: torch.Tensor, residual: Optional[torch.Tensor] = None,
                 out: Optional[torch.Tensor] = None):
         if out is None:
+            if x.is_cuda:
+                out = _lib.host().rms_norm(x, residual, self._parameters["weight"], self.eps)
+                if out is not None:
+                    return out if residual is None else (out, residual)
             out = torch.empty_like(x)
         if residual is None:
             ops.rms_norm(out, x, self.weight.data, self.eps)
