@@ -155,14 +155,15 @@ __device__ __forceinline__ int swizzled(int row, int chunk) {
 // Rounding follows the reference's storage points: the GEMM result is rounded to
 // the activation dtype, silu is rounded, the product is rounded
 // (nanovllm/layers/for_moe/fused_moe.py:216, csrc/activation_kernels.cu:11,23).
-template <typename El, bool GATED>
+// SCALED: e4m3 accumulators still carry the operands' scales here (p.a_scale, p.w_scale).
+template <typename El, bool GATED, bool SCALED = true>
 __device__ __forceinline__ void store_fragment(const GemmParams& p, int e, const f32x16& ga,
                                                const f32x16& ua, int tok, int slot, int ncol0, float rw) {
   using S = typename El::S;
   const S* bias = static_cast<const S*>(p.bias);
   // fp8: the accumulator is in units of (activation scale x weight scale)
-  const float as = p.a_scale ? p.a_scale[p.a_by_slot ? slot : tok / p.top_k] : 1.f;
-  const float* ws = p.w_scale ? p.w_scale + e * p.w_scale_stride_e : nullptr;
+  const float as = SCALED && p.a_scale ? p.a_scale[p.a_by_slot ? slot : tok / p.top_k] : 1.f;
+  const float* ws = SCALED && p.w_scale ? p.w_scale + e * p.w_scale_stride_e : nullptr;
   const int64_t crow = p.a_by_slot ? tok : slot;  // pass 2 writes by token, pass 1 by slot
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
@@ -1459,7 +1460,7 @@ __device__ __forceinline__ void stream_store(const GemmParams& p, int e, const f
 // The time of such a call is the time to pull every active expert's weights
 // out of HBM once, so the kernel is built around that stream: a workgroup owns
 // 64 weight rows of one expert and one alignment block of 32 slots, and walks
-// K in units of 64 elements.  A unit (64 weight rows and 32 token rows of
+// K in units of 128 bytes (64 elements of 16 bits, 128 of e4m3).  A unit (64 weight rows and 32 token rows of
 // 128 B: 8 KB + 4 KB) goes global->LDS by DMA into a ring of four units, three
 // of them in flight while the fourth is multiplied; three workgroups fit a CU,
 // which keeps about 100 KB per CU on its way from HBM and hides a workgroup's
@@ -1470,15 +1471,19 @@ __device__ __forceinline__ void stream_store(const GemmParams& p, int e, const f
 // out in LDS like the large-tile kernel's (16-byte chunk c of row r at chunk
 // c ^ ((r >> 1) & 7)).  Everything the start-up reads is wavefront-uniform and
 // comes through the scalar cache, in two round trips.
+// e4m3 runs here too (100 tokens of a 2048 x 128 x 768 top-8 layer: gate-up 45.6 -> 40.1 us, down 40.9 -> 25.9 us
+// against the register-staged kernel, whose two stages hold 36 KB per workgroup and drain at every K tile), its scales
+// fetched ahead of the stream like the routed weights.  Rows need whole 32-byte MFMA steps, not whole units.
 // ---------------------------------------------------------------------------
-constexpr int kStBK = 64, kStRowBytes = kStBK * 2, kStRows = 64, kStUnits = 4, kStBM = 32;
+constexpr int kStRowBytes = 128, kStRows = 64, kStUnits = 4, kStBM = 32;
 constexpr int kStWBytes = kStRows * kStRowBytes;               // 8 KB of weights per unit
 constexpr int kStUnitBytes = kStWBytes + kStBM * kStRowBytes;  // plus 4 KB of tokens
 constexpr int kStDmaPerUnit = 3;                               // requests per wavefront and unit
 
-template <typename Mma, bool GATED>
+template <typename Mma, bool GATED, bool TAIL>
 __global__ __launch_bounds__(kThreads, 3) void stream_gemm_kernel(const GemmParams p) {
   using El = typename Mma::El;
+  constexpr int ES = Mma::kEs;
   __shared__ __attribute__((aligned(1024))) char smem[kStUnits * kStUnitBytes];
   constexpr int BN_OUT = GATED ? kStRows / 2 : kStRows;
   // Per-XCD ranges of the (block major, n-tile minor) order, cut from the live
@@ -1530,16 +1535,23 @@ __global__ __launch_bounds__(kThreads, 3) void stream_gemm_kernel(const GemmPara
   // What the epilogue needs per slot is fetched now, ahead of the stream: a load
   // issued behind ~100 KB of queued DMA requests would take microseconds to return.
   int tok = p.numel;
-  float rw = 1.f;
+  float rw = 1.f, as = 1.f, wsc = 1.f;
   if (wave == 0) {
     tok = sid[l32];
     if (p.mul_weight && tok < p.numel) rw = p.topk_w[tok];
+    if constexpr (ES == 1) {
+      if (tok < p.numel) as = p.a_scale[p.a_by_slot ? mb * kStBM + l32 : tok / p.top_k];
+      // lane l holds the channel scale of the workgroup's weight row l
+      int n = n0 + (GATED ? l32 : lane);
+      n = n < p.N ? n : p.N - 1;
+      wsc = p.w_scale[e * p.w_scale_stride_e + (!GATED ? n : p.interleaved ? 2 * n + lhi : lhi * p.N + n)];
+    }
   }
 
   // DMA requests of this wavefront: token rows 8 * wave + lane / 8, weight rows
   // 16 * wave + 8 * j + lane / 8 (j < 2); lane % 8 is the chunk the lane's 16 bytes land in
   const char* a_base = static_cast<const char*>(p.a);
-  const char* w_base = static_cast<const char*>(p.w) + static_cast<int64_t>(e) * p.w_stride_e * 2;
+  const char* w_base = static_cast<const char*>(p.w) + static_cast<int64_t>(e) * p.w_stride_e * ES;
   int w_step = kStRowBytes;  // bytes from one K unit to the next
   uint32_t a_off, w_off[2];
   {
@@ -1552,14 +1564,15 @@ __global__ __launch_bounds__(kThreads, 3) void stream_gemm_kernel(const GemmPara
       const int tok = (q & 4) ? hi : lo;
       src = tok < p.numel ? tok / p.top_k : 0;
     }
-    a_off = static_cast<uint32_t>(src * p.lda * 2 + (((lane & 7) ^ ((rr >> 1) & 7)) << 4));
+    a_off = static_cast<uint32_t>(src * p.lda * ES + (((lane & 7) ^ ((rr >> 1) & 7)) << 4));
   }
+  const int row_bytes = p.Kd * ES;  // a multiple of 32
   if (p.w_tiled) {
     // Weights in 32 KB units of 256 rows (the large-tile kernel's): this workgroup's rows are one
     // or two contiguous pieces of every unit of its n-tile, 32 rows apart from a multiple of 32,
     // so a row's chunks already sit where this kernel's LDS rows want them.
     constexpr int kBigRows = GATED ? 128 : 256;  // output columns covered by one unit
-    w_base += static_cast<int64_t>(n0 / kBigRows) * (p.Kd / kStBK) * 32768;
+    w_base += static_cast<int64_t>(n0 / kBigRows) * (row_bytes / kStRowBytes) * 32768;
     w_step = 32768;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
@@ -1581,14 +1594,31 @@ __global__ __launch_bounds__(kThreads, 3) void stream_gemm_kernel(const GemmPara
       const int n = n0 + rr;
       wrow = n < p.N ? n : p.N - 1;
     }
-    w_off[j] = static_cast<uint32_t>(wrow * p.w_stride_n * 2 + (((lane & 7) ^ ((rr >> 1) & 7)) << 4));
+    w_off[j] = static_cast<uint32_t>(wrow * p.w_stride_n * ES + (((lane & 7) ^ ((rr >> 1) & 7)) << 4));
   }
   }
   const uint32_t lds0 = lds_offset_of(smem);
   const uint32_t dma_w = __builtin_amdgcn_readfirstlane(lds0 + 16 * wave * kStRowBytes);
   const uint32_t dma_a = __builtin_amdgcn_readfirstlane(lds0 + kStWBytes + 8 * wave * kStRowBytes);
+  // TAIL (plain layout only): the last unit of a row holds `tail` bytes, 32 to 96.  A lane whose chunk lies
+  // behind the row's end fetches the unit's first chunk instead, and no MFMA step reads that place.  (As a
+  // run-time branch this cost the rows of whole units 2 %.)
+  const int nu = TAIL ? row_bytes / kStRowBytes + 1 : row_bytes / kStRowBytes;
+  const int tail = row_bytes & (kStRowBytes - 1);
   auto issue = [&](int u) {
     const uint32_t ring = (u % kStUnits) * kStUnitBytes;
+    if (TAIL && u == nu - 1) {
+      const uint32_t ca = ((lane & 7) ^ (((8 * wave + (lane >> 3)) >> 1) & 7)) << 4;
+      const uint32_t back_a = static_cast<int>(ca) < tail ? 0u : ca;
+      lds_dma16(a_base + u * kStRowBytes, a_off - back_a, dma_a + ring);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const uint32_t cw = ((lane & 7) ^ (((16 * wave + 8 * j + (lane >> 3)) >> 1) & 7)) << 4;
+        const uint32_t back_w = static_cast<int>(cw) < tail ? 0u : cw;
+        lds_dma16(w_base + static_cast<int64_t>(u) * w_step, w_off[j] - back_w, dma_w + ring + j * 1024);
+      }
+      return;
+    }
     lds_dma16(a_base + u * kStRowBytes, a_off, dma_a + ring);
 #pragma unroll
     for (int j = 0; j < 2; ++j) lds_dma16(w_base + static_cast<int64_t>(u) * w_step, w_off[j], dma_w + ring + j * 1024);
@@ -1597,7 +1627,6 @@ __global__ __launch_bounds__(kThreads, 3) void stream_gemm_kernel(const GemmPara
   f32x16 acc0, acc1;
 #pragma unroll
   for (int r = 0; r < 16; ++r) { acc0[r] = 0.f; acc1[r] = 0.f; }
-  const int nu = p.Kd / kStBK;
   int rd_k[4];
 #pragma unroll
   for (int kk = 0; kk < 4; ++kk) rd_k[kk] = l32 * kStRowBytes + (((2 * kk + lhi) ^ ((l32 >> 1) & 7)) << 4);
@@ -1615,8 +1644,10 @@ __global__ __launch_bounds__(kThreads, 3) void stream_gemm_kernel(const GemmPara
     if (u + 3 < nu) issue(u + 3);
     if (wave == 0) {
       const char* st = smem + (u % kStUnits) * kStUnitBytes;
+      const int steps = TAIL && u == nu - 1 ? tail >> 5 : 4;
 #pragma unroll
       for (int kk = 0; kk < 4; ++kk) {
+        if (kk >= steps) break;
         const uint4 x = *reinterpret_cast<const uint4*>(st + kStWBytes + rd_k[kk]);
         const uint4 w0 = *reinterpret_cast<const uint4*>(st + rd_k[kk]);
         const uint4 w1 = *reinterpret_cast<const uint4*>(st + 32 * kStRowBytes + rd_k[kk]);
@@ -1627,11 +1658,19 @@ __global__ __launch_bounds__(kThreads, 3) void stream_gemm_kernel(const GemmPara
   }
 
   if (wave != 0) return;
+  if constexpr (ES == 1) {  // the accumulators back to the units of x . w
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int row = 8 * (r >> 2) + 4 * lhi + (r & 3);
+      acc0[r] *= as * __shfl(wsc, row, kWave);
+      acc1[r] *= as * __shfl(wsc, row + 32, kWave);
+    }
+  }
   const int slot = mb * kStBM + l32;
   if (tok < p.numel) {
-    const bool fast = n0 + BN_OUT <= p.N && (p.ldc & 3) == 0 && !p.w_scale;
+    const bool fast = n0 + BN_OUT <= p.N && (p.ldc & 3) == 0;
     if constexpr (GATED) {
-      if (!fast) store_fragment<El, true>(p, e, acc0, acc1, tok, slot, n0 + 4 * lhi, rw);
+      if (!fast) store_fragment<El, true, false>(p, e, acc0, acc1, tok, slot, n0 + 4 * lhi, rw);
       else if (p.activation == MOE_ACT_SILU) stream_store<El, true, MOE_ACT_SILU>(p, e, acc0, acc1, tok, slot, n0 + 4 * lhi, rw);
       else if (p.activation == MOE_ACT_SWIGLUOAI) stream_store<El, true, MOE_ACT_SWIGLUOAI>(p, e, acc0, acc1, tok, slot, n0 + 4 * lhi, rw);
       else stream_store<El, true, MOE_ACT_GELU>(p, e, acc0, acc1, tok, slot, n0 + 4 * lhi, rw);
@@ -1639,8 +1678,8 @@ __global__ __launch_bounds__(kThreads, 3) void stream_gemm_kernel(const GemmPara
       stream_store<El, false, 0>(p, e, acc0, acc0, tok, slot, n0 + 4 * lhi, rw);
       stream_store<El, false, 0>(p, e, acc1, acc1, tok, slot, n0 + 32 + 4 * lhi, rw);
     } else {
-      store_fragment<El, false>(p, e, acc0, acc0, tok, slot, n0 + 4 * lhi, rw);
-      store_fragment<El, false>(p, e, acc1, acc1, tok, slot, n0 + 32 + 4 * lhi, rw);
+      store_fragment<El, false, false>(p, e, acc0, acc0, tok, slot, n0 + 4 * lhi, rw);
+      store_fragment<El, false, false>(p, e, acc1, acc1, tok, slot, n0 + 32 + 4 * lhi, rw);
     }
   }
 }
@@ -1652,7 +1691,11 @@ int launch_stream(GemmParams& p, int64_t sorted_cap, hipStream_t s) {
   const int64_t tiles = static_cast<int64_t>(p.num_m_blocks) * p.num_n_tiles;
   const int64_t grid = (tiles + kXcds - 1) / kXcds * kXcds;
   if (grid > INT32_MAX) return moe_fail(MOE_ERR_ARG, "fused_experts: grid of %lld workgroups", static_cast<long long>(grid));
-  hipLaunchKernelGGL((stream_gemm_kernel<Mma, GATED>), dim3(static_cast<unsigned>(grid)), dim3(kThreads), 0, s, p);
+  const dim3 blocks(static_cast<unsigned>(grid)), threads(kThreads);
+  if (p.Kd * Mma::kEs % kStRowBytes)
+    hipLaunchKernelGGL((stream_gemm_kernel<Mma, GATED, true>), blocks, threads, 0, s, p);
+  else
+    hipLaunchKernelGGL((stream_gemm_kernel<Mma, GATED, false>), blocks, threads, 0, s, p);
   return moe_check_launch(GATED ? "fused_experts (gate-up pass)" : "fused_experts (down pass)");
 }
 
@@ -1776,7 +1819,9 @@ int launch_bm(GemmParams& p, int block_size, int64_t sorted_cap, hipStream_t s) 
       p.xcd_bounds = bounds;
       return launch_big<Mma, GATED>(p, sorted_cap, s);
     }
-    if (block_size == kStBM && p.Kd % kStBK == 0 && offsets_fit)
+  }
+  if constexpr (Mma::kEs <= 2) {
+    if (block_size == kStBM && p.Kd * Mma::kEs % 32 == 0 && offsets_fit)
       return launch_stream<Mma, GATED>(p, sorted_cap, s);
   }
   if (p.w_tiled)

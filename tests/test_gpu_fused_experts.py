@@ -288,7 +288,7 @@ def test_fused_experts_fp8_against_dequantised_oracle(moe, oracle, dev, E, H, I,
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_fp8_every_block_size_kernel(moe, oracle, dev, bm, dtype, monkeypatch):
     """Blocks of 256 slots run the large-tile e4m3 kernel (K = 64 MFMA steps),
-    smaller ones the register-staged kernels; both must agree with the oracle
+    blocks of 32 the streaming kernel, others the register-staged kernels; all must agree with the oracle
     that rounds where the kernels store."""
     x, w13, w2, logits = _layer(16, 512, 256, 700, 4, 77, dtype)
     tw, ids, _ = oracle.topk_softmax(logits, 4, renormalize=True)
@@ -302,6 +302,40 @@ def test_fp8_every_block_size_kernel(moe, oracle, dev, bm, dtype, monkeypatch):
         x, w13q.view(torch.uint8).cpu(), w13s.cpu(), w2q.view(torch.uint8).cpu(), w2s.cpu(), tw, ids,
         mirror_rounding=m), _mode(moe, 700, 16, 4, 512, dtype, fp8=True, bm=bm), rtol=2e-2,
         atol=0.03 * out.float().abs().max().item())
+
+
+@pytest.mark.parametrize("dt", ["bf16", "fp16", "e4m3"])
+@pytest.mark.parametrize("T,H,I", [(1, 32, 32), (33, 96, 160), (5, 1440, 416), (70, 256, 64), (9, 2880, 1440)])
+def test_streaming_kernel_row_tails(moe, oracle, dev, dt, T, H, I, monkeypatch):
+    """Reduction lengths that end inside a 128-byte unit of the streaming kernel (after 1 to 4 of its 32-byte steps),
+    shorter than one unit and longer than its ring, with 1 to 3 blocks of an expert; the weights sit in front of NaN
+    rows, which nothing may read."""
+    E, K = 4, 2
+    dtype = torch.float16 if dt == "fp16" else torch.bfloat16
+    x, w13, w2, logits = _layer(E, H, I, T, K, 3 + T + H, dtype)
+    tw, ids, _ = oracle.topk_softmax(logits, K, renormalize=True)
+    monkeypatch.setattr(moe.fused_moe, "try_get_optimal_moe_config", lambda *a, **k: {"BLOCK_SIZE_M": 32})
+    kw = dict(topk_weights=tw.to(dev), topk_ids=ids.to(dev))
+
+    def guarded(w):   # the same rows with NaN (codes 0x7f7f and 0x7fff) behind every expert's last one
+        g = torch.full((E, w.shape[1] + 1, w.shape[2]), 0x7f, dtype=torch.uint8, device=dev) if w.element_size() == 1 \
+            else torch.full((E, w.shape[1] + 1, w.shape[2]), 0x7fff, dtype=torch.int16, device=dev)
+        g = g.view(w.dtype)[:, :w.shape[1]]
+        g.copy_(w)
+        return g
+
+    if dt == "e4m3":
+        q13, s13, q2, s2 = moe.quantize_expert_weights(w13.to(dev), w2.to(dev))
+        out = moe.fused_experts(x.to(dev), guarded(q13), guarded(q2), None, None, per_channel_quant=True, w1_scale=s13,
+                                w2_scale=s2, **kw)
+        # one e4m3 step of an intermediate element next to a tie moves that term by 6 %
+        _close(out, oracle.fused_experts_fp8_ref(x, q13.view(torch.uint8).cpu(), s13.cpu(), q2.view(torch.uint8).cpu(),
+                                                 s2.cpu(), tw, ids, mirror_rounding=True),
+               rtol=2e-2, atol=0.03 * out.float().abs().max().item())
+    else:
+        out = moe.fused_experts(x.to(dev), guarded(w13.to(dev)), guarded(w2.to(dev)), None, None, **kw)
+        _close(out, oracle.fused_experts_ref(x, w13, w2, tw, ids, mirror_rounding=True), rtol=1.6e-2,
+               atol=2e-3 * max(1.0, out.float().abs().max().item()))
 
 
 def test_fp8_layered_prefill_batch_every_row(moe, oracle, dev):
