@@ -246,6 +246,17 @@ def test_quant_rows_e4m3_matches_oracle(moe, oracle, dev):
         assert not ((q.cpu() & 0x7f) == 0x7f).any() and s.cpu()[5] == 2.0 ** -100
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows", [1, 7, 9, 33])
+@pytest.mark.parametrize("cols", [8, 256, 512, 520, 768, 776, 1024, 1032, 2048, 2056, 4096, 4104])
+def test_quant_rows_e4m3_row_widths(moe, oracle, dev, dtype, rows, cols):
+    """Both sides of every width at which the kernel changes its lanes and steps per row; odd row counts."""
+    w = (torch.randn(rows, cols, generator=torch.Generator().manual_seed(rows + cols)) * 0.02).to(dtype)
+    q, s = moe.ops.quant_rows_e4m3(w.to(dev))
+    oq, os_ = oracle.quant_weight_per_channel(w[None])
+    assert torch.equal(s.cpu(), os_[0]) and torch.equal(q.cpu(), oq[0])
+
+
 # ------------------------------------------------------------------ fp8 e4m3 variant
 def _close_fp8(got, want, atol=1e-2):
     # north star: rtol 6e-2 against the fp32 dequantised oracle (atol 1e-2 as for bf16)
