@@ -296,6 +296,9 @@ int moe_fused_experts_plan_layout(int T, int H, int I, int E, int K, int block_s
  * tokens; plays the role of config["BLOCK_SIZE_M"] chosen by
  * try_get_optimal_moe_config (nanovllm/layers/for_moe/fused_moe.py:354-390). */
 int moe_preferred_block_size(int M, int E, int K, int act_dtype, int weight_dtype);
+/* The same for a layer whose intermediate size is known: a layer of few experts leaves the large
+ * tiles too few workgroups for the chip and keeps the small blocks longer. */
+int moe_layer_block_size(int M, int I, int E, int K, int act_dtype, int weight_dtype);
 
 /* One-time re-ordering of expert weights for the DMA kernels (no counterpart in the reference, whose
  * loader, nanovllm/layers/fused_moe.py:472-658, leaves `w13_weight [E, 2I, H]` / `w2_weight [E, H, I]`

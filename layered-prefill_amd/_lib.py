@@ -131,6 +131,8 @@ def _declare(L: ctypes.CDLL) -> None:
     L.moe_fused_experts_set_wait_limit.argtypes = [i32]
     L.moe_preferred_block_size.restype = i32
     L.moe_preferred_block_size.argtypes = [i32] * 5
+    L.moe_layer_block_size.restype = i32
+    L.moe_layer_block_size.argtypes = [i32] * 6
     L.moe_quant_rows_e4m3.restype = i32
     L.moe_quant_rows_e4m3.argtypes = [p, i32, i64, i32, p, p, p]
     L.moe_route_align_supported.restype = i32

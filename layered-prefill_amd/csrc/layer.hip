@@ -36,7 +36,7 @@ Layout layout_of(const MoeLayerArgs* a) {
     l.topk_w = a->topk_weights;
     l.topk_ids = a->topk_ids;
   }
-  l.block = a->block_size ? a->block_size : moe_preferred_block_size(a->T, a->E, a->K, a->act_dtype, a->weight_dtype);
+  l.block = a->block_size ? a->block_size : moe_layer_block_size(a->T, a->I, a->E, a->K, a->act_dtype, a->weight_dtype);
   l.sorted_cap = numel + static_cast<int64_t>(a->E) * (l.block - 1);
   l.expert_cap = (l.sorted_cap + l.block - 1) / l.block;
   l.align_bytes = moe_align_workspace_bytes(numel, a->E);
@@ -60,6 +60,27 @@ int check_layer_args(const MoeLayerArgs* a) {
 }
 
 }  // namespace
+
+// Blocks of 256 slots (large-tile kernel) or of 32 (streaming kernel).  What the large tile costs below its crossover
+// is idle CUs: an expert's weights are walked by I / 128 + H / 256 workgroups, each a serial chain of K tiles, and with
+// `tiles` = E * ceil(I / 128) gate-up tiles for the 256 CUs a layer of few experts leaves the chip half empty, however
+// many rows an expert has.  What the streaming kernel costs above it is re-reading the weights for every 32 rows.
+// The crossover measured, in routed rows per expert, both GEMM passes and the combine, MI355X, Zipf routing:
+//   bf16 tiles 768 (E 128, I 768): 24; 384 (E 64): 44; 256 (E 32, I 1024): 64; 96 (E 16, I 768; E 32, I 384): 97 and 115;
+//   64 (E 16, I 512): beyond 128.  e4m3 tiles 768: 34; 256: 84; 64: beyond 96.  The 16-bit line lies lower than these
+//   because tiled weights favour the large tile: at 768 tiles it leads from 16 rows on (183.4 us against 187.0 for the
+//   whole call of 256 tokens).
+// For instance E 32, H 2048, I 1024, 256 tokens top-4: 101.5 us against 122.2; 768 tokens: 169.6 against 139.8.
+// E 16, H 1024, I 512, 256 tokens top-4: 25.8 against 55.9.  Layers of more tiles keep the lines of
+// moe_preferred_block_size (16 and 32 rows).
+MOE_EXPORT int moe_layer_block_size(int M, int I, int E, int K, int act_dtype, int weight_dtype) {
+  if (act_dtype == MOE_F32 || E < 1 || I < 0) return moe_preferred_block_size(M, E, K, act_dtype, weight_dtype);
+  const int64_t tiles = static_cast<int64_t>(E) * ((static_cast<int64_t>(I) + 127) / 128);
+  const int64_t rows = static_cast<int64_t>(M) * K / E;
+  const int64_t line = weight_dtype == MOE_E4M3 ? 22528 : 12288, least = weight_dtype == MOE_E4M3 ? 32 : 16;
+  if (rows < least) return 32;
+  return rows >= 96 || rows * tiles >= line ? 256 : 32;
+}
 
 MOE_EXPORT int64_t moe_layer_workspace_bytes(const MoeLayerArgs* a) {
   if (check_layer_args(a)) return 0;

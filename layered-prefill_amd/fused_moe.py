@@ -76,7 +76,7 @@ def try_get_optimal_moe_config(w1_shape, w2_shape, top_k: int, dtype: Optional[s
     E = w2_shape[0]
     act_code = _lib.DTYPE_CODE[act_dtype]
     weight_code = _lib.E4M3_CODE if dtype == "fp8_w8a8" else act_code
-    bm = lib().moe_preferred_block_size(M, E, top_k, act_code, weight_code)
+    bm = lib().moe_layer_block_size(M, w1_shape[1] // 2, E, top_k, act_code, weight_code)
     return {"BLOCK_SIZE_M": bm}
 
 

@@ -235,3 +235,19 @@ def test_product_never_imports_the_oracle():
             if f.endswith((".py", ".hip", ".h", ".cpp")):
                 text = open(os.path.join(dirpath, f)).read()
                 assert "oracle" not in text.lower() or f == "__init__.py" and False, f
+
+
+@pytest.mark.parametrize("I,E,K,act,wgt,line", [(768, 128, 8, 2, 2, 16), (768, 64, 8, 2, 2, 32), (1024, 32, 4, 1, 1, 48),
+                                                (768, 16, 2, 2, 2, 96), (4096, 64, 2, 2, 2, 16), (768, 128, 8, 2, 3, 32),
+                                                (1024, 32, 4, 2, 3, 88), (512, 16, 4, 2, 3, 96)])
+def test_layer_block_size_changes_once_at_its_line(moe, I, E, K, act, wgt, line):
+    """Blocks of 32 below the line (in routed rows per expert), of 256 from it on."""
+    L = moe._lib.lib()
+    sizes = [L.moe_layer_block_size(rows * E // K, I, E, K, act, wgt) for rows in range(0, 300)]
+    assert sizes == [32] * line + [256] * (300 - line)
+
+
+def test_layer_block_size_of_fp32_is_the_old_rule(moe):
+    L = moe._lib.lib()
+    for m in (1, 256, 768, 2048, 8448):
+        assert L.moe_layer_block_size(m, 768, 128, 8, 0, 0) == L.moe_preferred_block_size(m, 128, 8, 0, 0)
