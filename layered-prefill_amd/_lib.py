@@ -26,7 +26,7 @@ WEIGHT_LAYOUT_CODE = {"plain": 0, "tiled": 1}   # MoeWeightLayout
 EXPORTS = (
     "moe_last_error", "moe_abi_version", "moe_topk_softmax", "moe_align_workspace_bytes",
     "moe_align_block_size", "moe_silu_and_mul", "moe_swigluoai_and_mul", "moe_sum",
-    "moe_fused_experts_workspace_bytes", "moe_fused_experts", "moe_preferred_block_size",
+    "moe_fused_experts_workspace_bytes", "moe_fused_experts", "moe_preferred_block_size", "moe_layer_block_size",
     "moe_quant_rows_e4m3", "moe_gate_topk_softmax", "moe_add_rms_norm",
     "moe_align_can_plan", "moe_align_block_size_planned", "moe_fused_experts_plan_layout",
     "moe_fused_experts_status", "moe_fused_experts_set_wait_limit", "moe_align_block_size_static",
