@@ -150,11 +150,11 @@ def test_moe_align_block_size_bit_exact(moe, oracle, dev, numel, E, bm):
     assert torch.equal(s.cpu(), os_)
 
 
-@pytest.mark.parametrize("bm", [1, 32, 64, 65])
-@pytest.mark.parametrize("numel", [0, 1, 63, 64, 65, 1023, 1024, 1025])
+@pytest.mark.parametrize("bm", [1, 32, 64, 65, 256])
+@pytest.mark.parametrize("numel", [0, 1, 63, 64, 65, 1023, 1024, 1025, 4096, 4097, 8191, 8192, 8193])
 @pytest.mark.parametrize("E", [1, 3, 64, 128, 256, 257])
-def test_alignment_of_a_decode_batch(moe, oracle, dev, numel, E, bm):
-    """Both sides of the sizes up to which one load per thread serves, with ids outside [0, E) among them."""
+def test_alignment_of_a_small_batch(moe, oracle, dev, numel, E, bm):
+    """Both sides of the sizes up to which one, four and eight loads per thread serve, with ids outside [0, E) among them."""
     ids = _skewed_ids(numel, E, numel + E)
     ids[5::11] = E
     ids[7::13] = -3
