@@ -296,7 +296,7 @@ int moe_fused_experts_plan_layout(int T, int H, int I, int E, int K, int block_s
  * tokens; plays the role of config["BLOCK_SIZE_M"] chosen by
  * try_get_optimal_moe_config (nanovllm/layers/for_moe/fused_moe.py:354-390). */
 int moe_preferred_block_size(int M, int E, int K, int act_dtype, int weight_dtype);
-/* The same for a layer whose intermediate size is known: a layer of few experts leaves the large
+/* The same for a layer of intermediate size I (0: not known; below 768 the same as 768): a layer of few experts leaves the large
  * tiles too few workgroups for the chip and keeps the small blocks longer. */
 int moe_layer_block_size(int M, int I, int E, int K, int act_dtype, int weight_dtype);
 

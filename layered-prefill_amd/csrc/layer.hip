@@ -75,7 +75,10 @@ int check_layer_args(const MoeLayerArgs* a) {
 // moe_preferred_block_size (16 and 32 rows).
 MOE_EXPORT int moe_layer_block_size(int M, int I, int E, int K, int act_dtype, int weight_dtype) {
   if (act_dtype == MOE_F32 || E < 1 || I < 0) return moe_preferred_block_size(M, E, K, act_dtype, weight_dtype);
-  const int64_t tiles = static_cast<int64_t>(E) * ((static_cast<int64_t>(I) + 127) / 128);
+  // An expert counts as six tiles at least: narrower ones (and a caller that passes 0 for a size it does not know) get
+  // the line of I = 768, on the safe side of the crossovers above.
+  const int64_t per_expert = (static_cast<int64_t>(I) + 127) / 128;
+  const int64_t tiles = static_cast<int64_t>(E) * (per_expert > 6 ? per_expert : 6);
   const int64_t rows = static_cast<int64_t>(M) * K / E;
   const int64_t line = weight_dtype == MOE_E4M3 ? 22528 : 12288, least = weight_dtype == MOE_E4M3 ? 32 : 16;
   if (rows < least) return 32;

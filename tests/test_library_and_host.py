@@ -239,7 +239,8 @@ def test_product_never_imports_the_oracle():
 
 @pytest.mark.parametrize("I,E,K,act,wgt,line", [(768, 128, 8, 2, 2, 16), (768, 64, 8, 2, 2, 32), (1024, 32, 4, 1, 1, 48),
                                                 (768, 16, 2, 2, 2, 96), (4096, 64, 2, 2, 2, 16), (768, 128, 8, 2, 3, 32),
-                                                (1024, 32, 4, 2, 3, 88), (512, 16, 4, 2, 3, 96)])
+                                                (1024, 32, 4, 2, 3, 88), (512, 16, 4, 2, 3, 96),
+                                                (0, 128, 8, 2, 2, 16), (256, 128, 8, 2, 2, 16), (0, 16, 2, 2, 2, 96)])
 def test_layer_block_size_changes_once_at_its_line(moe, I, E, K, act, wgt, line):
     """Blocks of 32 below the line (in routed rows per expert), of 256 from it on."""
     L = moe._lib.lib()
