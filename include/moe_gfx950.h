@@ -228,7 +228,11 @@ typedef struct MoeFusedExpertsArgs {
      workspace already holds the plan (moe_align_block_size_planned).  Bit 32 (for
      tests of the one-launch form): its down tiles run on the XCD next to the one
      that ran their block's gate-up tiles, so every hand-off crosses two L2s; the
-     result is the same, bit for bit. */
+     result is the same, bit for bit.  Bit 64: with SiLU and blocks of 32 slots the
+     gated product is rounded once, as with blocks of 256 (rows of x must be whole
+     multiples of 128 bytes; no effect elsewhere).  A caller that takes its block size
+     from moe_layer_block_size sets it when that is smaller than
+     moe_preferred_block_size, so that the choice does not decide the precision. */
   int32_t passes;
   int32_t weight_layout;     /* MoeWeightLayout of w13 and w2 (both): 0 = plain                   */
   void* stream;

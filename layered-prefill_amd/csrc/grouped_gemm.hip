@@ -123,6 +123,12 @@ struct GemmParams {
   int a_by_slot;     // A row = slot (pass 2) instead of tok / top_k (pass 1)
   int mul_weight;    // multiply by topk_w[tok] in the epilogue
   int activation;    // MoeActivation (gated pass only)
+  // Streaming kernel with SiLU, rows of whole units: the product is rounded once.  Those are the calls that
+  // moe_layer_block_size takes from the large-tile kernel, which forms silu(gate) * up on its fp32
+  // accumulators: which of the two runs must not decide the precision.  Error of the whole layer against
+  // float64, 32 experts, H 2048, I 1024, 256 tokens top-4: bf16 2.88e-3 on both kernels, 4.26e-3 with
+  // gate, up and silu rounded as well; fp16 3.61e-4 and 5.27e-4.
+  int silu_once;
   int interleaved;   // gate/up rows interleaved (2n, 2n+1) instead of halves (n, N+n)
   float alpha, limit;
   int64_t sorted_cap; // capacity of sorted_ids
@@ -156,7 +162,8 @@ __device__ __forceinline__ int swizzled(int row, int chunk) {
 // the activation dtype, silu is rounded, the product is rounded
 // (nanovllm/layers/for_moe/fused_moe.py:216, csrc/activation_kernels.cu:11,23).
 // SCALED: e4m3 accumulators still carry the operands' scales here (p.a_scale, p.w_scale).
-template <typename El, bool GATED, bool SCALED = true>
+// ONCE: p.silu_once may ask for one rounding of the SiLU product.
+template <typename El, bool GATED, bool SCALED = true, bool ONCE = false>
 __device__ __forceinline__ void store_fragment(const GemmParams& p, int e, const f32x16& ga,
                                                const f32x16& ua, int tok, int slot, int ncol0, float rw) {
   using S = typename El::S;
@@ -185,6 +192,10 @@ __device__ __forceinline__ void store_fragment(const GemmParams& p, int e, const
           uv += El::ld(bias[e * p.bias_stride_e + urow]);
         }
         if (p.mul_weight) { gv *= rw; uv *= rw; }
+        if (ONCE && p.silu_once) {
+          o[i] = El::st(moe_silu(gv) * uv);
+          continue;
+        }
         gv = El::ld(El::st(gv));
         uv = El::ld(El::st(uv));
         float r;
@@ -1417,8 +1428,10 @@ __global__ __launch_bounds__(kPlanThreads) void big_plan_kernel(const int32_t* _
 // Epilogue of the streaming kernel for full, aligned 16-bit tiles: same storage
 // points as store_fragment, with the hardware conversions and the fast SiLU of
 // the large-tile epilogue (one wavefront finishes the whole tile, so the
-// instruction count is the epilogue's latency).
-template <typename El, bool GATED, int ACT>
+// instruction count is the epilogue's latency).  ONCE (SiLU): gate and up are the
+// same accumulator element of two fragments, and silu(gate) * up is formed on the
+// fp32 values and rounded once, as the large-tile epilogue does.
+template <typename El, bool GATED, int ACT, bool ONCE = false>
 __device__ __forceinline__ void stream_store(const GemmParams& p, int e, const f32x16& ga, const f32x16& ua,
                                              int tok, int slot, int ncol0, float rw) {
   using S = typename El::S;
@@ -1444,7 +1457,10 @@ __device__ __forceinline__ void stream_store(const GemmParams& p, int e, const f
       uv[i] *= rw;
     }
     uint2 out;
-    if constexpr (GATED) {
+    if constexpr (ONCE) {
+      out.x = pack2<El>(silu_fast(gv[0]) * uv[0], silu_fast(gv[1]) * uv[1]);
+      out.y = pack2<El>(silu_fast(gv[2]) * uv[2], silu_fast(gv[3]) * uv[3]);
+    } else if constexpr (GATED) {
       out.x = gated_pair<El, ACT>(p, pack2<El>(gv[0], gv[1]), pack2<El>(uv[0], uv[1]));
       out.y = gated_pair<El, ACT>(p, pack2<El>(gv[2], gv[3]), pack2<El>(uv[2], uv[3]));
     } else {
@@ -1670,7 +1686,8 @@ __global__ __launch_bounds__(kThreads, 3) void stream_gemm_kernel(const GemmPara
   if (tok < p.numel) {
     const bool fast = n0 + BN_OUT <= p.N && (p.ldc & 3) == 0;
     if constexpr (GATED) {
-      if (!fast) store_fragment<El, true, false>(p, e, acc0, acc1, tok, slot, n0 + 4 * lhi, rw);
+      if (!fast) store_fragment<El, true, false, !TAIL>(p, e, acc0, acc1, tok, slot, n0 + 4 * lhi, rw);
+      else if (!TAIL && p.silu_once) stream_store<El, true, MOE_ACT_SILU, true>(p, e, acc0, acc1, tok, slot, n0 + 4 * lhi, rw);
       else if (p.activation == MOE_ACT_SILU) stream_store<El, true, MOE_ACT_SILU>(p, e, acc0, acc1, tok, slot, n0 + 4 * lhi, rw);
       else if (p.activation == MOE_ACT_SWIGLUOAI) stream_store<El, true, MOE_ACT_SWIGLUOAI>(p, e, acc0, acc1, tok, slot, n0 + 4 * lhi, rw);
       else stream_store<El, true, MOE_ACT_GELU>(p, e, acc0, acc1, tok, slot, n0 + 4 * lhi, rw);
@@ -2108,6 +2125,7 @@ MOE_EXPORT int moe_fused_experts(const MoeFusedExpertsArgs* a) {
   p.alpha = a->swiglu_alpha;
   p.limit = a->swiglu_limit;
   p.activation = a->activation;
+  p.silu_once = (a->passes & 64) && a->activation == MOE_ACT_SILU ? 1 : 0;
   p.interleaved = a->activation == MOE_ACT_SWIGLUOAI;
   p.w_tiled = a->weight_layout == MOE_WEIGHTS_TILED ? 1 : 0;
   p.ragged = fused_args_ragged(a) ? 1 : 0;

@@ -139,6 +139,8 @@ MOE_EXPORT int moe_layer(const MoeLayerArgs* a) {
   f.apply_router_weight_on_input = a->apply_router_weight_on_input;
   f.swiglu_alpha = a->swiglu_alpha; f.swiglu_limit = a->swiglu_limit;
   f.passes = plan ? 16 : 0;
+  // a block of 32 of the library's own choice where the large tile would also do: same roundings as that
+  if (!a->block_size && l.block < moe_preferred_block_size(a->T, a->E, a->K, a->act_dtype, a->weight_dtype)) f.passes |= 64;
   f.weight_layout = a->weight_layout;
   f.stream = a->stream;
   return moe_fused_experts(&f);

@@ -76,6 +76,8 @@ def try_get_optimal_moe_config(w1_shape, w2_shape, top_k: int, dtype: Optional[s
     E = w2_shape[0]
     act_code = _lib.DTYPE_CODE[act_dtype]
     weight_code = _lib.E4M3_CODE if dtype == "fp8_w8a8" else act_code
+    if w1_shape[1] == 0:   # the layer's width is not known
+        return {"BLOCK_SIZE_M": lib().moe_preferred_block_size(M, E, top_k, act_code, weight_code)}
     bm = lib().moe_layer_block_size(M, w1_shape[1] // 2, E, top_k, act_code, weight_code)
     return {"BLOCK_SIZE_M": bm}
 
@@ -421,11 +423,15 @@ def fused_experts_impl(hidden_states: torch.Tensor,
                                       act_code, weight_code, curr_ids.numel())
         sorted_token_ids, expert_ids, num_tokens_post_padded = _align_block_size(
             curr_ids, bm, global_num_experts, plan)
+        passes = 16 if plan is not None else 0
+        if try_get_optimal_moe_config is _LIBRARY_CONFIG and \
+                bm < L.moe_preferred_block_size(tokens_in_chunk, E, top_k_num, act_code, weight_code):
+            passes |= 64   # the library's choice of the smaller block keeps the larger one's roundings
         args = launch_fused_experts(hidden_states[begin:end], out_hidden_states[begin:end], w1, w2,
                                     w1_bias, w2_bias, w1_scale, w2_scale, curr_w, sorted_token_ids,
                                     expert_ids, num_tokens_post_padded, bm, activation,
                                     apply_router_weight_on_input, weight_code=weight_code,
-                                    workspace=workspace, passes=16 if plan is not None else 0,
+                                    workspace=workspace, passes=passes,
                                     weight_layout=weight_layout)
         if _CHECK_HANDOFF and not torch.cuda.is_current_stream_capturing():  # the check waits for the stream
             fused_experts_status(args)

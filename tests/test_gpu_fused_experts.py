@@ -88,6 +88,33 @@ def test_every_block_size_kernel(moe, oracle, dev, bm, monkeypatch):
     _close(out, oracle.fused_experts_ref(x, w13, w2, tw, ids))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,H,I", [(32, 128, 128), (150, 128, 120), (190, 320, 64), (300, 128, 128)])
+def test_silu_product_is_rounded_once_whatever_the_block_rule_picks(moe, dev, dtype, T, H, I, monkeypatch):
+    """Identity down weights and a routed weight of 1: the result is the gated intermediate itself, which must
+    be the float64 product rounded once, on the streaming kernel (16 to 95 rows per expert of a narrow layer;
+    tiles inside the matrix and at its edge) as on the large-tile kernel (150 rows).  The error of the fp32
+    sums, some 2^-20 of a value, moves it across a rounding boundary in fewer than one element in fifty (a step
+    of fp16 is 2^-11); with gate, up and silu rounded as well about half of the elements differ.  Entered both
+    natively and from Python."""
+    print(f"silu once {dtype} T={T} H={H} I={I}", flush=True)
+    E = 2
+    g = torch.Generator().manual_seed(H + T)
+    x = torch.randn(T, H, generator=g).to(dtype).to(dev)
+    w13 = (torch.randn(E, 2 * I, H, generator=g) / H ** 0.5).to(dtype).to(dev)
+    w2 = torch.eye(H, I, dtype=dtype, device=dev).expand(E, H, I).contiguous()
+    ids = (torch.arange(T, dtype=torch.int32) % E).view(T, 1).to(dev)
+    want = torch.zeros(T, H, dtype=torch.float64, device=dev)
+    for e in range(E):
+        gate, up = (x[e::E].double() @ w13[e].double().t()).chunk(2, dim=1)
+        want[e::E, :I] = torch.nn.functional.silu(gate) * up
+    for native in (True, False):
+        if not native:
+            monkeypatch.setattr(moe.fused_moe, "_layer_call", lambda *a: None)
+        out = moe.fused_experts(x, w13, w2, None, None, torch.ones(T, 1, device=dev), ids)
+        assert (out != want.to(dtype))[:, :I].double().mean().item() < 0.02
+
+
 def test_inplace_aliases_input_and_matches(moe, oracle, dev):
     x, w13, w2, logits = _layer(8, 256, 128, 200, 2, 9, torch.bfloat16)
     tw, ids, _ = oracle.topk_softmax(logits, 2, renormalize=True)
