@@ -24,6 +24,16 @@ __device__ __forceinline__ float wave_sum(float v) {
   return v;
 }
 
+// The product as an fp32 value, as the definition above has it: without this the compiler may fold the
+// multiplication into the conversion to fp16 (v_fma_mixlo_f16: one rounding of the exact product instead of two), and
+// it did so in one kernel here and not in the other, which then differed in one element in ten thousand.
+template <typename El>
+__device__ __forceinline__ float product(float a, float b) {
+  float v = a * b;
+  if constexpr (__is_same(El, ElemF16)) asm("" : "+v"(v));
+  return v;
+}
+
 // Two values rounded to the 16-bit dtype in one conversion instruction (written out with integers, the rounding of
 // an element took five operations and every element is rounded three times).
 template <typename El>
@@ -53,7 +63,9 @@ __global__ __launch_bounds__(kThreads) void rms_norm_vec_kernel(uint16_t* out, i
   // stored chunk by chunk a row took NV round trips to memory one after the other.  Rows stay packed, two
   // elements a register, so that several wavefronts of a SIMD still hold a row each (unpacked, 116 registers, the
   // same loads made it slower: 72 us at 16896 rows).  bf16 rows of 2048: 8.6 -> 4.8 us for 64 of them, 32.6 ->
-  // 25.5 us (5.4 TB/s) for 8448, 49.6 -> 44.8 us (6.2 TB/s) for 16896.
+  // 25.5 us (5.4 TB/s) for 8448, 49.6 -> 44.8 us (6.2 TB/s) for 16896.  Longer rows gain more, although NV = 8 and
+  // 16 take 138 and 284 registers, one wavefront a SIMD: the round trips of a row were its time (8448 rows of 4096
+  // 65.0 -> 57.0 us, of 8192 133.6 -> 107.1; 64 rows 11.9 -> 4.5 and 22.8 -> 6.8; fp16 59.0 -> 57.1, 113.7 -> 105.0).
   uint4 xv[NV], rv[NV];
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
@@ -97,7 +109,7 @@ __global__ __launch_bounds__(kThreads) void rms_norm_vec_kernel(uint16_t* out, i
   }
   const float r = rsqrtf(wave_sum(sq) / static_cast<float>(H) + eps);
   auto scale = [&](uint32_t v, uint32_t w) {
-    const uint32_t n = pack(lo(v) * r, hi(v) * r);
+    const uint32_t n = pack(product<El>(lo(v), r), product<El>(hi(v), r));
     return pack(lo(n) * lo(w), hi(n) * hi(w));
   };
 #pragma unroll
@@ -132,7 +144,7 @@ __global__ __launch_bounds__(kThreads) void rms_norm_any_kernel(typename El::S* 
   const float r = rsqrtf(wave_sum(sq) / static_cast<float>(H) + eps);
   for (int c = lane; c < H; c += kWave) {
     const float v = ADD ? El::ld(residual[row * res_stride + c]) : El::ld(x[row * x_stride + c]);
-    out[row * out_stride + c] = El::st(El::ld(El::st(v * r)) * El::ld(weight[c]));
+    out[row * out_stride + c] = El::st(El::ld(El::st(product<El>(v, r))) * El::ld(weight[c]));
   }
 }
 

@@ -312,6 +312,31 @@ def test_add_rms_norm_against_oracle(moe, oracle, dev, dtype, T, H):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("aligned", [True, False])   # the 16-byte kernel, the element kernel
+@pytest.mark.parametrize("add", [True, False])
+def test_rms_norm_fp16_rounds_where_the_definition_says(moe, dev, aligned, add):
+    """T(T(s * r) * weight) with s * r an fp32 value before it is narrowed.  Whole numbers of up to 63 make the sum
+    of squares exact in any order, so fp32 rows give r and the products bit for bit (their weight is 1); half a
+    million distinct products hold some tens that a single rounding to fp16 would take the other way."""
+    T, H = 8192, 2048
+    g = torch.Generator().manual_seed(5)
+    s = torch.randint(-63, 64, (T, H), generator=g).float().to(dev)
+    res = torch.randint(-20, 21, (T, H), generator=g).float().clamp(-63 - s.cpu(), 63 - s.cpu()).to(dev) if add \
+        else torch.zeros_like(s)
+    one = torch.ones(H, device=dev)
+    want = torch.empty_like(s)
+    moe.ops.rms_norm(want, s, one, 1e-6)
+    x, residual = (s - res).half(), res.half()
+    buf = torch.empty(T * H + 1, dtype=torch.float16, device=dev)
+    out = (buf[:-1] if aligned else buf[1:]).view(T, H)
+    if add:
+        moe.ops.add_rms_norm(out, residual, x, one.half(), 1e-6)
+        assert torch.equal(residual, s.half())
+    else:
+        moe.ops.rms_norm(out, x, one.half(), 1e-6)
+    assert torch.equal(out, want.half())
+
+
 def test_rms_norm_module_mirrors_the_reference_interface(moe, oracle, dev):
     """nanovllm/layers/layernorm.py:7-34: forward(x) -> out; forward(x, residual) ->
     (out, residual) with the residual updated in place."""
