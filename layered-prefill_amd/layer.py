@@ -54,6 +54,13 @@ class MoEConfig:
         return self.moe_parallel_config.tp_rank
 
 
+def _held(module: torch.nn.Module, name: str, *default):
+    """``getattr(module, name, *default)``: a parameter, a buffer, a plain attribute or a parametrised tensor.  The
+    module's own lookup costs a microsecond for each registered parameter, which is found directly here."""
+    t = module._parameters.get(name)
+    return t if t is not None and name not in module.__dict__ else getattr(module, name, *default)
+
+
 class UnquantizedFusedMoEMethod:
     """nanovllm/layers/fused_moe.py:108-216."""
 
@@ -97,10 +104,9 @@ class UnquantizedFusedMoEMethod:
                 and e_score_correction_bias is None and expert_map is None
                 and self.topk_indices_dtype is None and self.fused_experts is fused_experts):
             # plain softmax routing: select_experts + fused_experts as one function
-            params = layer._parameters   # (the module's own attribute lookup costs a microsecond per name)
             return fused_topk_experts(
-                x, router_logits, params["w13_weight"], params["w2_weight"], top_k, renormalize,
-                w1_bias=params.get("w13_bias"), w2_bias=params.get("w2_bias"),
+                x, router_logits, _held(layer, "w13_weight"), _held(layer, "w2_weight"), top_k, renormalize,
+                w1_bias=_held(layer, "w13_bias", None), w2_bias=_held(layer, "w2_bias", None),
                 inplace=True, activation=activation,
                 apply_router_weight_on_input=apply_router_weight_on_input, weight_layout=layout)
         topk_weights, topk_ids = FusedMoE.select_experts(
@@ -161,16 +167,16 @@ class Fp8E4M3FusedMoEMethod(UnquantizedFusedMoEMethod):
               apply_router_weight_on_input: bool = False, global_num_experts: int = -1,
               expert_map: Optional[torch.Tensor] = None,
               custom_routing_function: Optional[Callable] = None, **unused) -> torch.Tensor:
-        params = layer._parameters
-        if "w13_weight_scale" not in params:
+        w13_scale = _held(layer, "w13_weight_scale", None)
+        if w13_scale is None:
             raise RuntimeError("Fp8E4M3FusedMoEMethod.apply before process_weights_after_loading")
         if (custom_routing_function is None and expert_map is None and self.topk_indices_dtype is None
                 and self.fused_experts is fused_experts):
             return fused_topk_experts(
-                x, router_logits, params["w13_weight"], params["w2_weight"], top_k, renormalize,
-                w1_bias=params.get("w13_bias"), w2_bias=params.get("w2_bias"), inplace=True, activation=activation,
-                apply_router_weight_on_input=apply_router_weight_on_input,
-                w1_scale=params["w13_weight_scale"], w2_scale=params["w2_weight_scale"])
+                x, router_logits, _held(layer, "w13_weight"), _held(layer, "w2_weight"), top_k, renormalize,
+                w1_bias=_held(layer, "w13_bias", None), w2_bias=_held(layer, "w2_bias", None), inplace=True,
+                activation=activation, apply_router_weight_on_input=apply_router_weight_on_input,
+                w1_scale=w13_scale, w2_scale=_held(layer, "w2_weight_scale"))
         topk_weights, topk_ids = FusedMoE.select_experts(
             hidden_states=x, router_logits=router_logits, use_grouped_topk=False, top_k=top_k,
             renormalize=renormalize, custom_routing_function=custom_routing_function,
@@ -495,7 +501,7 @@ class RMSNorm(torch.nn.Module):
                 out: Optional[torch.Tensor] = None):
         if out is None:
             if x.is_cuda:
-                out = _lib.host().rms_norm(x, residual, self._parameters["weight"], self.eps)
+                out = _lib.host().rms_norm(x, residual, _held(self, "weight"), self.eps)
                 if out is not None:
                     return out if residual is None else (out, residual)
             out = torch.empty_like(x)

@@ -252,3 +252,70 @@ def test_layer_block_size_of_fp32_is_the_old_rule(moe):
     L = moe._lib.lib()
     for m in (1, 256, 768, 2048, 8448):
         assert L.moe_layer_block_size(m, 768, 128, 8, 0, 0) == L.moe_preferred_block_size(m, 128, 8, 0, 0)
+
+
+def _hold(module, name, how):
+    """Re-registers a parameter as what else a module can hold under that name; returns the tensor it now stands for."""
+    t = getattr(module, name).detach()
+    if how == "parameter":
+        return getattr(module, name)
+    if how == "parametrised":
+        class Twice(torch.nn.Module):
+            def forward(self, w):
+                return w + w
+        torch.nn.utils.parametrize.register_parametrization(module, name, Twice())
+        return t + t
+    delattr(module, name)
+    if how == "buffer":
+        module.register_buffer(name, t)
+    else:
+        setattr(module, name, t)
+    return t
+
+
+@pytest.mark.parametrize("quantization", [None, "fp8_e4m3"])
+@pytest.mark.parametrize("how", ["parameter", "buffer", "attribute", "parametrised"])
+def test_layer_takes_weights_however_the_module_holds_them(moe, monkeypatch, how, quantization):
+    layer = moe.FusedMoE(4, 2, 32, 16, params_dtype=torch.bfloat16, has_bias=quantization is None,
+                         quantization=quantization)
+    names = {"w13_weight": 2, "w2_weight": 3}
+    if quantization:
+        names.update(w13_weight_scale="w1_scale", w2_weight_scale="w2_scale")
+        for name, shape in (("w13_weight_scale", (4, 32)), ("w2_weight_scale", (4, 32))):
+            layer.register_parameter(name, torch.nn.Parameter(torch.rand(shape), requires_grad=False))
+    else:
+        names.update(w13_bias="w1_bias", w2_bias="w2_bias")
+    for name in names:
+        getattr(layer, name).data.fill_(0.25)
+    want = {name: _hold(layer, name, how) for name in names}
+    seen = []
+    monkeypatch.setattr(moe.layer, "fused_topk_experts", lambda *a, **k: seen.append((a, k)) or a[0])
+    layer(torch.zeros(3, 32, dtype=torch.bfloat16), torch.zeros(3, 4))
+    args, kwargs = seen[0]
+    for name, where in names.items():
+        assert torch.equal(args[where] if isinstance(where, int) else kwargs[where], want[name]), name
+
+
+@pytest.mark.parametrize("how", ["parameter", "buffer", "attribute", "parametrised"])
+def test_norm_takes_its_weight_however_the_module_holds_it(moe, monkeypatch, how):
+    norm = moe.RMSNorm(8)
+    want = _hold(norm, "weight", how)
+
+    class Host:
+        rms_norm = staticmethod(lambda x, residual, weight, eps: weight)
+
+    class OnGpu:
+        is_cuda = True
+
+    monkeypatch.setattr(moe.layer._lib, "host", lambda: Host)
+    assert torch.equal(norm(OnGpu()), want)
+
+
+def test_layer_without_weights_says_so(moe):
+    layer = moe.FusedMoE(4, 2, 32, 16, params_dtype=torch.bfloat16)
+    del layer.w2_weight
+    with pytest.raises(AttributeError, match="w2_weight"):
+        layer(torch.zeros(3, 32, dtype=torch.bfloat16), torch.zeros(3, 4))
+    quantised = moe.FusedMoE(4, 2, 32, 16, params_dtype=torch.bfloat16, quantization="fp8_e4m3")
+    with pytest.raises(RuntimeError, match="before process_weights_after_loading"):
+        quantised(torch.zeros(3, 32, dtype=torch.bfloat16), torch.zeros(3, 4))
