@@ -44,6 +44,25 @@ bool optional_tensor(PyObject* o, const at::Device& dev, at::ScalarType type, at
   return true;
 }
 
+// Plain ints, bools and floats, or false, with no Python error set: the Python caller's own path then converts
+// what can be converted and names what cannot.
+bool int_arg(PyObject* o, int64_t* v) {
+  int overflow = 0;
+  if (!PyLong_CheckExact(o)) return false;
+  *v = PyLong_AsLongAndOverflow(o, &overflow);
+  return !overflow;
+}
+bool flag_arg(PyObject* o, bool* v) {
+  if (!PyBool_Check(o)) return false;
+  *v = o == Py_True;
+  return true;
+}
+bool float_arg(PyObject* o, float* v) {
+  if (!PyFloat_CheckExact(o)) return false;
+  *v = static_cast<float>(PyFloat_AS_DOUBLE(o));
+  return true;
+}
+
 void* current_stream(const at::Device& dev) {
   PyObject* idx = PyLong_FromLong(dev.index());
   PyObject* r = idx ? PyObject_CallOneArg(g_raw_stream, idx) : nullptr;
@@ -80,7 +99,11 @@ PyObject* tuple_of(const at::Tensor& a, const at::Tensor& b, const at::Tensor& c
 // -> result tensor, or None.  Codes as in moe_gfx950.h.
 PyObject* layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  if (n != 16) MOE_NONE;
+  int64_t K, activation, weight_layout;
+  bool renormalize, weight_on_input, inplace;
+  if (n != 16 || !int_arg(a[10], &K) || !flag_arg(a[11], &renormalize) || !int_arg(a[12], &activation) ||
+      !flag_arg(a[13], &weight_on_input) || !int_arg(a[14], &weight_layout) || !flag_arg(a[15], &inplace))
+    MOE_NONE;
   const at::Tensor *x = gpu_tensor(a[0]), *w13 = gpu_tensor(a[2]), *w2 = gpu_tensor(a[3]);
   if (!x || !w13 || !w2 || x->dim() != 2 || w13->dim() != 3 || w2->dim() != 3) MOE_NONE;
   const at::Device dev = x->device();
@@ -108,7 +131,6 @@ PyObject* layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
     MOE_NONE;
   }
   MoeLayerArgs m{};
-  const int64_t K = PyLong_AsLong(a[10]);
   if (K < 1 || K > E || T * K > INT32_MAX) MOE_NONE;
   if (a[1] != Py_None) {
     const at::Tensor* g = gpu_tensor(a[1]);
@@ -116,7 +138,7 @@ PyObject* layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
     m.logits_dtype = dtype_code(g->scalar_type());
     if (m.logits_dtype < 0) MOE_NONE;
     m.router_logits = g->data_ptr();
-    m.renormalize = PyObject_IsTrue(a[11]);
+    m.renormalize = renormalize;
   } else {
     const at::Tensor *w, *ids;
     const int64_t tk[2] = {T, K};
@@ -124,10 +146,9 @@ PyObject* layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
     m.topk_weights = static_cast<float*>(w->data_ptr());
     m.topk_ids = static_cast<int32_t*>(ids->data_ptr());
   }
-  m.activation = static_cast<int32_t>(PyLong_AsLong(a[12]));
-  m.apply_router_weight_on_input = PyObject_IsTrue(a[13]);
-  m.weight_layout = static_cast<int32_t>(PyLong_AsLong(a[14]));
-  const bool inplace = PyObject_IsTrue(a[15]);
+  m.activation = static_cast<int32_t>(activation);
+  m.apply_router_weight_on_input = weight_on_input;
+  m.weight_layout = static_cast<int32_t>(weight_layout);
   c10::OptionalDeviceGuard guard(dev);
   const at::Tensor out = inplace ? *x : empty({T, H}, x->scalar_type(), dev);
   m.x = x->data_ptr();
@@ -168,18 +189,20 @@ PyObject* layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
 // topk(router_logits, top_k, renormalize) -> (weights, ids, token_expert_indices), or None.
 PyObject* topk(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  if (n != 3) MOE_NONE;
+  int64_t K;
+  bool renormalize;
+  if (n != 3 || !int_arg(a[1], &K) || !flag_arg(a[2], &renormalize)) MOE_NONE;
   const at::Tensor* g = gpu_tensor(a[0]);
   if (!g || g->dim() != 2 || !g->is_contiguous() || g->size(0) < 1) MOE_NONE;
   const int dtype = dtype_code(g->scalar_type());
-  const int64_t T = g->size(0), E = g->size(1), K = PyLong_AsLong(a[1]);
+  const int64_t T = g->size(0), E = g->size(1);
   if (dtype < 0 || K < 1 || K > E || T * K > INT32_MAX) MOE_NONE;
   const at::Device dev = g->device();
   c10::OptionalDeviceGuard guard(dev);
   const at::Tensor w = empty({T, K}, at::kFloat, dev), ids = empty({T, K}, at::kInt, dev), tei = empty({T, K}, at::kInt, dev);
   check(moe_topk_softmax_typed(g->data_ptr(), dtype, static_cast<float*>(w.data_ptr()), static_cast<int32_t*>(ids.data_ptr()),
                                static_cast<int32_t*>(tei.data_ptr()), static_cast<int>(T), static_cast<int>(E),
-                               static_cast<int>(K), PyObject_IsTrue(a[2]), current_stream(dev)));
+                               static_cast<int>(K), renormalize, current_stream(dev)));
   return tuple_of(w, ids, tei);
   END_HANDLE_TH_ERRORS
 }
@@ -187,7 +210,8 @@ PyObject* topk(PyObject*, PyObject* const* a, Py_ssize_t n) {
 // rms_norm(x, residual | None, weight, eps) -> the normalised tensor (residual updated in place), or None.
 PyObject* rms_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  if (n != 4) MOE_NONE;
+  float eps;
+  if (n != 4 || !float_arg(a[3], &eps)) MOE_NONE;
   const at::Tensor *x = gpu_tensor(a[0]), *w = gpu_tensor(a[2]);
   const at::Tensor* res = a[1] == Py_None ? nullptr : gpu_tensor(a[1]);
   if (!x || !w || (!res && a[1] != Py_None) || x->dim() != 2) MOE_NONE;
@@ -202,7 +226,7 @@ PyObject* rms_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
   c10::OptionalDeviceGuard guard(dev);
   const at::Tensor out = empty({T, H}, x->scalar_type(), dev);
   check(moe_add_rms_norm(out.data_ptr(), H, res ? res->data_ptr() : nullptr, H, x->data_ptr(), H, w->data_ptr(), dtype, T,
-                         static_cast<int>(H), static_cast<float>(PyFloat_AsDouble(a[3])), current_stream(dev)));
+                         static_cast<int>(H), eps, current_stream(dev)));
   return THPVariable_Wrap(out);
   END_HANDLE_TH_ERRORS
 }
@@ -210,12 +234,14 @@ PyObject* rms_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
 // gate_topk(x, gate_weight, top_k, renormalize) -> (weights, ids, token_expert_indices), or None.
 PyObject* gate_topk(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  if (n != 4) MOE_NONE;
+  int64_t K;
+  bool renormalize;
+  if (n != 4 || !int_arg(a[2], &K) || !flag_arg(a[3], &renormalize)) MOE_NONE;
   const at::Tensor *x = gpu_tensor(a[0]), *g = gpu_tensor(a[1]);
   if (!x || !g || x->dim() != 2 || g->dim() != 2 || !x->is_contiguous() || !g->is_contiguous()) MOE_NONE;
   const at::Device dev = x->device();
   const int dtype = dtype_code(x->scalar_type());
-  const int64_t T = x->size(0), H = x->size(1), E = g->size(0), K = PyLong_AsLong(a[2]);
+  const int64_t T = x->size(0), H = x->size(1), E = g->size(0);
   if (T < 1 || g->device() != dev || g->scalar_type() != x->scalar_type() || g->size(1) != H || K < 1 || K > E ||
       T * K > INT32_MAX || T * H * 2 >= (int64_t{1} << 32))
     MOE_NONE;
@@ -226,7 +252,7 @@ PyObject* gate_topk(PyObject*, PyObject* const* a, Py_ssize_t n) {
   check(moe_gate_topk_softmax(x->data_ptr(), g->data_ptr(), dtype, nullptr, static_cast<float*>(w.data_ptr()),
                               static_cast<int32_t*>(ids.data_ptr()), static_cast<int32_t*>(tei.data_ptr()),
                               static_cast<int>(T), static_cast<int>(H), static_cast<int>(E), static_cast<int>(K),
-                              PyObject_IsTrue(a[3]), current_stream(dev)));
+                              renormalize, current_stream(dev)));
   return tuple_of(w, ids, tei);
   END_HANDLE_TH_ERRORS
 }

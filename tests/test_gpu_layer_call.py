@@ -1,4 +1,5 @@
 """The layer as one call into native code: the same results as its steps, and the kernels it picks by the sizes."""
+import numpy as np
 import pytest
 import torch
 
@@ -32,3 +33,42 @@ def test_one_call_is_its_steps(moe, dev, monkeypatch, T, activation, on_input):
     monkeypatch.setattr(moe.fused_moe, "try_get_optimal_moe_config", lambda *a, **k: own(*a, **k))
     steps = moe.fused_topk_experts(x, logits, w13, w2, K, True, **kw)
     assert (one.float() - steps.float()).norm() <= 2e-3 * steps.float().norm()
+
+
+def test_arguments_are_converted_or_refused_as_python_does(moe, dev):
+    """What is no plain int, bool or float takes the Python path: what converts, converts; what does not is that
+    path's error, in front of any launch."""
+    g = torch.Generator().manual_seed(3)
+    x = torch.randn(5, 32, generator=g).bfloat16().to(dev)
+    logits = torch.randn(5, 8, generator=g).bfloat16().to(dev)
+    w13 = (torch.randn(8, 64, 32, generator=g) * 0.1).bfloat16().to(dev)
+    w2 = (torch.randn(8, 32, 32, generator=g) * 0.1).bfloat16().to(dev)
+    gate = torch.randn(32, 64, generator=g).bfloat16().to(dev)
+    many = torch.randn(2048, 64, generator=g).bfloat16().to(dev)
+    plain = moe.fused_topk(x, logits, 2, True)
+    for topk, renormalize in ((np.int64(2), True), (2, np.bool_(True)), (2, 1)):
+        assert all(torch.equal(a, b) for a, b in zip(moe.fused_topk(x, logits, topk, renormalize), plain))
+    for topk in (2.0, "2", None):
+        with pytest.raises(TypeError):
+            moe.fused_topk(x, logits, topk, True)
+        with pytest.raises(TypeError):
+            moe.fused_topk_experts(x, logits, w13, w2, topk, True)
+        with pytest.raises(TypeError):
+            moe.fused_gate_topk(many, gate, topk, True)
+    with pytest.raises((RuntimeError, OverflowError, TypeError)):
+        moe.fused_topk(x, logits, 1 << 70, True)
+    for renormalize in (None, [1]):
+        with pytest.raises(TypeError):
+            moe.fused_topk(x, logits, 2, renormalize)
+    out = moe.fused_topk_experts(x, logits, w13, w2, 2, True)
+    for kw in (dict(apply_router_weight_on_input=np.bool_(False)), dict(inplace=0), dict(inplace=None)):
+        assert torch.equal(moe.fused_topk_experts(x, logits, w13, w2, np.int64(2), np.bool_(True), **kw), out)
+
+    norm, res = moe.RMSNorm(32, eps="1e-6").bfloat16().to(dev), x.clone()
+    want, want_res = moe.RMSNorm(32).bfloat16().to(dev)(x, x.clone())
+    got, _ = norm(x, res)
+    assert torch.equal(got, want) and torch.equal(res, want_res)
+    norm.eps, res = None, x.clone()
+    with pytest.raises(TypeError):
+        norm(x, res)
+    assert torch.equal(res, x)
