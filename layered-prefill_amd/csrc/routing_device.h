@@ -56,9 +56,11 @@ __device__ __forceinline__ void argmax_level(float& best, int& bidx) {
 }
 
 // The logits of row `row` as route_row wants them, widened to fp32: lane t of the row loads columns
-// (i / EPL) * EPL * TPR + t * EPL + i % EPL into v[i], EPL at a time.
+// (i / EPL) * EPL * TPR + t * EPL + i % EPL into v[i], EPL at a time.  A caller's rows need no more than the
+// alignment of an element, and the type says so; the load is one instruction all the same (a global load takes
+// any address).
 template <typename S, int N>
-struct alignas(sizeof(S) * N) RowVec {
+struct __attribute__((packed, aligned(sizeof(S)))) RowVec {
   S v[N];
 };
 template <int E, typename El = ElemF32>

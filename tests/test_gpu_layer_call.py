@@ -16,6 +16,27 @@ def test_topk_of_16bit_logits_is_topk_of_their_float(moe, dev, dtype, T, E, K):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("E,K", [(1, 1), (2, 1), (4, 2), (8, 2), (32, 4), (128, 8), (256, 8), (60, 4), (1100, 2)])
+@pytest.mark.parametrize("offset", [1, 2, 3])
+def test_logits_need_the_alignment_of_an_element_only(moe, dev, dtype, E, K, offset):
+    print(f"logits {dtype} E={E} offset={offset}", flush=True)
+    T, H, I = 9, 32, 32
+    g = torch.Generator().manual_seed(E + offset)
+    aligned = torch.randn(T, E, generator=g).to(dtype).to(dev)
+    buf = torch.full((T * E + 8,), 50.0, dtype=dtype, device=dev)
+    logits = buf[offset:offset + T * E].view(T, E).copy_(aligned)
+    assert logits.is_contiguous() and logits.data_ptr() % 16 == offset * logits.element_size()
+    x = torch.randn(T, H, generator=g).bfloat16().to(dev)
+    for a, b in zip(moe.fused_topk(x, logits, K, True), moe.fused_topk(x, aligned, K, True)):
+        assert torch.equal(a, b)
+    if E <= 256:
+        w13 = torch.randn(E, 2 * I, H, generator=g).bfloat16().to(dev)
+        w2 = torch.randn(E, H, I, generator=g).bfloat16().to(dev)
+        assert torch.equal(moe.fused_topk_experts(x, logits, w13, w2, K, True),
+                           moe.fused_topk_experts(x, aligned, w13, w2, K, True))
+
+
 @pytest.mark.parametrize("T,activation,on_input", [(1, "silu", False), (40, "gelu", True), (700, "swigluoai", False)])
 def test_one_call_is_its_steps(moe, dev, monkeypatch, T, activation, on_input):
     """``fused_topk_experts`` against alignment and experts enqueued from Python (what a block size of the
