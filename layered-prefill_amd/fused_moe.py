@@ -103,11 +103,11 @@ def fused_topk(hidden_states: torch.Tensor, gating_output: torch.Tensor, topk: i
                renormalize: bool):
     """nanovllm/layers/for_moe/fused_moe.py:393-419."""
     assert hidden_states.shape[0] == gating_output.shape[0], "Number of tokens mismatch"
+    M, _ = hidden_states.shape
     if gating_output.is_cuda and hidden_states.device == gating_output.device:
         routed = _lib.host().topk(gating_output, topk, renormalize)
         if routed is not None:
             return routed
-    M, _ = hidden_states.shape
     topk_weights = torch.empty(M, topk, dtype=torch.float32, device=hidden_states.device)
     topk_ids = torch.empty(M, topk, dtype=torch.int32, device=hidden_states.device)
     token_expert_indicies = torch.empty(M, topk, dtype=torch.int32, device=hidden_states.device)

@@ -37,6 +37,17 @@ def test_logits_need_the_alignment_of_an_element_only(moe, dev, dtype, E, K, off
                            moe.fused_topk_experts(x, aligned, w13, w2, K, True))
 
 
+@pytest.mark.parametrize("shape", [(4,), (4, 2, 8)])
+def test_routing_refuses_hidden_states_that_are_no_matrix(moe, dev, shape):
+    x = torch.zeros(shape, dtype=torch.bfloat16, device=dev)
+    logits = torch.zeros(4, 8, device=dev)
+    with pytest.raises(ValueError):
+        moe.fused_topk(x, logits, 2, True)
+    w = torch.zeros(8, 16, 8, dtype=torch.bfloat16, device=dev)
+    with pytest.raises(ValueError):
+        moe.fused_topk_experts(x, logits, w, w[:, :, :8], 2, True)
+
+
 @pytest.mark.parametrize("T,activation,on_input", [(1, "silu", False), (40, "gelu", True), (700, "swigluoai", False)])
 def test_one_call_is_its_steps(moe, dev, monkeypatch, T, activation, on_input):
     """``fused_topk_experts`` against alignment and experts enqueued from Python (what a block size of the
