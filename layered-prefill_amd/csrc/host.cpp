@@ -63,6 +63,22 @@ bool float_arg(PyObject* o, float* v) {
   return true;
 }
 
+// Other Python threads run while a call allocates and enqueues (fresh memory and the first launch of a kernel take
+// milliseconds, a full queue makes a launch wait).  Nothing of Python is touched meanwhile.
+struct WithoutGil {
+  PyThreadState* state = PyEval_SaveThread();
+  WithoutGil() = default;
+  WithoutGil(const WithoutGil&) = delete;
+  ~WithoutGil() { PyEval_RestoreThread(state); }
+};
+
+// Allocations and the library call at their end, made without the GIL; its return code.
+template <typename Call>
+int enqueue(const Call& call) {
+  const WithoutGil nogil;
+  return call();
+}
+
 void* current_stream(const at::Device& dev) {
   PyObject* idx = PyLong_FromLong(dev.index());
   PyObject* r = idx ? PyObject_CallOneArg(g_raw_stream, idx) : nullptr;
@@ -150,9 +166,7 @@ PyObject* layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
   m.apply_router_weight_on_input = weight_on_input;
   m.weight_layout = static_cast<int32_t>(weight_layout);
   c10::OptionalDeviceGuard guard(dev);
-  const at::Tensor out = inplace ? *x : empty({T, H}, x->scalar_type(), dev);
   m.x = x->data_ptr();
-  m.out = out.data_ptr();
   m.w13 = w13->data_ptr();
   m.w2 = w2->data_ptr();
   m.w13_bias = b13 ? b13->data_ptr() : nullptr;
@@ -175,9 +189,15 @@ PyObject* layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
   m.stream = current_stream(dev);
   m.workspace_bytes = moe_layer_workspace_bytes(&m);
   if (m.workspace_bytes <= 0) MOE_NONE;
-  const at::Tensor ws = empty({m.workspace_bytes}, at::kByte, dev);
-  m.workspace = ws.data_ptr();
-  check(moe_layer(&m));
+  const at::ScalarType type = x->scalar_type();
+  at::Tensor out = *x;
+  check(enqueue([&] {
+    if (!inplace) out = empty({T, H}, type, dev);
+    m.out = out.data_ptr();
+    const at::Tensor ws = empty({m.workspace_bytes}, at::kByte, dev);
+    m.workspace = ws.data_ptr();
+    return moe_layer(&m);
+  }));
   if (inplace) {
     Py_INCREF(a[0]);
     return a[0];
@@ -199,10 +219,15 @@ PyObject* topk(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (dtype < 0 || K < 1 || K > E || T * K > INT32_MAX) MOE_NONE;
   const at::Device dev = g->device();
   c10::OptionalDeviceGuard guard(dev);
-  const at::Tensor w = empty({T, K}, at::kFloat, dev), ids = empty({T, K}, at::kInt, dev), tei = empty({T, K}, at::kInt, dev);
-  check(moe_topk_softmax_typed(g->data_ptr(), dtype, static_cast<float*>(w.data_ptr()), static_cast<int32_t*>(ids.data_ptr()),
-                               static_cast<int32_t*>(tei.data_ptr()), static_cast<int>(T), static_cast<int>(E),
-                               static_cast<int>(K), renormalize, current_stream(dev)));
+  void* const stream = current_stream(dev);
+  const void* const logits = g->data_ptr();
+  at::Tensor w, ids, tei;
+  check(enqueue([&] {
+    w = empty({T, K}, at::kFloat, dev), ids = empty({T, K}, at::kInt, dev), tei = empty({T, K}, at::kInt, dev);
+    return moe_topk_softmax_typed(logits, dtype, static_cast<float*>(w.data_ptr()),
+                                  static_cast<int32_t*>(ids.data_ptr()), static_cast<int32_t*>(tei.data_ptr()),
+                                  static_cast<int>(T), static_cast<int>(E), static_cast<int>(K), renormalize, stream);
+  }));
   return tuple_of(w, ids, tei);
   END_HANDLE_TH_ERRORS
 }
@@ -224,9 +249,15 @@ PyObject* rms_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (res && (res->device() != dev || res->scalar_type() != x->scalar_type() || res->sizes() != x->sizes() || !res->is_contiguous()))
     MOE_NONE;
   c10::OptionalDeviceGuard guard(dev);
-  const at::Tensor out = empty({T, H}, x->scalar_type(), dev);
-  check(moe_add_rms_norm(out.data_ptr(), H, res ? res->data_ptr() : nullptr, H, x->data_ptr(), H, w->data_ptr(), dtype, T,
-                         static_cast<int>(H), eps, current_stream(dev)));
+  void* const stream = current_stream(dev);
+  void* const r = res ? res->data_ptr() : nullptr;
+  const void *const in = x->data_ptr(), *const weight = w->data_ptr();
+  const at::ScalarType type = x->scalar_type();
+  at::Tensor out;
+  check(enqueue([&] {
+    out = empty({T, H}, type, dev);
+    return moe_add_rms_norm(out.data_ptr(), H, r, H, in, H, weight, dtype, T, static_cast<int>(H), eps, stream);
+  }));
   return THPVariable_Wrap(out);
   END_HANDLE_TH_ERRORS
 }
@@ -248,11 +279,16 @@ PyObject* gate_topk(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if ((dtype != MOE_BF16 && dtype != MOE_F16) || (E != 32 && E != 64 && E != 128) || H % 64) MOE_NONE;
   if ((reinterpret_cast<uintptr_t>(x->data_ptr()) | reinterpret_cast<uintptr_t>(g->data_ptr())) & 15u) MOE_NONE;
   c10::OptionalDeviceGuard guard(dev);
-  const at::Tensor w = empty({T, K}, at::kFloat, dev), ids = empty({T, K}, at::kInt, dev), tei = empty({T, K}, at::kInt, dev);
-  check(moe_gate_topk_softmax(x->data_ptr(), g->data_ptr(), dtype, nullptr, static_cast<float*>(w.data_ptr()),
-                              static_cast<int32_t*>(ids.data_ptr()), static_cast<int32_t*>(tei.data_ptr()),
-                              static_cast<int>(T), static_cast<int>(H), static_cast<int>(E), static_cast<int>(K),
-                              renormalize, current_stream(dev)));
+  void* const stream = current_stream(dev);
+  const void *const in = x->data_ptr(), *const gate = g->data_ptr();
+  at::Tensor w, ids, tei;
+  check(enqueue([&] {
+    w = empty({T, K}, at::kFloat, dev), ids = empty({T, K}, at::kInt, dev), tei = empty({T, K}, at::kInt, dev);
+    return moe_gate_topk_softmax(in, gate, dtype, nullptr, static_cast<float*>(w.data_ptr()),
+                                 static_cast<int32_t*>(ids.data_ptr()), static_cast<int32_t*>(tei.data_ptr()),
+                                 static_cast<int>(T), static_cast<int>(H), static_cast<int>(E), static_cast<int>(K),
+                                 renormalize, stream);
+  }));
   return tuple_of(w, ids, tei);
   END_HANDLE_TH_ERRORS
 }

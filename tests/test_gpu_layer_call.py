@@ -1,4 +1,7 @@
 """The layer as one call into native code: the same results as its steps, and the kernels it picks by the sizes."""
+import sys
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -104,3 +107,60 @@ def test_arguments_are_converted_or_refused_as_python_does(moe, dev):
     with pytest.raises(TypeError):
         norm(x, res)
     assert torch.equal(res, x)
+
+
+@pytest.mark.parametrize("call", ["layer", "topk", "norm", "gate"])
+def test_other_python_threads_run_during_a_call(moe, dev, call):
+    """With a switch interval of minutes a thread gets the interpreter only when the other gives it up: the calls
+    have to.  (A release of microseconds may pass before the waiting thread is awake, hence the many
+    calls; their results are kept, because torch gives the interpreter up where it frees a tensor.)"""
+    x = torch.zeros(2048, 64, dtype=torch.bfloat16, device=dev)
+    logits = torch.zeros(2048, 32, dtype=torch.bfloat16, device=dev)
+    w13, w2 = (torch.zeros(32, n, k, dtype=torch.bfloat16, device=dev) for n, k in ((64, 64), (64, 32)))
+    norm = moe.RMSNorm(64).bfloat16().to(dev)
+    run = {"layer": lambda: moe.fused_topk_experts(x[:1], logits[:1], w13, w2, 2, True),
+           "topk": lambda: moe.fused_topk(x, logits, 2, True),
+           "norm": lambda: norm(x),
+           "gate": lambda: moe.fused_gate_topk(x, x[:32], 2, True)}[call]
+    native = {"layer": "layer", "topk": "topk", "norm": "rms_norm", "gate": "gate_topk"}[call]
+    args = []
+    host = moe._lib.host()
+
+    class Recorder:   # the arguments of the native call, so that the loop below makes nothing but that call
+        def __getattr__(self, name):
+            def f(*a):
+                args.append((name, a))
+                return getattr(host, name)(*a)
+            return f
+
+    own = moe._lib.host
+    moe._lib.host = lambda: Recorder()
+    try:
+        run()
+    finally:
+        moe._lib.host = own
+    a = next(a for name, a in args if name == native)
+    enter = getattr(host, native)
+    assert enter(*a) is not None
+    torch.cuda.synchronize()
+    ran, go = [], threading.Event()
+
+    def other():
+        go.wait()
+        ran.append(1)
+
+    interval = sys.getswitchinterval()
+    thread = threading.Thread(target=other)
+    thread.start()
+    sys.setswitchinterval(600.0)
+    try:
+        go.set()
+        results = []
+        for _ in range(10000):
+            results.append(enter(*a))
+            if ran:
+                break
+    finally:
+        sys.setswitchinterval(interval)
+    assert ran
+    thread.join()
