@@ -268,8 +268,8 @@ typedef struct MoeLayerArgs {
   int32_t weight_layout;
   void* stream;
 } MoeLayerArgs;
-/* Workspace of a call with these arguments (pointers other than null / non-null do not matter, except
- * that tensors of a 16-bit or e4m3 call that are not 16-byte aligned choose other kernels). */
+/* Workspace of a call with these arguments, by the sizes, dtypes and block_size; of the pointers only whether
+ * router_logits is NULL matters. */
 int64_t moe_layer_workspace_bytes(const MoeLayerArgs* args);
 int moe_layer(const MoeLayerArgs* args);
 

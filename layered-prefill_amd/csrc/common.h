@@ -114,19 +114,6 @@ __device__ __forceinline__ float moe_expf(float x) {
   return __uint_as_float(__float_as_uint(p) + (static_cast<uint32_t>(ni) << 23));
 }
 
-// Two fp32 values -> OCP e4m3fn codes (bits 0-7 the code of a, bits 8-15 the code of b), saturating at
-// +-448, round to nearest even (v_cvt_pk_fp8_f32 produces the OCP encoding on gfx950).
-__device__ __forceinline__ uint32_t moe_f32x2_to_e4m3(float a, float b) {
-  a = __builtin_amdgcn_fmed3f(a, -448.f, 448.f);
-  b = __builtin_amdgcn_fmed3f(b, -448.f, 448.f);
-  return static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false)) & 0xffffu;
-}
-
-// Smallest e4m3 row scale: a row whose largest magnitude is tiny but not zero would get
-// a scale whose reciprocal overflows (amax below about 1.3e-36); from 2^-100 down
-// the scale stays 2^-100 and the row's codes are simply small.
-constexpr float kMoeMinE4m3Scale = 7.888609052210118e-31f;  // 2^-100
-
 __device__ __forceinline__ float moe_silu(float x) { return x / (1.0f + moe_expf(-x)); }
 
 __device__ __forceinline__ float moe_swigluoai(float g, float u, float alpha, float limit) {
