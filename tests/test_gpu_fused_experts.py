@@ -31,9 +31,11 @@ def _mode(moe, T, E, K, H, dtype, fp8=False, bm=None, activation="silu"):
     large-tile kernel (alignment blocks that are multiples of 256 slots, reduction
     length of the gate-up pass a multiple of its K tile: 64 elements of 16 bits, 128
     of e4m3) forms silu(gate) * up on its fp32 accumulators and rounds the
-    intermediate once (``mirror_rounding="fused"``); every other kernel, and the
-    large-tile kernel with the other activations, rounds at every store the
-    reference has (``True``)."""
+    intermediate once (``mirror_rounding="fused"``), and so does the streaming kernel
+    where the library picks it for a narrow layer in place of the large tile (the
+    width is left out here, so ``bm`` is then the large tile's); every other kernel,
+    and these with the other activations, rounds at every store the reference has
+    (``True``)."""
     if bm is None:
         bm = moe.fused_moe.try_get_optimal_moe_config(
             (E, 0, H), (E, H, 0), K, "fp8_w8a8" if fp8 else None, min(T, 65536), act_dtype=dtype)["BLOCK_SIZE_M"]

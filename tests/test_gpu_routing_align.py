@@ -404,6 +404,13 @@ def test_planned_alignment_leaves_the_plan_of_the_plan_kernel(moe, oracle, dev, 
     assert int((bounds[1:] - bounds[:-1]).max()) <= cap_mb
 
 
+@pytest.mark.parametrize("T,E,K", [(1, 128, 8), (512, 128, 8), (513, 128, 8), (741, 128, 8), (1024, 128, 8), (1025, 128, 8),
+                                   (4096, 1, 1), (4097, 1, 1), (2048, 256, 4), (2049, 256, 4), (100, 257, 4)])
+def test_planned_alignment_of_a_small_batch(moe, oracle, dev, T, E, K):
+    """The same check on both sides of 4096 and 8192 ids and of 256 experts, where the kernel changes."""
+    test_planned_alignment_leaves_the_plan_of_the_plan_kernel(moe, oracle, dev, T, E, K, E > 1)
+
+
 @pytest.mark.parametrize("E,K", [(128, 8), (8, 2), (256, 6), (64, 1), (16, 16)])
 @pytest.mark.parametrize("T", [1, 7, 20, 32])
 @pytest.mark.parametrize("bm,renorm", [(32, True), (256, True), (64, False)])
@@ -446,8 +453,8 @@ def test_route_align_rejects_what_it_does_not_serve(moe, dev):
 @pytest.mark.parametrize("layout", ["plain", "tiled"])
 @pytest.mark.parametrize("E,K", [(128, 8), (4, 4)])   # (4, 4) at 32 tokens: blocks of 256, the alignment also plans
 def test_fused_topk_experts_equals_the_two_calls(moe, dev, T, layout, E, K):
-    """``fused_topk_experts`` (routing + alignment in one launch up to 32 tokens, the two
-    calls beyond) gives the bits of ``fused_topk`` followed by ``fused_experts``."""
+    """``fused_topk_experts`` (one entry into native code) gives the bits of ``fused_topk``
+    followed by ``fused_experts``."""
     H, I = 512, 256
     g = torch.Generator().manual_seed(T)
     x = torch.randn(T, H, generator=g).bfloat16().to(dev)
@@ -467,9 +474,9 @@ def test_fused_topk_experts_equals_the_two_calls(moe, dev, T, layout, E, K):
 
 
 def test_fused_topk_experts_inside_a_hip_graph(moe, dev):
-    """A call made while the stream is captured enqueues the two kernels (routing, alignment)
-    instead of the one launch; every replay gives the bits of the eager call, with eager
-    work and synchronisations of the program's own between the replays."""
+    """A call made while the stream is captured enqueues the same kernels as an eager one; every
+    replay gives the bits of the eager call, with eager work and synchronisations of the
+    program's own between the replays."""
     T, H, I, E, K = 16, 512, 256, 128, 8
     g = torch.Generator().manual_seed(16)
     x = torch.randn(T, H, generator=g).bfloat16().to(dev)

@@ -319,3 +319,40 @@ def test_layer_without_weights_says_so(moe):
     quantised = moe.FusedMoE(4, 2, 32, 16, params_dtype=torch.bfloat16, quantization="fp8_e4m3")
     with pytest.raises(RuntimeError, match="before process_weights_after_loading"):
         quantised(torch.zeros(3, 32, dtype=torch.bfloat16), torch.zeros(3, 4))
+
+
+def test_layer_struct_layout_matches_header(moe):
+    text = open(os.path.join(ROOT, "include", "moe_gfx950.h")).read()
+    body = text[text.index("typedef struct MoeLayerArgs {") + len("typedef struct MoeLayerArgs {"):text.index("} MoeLayerArgs;")]
+    body = re.sub(r"/\*.*?\*/", "", body, flags=re.S)
+    names = [n.split()[-1].lstrip("*") for decl in body.split(";") if decl.strip() for n in decl.split(",")]
+    assert names == [f[0] for f in moe._lib.MoeLayerArgs._fields_]
+
+
+def test_layer_entry_rejects_bad_calls_without_a_gpu(moe):
+    """The C entry of the whole layer checks its sizes, pointers and workspace in front of any launch."""
+    L, A = moe._lib.lib(), moe._lib.MoeLayerArgs
+    sizes = dict(T=64, H=256, I=128, E=16, K=4, act_dtype=2, weight_dtype=2, logits_dtype=2, w13_stride_e=2 * 128 * 256,
+                 w13_stride_n=256, w2_stride_e=256 * 128, w2_stride_n=128)
+    tensors = {n: 1 << 20 for n in ("x", "out", "w13", "w2", "router_logits")}   # never followed
+    assert L.moe_layer(None) == -1 and L.moe_layer_workspace_bytes(None) == 0
+    assert L.moe_layer(A(**{**sizes, "T": 0})) == 0 and L.moe_layer_workspace_bytes(A(**{**sizes, "T": 0})) == 0
+    for bad in (dict(T=-1), dict(H=0), dict(E=0), dict(K=0), dict(T=1 << 30), dict(block_size=-1)):
+        assert L.moe_layer(A(**{**sizes, **tensors, **bad})) == -1
+        assert L.moe_layer_workspace_bytes(A(**{**sizes, **tensors, **bad})) == 0
+    for name in ("x", "out", "w13", "w2"):
+        assert L.moe_layer(A(**{**sizes, **tensors, name: None})) == -1 and b"null" in L.moe_last_error()
+    assert L.moe_layer(A(**{**sizes, **tensors, "router_logits": None})) == -1 and b"topk_ids" in L.moe_last_error()
+    need = L.moe_layer_workspace_bytes(A(**sizes, **tensors))
+    # without logits the routing's weights and ids come from the caller
+    assert need - L.moe_layer_workspace_bytes(A(**{**sizes, **tensors, "router_logits": None})) == 2 * 64 * 4 * 4
+    # x's place does not matter, the block size does
+    assert L.moe_layer_workspace_bytes(A(**{**sizes, **tensors, "x": (1 << 20) + 2})) == need
+    assert L.moe_layer_workspace_bytes(A(**sizes, **tensors, block_size=256)) > need
+    assert L.moe_layer(A(**sizes, **tensors)) == -3
+    assert L.moe_layer(A(**sizes, **tensors, workspace=1 << 20, workspace_bytes=need - 1)) == -3
+    assert L.moe_layer(A(**sizes, **tensors, workspace=(1 << 20) + 128, workspace_bytes=need)) == -3
+    assert b"256-byte" in L.moe_last_error()
+    assert L.moe_topk_softmax_typed(None, 2, None, None, None, 4, 8, 9, 0, None) == -1
+    assert L.moe_topk_softmax_typed(1 << 20, 3, 1 << 20, 1 << 20, None, 4, 8, 2, 0, None) == -1
+    assert b"dtype code 3" in L.moe_last_error()
