@@ -25,9 +25,10 @@ constexpr int kMaxExperts = 1024;
 // side in about 6 us (one CU's instruction throughput: a row is ~750 instructions), and every further
 // 32 rows cost as much again, while the stand-alone router spreads its rows over the whole chip:
 // measured on the Qwen3-30B-A3B router (128 experts, top-8), launches included, 14.8 us against
-// 17.7 us for the two kernels at 32 rows, 21.0 against 17.6 at 64, 59.7 against 17.2 at 256.
-// What it saves at 32 rows is host time only: replayed from a HIP graph the one launch takes 14.7 us
-// and the two kernels 13.2 us (they follow each other within about a microsecond).  Spreading the
+// 17.7 us for the router and align_small_kernel at 32 rows, 21.0 against 17.6 at 64, 59.7 against 17.2 at 256.
+// What it saves is a launch from Python, not GPU time: 14.4 us against 5.9 + 4.3 us of the router and
+// align_tiny_kernel, which the layer's call enqueues from native code (they follow each other within about a
+// microsecond).  Spreading the
 // routing over several workgroups and letting the last one to finish align (release fence, arrival
 // counter, acquire fence) cost 4.5 us more than the two kernels from 64 to 256 rows.
 constexpr int kRouteAlignMaxTokens = 32;
