@@ -25,6 +25,7 @@ namespace {
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 struct MmaBF16 {
   using El = ElemBF16;
@@ -37,6 +38,10 @@ struct MmaBF16 {
   static __device__ __forceinline__ f32x16 mma_big(const uint4 (&a)[1], const uint4 (&b)[1], f32x16 c) {
     return mma(a[0], b[0], c);
   }
+  // 16 x 16, four 16-byte chunks of a row (lane / 16 says which of them a lane holds)
+  static __device__ __forceinline__ f32x4 mma16(const uint4& a, const uint4& b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  }
 };
 struct MmaF16 {
   using El = ElemF16;
@@ -48,6 +53,9 @@ struct MmaF16 {
   }
   static __device__ __forceinline__ f32x16 mma_big(const uint4 (&a)[1], const uint4 (&b)[1], f32x16 c) {
     return mma(a[0], b[0], c);
+  }
+  static __device__ __forceinline__ f32x4 mma16(const uint4& a, const uint4& b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
   }
 };
 
@@ -78,6 +86,14 @@ struct MmaE4M3 {
     const long b1 = static_cast<long>(b.z) | (static_cast<long>(b.w) << 32);
     c = __builtin_amdgcn_mfma_f32_32x32x16_fp8_fp8(a0, b0, c, 0, 0, 0);
     return __builtin_amdgcn_mfma_f32_32x32x16_fp8_fp8(a1, b1, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ f32x4 mma16(const uint4& a, const uint4& b, f32x4 c) {
+    const long a0 = static_cast<long>(a.x) | (static_cast<long>(a.y) << 32);
+    const long a1 = static_cast<long>(a.z) | (static_cast<long>(a.w) << 32);
+    const long b0 = static_cast<long>(b.x) | (static_cast<long>(b.y) << 32);
+    const long b1 = static_cast<long>(b.z) | (static_cast<long>(b.w) << 32);
+    c = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(a0, b0, c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(a1, b1, c, 0, 0, 0);
   }
 };
 
@@ -161,16 +177,14 @@ __device__ __forceinline__ int swizzled(int row, int chunk) {
 // Rounding follows the reference's storage points: the GEMM result is rounded to
 // the activation dtype, silu is rounded, the product is rounded
 // (nanovllm/layers/for_moe/fused_moe.py:216, csrc/activation_kernels.cu:11,23).
-// SCALED: e4m3 accumulators still carry the operands' scales here (p.a_scale, p.w_scale).
-// ONCE: with SiLU, silu(gate) * up is rounded once.
-template <typename El, bool GATED, bool SCALED = true, bool ONCE = false>
+template <typename El, bool GATED>
 __device__ __forceinline__ void store_fragment(const GemmParams& p, int e, const f32x16& ga,
                                                const f32x16& ua, int tok, int slot, int ncol0, float rw) {
   using S = typename El::S;
   const S* bias = static_cast<const S*>(p.bias);
   // fp8: the accumulator is in units of (activation scale x weight scale)
-  const float as = SCALED && p.a_scale ? p.a_scale[p.a_by_slot ? slot : tok / p.top_k] : 1.f;
-  const float* ws = SCALED && p.w_scale ? p.w_scale + e * p.w_scale_stride_e : nullptr;
+  const float as = p.a_scale ? p.a_scale[p.a_by_slot ? slot : tok / p.top_k] : 1.f;
+  const float* ws = p.w_scale ? p.w_scale + e * p.w_scale_stride_e : nullptr;
   const int64_t crow = p.a_by_slot ? tok : slot;  // pass 2 writes by token, pass 1 by slot
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
@@ -192,10 +206,6 @@ __device__ __forceinline__ void store_fragment(const GemmParams& p, int e, const
           uv += El::ld(bias[e * p.bias_stride_e + urow]);
         }
         if (p.mul_weight) { gv *= rw; uv *= rw; }
-        if constexpr (ONCE) {
-          o[i] = El::st(moe_silu(gv) * uv);
-          continue;
-        }
         gv = El::ld(El::st(gv));
         uv = El::ld(El::st(uv));
         float r;
@@ -1425,49 +1435,31 @@ __global__ __launch_bounds__(kPlanThreads) void big_plan_kernel(const int32_t* _
   }
 }
 
-// Epilogue of the streaming kernel for full, aligned 16-bit tiles: same storage
-// points as store_fragment, with the hardware conversions and the fast SiLU of
-// the large-tile epilogue (one wavefront finishes the whole tile, so the
-// instruction count is the epilogue's latency).  ONCE (SiLU): gate and up are the
-// same accumulator element of two fragments, and silu(gate) * up is formed on the
-// fp32 values and rounded once, as the large-tile epilogue does.
+// What a lane of the streaming kernel computed for one token: gate and up of columns n and n + 1 (v = g0, g1, u0,
+// u1), or columns n .. n + 3.  Same storage points as store_fragment, with the hardware conversions and the fast
+// SiLU of the large-tile epilogue.  ONCE (SiLU): silu(gate) * up is formed on the fp32 values and rounded once, as
+// the large-tile epilogue does.
 template <typename El, bool GATED, int ACT, bool ONCE = false>
-__device__ __forceinline__ void stream_store(const GemmParams& p, int e, const f32x16& ga, const f32x16& ua,
-                                             int tok, int slot, int ncol0, float rw) {
+__device__ __forceinline__ void stream_store(const GemmParams& p, const float (&v)[4], int64_t crow, int n) {
   using S = typename El::S;
-  const S* bias = static_cast<const S*>(p.bias);
-  const int64_t crow = p.a_by_slot ? tok : slot;
+  constexpr int COLS = GATED ? 2 : 4;
+  uint32_t out[2];
+  if constexpr (!GATED) {
+    out[0] = pack2<El>(v[0], v[1]);
+    out[1] = pack2<El>(v[2], v[3]);
+  } else if constexpr (ONCE) {
+    out[0] = pack2<El>(silu_fast(v[0]) * v[2], silu_fast(v[1]) * v[3]);
+  } else {
+    out[0] = gated_pair<El, ACT>(p, pack2<El>(v[0], v[1]), pack2<El>(v[2], v[3]));
+  }
+  S* dst = static_cast<S*>(p.c) + crow * p.ldc + n;
+  if (n + COLS <= p.N && p.ldc % COLS == 0) {
+    if constexpr (GATED) *reinterpret_cast<uint32_t*>(dst) = out[0];
+    else *reinterpret_cast<uint2*>(dst) = uint2{out[0], out[1]};
+  } else {
 #pragma unroll
-  for (int g = 0; g < 4; ++g) {
-    const int n = ncol0 + 8 * g;
-    float gv[4], uv[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      gv[i] = ga[4 * g + i];
-      uv[i] = ua[4 * g + i];
-      if (bias) {
-        if constexpr (GATED) {
-          gv[i] += El::ld(bias[e * p.bias_stride_e + (p.interleaved ? 2 * (n + i) : n + i)]);
-          uv[i] += El::ld(bias[e * p.bias_stride_e + (p.interleaved ? 2 * (n + i) + 1 : p.N + n + i)]);
-        } else {
-          gv[i] += El::ld(bias[e * p.bias_stride_e + n + i]);
-        }
-      }
-      gv[i] *= rw;
-      uv[i] *= rw;
-    }
-    uint2 out;
-    if constexpr (ONCE) {
-      out.x = pack2<El>(silu_fast(gv[0]) * uv[0], silu_fast(gv[1]) * uv[1]);
-      out.y = pack2<El>(silu_fast(gv[2]) * uv[2], silu_fast(gv[3]) * uv[3]);
-    } else if constexpr (GATED) {
-      out.x = gated_pair<El, ACT>(p, pack2<El>(gv[0], gv[1]), pack2<El>(uv[0], uv[1]));
-      out.y = gated_pair<El, ACT>(p, pack2<El>(gv[2], gv[3]), pack2<El>(uv[2], uv[3]));
-    } else {
-      out.x = pack2<El>(gv[0], gv[1]);
-      out.y = pack2<El>(gv[2], gv[3]);
-    }
-    *reinterpret_cast<uint2*>(static_cast<S*>(p.c) + crow * p.ldc + n) = out;
+    for (int i = 0; i < COLS; ++i)
+      if (n + i < p.N) dst[i] = static_cast<S>(out[i >> 1] >> (16 * (i & 1)));
   }
 }
 
@@ -1482,14 +1474,24 @@ __device__ __forceinline__ void stream_store(const GemmParams& p, int e, const f
 // which keeps about 100 KB per CU on its way from HBM and hides a workgroup's
 // start-up and epilogue behind its neighbours' streams.  Small tiles (256 KB of
 // weights in the gate-up pass) also keep the last wave of workgroups short.
-// All four wavefronts issue DMA requests; the MFMA work of a 32-slot block is
-// so small (8 MFMAs per unit) that wavefront 0 does all of it.  Rows are laid
+// All four wavefronts issue DMA requests, and each multiplies 16 of the weight
+// rows (16x16 products, two per 16 tokens and unit), so that a unit's way through
+// the workgroup and the epilogue are short: they are what a call of few workgroups
+// and the first and last workgroups of any call wait for.  (One wavefront for all
+// rows: 0.29 us a unit and 0.9 to 1.5 us of epilogue, now 0.2 and 0.4.)  Both passes
+// of a 2048 x 128 x 768 top-8 layer, this way and with one wavefront: 18.7 and 20.2 us
+// at 1 token, 101.8 and 103.7 at 64, 124.9 and 129.0 at 128, 154.8 and 158.5 at 256.
+// Biases are fetched ahead of the stream, too: behind it they held every epilogue up (the whole call of 301 tokens,
+// 32 experts, I 1024, top-4, with biases: 146.4 -> 119.4 us).
+// Token rows of padding slots are not requested: in the down pass each slot has a row
+// of its own and they were up to a fifth of the pass's traffic (50.3 -> 47.8 us at 128 tokens).
+// Rows are laid
 // out in LDS like the large-tile kernel's (16-byte chunk c of row r at chunk
 // c ^ ((r >> 1) & 7)).  Everything the start-up reads is wavefront-uniform and
 // comes through the scalar cache, in two round trips.
-// e4m3 runs here too (100 tokens of a 2048 x 128 x 768 top-8 layer: gate-up 45.6 -> 40.1 us, down 40.9 -> 25.9 us
+// e4m3 runs here too (100 tokens of that layer: gate-up 45.6 -> 40.1 us, down 40.9 -> 25.9 us
 // against the register-staged kernel, whose two stages hold 36 KB per workgroup and drain at every K tile), its scales
-// fetched ahead of the stream like the routed weights.  Rows need whole 32-byte MFMA steps, not whole units.
+// fetched ahead of the stream like the routed weights.  Rows need whole 32-byte steps, not whole units.
 // ---------------------------------------------------------------------------
 constexpr int kStRowBytes = 128, kStRows = 64, kStUnits = 4, kStBM = 32;
 constexpr int kStWBytes = kStRows * kStRowBytes;               // 8 KB of weights per unit
@@ -1540,166 +1542,171 @@ __global__ __launch_bounds__(kThreads, 3) void stream_gemm_kernel(const GemmPara
   }
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int l32 = lane & 31, lhi = lane >> 5;
+  const int l15 = lane & 15, lq = lane >> 4;
   const int n0 = nt * BN_OUT;
 
-  // second round trip: the expert, and the eight slots whose token rows this wavefront requests
+  // second round trip: the expert, the slots of this lane's results (tokens lane % 16 and 16 + lane % 16 of the
+  // block) and the eight slots whose token rows this wavefront requests
   const int32_t* sid = p.sorted_ids + static_cast<int64_t>(mb) * kStBM;
+  int tok[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) tok[h] = sid[16 * h + l15];
   const int e = __builtin_amdgcn_readfirstlane(p.expert_ids[mb]);
   const int first = sid[0];
   const int4 s0 = *reinterpret_cast<const int4*>(sid + 8 * wave);
   const int4 s1 = *reinterpret_cast<const int4*>(sid + 8 * wave + 4);
   if (first >= p.numel) return;  // real slots come first: the block is empty
-  // What the epilogue needs per slot is fetched now, ahead of the stream: a load
+  // The lane's results: columns n_out and n_out + 1 (their gate and up rows), or n_out .. n_out + 3.
+  const int n_out = n0 + (GATED ? 8 * wave + 2 * lq : 16 * wave + 4 * lq);
+  auto result_row = [&](int i) {  // weight row behind accumulator element i
+    const int half = GATED ? i >> 1 : 0;
+    int n = n_out + (GATED ? i & 1 : i);
+    n = n < p.N ? n : p.N - 1;
+    return static_cast<int64_t>(!GATED ? n : p.interleaved ? 2 * n + half : half * p.N + n);
+  };
+  // What the epilogue needs per slot and per weight row is fetched now, ahead of the stream: a load
   // issued behind ~100 KB of queued DMA requests would take microseconds to return.
-  int tok = p.numel;
-  float rw = 1.f, as = 1.f, wsc = 1.f;
-  if (wave == 0) {
-    tok = sid[l32];
-    if (p.mul_weight && tok < p.numel) rw = p.topk_w[tok];
-    if constexpr (ES == 1) {
-      if (tok < p.numel) as = p.a_scale[p.a_by_slot ? mb * kStBM + l32 : tok / p.top_k];
-      // lane l holds the channel scale of the workgroup's weight row l
-      int n = n0 + (GATED ? l32 : lane);
-      n = n < p.N ? n : p.N - 1;
-      wsc = p.w_scale[e * p.w_scale_stride_e + (!GATED ? n : p.interleaved ? 2 * n + lhi : lhi * p.N + n)];
-    }
+  float rw[2] = {1.f, 1.f}, as[2] = {1.f, 1.f}, ws[4], bias[4];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    if (p.mul_weight && tok[h] < p.numel) rw[h] = p.topk_w[tok[h]];
+    if constexpr (ES == 1)
+      if (tok[h] < p.numel) as[h] = p.a_scale[p.a_by_slot ? mb * kStBM + 16 * h + l15 : tok[h] / p.top_k];
   }
+  if constexpr (ES == 1)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) ws[i] = p.w_scale[e * p.w_scale_stride_e + result_row(i)];
+  if (p.bias)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      bias[i] = El::ld(static_cast<const typename El::S*>(p.bias)[e * p.bias_stride_e + result_row(i)]);
 
   // DMA requests of this wavefront: token rows 8 * wave + lane / 8, weight rows
-  // 16 * wave + 8 * j + lane / 8 (j < 2); lane % 8 is the chunk the lane's 16 bytes land in
+  // 16 * wave + 8 * j + lane / 8 (j < 2); lane % 8 is the place the lane's 16 bytes land in.
   const char* a_base = static_cast<const char*>(p.a);
   const char* w_base = static_cast<const char*>(p.w) + static_cast<int64_t>(e) * p.w_stride_e * ES;
   int w_step = kStRowBytes;  // bytes from one K unit to the next
   uint32_t a_off, w_off[2];
+  bool a_live;   // lane 0 always: a request with no lane at all would not count
   {
     const int q = lane >> 3;
     const int rr = 8 * wave + q;
     int64_t src = mb * kStBM + rr;
-    if (!p.a_by_slot) {
-      const int lo = (q & 2) ? ((q & 1) ? s0.w : s0.z) : ((q & 1) ? s0.y : s0.x);
-      const int hi = (q & 2) ? ((q & 1) ? s1.w : s1.z) : ((q & 1) ? s1.y : s1.x);
-      const int tok = (q & 4) ? hi : lo;
-      src = tok < p.numel ? tok / p.top_k : 0;
-    }
+    const int lo = (q & 2) ? ((q & 1) ? s0.w : s0.z) : ((q & 1) ? s0.y : s0.x);
+    const int hi = (q & 2) ? ((q & 1) ? s1.w : s1.z) : ((q & 1) ? s1.y : s1.x);
+    const int slot_tok = (q & 4) ? hi : lo;
+    if (!p.a_by_slot) src = slot_tok < p.numel ? slot_tok / p.top_k : 0;
+    a_live = slot_tok < p.numel || lane == 0;
     a_off = static_cast<uint32_t>(src * p.lda * ES + (((lane & 7) ^ ((rr >> 1) & 7)) << 4));
   }
   const int row_bytes = p.Kd * ES;  // a multiple of 32
+  constexpr int kBigRows = GATED ? 128 : 256;  // output columns covered by one 32 KB unit of tiled weights
   if (p.w_tiled) {
     // Weights in 32 KB units of 256 rows (the large-tile kernel's): this workgroup's rows are one
-    // or two contiguous pieces of every unit of its n-tile, 32 rows apart from a multiple of 32,
-    // so a row's chunks already sit where this kernel's LDS rows want them.
-    constexpr int kBigRows = GATED ? 128 : 256;  // output columns covered by one unit
+    // or two contiguous pieces of every unit of its n-tile.
     w_base += static_cast<int64_t>(n0 / kBigRows) * (row_bytes / kStRowBytes) * 32768;
     w_step = 32768;
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int rr = 16 * wave + 8 * j + (lane >> 3);
-      const int R = GATED ? ((rr >> 5) * 128 + (n0 % kBigRows) + (rr & 31)) : ((n0 % kBigRows) + rr);
-      w_off[j] = static_cast<uint32_t>(R * kStRowBytes + ((lane & 7) << 4));
-    }
-  } else {
+  }
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
+    // LDS row rr: rows 0 .. 31 gate, 32 .. 63 up when gated.  The up rows sit eight places apart from their gate
+    // rows (modulo 16), so that the 16 rows that a wavefront reads together touch 16 distinct bank groups.
     const int rr = 16 * wave + 8 * j + (lane >> 3);
-    int64_t wrow;
-    if constexpr (GATED) {
-      const int half = rr >> 5;
-      int n = n0 + (rr & 31);
-      n = n < p.N ? n : p.N - 1;
-      wrow = p.interleaved ? (2 * n + half) : (half * p.N + n);
+    const int half = GATED ? rr >> 5 : 0, nl = !GATED ? rr : half ? (rr & 31) ^ 8 : rr & 31;
+    const int chunk = (lane & 7) ^ ((rr >> 1) & 7);   // the row's chunk that belongs there
+    if (p.w_tiled) {
+      const int R = half * 128 + n0 % kBigRows + nl;
+      w_off[j] = static_cast<uint32_t>(R * kStRowBytes + ((chunk ^ ((R >> 1) & 7)) << 4));
     } else {
-      const int n = n0 + rr;
-      wrow = n < p.N ? n : p.N - 1;
+      const int n = n0 + nl < p.N ? n0 + nl : p.N - 1;
+      const int64_t wrow = !GATED ? n : p.interleaved ? 2 * n + half : half * p.N + n;
+      w_off[j] = static_cast<uint32_t>(wrow * p.w_stride_n * ES + (chunk << 4));
     }
-    w_off[j] = static_cast<uint32_t>(wrow * p.w_stride_n * ES + (((lane & 7) ^ ((rr >> 1) & 7)) << 4));
-  }
   }
   const uint32_t lds0 = lds_offset_of(smem);
   const uint32_t dma_w = __builtin_amdgcn_readfirstlane(lds0 + 16 * wave * kStRowBytes);
   const uint32_t dma_a = __builtin_amdgcn_readfirstlane(lds0 + kStWBytes + 8 * wave * kStRowBytes);
   // TAIL (plain layout only): the last unit of a row holds `tail` bytes, 32 to 96.  A lane whose chunk lies
-  // behind the row's end fetches the unit's first chunk instead, and no MFMA step reads that place.  (As a
+  // behind the row's end fetches the unit's first chunk instead, and the product takes zeros in that place.  (As a
   // run-time branch this cost the rows of whole units 2 %.)
   const int nu = TAIL ? row_bytes / kStRowBytes + 1 : row_bytes / kStRowBytes;
   const int tail = row_bytes & (kStRowBytes - 1);
   auto issue = [&](int u) {
     const uint32_t ring = (u % kStUnits) * kStUnitBytes;
+    uint32_t a = a_off, w[2] = {w_off[0], w_off[1]};
     if (TAIL && u == nu - 1) {
       const uint32_t ca = ((lane & 7) ^ (((8 * wave + (lane >> 3)) >> 1) & 7)) << 4;
-      const uint32_t back_a = static_cast<int>(ca) < tail ? 0u : ca;
-      lds_dma16(a_base + u * kStRowBytes, a_off - back_a, dma_a + ring);
+      a -= static_cast<int>(ca) < tail ? 0u : ca;
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         const uint32_t cw = ((lane & 7) ^ (((16 * wave + 8 * j + (lane >> 3)) >> 1) & 7)) << 4;
-        const uint32_t back_w = static_cast<int>(cw) < tail ? 0u : cw;
-        lds_dma16(w_base + static_cast<int64_t>(u) * w_step, w_off[j] - back_w, dma_w + ring + j * 1024);
+        w[j] -= static_cast<int>(cw) < tail ? 0u : cw;
       }
-      return;
     }
-    lds_dma16(a_base + u * kStRowBytes, a_off, dma_a + ring);
+    if (a_live) lds_dma16(a_base + u * kStRowBytes, a, dma_a + ring);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) lds_dma16(w_base + static_cast<int64_t>(u) * w_step, w_off[j], dma_w + ring + j * 1024);
+    for (int j = 0; j < 2; ++j) lds_dma16(w_base + static_cast<int64_t>(u) * w_step, w[j], dma_w + ring + j * 1024);
   };
 
-  f32x16 acc0, acc1;
+  // Fragments: row lane % 16, chunk 4 * kk + lane / 16 of step kk.  Accumulator element i of a lane is weight row
+  // 4 * (lane / 16) + i of the wavefront's sixteen, token lane % 16: gated rows are ordered g, g + 1, u, u + 1.
+  f32x4 acc[2];
 #pragma unroll
-  for (int r = 0; r < 16; ++r) { acc0[r] = 0.f; acc1[r] = 0.f; }
-  int rd_k[4];
+  for (int h = 0; h < 2; ++h)
 #pragma unroll
-  for (int kk = 0; kk < 4; ++kk) rd_k[kk] = l32 * kStRowBytes + (((2 * kk + lhi) ^ ((l32 >> 1) & 7)) << 4);
+    for (int r = 0; r < 4; ++r) acc[h][r] = 0.f;
+  int rd_w[2], rd_x[2];
+  {
+    const int col = 8 * wave + 2 * (l15 >> 2) + (l15 & 1);
+    const int row = !GATED ? 16 * wave + l15 : (l15 & 2) ? 32 + (col ^ 8) : col;
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      rd_w[kk] = row * kStRowBytes + (((4 * kk + lq) ^ ((row >> 1) & 7)) << 4);
+      rd_x[kk] = kStWBytes + l15 * kStRowBytes + (((4 * kk + lq) ^ ((l15 >> 1) & 7)) << 4);
+    }
+  }
 
   issue(0);
   if (1 < nu) issue(1);
   if (2 < nu) issue(2);
   for (int u = 0; u < nu; ++u) {
-    // unit u has landed (only the two younger units may be outstanding) and
-    // wavefront 0 is done reading unit u-1, whose ring slot the next request reuses
+    // unit u has landed (only the two younger units may be outstanding) and nobody
+    // reads unit u-1 any more, whose ring slot the next request reuses
     if (u + 2 < nu) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(2 * kStDmaPerUnit) : "memory");
     else if (u + 1 < nu) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kStDmaPerUnit) : "memory");
     else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     bare_barrier();
     if (u + 3 < nu) issue(u + 3);
-    if (wave == 0) {
-      const char* st = smem + (u % kStUnits) * kStUnitBytes;
-      const int steps = TAIL && u == nu - 1 ? tail >> 5 : 4;
+    const char* st = smem + (u % kStUnits) * kStUnitBytes;
+    uint4 w[2], x[2][2];
 #pragma unroll
-      for (int kk = 0; kk < 4; ++kk) {
-        if (kk >= steps) break;
-        const uint4 x = *reinterpret_cast<const uint4*>(st + kStWBytes + rd_k[kk]);
-        const uint4 w0 = *reinterpret_cast<const uint4*>(st + rd_k[kk]);
-        const uint4 w1 = *reinterpret_cast<const uint4*>(st + 32 * kStRowBytes + rd_k[kk]);
-        acc0 = Mma::mma(w0, x, acc0);
-        acc1 = Mma::mma(w1, x, acc1);
-      }
+    for (int kk = 0; kk < 2; ++kk) {
+      w[kk] = *reinterpret_cast<const uint4*>(st + rd_w[kk]);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) x[kk][h] = *reinterpret_cast<const uint4*>(st + rd_x[kk] + h * 16 * kStRowBytes);
+      if (TAIL && u == nu - 1 && (4 * kk + lq) * 16 >= tail) w[kk] = x[kk][0] = x[kk][1] = uint4{0, 0, 0, 0};
     }
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) acc[h] = Mma::mma16(w[kk], x[kk][h], acc[h]);
   }
 
-  if (wave != 0) return;
-  if constexpr (ES == 1) {  // the accumulators back to the units of x . w
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int row = 8 * (r >> 2) + 4 * lhi + (r & 3);
-      acc0[r] *= as * __shfl(wsc, row, kWave);
-      acc1[r] *= as * __shfl(wsc, row + 32, kWave);
+  for (int h = 0; h < 2; ++h) {
+    if (tok[h] >= p.numel) continue;
+    float v[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      v[i] = acc[h][i];
+      if constexpr (ES == 1) v[i] *= as[h] * ws[i];  // the accumulators back to the units of x . w
+      if (p.bias) v[i] += bias[i];
+      v[i] *= rw[h];
     }
-  }
-  const int slot = mb * kStBM + l32;
-  if (tok < p.numel) {
-    const bool fast = n0 + BN_OUT <= p.N && (p.ldc & 3) == 0;
-    if constexpr (GATED) {
-      if (!fast) store_fragment<El, true, false, ONCE>(p, e, acc0, acc1, tok, slot, n0 + 4 * lhi, rw);
-      else if (ONCE) stream_store<El, true, MOE_ACT_SILU, true>(p, e, acc0, acc1, tok, slot, n0 + 4 * lhi, rw);
-      else if (p.activation == MOE_ACT_SILU) stream_store<El, true, MOE_ACT_SILU>(p, e, acc0, acc1, tok, slot, n0 + 4 * lhi, rw);
-      else if (p.activation == MOE_ACT_SWIGLUOAI) stream_store<El, true, MOE_ACT_SWIGLUOAI>(p, e, acc0, acc1, tok, slot, n0 + 4 * lhi, rw);
-      else stream_store<El, true, MOE_ACT_GELU>(p, e, acc0, acc1, tok, slot, n0 + 4 * lhi, rw);
-    } else if (fast) {
-      stream_store<El, false, 0>(p, e, acc0, acc0, tok, slot, n0 + 4 * lhi, rw);
-      stream_store<El, false, 0>(p, e, acc1, acc1, tok, slot, n0 + 32 + 4 * lhi, rw);
-    } else {
-      store_fragment<El, false, false>(p, e, acc0, acc0, tok, slot, n0 + 4 * lhi, rw);
-      store_fragment<El, false, false>(p, e, acc1, acc1, tok, slot, n0 + 32 + 4 * lhi, rw);
-    }
+    const int64_t crow = p.a_by_slot ? tok[h] : mb * kStBM + 16 * h + l15;
+    if (!GATED || ONCE || p.activation == MOE_ACT_SILU) stream_store<El, GATED, MOE_ACT_SILU, ONCE>(p, v, crow, n_out);
+    else if (p.activation == MOE_ACT_SWIGLUOAI) stream_store<El, GATED, MOE_ACT_SWIGLUOAI>(p, v, crow, n_out);
+    else stream_store<El, GATED, MOE_ACT_GELU>(p, v, crow, n_out);
   }
 }
 
