@@ -528,6 +528,15 @@ __device__ __forceinline__ uint32_t pack2<ElemF16>(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, f16x2));
 }
 
+// The lane number, computed where it stands: what is derived from it before and after the large-tile main loop is
+// not the same value to the compiler, which would otherwise keep it, and every address made of it, in registers
+// that the loop's 256 accumulators do not leave.
+__device__ __forceinline__ int fresh_lane() {
+  int zero = 0;
+  asm volatile("" : "+s"(zero));
+  return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, zero));
+}
+
 struct BigCtx {
   const char* a_base;   // wave-uniform base of the A rows
   const char* w_base;   // wave-uniform base of this expert's weights
@@ -536,7 +545,7 @@ struct BigCtx {
   uint32_t dma_lds;     // LDS address of the middle of this wavefront's 8 KB DMA window in unit slot 0
   uint32_t dma_lds_light_a;  // the same for the 2 KB window of the first 64-row token unit of a weight-streaming tile
   int rd_k[4];          // fragment read offsets for the four MFMA steps of a K tile
-  int x_row;            // byte offset of this wavefront's first token row in a token unit
+  int x_row;            // byte offset of this wavefront's first token fragment in a token unit
   int w_row[4];         // byte offsets of this wavefront's weight fragments in a weight unit
   int a_step, w_step;   // bytes from one K tile to the next: 128 along a row, 32768 from unit to unit
 };
@@ -586,6 +595,12 @@ __device__ __forceinline__ void lds_dma16_win(const char* base, uint32_t lane_by
 // the offset field's share taken out again, and 4096 that the base pointers are short of (so that
 // no offset is negative).
 constexpr uint32_t dma_win_bias(int j) { return static_cast<uint32_t>(4096 - (j - 4) * 1024); }
+
+// The 32-row token fragments of a block go to the two halves of the wavefronts in turn (wavefront half wm has
+// fragments wm, wm + 2, ..), so that a partly filled block, whose fragments without a real slot are skipped, keeps
+// both halves busy: with the first 128 rows in one half and the rest in the other, a block of 128 rows took as
+// long as one of 256.
+constexpr int kFragStep = 2 * 32 * kBigRowBytes;
 
 // Main loop for a wavefront that has FMC live token fragments (0..4).
 // Unit j of the stream  A(0) W(0) A(1) W(1) ...  lives in ring slot j % 5.
@@ -643,7 +658,7 @@ __device__ __forceinline__ void big_mainloop(const BigCtx& c, const char* smem, 
           const char* stw = smem + (yw + wl[YKK * CH + ch]);
           if constexpr (r == 0) xfY[0][ch] = *reinterpret_cast<const uint4*>(sta);
           else if constexpr (r <= 4) wfY[r - 1][ch] = *reinterpret_cast<const uint4*>(stw + woff(r - 1));
-          else if constexpr (r - 4 < FMC) xfY[r - 4][ch] = *reinterpret_cast<const uint4*>(sta + (r - 4) * 4096);
+          else if constexpr (r - 4 < FMC) xfY[r - 4][ch] = *reinterpret_cast<const uint4*>(sta + (r - 4) * kFragStep);
         }
       }
     };
@@ -736,7 +751,7 @@ __device__ __forceinline__ void big_mainloop(const BigCtx& c, const char* smem, 
 #pragma unroll
       for (int fn = 0; fn < 4; ++fn) wfP[fn][ch] = *reinterpret_cast<const uint4*>(stw + woff(fn));
 #pragma unroll
-      for (int fm = 0; fm < FMC; ++fm) xfP[fm][ch] = *reinterpret_cast<const uint4*>(sta + fm * 4096);
+      for (int fm = 0; fm < FMC; ++fm) xfP[fm][ch] = *reinterpret_cast<const uint4*>(sta + fm * kFragStep);
     }
   }
   __builtin_amdgcn_sched_barrier(0);
@@ -758,7 +773,7 @@ __device__ __forceinline__ void big_mainloop(const BigCtx& c, const char* smem, 
 template <typename Mma, int FMC>
 __device__ __forceinline__ void big_light_mainloop(const BigCtx& c, const char* smem, int nk,
                                                    f32x16 (&acc)[4][4]) {
-  static_assert(FMC <= 2, "at most 64 token rows");
+  static_assert(FMC <= 1, "at most 64 token rows: one fragment for each half of the wavefronts");
   constexpr int CH = Mma::kBigChunks, STEPS = 4 / CH;
   constexpr int kTokUnit = 2 * 4096;  // 64 rows
   auto w_slot = [](int k) {
@@ -816,7 +831,7 @@ __device__ __forceinline__ void big_light_mainloop(const BigCtx& c, const char* 
         for (int ch = 0; ch < CH; ++ch) {
 #pragma unroll
           for (int fm = 0; fm < FMC; ++fm)
-            xf[fm][ch] = *reinterpret_cast<const uint4*>(sa + fm * 32 * kBigRowBytes + c.rd_k[kk * CH + ch]);
+            xf[fm][ch] = *reinterpret_cast<const uint4*>(sa + c.x_row + c.rd_k[kk * CH + ch]);
 #pragma unroll
           for (int fn = 0; fn < 4; ++fn)
             wf[fn][ch] = *reinterpret_cast<const uint4*>(sw + c.w_row[fn] + c.rd_k[kk * CH + ch]);
@@ -873,9 +888,9 @@ __device__ __forceinline__ uint32_t gated_pair(const GemmParams& p, uint32_t gw,
 // The other activations park gate and up rounded, as the stand-alone activation
 // kernels see them, and the flush combines them.
 template <typename El, int FMC, bool GATED, bool SCALED, bool BIAS, bool FAST_SILU>
-__device__ __forceinline__ void big_park(const GemmParams& p, int e, int n0, int wn, int lhi, int l32,
+__device__ __forceinline__ void big_park(const GemmParams& p, int e, int n0, int wn, int wm, int lhi, int l32,
                                          const float* s_rw, const float* s_as, const float* s_ws,
-                                         const float* s_bias, char* epi, const f32x16 (&acc)[4][4]) {
+                                         const float* s_bias, char* epi, f32x16 (&acc)[4][4]) {
   // e4m3: the accumulator is in units of (row scale of the A operand) x (weight row scale).
   // Scales and biases of the weight rows were put into LDS in the order of the weight unit's rows.
   [[maybe_unused]] int ws_row[4];
@@ -902,8 +917,15 @@ __device__ __forceinline__ void big_park(const GemmParams& p, int e, int n0, int
   };
 #pragma unroll
   for (int fm = 0; fm < FMC; ++fm) {
-    const float rw = s_rw[fm * 32 + l32];
-    [[maybe_unused]] const float as = SCALED ? s_as[fm * 32 + l32] : 1.f;
+    // e4m3: the accumulators stay where they are until their turn.  (The compiler copies them out of the accumulation
+    // registers behind the last product of each, in front of the branches that lead here, which takes 256 more
+    // registers than its main loop leaves.  The 16-bit loop leaves enough, and there the copies are as well placed.)
+    if constexpr (SCALED)
+#pragma unroll
+      for (int fn = 0; fn < 4; ++fn) asm volatile("" : "+a"(acc[fn][fm]));
+    const int slot = (2 * fm + wm) * 32 + l32;   // of the block
+    const float rw = s_rw[slot];
+    [[maybe_unused]] const float as = SCALED ? s_as[slot] : 1.f;
     char* row = epi + (fm * 32 + l32) * kEpiRowBytes;
 #pragma unroll
     for (int fn = 0; fn < (FAST_SILU ? 2 : 4); ++fn) {
@@ -919,7 +941,9 @@ __device__ __forceinline__ void big_park(const GemmParams& p, int e, int n0, int
         }
         *reinterpret_cast<uint2*>(row + (fn * 32 + 8 * g + 4 * lhi) * 2) =
             uint2{pack2<El>(v[0], v[1]), pack2<El>(v[2], v[3])};
+        if constexpr (SCALED) __builtin_amdgcn_sched_barrier(0);
       }
+      __builtin_amdgcn_sched_barrier(0);  // no accumulators copied further ahead than the registers hold
     }
   }
 }
@@ -929,14 +953,16 @@ __device__ __forceinline__ void big_park(const GemmParams& p, int e, int n0, int
 // row are parked ready; with the other activations columns [0,64) of a row are
 // gate values and [64,128) the matching up values, combined here.
 template <typename El, bool GATED, int ACT>
-__device__ __forceinline__ void big_flush(const GemmParams& p, int n0, int wn, int lane, int slot0,
-                                          int rows, const int* s_tok, const char* epi) {
+__device__ __forceinline__ void big_flush(const GemmParams& p, int n0, int wn, int wm, int lane, int slot0,
+                                          int nvalid, const int* s_tok, const char* epi) {
   using S = typename El::S;
   constexpr int COLS = GATED ? 64 : 128;      // output columns of the wavefront tile
   constexpr int LPR = COLS / 8;               // lanes per row
   constexpr int RPS = kWave / LPR;            // rows per step
   constexpr bool PAIRS = GATED && ACT != MOE_ACT_SILU;  // gate and up parked side by side, activation applied here
   constexpr int UNR = PAIRS ? 4 : 8;          // steps in flight: LDS reads, math and stores overlap
+  const int frags = ((nvalid + 31) / 32 + 1 - wm) >> 1;   // parked by this wavefront, 32 rows each
+  auto slot_of = [&](int r) { return r + (r & ~31) + 32 * wm; };  // parked row r's slot of the block
   const int c8 = (lane % LPR) * 8;
   const int ncol = n0 + wn * COLS + c8;
   const bool vec_ok = ncol + 7 < p.N && (p.ldc & 7) == 0;
@@ -947,28 +973,25 @@ __device__ __forceinline__ void big_flush(const GemmParams& p, int n0, int wn, i
   if constexpr (GATED) tiled = p.c_tiled != 0;
   if (tiled && n0 + wn * COLS >= p.N) return;
   // Whole wavefront inside the matrix: no per-lane edge handling.  Real slots come
-  // first in a block, so row r is live exactly when r < rows.
+  // first in a block, so a slot is live exactly when it is below nvalid.
   if (tiled || (n0 + wn * COLS + COLS <= p.N && (p.ldc & 7) == 0)) {
     const int lrow = lane / LPR;
     char* cbase = static_cast<char*>(p.c) + static_cast<int64_t>(ncol) * 2;
     int64_t ldc_bytes = static_cast<int64_t>(p.ldc) * 2;
     if (tiled) {
-      const int64_t unit = static_cast<int64_t>(slot0 >> 8) * (p.N >> 6) + (n0 >> 6) + wn;
+      const int64_t unit = static_cast<int64_t>(slot0 / kBigBM) * (p.N >> 6) + (n0 >> 6) + wn;
       cbase = static_cast<char*>(p.c) + unit * kBigUnitBytes;
       ldc_bytes = kBigRowBytes;
     }
     const char* src = epi + lrow * kEpiRowBytes + c8 * 2;
-    for (int r0 = 0; r0 < rows; r0 += RPS * UNR) {
+    for (int r0 = 0; r0 < frags * 32; r0 += RPS * UNR) {
       int crow[UNR];
       uint4 gq[UNR], uq[UNR];
 #pragma unroll
       for (int u = 0; u < UNR; ++u) {
-        const int r = r0 + u * RPS + lrow;  // < 128: rows <= 128 and 128 is a multiple of RPS * UNR
-        crow[u] = p.a_by_slot ? s_tok[r] : slot0 + r;
-        if (tiled) {
-          const int rb = (slot0 & 255) + r;  // row inside the block; the row's byte offset carries the chunk
-          crow[u] = rb;
-        }
+        const int b = slot_of(r0 + u * RPS + lrow);  // < 256: a wavefront parks 128 rows, a multiple of RPS * UNR
+        crow[u] = p.a_by_slot ? s_tok[b] : slot0 + b;
+        if (tiled) crow[u] = b;  // row inside the block; the row's byte offset carries the chunk
         gq[u] = *reinterpret_cast<const uint4*>(src + (r0 + u * RPS) * kEpiRowBytes);
         if constexpr (PAIRS) uq[u] = *reinterpret_cast<const uint4*>(src + (r0 + u * RPS) * kEpiRowBytes + 128);
       }
@@ -978,7 +1001,7 @@ __device__ __forceinline__ void big_flush(const GemmParams& p, int n0, int wn, i
         if constexpr (PAIRS)
           out = uint4{gated_pair<El, ACT>(p, gq[u].x, uq[u].x), gated_pair<El, ACT>(p, gq[u].y, uq[u].y),
                       gated_pair<El, ACT>(p, gq[u].z, uq[u].z), gated_pair<El, ACT>(p, gq[u].w, uq[u].w)};
-        if (r0 + u * RPS + lrow < rows) {
+        if (slot_of(r0 + u * RPS + lrow) < nvalid) {
           char* dst = cbase + crow[u] * ldc_bytes;
           if (tiled) dst += ((lane & 7) ^ ((crow[u] >> 1) & 7)) << 4;
           if (p.wt_stores) store16_device_scope(dst, out);
@@ -988,13 +1011,13 @@ __device__ __forceinline__ void big_flush(const GemmParams& p, int n0, int wn, i
     }
     return;
   }
-  for (int r0 = 0; r0 < rows; r0 += RPS * UNR) {
+  for (int r0 = 0; r0 < frags * 32; r0 += RPS * UNR) {
     int tok[UNR];
     uint4 gq[UNR], uq[UNR];
 #pragma unroll
     for (int u = 0; u < UNR; ++u) {
-      const int r = r0 + u * RPS + lane / LPR;
-      tok[u] = r < rows ? s_tok[r] : p.numel;
+      const int r = r0 + u * RPS + lane / LPR, b = slot_of(r);
+      tok[u] = b < nvalid ? s_tok[b] : p.numel;
       const char* row = epi + (r < 128 ? r : 127) * kEpiRowBytes;
       gq[u] = *reinterpret_cast<const uint4*>(row + c8 * 2);
       if constexpr (PAIRS) uq[u] = *reinterpret_cast<const uint4*>(row + (64 + c8) * 2);
@@ -1006,7 +1029,7 @@ __device__ __forceinline__ void big_flush(const GemmParams& p, int n0, int wn, i
       if constexpr (PAIRS)
         out = uint4{gated_pair<El, ACT>(p, gq[u].x, uq[u].x), gated_pair<El, ACT>(p, gq[u].y, uq[u].y),
                     gated_pair<El, ACT>(p, gq[u].z, uq[u].z), gated_pair<El, ACT>(p, gq[u].w, uq[u].w)};
-      const int slot = slot0 + r0 + u * RPS + lane / LPR;
+      const int slot = slot0 + slot_of(r0 + u * RPS + lane / LPR);
       const int64_t crow = p.a_by_slot ? tok[u] : slot;
       S* dst = static_cast<S*>(p.c) + crow * p.ldc + ncol;
       if (vec_ok) {
@@ -1021,11 +1044,19 @@ __device__ __forceinline__ void big_flush(const GemmParams& p, int n0, int wn, i
   }
 }
 
-template <typename Mma, int FMC, bool GATED, bool LIGHT = false>
-__device__ __forceinline__ void big_wave(const GemmParams& p, const BigCtx& c, char* smem, int nk,
-                                         int e, int n0, int wn, int wm, int lane, int my_tok, float my_rw,
+template <typename Mma, int FMC, bool GATED, bool LIGHT>
+__device__ __forceinline__ void big_wave(const GemmParams& p, BigCtx& c, char* smem, int nk,
+                                         int e, int n0, int wn, int wm, int my_tok, float my_rw,
                                          float my_as, float my_ws, float my_bias, int* s_tok_all, float* s_rw_all, char* epi) {
   using El = typename Mma::El;
+  {
+    // chunk ch of MFMA step kk: lane half lhi owns the K elements of chunks CH * (2 kk + lhi) .. + CH - 1
+    constexpr int CH = Mma::kBigChunks;
+    const int lane = fresh_lane(), l32 = lane & 31, lhi = lane >> 5;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      c.rd_k[q] = l32 * kBigRowBytes + (((CH * (2 * (q / CH) + lhi) + q % CH) ^ ((l32 >> 1) & 7)) << 4);
+  }
   f32x16 acc[4][4];
 #pragma unroll
   for (int fn = 0; fn < 4; ++fn)
@@ -1039,19 +1070,22 @@ __device__ __forceinline__ void big_wave(const GemmParams& p, const BigCtx& c, c
     big_mainloop<Mma, FMC, GATED>(c, smem, nk, acc);
   }
   bare_barrier();  // every wavefront is done reading the ring before it is reused
-  s_tok_all[threadIdx.x] = my_tok;
-  s_rw_all[threadIdx.x] = my_rw;  // requested before the main loop, needed only now
-  s_rw_all[kBigBM + threadIdx.x] = my_as;
-  s_rw_all[2 * kBigBM + threadIdx.x] = my_ws;
-  s_rw_all[3 * kBigBM + threadIdx.x] = my_bias;
+  const int lane = fresh_lane(), tid = (2 * wn + wm) * kWave + lane;
+  s_tok_all[tid] = my_tok;
+  s_rw_all[tid] = my_rw;  // requested before the main loop, needed only now
+  if constexpr (Mma::kEs == 1) {
+    s_rw_all[kBigBM + tid] = my_as;
+    s_rw_all[2 * kBigBM + tid] = my_ws;
+  }
+  s_rw_all[3 * kBigBM + tid] = my_bias;
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   bare_barrier();
   if constexpr (FMC > 0) {
     // one straight-line body per case: a test per element costs more than the element
     auto park = [&](auto bias_tag, auto silu_tag) {
       big_park<El, FMC, GATED, Mma::kEs == 1, decltype(bias_tag)::value != 0, decltype(silu_tag)::value != 0>(
-          p, e, n0, wn, lane >> 5, lane & 31, s_rw_all + wm * 128, s_rw_all + kBigBM + wm * 128,
-          s_rw_all + 2 * kBigBM, s_rw_all + 3 * kBigBM, epi, acc);
+          p, e, n0, wn, wm, lane >> 5, lane & 31, s_rw_all, s_rw_all + kBigBM, s_rw_all + 2 * kBigBM,
+          s_rw_all + 3 * kBigBM, epi, acc);
     };
     bool fast_silu = false;
     if constexpr (GATED) fast_silu = p.activation == MOE_ACT_SILU;
@@ -1072,8 +1106,9 @@ __device__ __forceinline__ void big_wave(const GemmParams& p, const BigCtx& c, c
 template <typename Mma, bool GATED>
 __device__ __forceinline__ void big_tile(const GemmParams& p, int mb, int nt, char* smem) {
   using El = typename Mma::El;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int l32 = lane & 31, lhi = lane >> 5;
+  // (uniform, and known to the compiler as such: a branch on a vector register keeps the operands of the bodies not
+  // taken alive through the one that is)
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave & 1, wn = wave >> 1;
   // the two loads below do not depend on each other: one memory latency, not two
   const int e = __builtin_amdgcn_readfirstlane(p.expert_ids[(mb * kBigBM) / p.align_bs]);
@@ -1087,7 +1122,7 @@ __device__ __forceinline__ void big_tile(const GemmParams& p, int mb, int nt, ch
   int* s_cnt = reinterpret_cast<int*>(smem + kBigLdsBytes + kBigSideBytes);
   const int wave_cnt = __popcll(__ballot(my_tok < p.numel));
   if (lane == 0) s_cnt[wave] = wave_cnt;
-  constexpr int ES = Mma::kEs, CH = Mma::kBigChunks;
+  constexpr int ES = Mma::kEs;
   const int nk = p.Kd / (kBigRowBytes / ES);
   BigCtx c;
   // DMA geometry: wavefront w fills bytes [8192 w, 8192 w + 8192) of every unit with eight requests
@@ -1139,7 +1174,7 @@ __device__ __forceinline__ void big_tile(const GemmParams& p, int mb, int nt, ch
     });
   }
   __syncthreads();
-  const int nvalid = s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3];
+  const int nvalid = __builtin_amdgcn_readfirstlane(s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3]);
   if (nvalid == 0) {
     wait_vmcnt<0>();  // nothing may still be landing in LDS when the workgroup ends
     return;
@@ -1190,11 +1225,7 @@ __device__ __forceinline__ void big_tile(const GemmParams& p, int mb, int nt, ch
     }
     c.a_off[i] = static_cast<uint32_t>(src * p.lda * ES + dma_chunk(pos_row) * 16) + bias;
   }
-  // chunk ch of MFMA step kk: lane half lhi owns the K elements of chunks CH * (2 kk + lhi) .. + CH - 1
-#pragma unroll
-  for (int q = 0; q < 4; ++q)
-    c.rd_k[q] = l32 * kBigRowBytes + (((CH * (2 * (q / CH) + lhi) + q % CH) ^ ((l32 >> 1) & 7)) << 4);
-  c.x_row = wm * 128 * kBigRowBytes;
+  c.x_row = wm * 32 * kBigRowBytes;
 #pragma unroll
   for (int fn = 0; fn < 4; ++fn) {
     int r;
@@ -1204,34 +1235,38 @@ __device__ __forceinline__ void big_tile(const GemmParams& p, int mb, int nt, ch
       r = wn * 128 + fn * 32;
     c.w_row[fn] = r * kBigRowBytes;
   }
-  const int slot0 = mb * kBigBM + wm * 128;
+  const int slot0 = mb * kBigBM;
   char* epi = smem + wave * kEpiWaveBytes;
-  const int rows = min(128, max(0, nvalid - wm * 128));  // real slots of this wavefront
+  const int frags = ((nvalid + 31) / 32 + 1 - wm) >> 1;  // token fragments of this wavefront that hold a real slot
   __syncthreads();  // s_tok sits inside the ring: everyone has read it before any DMA may land there
-  if (nvalid <= 64) {
-    // a workgroup-wide choice: every wavefront runs the streaming-shaped loop
-    switch ((rows + 31) >> 5) {
-      case 0: big_wave<Mma, 0, GATED, true>(p, c, smem, nk, e, n0, wn, wm, lane, my_tok, my_rw, my_as, my_ws, my_bias, s_tok, s_rw_all, epi); break;
-      case 1: big_wave<Mma, 1, GATED, true>(p, c, smem, nk, e, n0, wn, wm, lane, my_tok, my_rw, my_as, my_ws, my_bias, s_tok, s_rw_all, epi); break;
-      default: big_wave<Mma, 2, GATED, true>(p, c, smem, nk, e, n0, wn, wm, lane, my_tok, my_rw, my_as, my_ws, my_bias, s_tok, s_rw_all, epi); break;
-    }
-  } else
-  switch ((rows + 31) >> 5) {
-    case 0: big_wave<Mma, 0, GATED>(p, c, smem, nk, e, n0, wn, wm, lane, my_tok, my_rw, my_as, my_ws, my_bias, s_tok, s_rw_all, epi); break;
-    case 1: big_wave<Mma, 1, GATED>(p, c, smem, nk, e, n0, wn, wm, lane, my_tok, my_rw, my_as, my_ws, my_bias, s_tok, s_rw_all, epi); break;
-    case 2: big_wave<Mma, 2, GATED>(p, c, smem, nk, e, n0, wn, wm, lane, my_tok, my_rw, my_as, my_ws, my_bias, s_tok, s_rw_all, epi); break;
-    case 3: big_wave<Mma, 3, GATED>(p, c, smem, nk, e, n0, wn, wm, lane, my_tok, my_rw, my_as, my_ws, my_bias, s_tok, s_rw_all, epi); break;
-    default: big_wave<Mma, 4, GATED>(p, c, smem, nk, e, n0, wn, wm, lane, my_tok, my_rw, my_as, my_ws, my_bias, s_tok, s_rw_all, epi); break;
-  }
+  auto wave_tile = [&](auto fm_tag, auto light_tag) {
+    big_wave<Mma, decltype(fm_tag)::value, GATED, decltype(light_tag)::value != 0>(
+        p, c, smem, nk, e, n0, wn, wm, my_tok, my_rw, my_as, my_ws, my_bias, s_tok, s_rw_all, epi);
+  };
+  using Yes = IntTag<1>;
+  using No = IntTag<0>;
+  // The streaming-shaped loop is a workgroup-wide choice.  The compiler lays the bodies out one behind the other and
+  // keeps the operands of the later ones through the earlier, so the one of four fragments, which has no register to
+  // spare, comes last.  One VGPR too many is not cheap: a spilled value that is still being loaded, or one that is
+  // loaded back, waits for every request in flight.  As a switch over wavefront numbers in vector registers the
+  // 16-bit kernel spilled 25 of them, now none.  With the fragments dealt in turn: 8448 tokens 817 -> 797 us, 16896
+  // 1481 -> 1428, 1024 256 -> 247, with e4m3 weights 8448 605 -> 584, 600 161 -> 153 (both passes and the combine).
+  if (light_a && frags == 0) wave_tile(IntTag<0>{}, Yes{});
+  if (light_a && frags == 1) wave_tile(IntTag<1>{}, Yes{});
+  if (!light_a && frags == 1) wave_tile(IntTag<1>{}, No{});
+  if (!light_a && frags == 2) wave_tile(IntTag<2>{}, No{});
+  if (!light_a && frags == 3) wave_tile(IntTag<3>{}, No{});
+  if (!light_a && frags == 4) wave_tile(IntTag<4>{}, No{});
+  const int flush_lane = fresh_lane();
   if constexpr (GATED) {
     if (p.activation == MOE_ACT_SILU)
-      big_flush<El, true, MOE_ACT_SILU>(p, n0, wn, lane, slot0, rows, s_tok + wm * 128, epi);
+      big_flush<El, true, MOE_ACT_SILU>(p, n0, wn, wm, flush_lane, slot0, nvalid, s_tok, epi);
     else if (p.activation == MOE_ACT_SWIGLUOAI)
-      big_flush<El, true, MOE_ACT_SWIGLUOAI>(p, n0, wn, lane, slot0, rows, s_tok + wm * 128, epi);
+      big_flush<El, true, MOE_ACT_SWIGLUOAI>(p, n0, wn, wm, flush_lane, slot0, nvalid, s_tok, epi);
     else
-      big_flush<El, true, MOE_ACT_GELU>(p, n0, wn, lane, slot0, rows, s_tok + wm * 128, epi);
+      big_flush<El, true, MOE_ACT_GELU>(p, n0, wn, wm, flush_lane, slot0, nvalid, s_tok, epi);
   } else {
-    big_flush<El, false, MOE_ACT_SILU>(p, n0, wn, lane, slot0, rows, s_tok + wm * 128, epi);
+    big_flush<El, false, MOE_ACT_SILU>(p, n0, wn, wm, flush_lane, slot0, nvalid, s_tok, epi);
   }
 }
 

@@ -592,6 +592,30 @@ def test_large_tile_ranges_on_lopsided_routing(moe, oracle, dev, pattern, monkey
                     "fused", rtol=1.6e-2, atol=2e-3 + 4e-3 * out.float().abs().max().item())
 
 
+@pytest.mark.parametrize("dt", ["bf16", "e4m3"])
+@pytest.mark.parametrize("rows", [1, 32, 33, 64, 65, 96, 97, 128, 129, 160, 161, 192, 193, 224, 225])
+def test_partly_filled_blocks_of_the_large_tile(moe, oracle, dev, dt, rows, monkeypatch):
+    """The 32-row fragments of a block of 256 go to the two halves of a workgroup's wavefronts in turn: every number
+    of fragments, full and with a single row in the last one, in both passes.  Tolerances as of the tests with other
+    row counts: one rounding of the intermediate; with e4m3 one step of an element next to a tie moves it by 6 %."""
+    E, H, I = 2, 512, 256
+    monkeypatch.setattr(moe.fused_moe, "try_get_optimal_moe_config", lambda *a, **k: {"BLOCK_SIZE_M": 256})
+    x, w13, w2, _ = _layer(E, H, I, E * rows, 1, 300 + rows, torch.bfloat16)
+    ids = (torch.arange(E * rows, dtype=torch.int32) % E).view(-1, 1)
+    tw = torch.rand(E * rows, 1, generator=torch.Generator().manual_seed(rows)) + 0.5
+    kw = dict(topk_weights=tw.to(dev), topk_ids=ids.to(dev))
+    if dt == "e4m3":
+        q13, s13, q2, s2 = moe.quantize_expert_weights(w13.to(dev), w2.to(dev))
+        out = moe.fused_experts(x.to(dev), q13, q2, None, None, per_channel_quant=True, w1_scale=s13, w2_scale=s2, **kw)
+        want = oracle.fused_experts_fp8_ref(x, q13.view(torch.uint8).cpu(), s13.cpu(), q2.view(torch.uint8).cpu(),
+                                            s2.cpu(), tw, ids, mirror_rounding="fused")
+        _close(out, want, rtol=2e-2, atol=0.03 * out.float().abs().max().item())
+    else:
+        out = moe.fused_experts(x.to(dev), w13.to(dev), w2.to(dev), None, None, **kw)
+        want = oracle.fused_experts_ref(x, w13, w2, tw, ids, mirror_rounding="fused")
+        _close(out, want, rtol=1.6e-2, atol=2e-3 * max(1.0, out.float().abs().max().item()))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("rows_per_expert", [256, 512, 32, 255, 257])
 def test_experts_with_exactly_full_blocks(moe, oracle, dev, rows_per_expert):
