@@ -528,6 +528,12 @@ __device__ __forceinline__ uint32_t pack2<ElemF16>(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, f16x2));
 }
 
+// A word that no workgroup of the launch writes, at an address that is the same for the whole wavefront: as a scalar
+// load, so that it does not stand in the queue of the vector requests.
+__device__ __forceinline__ int uniform_load(const int32_t* at) {
+  return *reinterpret_cast<const __attribute__((address_space(4))) int32_t*>(reinterpret_cast<uintptr_t>(at));
+}
+
 // The lane number, computed where it stands: what is derived from it before and after the large-tile main loop is
 // not the same value to the compiler, which would otherwise keep it, and every address made of it, in registers
 // that the loop's 256 accumulators do not leave.
@@ -1102,22 +1108,32 @@ __device__ __forceinline__ void big_wave(const GemmParams& p, BigCtx& c, char* s
   }
 }
 
-// One output tile of the large-tile kernel: m-block mb, n-tile nt.
-template <typename Mma, bool GATED>
-__device__ __forceinline__ void big_tile(const GemmParams& p, int mb, int nt, char* smem) {
+// One output tile of the large-tile kernel: m-block mb, n-tile nt.  `wait.ready()` is called by the workgroup's first
+// wavefront before any row of the A operand is read; it returns whether that operand is complete.  Where it is not, the
+// workgroup calls `wait.expired(p, mb, nt)` instead of multiplying.
+// The start of a tile is a chain of memory latencies with idle matrix pipes.  The expert's id and the slot ids are one
+// of them, the first weights and the wait for the A operand another, the A operand's rows the third: the rows' numbers
+// are divided out by one thread each behind the requests for weights, not by every thread for its eight requests, and
+// of the four wavefronts only the one that waits asks for its weights late.  With the wait ahead of everything, the two
+// ids one after the other and eight divisions between the requests: 8448 tokens 766 us, 757 now, 256 tokens 166.5 and
+// 164.1, e4m3 8448 554 and 548 (both passes and the combine).
+template <typename Mma, bool GATED, typename Wait>
+__device__ __forceinline__ void big_tile(const GemmParams& p, int mb, int nt, char* smem, Wait wait) {
   using El = typename Mma::El;
   // (uniform, and known to the compiler as such: a branch on a vector register keeps the operands of the bodies not
   // taken alive through the one that is)
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave & 1, wn = wave >> 1;
-  // the two loads below do not depend on each other: one memory latency, not two
-  const int e = __builtin_amdgcn_readfirstlane(p.expert_ids[(mb * kBigBM) / p.align_bs]);
+  // the two loads below do not depend on each other: one memory latency, not two (the expert's id through the scalar
+  // cache: as a vector load it was waited for before the slot ids were asked for)
+  const int eb = __builtin_amdgcn_readfirstlane(p.align_bs == kBigBM ? mb : (mb * kBigBM) / p.align_bs);
+  const int e = uniform_load(p.expert_ids + eb);
   const int64_t my_slot = static_cast<int64_t>(mb) * kBigBM + tid;
   const int my_tok = p.sorted_ids[my_slot < p.sorted_cap ? my_slot : p.sorted_cap - 1];
   const int n0 = nt * (GATED ? kBigBNW / 2 : kBigBNW);
   int* s_tok = reinterpret_cast<int*>(smem + kBigLdsBytes);
   float* s_rw_all = reinterpret_cast<float*>(smem + kBigLdsBytes + kBigBM * 4);
-  s_tok[tid] = my_tok;
+  int* s_src = s_tok;  // until the ring takes the place over
   // real slots come first in a block: count them (dynamic LDS only, the ring needs all 160 KB)
   int* s_cnt = reinterpret_cast<int*>(smem + kBigLdsBytes + kBigSideBytes);
   const int wave_cnt = __popcll(__ballot(my_tok < p.numel));
@@ -1147,7 +1163,7 @@ __device__ __forceinline__ void big_tile(const GemmParams& p, int mb, int nt, ch
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const int rr = dma_row0 + 8 * i;
-    int64_t wrow;
+    int wrow;
     if constexpr (GATED) {
       const int half = rr >> 7;
       int n = n0 + (rr & 127);
@@ -1157,8 +1173,14 @@ __device__ __forceinline__ void big_tile(const GemmParams& p, int mb, int nt, ch
       const int n = n0 + rr;
       wrow = n < p.N ? n : p.N - 1;
     }
-    c.w_off[i] = static_cast<uint32_t>(wrow * p.w_stride_n * ES + dma_chunk(rr) * 16) + dma_win_bias(i);
+    c.w_off[i] = static_cast<uint32_t>(wrow) * (static_cast<uint32_t>(p.w_stride_n) * ES) + dma_chunk(rr) * 16 + dma_win_bias(i);
   }
+  }
+  if constexpr (Wait::kWaits) {
+    if (wave == 0) {
+      const int ready = wait.ready() ? 1 : 0;
+      if (lane == 0) s_cnt[4] = ready;
+    }
   }
   // The weights of the first K tile and a half are on their way (ring slots 1 and 3) while
   // the slot ids are still being looked at: they are the cold half of the fill.
@@ -1173,7 +1195,20 @@ __device__ __forceinline__ void big_tile(const GemmParams& p, int mb, int nt, ch
       lds_dma16_win<i, i == 0>(c.w_base + c.w_step, c.w_off[i], c.dma_lds + 3 * kBigUnitBytes);
     });
   }
+  // row of the A operand that this thread's slot reads (one division a thread, while the weights are on their way)
+  if (!p.a_by_slot) s_src[tid] = my_tok < p.numel ? my_tok / p.top_k : 0;
   __syncthreads();
+  if constexpr (Wait::kWaits) {
+    // Every wavefront orders its own loads of the block's rows behind the count it has just been told
+    // of: the acquire fence drops the cached lines (and completes, vmcnt(0)) in the wavefront that
+    // issues it, and a workgroup barrier alone does not extend that to the other three.
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    if (__builtin_amdgcn_readfirstlane(s_cnt[4]) == 0) {
+      wait_vmcnt<0>();  // nothing may still be landing in LDS when the workgroup ends
+      wait.template expired<typename Mma::El>(p, mb, nt);
+      return;
+    }
+  }
   const int nvalid = __builtin_amdgcn_readfirstlane(s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3]);
   if (nvalid == 0) {
     wait_vmcnt<0>();  // nothing may still be landing in LDS when the workgroup ends
@@ -1204,26 +1239,24 @@ __device__ __forceinline__ void big_tile(const GemmParams& p, int mb, int nt, ch
   // A weight-streaming tile (at most 64 real slots) loads token units of 64 rows: there the
   // wavefront's window is 2 KB, rows 16 w + 8 j + l / 8, two requests with the offsets -1024 and 0.
   const bool light_a = nvalid <= 64;
+  // row of request i whose data is asked for: a request whose eight rows are all padding asks for rows 0..7 again (an
+  // L1 hit), so that every token unit is the same number of loads and the vmcnt bookkeeping stays fixed
+  auto place = [&](int i) { return light_a ? 16 * wave + 8 * (i & 1) + (lane >> 3) : dma_row0 + 8 * i; };
+  auto live_row = [&](int i) { const int r = place(i); return (r & ~7) >= nvalid ? lane >> 3 : r; };
+  auto win_bias = [&](int i) { return light_a ? static_cast<uint32_t>(4096 - ((i & 1) - 1) * 1024) : dma_win_bias(i); };
+  if (p.a_tiled) {
+    // (a dead request reads the bytes of live rows 0..7 into its own place: never looked at)
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    int row = light_a ? 16 * wave + 8 * (i & 1) + (lane >> 3) : dma_row0 + 8 * i;
-    const uint32_t bias = light_a ? static_cast<uint32_t>(4096 - ((i & 1) - 1) * 1024) : dma_win_bias(i);
-    // a request whose eight rows are all padding asks for rows 0..7 again (an L1 hit), so that
-    // every token unit is the same number of loads and the vmcnt bookkeeping stays fixed
-    const bool dead = (row & ~7) >= nvalid;
-    const int pos_row = row;   // the row whose place in LDS the data takes (it decides the chunk order)
-    if (dead) row = lane >> 3;
-    if (p.a_tiled) {
-      // (a dead request reads the bytes of live rows 0..7 into its own place: never looked at)
-      c.a_off[i] = static_cast<uint32_t>(row * kBigRowBytes + (lane & 7) * 16) + bias;
-      continue;
-    }
-    int64_t src = static_cast<int64_t>(mb) * kBigBM + row;
-    if (!p.a_by_slot) {
-      const int tok = s_tok[row];
-      src = tok < p.numel ? tok / p.top_k : 0;
-    }
-    c.a_off[i] = static_cast<uint32_t>(src * p.lda * ES + dma_chunk(pos_row) * 16) + bias;
+    for (int i = 0; i < 8; ++i)
+      c.a_off[i] = static_cast<uint32_t>(live_row(i) * kBigRowBytes + (lane & 7) * 16) + win_bias(i);
+  } else {
+    uint32_t src[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) src[i] = p.a_by_slot ? mb * kBigBM + live_row(i) : s_src[live_row(i)];
+    // (the place in LDS decides the chunk order; the offset fits 32 bits: dma_offsets_fit)
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      c.a_off[i] = src[i] * (static_cast<uint32_t>(p.lda) * ES) + dma_chunk(place(i)) * 16 + win_bias(i);
   }
   c.x_row = wm * 32 * kBigRowBytes;
 #pragma unroll
@@ -1238,7 +1271,7 @@ __device__ __forceinline__ void big_tile(const GemmParams& p, int mb, int nt, ch
   const int slot0 = mb * kBigBM;
   char* epi = smem + wave * kEpiWaveBytes;
   const int frags = ((nvalid + 31) / 32 + 1 - wm) >> 1;  // token fragments of this wavefront that hold a real slot
-  __syncthreads();  // s_tok sits inside the ring: everyone has read it before any DMA may land there
+  __syncthreads();  // s_src sits inside the ring: everyone has read it before any DMA may land there
   auto wave_tile = [&](auto fm_tag, auto light_tag) {
     big_wave<Mma, decltype(fm_tag)::value, GATED, decltype(light_tag)::value != 0>(
         p, c, smem, nk, e, n0, wn, wm, my_tok, my_rw, my_as, my_ws, my_bias, s_tok, s_rw_all, epi);
@@ -1270,6 +1303,10 @@ __device__ __forceinline__ void big_tile(const GemmParams& p, int mb, int nt, ch
   }
 }
 
+struct NoWait {
+  static constexpr bool kWaits = false;
+};
+
 template <typename Mma, bool GATED>
 __global__ __launch_bounds__(kThreads, 1) void big_gemm_kernel(const GemmParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -1299,7 +1336,7 @@ __global__ __launch_bounds__(kThreads, 1) void big_gemm_kernel(const GemmParams 
     mb = logical - nt * live_mb;
   }
   }
-  big_tile<Mma, GATED>(p, mb, nt, smem);
+  big_tile<Mma, GATED>(p, mb, nt, smem, NoWait{});
 }
 
 // Both passes in one launch, for the 16-bit dtypes.  Workgroup ids go to the XCDs
@@ -1322,7 +1359,9 @@ __global__ __launch_bounds__(kThreads, 1) void big_gemm_kernel(const GemmParams 
 template <typename El>
 __device__ __forceinline__ void big_poison_tile(const GemmParams& p, int mb, int nt) {
   using S = typename El::S;
-  const int64_t slot = static_cast<int64_t>(mb) * kBigBM + threadIdx.x;
+  // (not the slot that big_tile started with: as the same value it would be kept in registers through the main loop)
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
+  const int64_t slot = static_cast<int64_t>(mb) * kBigBM + wave * kWave + fresh_lane();
   if (slot >= p.sorted_cap) return;
   const int tok = p.sorted_ids[slot];
   if (tok >= p.numel) return;
@@ -1331,6 +1370,26 @@ __device__ __forceinline__ void big_poison_tile(const GemmParams& p, int mb, int
   const int n0 = nt * kBigBNW;
   for (int n = n0; n < n0 + kBigBNW && n < p.N; ++n) row[n] = nan;
 }
+
+// Wait of a down tile for the gate-up tiles of its m-block.
+struct GateUpWait {
+  static constexpr bool kWaits = true;
+  const int32_t* done;
+  int32_t* status;
+  int tiles, spin_limit;
+  __device__ bool ready() const {
+    int spins = 0;
+    bool ready;
+    while (!(ready = __builtin_amdgcn_readfirstlane(__hip_atomic_load(done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) >= tiles) && spins++ < spin_limit)
+      __builtin_amdgcn_s_sleep(32);
+    return ready;
+  }
+  template <typename El>
+  __device__ void expired(const GemmParams& p, int mb, int nt) const {
+    big_poison_tile<El>(p, mb, nt);
+    if (threadIdx.x == 0) __hip_atomic_fetch_add(status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+};
 
 template <typename Mma>
 __global__ __launch_bounds__(kThreads, 1) void big_fused_kernel(const GemmParams p1, const GemmParams p2,
@@ -1348,7 +1407,7 @@ __global__ __launch_bounds__(kThreads, 1) void big_fused_kernel(const GemmParams
   if (xslot < n1) {
     const int mb = lo + xslot / p1.num_n_tiles, nt = xslot % p1.num_n_tiles;
     if (mb >= hi || lo < 0 || mb >= p1.num_m_blocks) return;  // (an unwritten plan must not send a tile out of range)
-    big_tile<Mma, true>(p1, mb, nt, smem);
+    big_tile<Mma, true>(p1, mb, nt, smem, NoWait{});
     // Every store of this workgroup is complete before the barrier.  With write-through stores
     // (whole tiles inside the matrix) that means visible device-wide; otherwise the release
     // writes the L2 back first.  Measured at 8448 tokens, both passes: 766 us with no ordering
@@ -1363,28 +1422,7 @@ __global__ __launch_bounds__(kThreads, 1) void big_fused_kernel(const GemmParams
     const int j = xslot - n1;
     const int mb = lo + j / p2.num_n_tiles, nt = j % p2.num_n_tiles;
     if (mb >= hi || lo < 0 || mb >= p1.num_m_blocks) return;
-    int* s_flag = reinterpret_cast<int*>(smem + kBigLdsBytes + kBigSideBytes + 16);
-    if (threadIdx.x == 0) {
-      int spins = 0;
-      bool ready;
-      while (!(ready = __hip_atomic_load(done + mb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= p1.num_n_tiles) &&
-             spins++ < spin_limit)
-        __builtin_amdgcn_s_sleep(32);
-      *s_flag = ready ? 1 : 0;
-    }
-    __syncthreads();
-    // Every wavefront orders its own loads of the block's rows behind the count it has just been told
-    // of: the acquire fence drops the cached lines (and completes, vmcnt(0)) in the wavefront that
-    // issues it, and a workgroup barrier alone does not extend that to the other three.
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    if (*s_flag == 0) {  // workgroup-uniform
-      big_poison_tile<typename Mma::El>(p2, mb, nt);
-      if (threadIdx.x == 0) __hip_atomic_fetch_add(status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      return;
-    }
-    // (the flag word lies behind the epilogue's staging area and side arrays, in the ring's last unit,
-    // which big_tile writes only behind its own barriers)
-    big_tile<Mma, false>(p2, mb, nt, smem);
+    big_tile<Mma, false>(p2, mb, nt, smem, GateUpWait{done + mb, status, p1.num_n_tiles, spin_limit});
   }
 }
 
