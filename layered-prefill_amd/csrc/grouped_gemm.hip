@@ -136,6 +136,7 @@ struct GemmParams {
   int top_k;
   int num_m_blocks;  // ceil(sorted_cap / BM)
   int num_n_tiles;
+  uint32_t n_tiles_rcp;  // streaming kernel: floor(2^32 / num_n_tiles) + 1 (of more than one tile)
   int a_by_slot;     // A row = slot (pass 2) instead of tok / top_k (pass 1)
   int mul_weight;    // multiply by topk_w[tok] in the epilogue
   int activation;    // MoeActivation (gated pass only)
@@ -1560,8 +1561,11 @@ __device__ __forceinline__ void stream_store(const GemmParams& p, const float (&
 // of its own and they were up to a fifth of the pass's traffic (50.3 -> 47.8 us at 128 tokens).
 // Rows are laid
 // out in LDS like the large-tile kernel's (16-byte chunk c of row r at chunk
-// c ^ ((r >> 1) & 7)).  Everything the start-up reads is wavefront-uniform and
-// comes through the scalar cache, in two round trips.
+// c ^ ((r >> 1) & 7)).  The start-up is a chain of latencies that nothing hides in a call of few workgroups: the count
+// of blocks, the experts of the four blocks around, and the first weights, which need nothing else; the slot ids come
+// through the scalar cache meanwhile, as everything before them does, and what hangs on them follows the weights.  No
+// branch and no division in it.  (Slot ids and the expert once more in front of the weights, a run of branches and two
+// divisions: 64 tokens of the layer above 104.4 us, 103.1 this way, e4m3 100 tokens 73.9 and 71.8.)
 // e4m3 runs here too (100 tokens of that layer: gate-up 45.6 -> 40.1 us, down 40.9 -> 25.9 us
 // against the register-staged kernel, whose two stages hold 36 KB per workgroup and drain at every K tile), its scales
 // fetched ahead of the stream like the routed weights.  Rows need whole 32-byte steps, not whole units.
@@ -1589,46 +1593,41 @@ __global__ __launch_bounds__(kThreads, 3) void stream_gemm_kernel(const GemmPara
   const int xslot = blockIdx.x / kXcds;
   const int logical = (blockIdx.x % kXcds) * per_xcd + xslot;
   if (xslot >= per_xcd || logical >= live) return;
-  int mb = logical / p.num_n_tiles;
+  int mb = p.num_n_tiles > 1 ? __umulhi(logical, p.n_tiles_rcp) : logical;  // logical / num_n_tiles, or one more
   int nt = logical - mb * p.num_n_tiles;
-  {
-    // Blocks of one expert (it has more than 32 tokens) stream the same weights.
-    // Inside an aligned group of four blocks, reorder a run of g same-expert
-    // blocks from (block, n-tile) to (n-tile, block): the g workgroups that
-    // read one weight tile then start back to back on one XCD and the second
-    // to g-th find the lines in L2 (or already requested).
-    const int q0 = mb & ~3;
-    int eq[4];
+  if (nt < 0) { mb -= 1; nt += p.num_n_tiles; }
+  // Blocks of one expert (it has more than 32 tokens) stream the same weights.
+  // Inside an aligned group of four blocks, reorder a run of g same-expert
+  // blocks from (block, n-tile) to (n-tile, block): the g workgroups that
+  // read one weight tile then start back to back on one XCD and the second
+  // to g-th find the lines in L2 (or already requested).
+  const int q0 = mb & ~3, me = mb & 3;
+  int eq[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) eq[i] = q0 + i < live_mb ? p.expert_ids[q0 + i] : -1 - i;
-    const int me = mb - q0;
-    int lo = me, hi = me;
+  for (int i = 0; i < 4; ++i) eq[i] = uniform_load(p.expert_ids + (q0 + i < live_mb ? q0 + i : live_mb - 1));
+  uint32_t links = 0;  // bit i: blocks i and i + 1 of the group belong to one expert
 #pragma unroll
-    for (int i = 1; i < 4; ++i) {
-      if (lo == me - i + 1 && lo > 0 && eq[lo - 1] == eq[me]) lo = me - i;
-      if (hi == me + i - 1 && hi < 3 && eq[hi + 1] == eq[me]) hi = me + i;
-    }
-    const int g = hi - lo + 1;
-    const int li = (me - lo) * p.num_n_tiles + nt;
-    nt = li / g;
-    mb = q0 + lo + (li - nt * g);
-  }
+  for (int i = 0; i < 3; ++i) links |= (q0 + i + 1 < live_mb && eq[i] == eq[i + 1]) ? 1u << i : 0u;
+  const int lo = me - __builtin_clz(~(links << (31 - me) << 1)), hi = me + __builtin_ctz(~(links >> me));
+  const int e = me == 0 ? eq[0] : me == 1 ? eq[1] : me == 2 ? eq[2] : eq[3];
+  const int g = hi - lo + 1;
+  const int li = (me - lo) * p.num_n_tiles + nt;
+  nt = g == 1 ? li : static_cast<int>(__umulhi(li, g == 2 ? 0x80000000u : g == 3 ? 0x55555556u : 0x40000000u));  // li / g
+  mb = q0 + lo + (li - nt * g);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l15 = lane & 15, lq = lane >> 4;
   const int n0 = nt * BN_OUT;
 
-  // second round trip: the expert, the slots of this lane's results (tokens lane % 16 and 16 + lane % 16 of the
-  // block) and the eight slots whose token rows this wavefront requests
+  // second round trip, scalar: the block's slots and the eight whose token rows this wavefront requests.  The first
+  // weights are asked for meanwhile: vector loads whose results are needed this early would wait for them, too
   const int32_t* sid = p.sorted_ids + static_cast<int64_t>(mb) * kStBM;
-  int tok[2];
+  int slots[kStBM], mine[8];
 #pragma unroll
-  for (int h = 0; h < 2; ++h) tok[h] = sid[16 * h + l15];
-  const int e = __builtin_amdgcn_readfirstlane(p.expert_ids[mb]);
-  const int first = sid[0];
-  const int4 s0 = *reinterpret_cast<const int4*>(sid + 8 * wave);
-  const int4 s1 = *reinterpret_cast<const int4*>(sid + 8 * wave + 4);
-  if (first >= p.numel) return;  // real slots come first: the block is empty
+  for (int i = 0; i < kStBM; ++i) slots[i] = uniform_load(sid + i);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) mine[i] = uniform_load(sid + 8 * wave + i);
+  const char* w_base = static_cast<const char*>(p.w) + static_cast<int64_t>(e < 0 ? 0 : e) * p.w_stride_e * ES;
   // The lane's results: columns n_out and n_out + 1 (their gate and up rows), or n_out .. n_out + 3.
   const int n_out = n0 + (GATED ? 8 * wave + 2 * lq : 16 * wave + 4 * lq);
   auto result_row = [&](int i) {  // weight row behind accumulator element i
@@ -1637,41 +1636,12 @@ __global__ __launch_bounds__(kThreads, 3) void stream_gemm_kernel(const GemmPara
     n = n < p.N ? n : p.N - 1;
     return static_cast<int64_t>(!GATED ? n : p.interleaved ? 2 * n + half : half * p.N + n);
   };
-  // What the epilogue needs per slot and per weight row is fetched now, ahead of the stream: a load
-  // issued behind ~100 KB of queued DMA requests would take microseconds to return.
-  float rw[2] = {1.f, 1.f}, as[2] = {1.f, 1.f}, ws[4], bias[4];
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    if (p.mul_weight && tok[h] < p.numel) rw[h] = p.topk_w[tok[h]];
-    if constexpr (ES == 1)
-      if (tok[h] < p.numel) as[h] = p.a_scale[p.a_by_slot ? mb * kStBM + 16 * h + l15 : tok[h] / p.top_k];
-  }
-  if constexpr (ES == 1)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) ws[i] = p.w_scale[e * p.w_scale_stride_e + result_row(i)];
-  if (p.bias)
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      bias[i] = El::ld(static_cast<const typename El::S*>(p.bias)[e * p.bias_stride_e + result_row(i)]);
-
   // DMA requests of this wavefront: token rows 8 * wave + lane / 8, weight rows
   // 16 * wave + 8 * j + lane / 8 (j < 2); lane % 8 is the place the lane's 16 bytes land in.
   const char* a_base = static_cast<const char*>(p.a);
-  const char* w_base = static_cast<const char*>(p.w) + static_cast<int64_t>(e) * p.w_stride_e * ES;
   int w_step = kStRowBytes;  // bytes from one K unit to the next
-  uint32_t a_off, w_off[2];
-  bool a_live;   // lane 0 always: a request with no lane at all would not count
-  {
-    const int q = lane >> 3;
-    const int rr = 8 * wave + q;
-    int64_t src = mb * kStBM + rr;
-    const int lo = (q & 2) ? ((q & 1) ? s0.w : s0.z) : ((q & 1) ? s0.y : s0.x);
-    const int hi = (q & 2) ? ((q & 1) ? s1.w : s1.z) : ((q & 1) ? s1.y : s1.x);
-    const int slot_tok = (q & 4) ? hi : lo;
-    if (!p.a_by_slot) src = slot_tok < p.numel ? slot_tok / p.top_k : 0;
-    a_live = slot_tok < p.numel || lane == 0;
-    a_off = static_cast<uint32_t>(src * p.lda * ES + (((lane & 7) ^ ((rr >> 1) & 7)) << 4));
-  }
+  uint32_t a_off = 0, w_off[2];
+  bool a_live = false;  // lane 0 always: a request with no lane at all would not count
   const int row_bytes = p.Kd * ES;  // a multiple of 32
   constexpr int kBigRows = GATED ? 128 : 256;  // output columns covered by one 32 KB unit of tiled weights
   if (p.w_tiled) {
@@ -1704,7 +1674,8 @@ __global__ __launch_bounds__(kThreads, 3) void stream_gemm_kernel(const GemmPara
   // run-time branch this cost the rows of whole units 2 %.)
   const int nu = TAIL ? row_bytes / kStRowBytes + 1 : row_bytes / kStRowBytes;
   const int tail = row_bytes & (kStRowBytes - 1);
-  auto issue = [&](int u) {
+  auto issue = [&](int u, auto part) {
+    constexpr int PART = decltype(part)::value;  // 1 tokens, 2 weights
     const uint32_t ring = (u % kStUnits) * kStUnitBytes;
     uint32_t a = a_off, w[2] = {w_off[0], w_off[1]};
     if (TAIL && u == nu - 1) {
@@ -1716,11 +1687,60 @@ __global__ __launch_bounds__(kThreads, 3) void stream_gemm_kernel(const GemmPara
         w[j] -= static_cast<int>(cw) < tail ? 0u : cw;
       }
     }
-    if (a_live) lds_dma16(a_base + u * kStRowBytes, a, dma_a + ring);
+    if constexpr ((PART & 1) != 0)
+      if (a_live) lds_dma16(a_base + u * kStRowBytes, a, dma_a + ring);
+    if constexpr ((PART & 2) != 0) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) lds_dma16(w_base + static_cast<int64_t>(u) * w_step, w[j], dma_w + ring + j * 1024);
+      for (int j = 0; j < 2; ++j) lds_dma16(w_base + static_cast<int64_t>(u) * w_step, w[j], dma_w + ring + j * 1024);
+    }
   };
 
+  using Tokens = IntTag<1>;
+  using Weights = IntTag<2>;
+  using Both = IntTag<3>;
+  issue(0, Weights{});
+  if (1 < nu) issue(1, Weights{});
+  if (slots[0] >= p.numel) {  // real slots come first: the block is empty
+    wait_vmcnt<0>();          // nothing may still be landing in LDS when the workgroup ends
+    return;
+  }
+  // slots of this lane's results: tokens lane % 16 and 16 + lane % 16 of the block
+  int tok[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    int v = slots[16 * h];
+#pragma unroll
+    for (int i = 1; i < 16; ++i) v = l15 == i ? slots[16 * h + i] : v;
+    tok[h] = v;
+  }
+  // What the epilogue needs per slot and per weight row is fetched now, ahead of the stream: a load
+  // issued behind ~100 KB of queued DMA requests would take microseconds to return.
+  float rw[2] = {1.f, 1.f}, as[2] = {1.f, 1.f}, ws[4], bias[4];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    if (p.mul_weight && tok[h] < p.numel) rw[h] = p.topk_w[tok[h]];
+    if constexpr (ES == 1)
+      if (tok[h] < p.numel) as[h] = p.a_scale[p.a_by_slot ? mb * kStBM + 16 * h + l15 : tok[h] / p.top_k];
+  }
+  if constexpr (ES == 1)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) ws[i] = p.w_scale[e * p.w_scale_stride_e + result_row(i)];
+  if (p.bias)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      bias[i] = El::ld(static_cast<const typename El::S*>(p.bias)[e * p.bias_stride_e + result_row(i)]);
+
+  {
+    const int q = lane >> 3;
+    const int rr = 8 * wave + q;
+    int64_t src = mb * kStBM + rr;
+    int slot_tok = mine[0];
+#pragma unroll
+    for (int i = 1; i < 8; ++i) slot_tok = q == i ? mine[i] : slot_tok;
+    if (!p.a_by_slot) src = slot_tok < p.numel ? slot_tok / p.top_k : 0;
+    a_live = slot_tok < p.numel || lane == 0;
+    a_off = static_cast<uint32_t>(src * p.lda * ES + (((lane & 7) ^ ((rr >> 1) & 7)) << 4));
+  }
   // Fragments: row lane % 16, chunk 4 * kk + lane / 16 of step kk.  Accumulator element i of a lane is weight row
   // 4 * (lane / 16) + i of the wavefront's sixteen, token lane % 16: gated rows are ordered g, g + 1, u, u + 1.
   f32x4 acc[2];
@@ -1739,17 +1759,20 @@ __global__ __launch_bounds__(kThreads, 3) void stream_gemm_kernel(const GemmPara
     }
   }
 
-  issue(0);
-  if (1 < nu) issue(1);
-  if (2 < nu) issue(2);
+  issue(0, Tokens{});
+  if (1 < nu) issue(1, Tokens{});
+  if (2 < nu) issue(2, Both{});
   for (int u = 0; u < nu; ++u) {
-    // unit u has landed (only the two younger units may be outstanding) and nobody
+    // unit u has landed (only the two younger units may be outstanding; behind the token rows of unit 0, which were
+    // asked for after two units of weights, are those of unit 1 and all of unit 2) and nobody
     // reads unit u-1 any more, whose ring slot the next request reuses
-    if (u + 2 < nu) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(2 * kStDmaPerUnit) : "memory");
+    if (u == 0 && nu > 2) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(1 + kStDmaPerUnit) : "memory");
+    else if (u == 0 && nu > 1) asm volatile("s_waitcnt vmcnt(1) lgkmcnt(0)" ::: "memory");
+    else if (u + 2 < nu) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(2 * kStDmaPerUnit) : "memory");
     else if (u + 1 < nu) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kStDmaPerUnit) : "memory");
     else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     bare_barrier();
-    if (u + 3 < nu) issue(u + 3);
+    if (u + 3 < nu) issue(u + 3, Both{});
     const char* st = smem + (u % kStUnits) * kStUnitBytes;
     uint4 w[2], x[2][2];
 #pragma unroll
@@ -1787,6 +1810,7 @@ template <typename Mma, bool GATED>
 int launch_stream(GemmParams& p, int64_t sorted_cap, hipStream_t s) {
   p.num_m_blocks = static_cast<int>((sorted_cap + kStBM - 1) / kStBM);
   p.num_n_tiles = (p.N + (GATED ? kStRows / 2 : kStRows) - 1) / (GATED ? kStRows / 2 : kStRows);
+  p.n_tiles_rcp = static_cast<uint32_t>((1LL << 32) / p.num_n_tiles + 1);
   const int64_t tiles = static_cast<int64_t>(p.num_m_blocks) * p.num_n_tiles;
   const int64_t grid = (tiles + kXcds - 1) / kXcds * kXcds;
   if (grid > INT32_MAX) return moe_fail(MOE_ERR_ARG, "fused_experts: grid of %lld workgroups", static_cast<long long>(grid));

@@ -410,6 +410,22 @@ def test_streaming_kernel_keeps_slots_apart(moe, oracle, dev, dt, rows, monkeypa
     assert torch.equal(again[~bad], out[~bad])
 
 
+@pytest.mark.parametrize("I", [8, 16, 24, 32, 40, 72])
+@pytest.mark.parametrize("H", [32, 64, 96, 128, 192, 256])
+def test_streaming_kernel_finds_its_tile(moe, oracle, dev, H, I, monkeypatch):
+    """Runs of one to six blocks of one expert that begin at every place of a group of four, one to five column tiles
+    and rows of one to four units: every output element within tolerance of the oracle."""
+    monkeypatch.setattr(moe.fused_moe, "try_get_optimal_moe_config", lambda *a, **k: {"BLOCK_SIZE_M": 32})
+    blocks = [1, 2, 3, 4, 5, 6, 1, 1, 3, 2, 0, 4, 1]
+    ids = torch.cat([torch.full((32 * b - (7 if b else 0),), i, dtype=torch.int32) for i, b in enumerate(blocks)])
+    T = ids.numel()
+    ids = ids[torch.randperm(T, generator=torch.Generator().manual_seed(H + I))].view(T, 1)
+    x, w13, w2, _ = _layer(len(blocks), H, I, T, 1, H * I, torch.bfloat16)
+    tw = torch.rand(T, 1, generator=torch.Generator().manual_seed(I)) + 0.5
+    out = moe.fused_experts(x.to(dev), w13.to(dev), w2.to(dev), None, None, tw.to(dev), ids.to(dev))
+    _close(out, oracle.fused_experts_ref(x, w13, w2, tw, ids))
+
+
 def test_fp8_layered_prefill_batch_every_row(moe, oracle, dev):
     """Config 5: the 8192+256 batch with e4m3 weights and per-token e4m3
     activations, against the fp32 dequantised oracle and the one that rounds where the
