@@ -18,6 +18,8 @@
 #include "common.h"
 #include "routing_device.h"
 
+#include <type_traits>
+
 namespace {
 
 constexpr int kMaxExperts = 1024;
@@ -258,15 +260,13 @@ __device__ void align_small_body(const void* __restrict__ ids, int dtype, int nu
 // 8 to 1024 ids of 128 experts, blocks of 32: 8.0 to 10.2 us in align_small_kernel, 4.3 to 5.0 us here; registers and
 // skipped tail stores inside that kernel had changed nothing.
 constexpr int kTinyNumel = kScanThreads, kTinyExperts = 256;
-__global__ __launch_bounds__(kScanThreads) void align_tiny_kernel(
-    const int32_t* __restrict__ ids, int numel, int E, int BM, int id_bits, int32_t* __restrict__ sorted_ids,
-    int sorted_cap, int32_t* __restrict__ expert_ids, int expert_cap, int32_t* __restrict__ num_post_pad) {
-  __shared__ int cnt[kScanWaves * kTinyExperts];   // [wave][expert]: counts, then the first slot of the wave's ids
+// Thread i brings id i; `cnt` ([wave][expert] counts, then the first slot of the wave's ids) is zero.  Called by all
+// kScanThreads threads behind a barrier; contains barriers.
+__device__ __forceinline__ void align_tiny_body(
+    int id, int numel, int E, int BM, int id_bits, int32_t* __restrict__ sorted_ids, int sorted_cap,
+    int32_t* __restrict__ expert_ids, int expert_cap, int32_t* __restrict__ num_post_pad, int* cnt) {
   __shared__ int wave_tot[kTinyExperts / kWave];
   const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
-  const int id = tid < numel ? ids[tid] : -1;
-  for (int i = tid; i < kScanWaves * E; i += kScanThreads) cnt[i] = 0;
-  __syncthreads();
   const bool valid = id >= 0 && id < E;
   const uint64_t grp = same_id_lanes(id, valid, id_bits);
   const int below = __popcll(grp & lanes_below(lane));
@@ -312,6 +312,40 @@ __global__ __launch_bounds__(kScanThreads) void align_tiny_kernel(
   for (int b = all / BM + tid; b < expert_cap; b += kScanThreads) expert_ids[b] = 0;
   __syncthreads();
   if (valid) sorted_ids[cnt[wave * E + id] + below] = tid;
+}
+__global__ __launch_bounds__(kScanThreads) void align_tiny_kernel(
+    const int32_t* __restrict__ ids, int numel, int E, int BM, int id_bits, int32_t* __restrict__ sorted_ids,
+    int sorted_cap, int32_t* __restrict__ expert_ids, int expert_cap, int32_t* __restrict__ num_post_pad) {
+  __shared__ int cnt[kScanWaves * kTinyExperts];
+  const int tid = threadIdx.x;
+  const int id = tid < numel ? ids[tid] : -1;
+  for (int i = tid; i < kScanWaves * E; i += kScanThreads) cnt[i] = 0;
+  __syncthreads();
+  align_tiny_body(id, numel, E, BM, id_bits, sorted_ids, sorted_cap, expert_ids, expert_cap, num_post_pad, cnt);
+}
+
+// Routing in front of it, for the layer call: the ids stay in LDS.  The one workgroup routes its rows with the lane
+// layout, reduction order and results of topk_softmax_pow2_kernel, sixteen wavefronts side by side.
+template <int E, typename El>
+__global__ __launch_bounds__(kScanThreads) void route_align_tiny_kernel(
+    const typename El::S* __restrict__ gating, float* __restrict__ topk_w, int32_t* __restrict__ sorted_ids,
+    int32_t* __restrict__ expert_ids, int32_t* __restrict__ num_post_pad, int T, int K, int renormalize, int BM, int id_bits,
+    int sorted_cap, int expert_cap) {
+  using G = Pow2Geom<E>;
+  constexpr int VPT = G::kVpt, TPR = G::kTpr, RPW = G::kRowsPerWave;
+  __shared__ int cnt[kScanWaves * kTinyExperts], s_ids[kTinyNumel];
+  const int tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  for (int r0 = wave * RPW; r0 < T; r0 += kScanWaves * RPW) {  // (whole wavefronts take part in a row's exchanges)
+    const int row = r0 + lane / TPR;
+    float v[VPT];
+    load_row<E, El>(gating, row < T ? row : T - 1, lane % TPR, v);
+    route_row<E>(v, lane % TPR, row, row < T, topk_w, s_ids, nullptr, T, K, renormalize);
+  }
+  for (int i = tid; i < kScanWaves * E; i += kScanThreads) cnt[i] = 0;
+  __syncthreads();
+  const int numel = T * K;
+  align_tiny_body(tid < numel ? s_ids[tid] : -1, numel, E, BM, id_bits, sorted_ids, sorted_cap, expert_ids, expert_cap,
+                  num_post_pad, cnt);
 }
 
 __global__ __launch_bounds__(kScanThreads) void align_small_kernel(
@@ -774,6 +808,45 @@ MOE_EXPORT int moe_align_block_size_planned(const void* topk_ids, int ids_dtype,
   return align_impl(topk_ids, ids_dtype, numel, E, block_size, sorted_token_ids, sorted_cap, expert_ids,
                     expert_cap, num_tokens_post_pad, workspace, workspace_bytes, stream, plan_bounds,
                     plan_done, plan_num_done, plan_cap_mb);
+}
+
+// Routing and alignment of a layer call in one launch, where that is the faster way; see common.h.
+template <int E>
+static int launch_route_align_tiny(const void* logits, int dtype, float* topk_w, int T, int K, int renormalize, int block_size,
+                                   int32_t* sorted_ids, int sorted_cap, int32_t* expert_ids, int expert_cap, int32_t* npp,
+                                   hipStream_t s) {
+  auto go = [&](auto kernel, auto* gating) {
+    hipLaunchKernelGGL(kernel, dim3(1), dim3(kScanThreads), 0, s, gating, topk_w, sorted_ids, expert_ids, npp, T, K, renormalize,
+                       block_size, bits_for(E), sorted_cap, expert_cap);
+  };
+  if (dtype == MOE_BF16) go(route_align_tiny_kernel<E, ElemBF16>, static_cast<const ElemBF16::S*>(logits));
+  else if (dtype == MOE_F16) go(route_align_tiny_kernel<E, ElemF16>, static_cast<const ElemF16::S*>(logits));
+  else go(route_align_tiny_kernel<E, ElemF32>, static_cast<const ElemF32::S*>(logits));
+  return moe_check_launch("layer (routing and alignment)");
+}
+bool moe_layer_route_align(const void* logits, int dtype, float* topk_w, int T, int E, int K, int renormalize, int block_size,
+                           int32_t* sorted_ids, int64_t sorted_cap, int32_t* expert_ids, int64_t expert_cap, int32_t* npp,
+                           hipStream_t s, int* rc) {
+  // One CU routes all rows: with up to half its wavefronts at work that costs less than a launch and a trip of the ids
+  // through memory, with more of them the rows queue up.  Whole layer, us, against the two launches: E 128, H 2048,
+  // I 768, top-8: 28.1 and 29.2 at 1 token, 34.2 and 35.5 at 2, 54.0 and 54.8 at 9, 63.4 and 63.9 at 16, but 74.6 and
+  // 74.4 at 24, 96.6 and 95.7 at 32; E 32, I 1024, top-4: 23.8 and 25.5 at 1, 61.7 and 63.1 at 64, 75.4 and 75.4 at 128.
+  if (static_cast<int64_t>(T) * E > 2048 || static_cast<int64_t>(T) * K > kTinyNumel || K > E || K < 1 || block_size > 64 || !logits || sorted_cap > INT32_MAX ||
+      expert_cap > INT32_MAX || (dtype != MOE_BF16 && dtype != MOE_F16 && dtype != MOE_F32))
+    return false;
+  auto go = [&](auto tag) {
+    *rc = launch_route_align_tiny<decltype(tag)::value>(logits, dtype, topk_w, T, K, renormalize, block_size, sorted_ids,
+                                                        static_cast<int>(sorted_cap), expert_ids, static_cast<int>(expert_cap),
+                                                        npp, s);
+    return true;
+  };
+  switch (E) {
+    case 32: return go(std::integral_constant<int, 32>{});
+    case 64: return go(std::integral_constant<int, 64>{});
+    case 128: return go(std::integral_constant<int, 128>{});
+    case 256: return go(std::integral_constant<int, 256>{});
+    default: return false;
+  }
 }
 
 // Routing (moe_topk_softmax) and alignment (moe_align_block_size, with the plan of

@@ -29,6 +29,12 @@ struct MoeLdsOptIn {
 };
 int moe_opt_in_lds(MoeLdsOptIn& flags, const void* kernel, int lds_bytes, const char* what);
 
+// Router and alignment of a layer call in one launch, for the batches and layers where that is the faster way (align.hip);
+// false, and nothing enqueued, elsewhere.  `rc` is the launch's status.
+bool moe_layer_route_align(const void* logits, int dtype, float* topk_w, int T, int E, int K, int renormalize, int block_size,
+                           int32_t* sorted_ids, int64_t sorted_cap, int32_t* expert_ids, int64_t expert_cap, int32_t* npp,
+                           hipStream_t s, int* rc);
+
 // int32 index, inside the 256-byte table of per-XCD ranges at the end of a moe_fused_experts
 // workspace, of the count of expired waits of the one-launch form (cleared with the plan).
 constexpr int kMoeStatusWord = 16;

@@ -109,7 +109,13 @@ MOE_EXPORT int moe_layer(const MoeLayerArgs* a) {
   if (reinterpret_cast<uintptr_t>(a->workspace) & 255u)
     return moe_fail(MOE_ERR_WORKSPACE, "layer: workspace must be 256-byte aligned");
   const int64_t numel = static_cast<int64_t>(a->T) * a->K;
-  if (a->router_logits) {
+  int rc = MOE_OK;
+  const bool routed = a->router_logits &&
+                      moe_layer_route_align(a->router_logits, a->logits_dtype, l.topk_w, a->T, a->E, a->K, a->renormalize, l.block,
+                                            l.sorted, l.sorted_cap, l.experts, l.expert_cap, l.npp,
+                                            static_cast<hipStream_t>(a->stream), &rc);
+  if (rc) return rc;
+  if (a->router_logits && !routed) {
     if (int rc = moe_topk_softmax_typed(a->router_logits, a->logits_dtype, l.topk_w, l.topk_ids, nullptr, a->T, a->E, a->K,
                                         a->renormalize, a->stream))
       return rc;
@@ -121,13 +127,12 @@ MOE_EXPORT int moe_layer(const MoeLayerArgs* a) {
                     moe_fused_experts_plan_layout(a->T, a->H, a->I, a->E, a->K, l.block, a->act_dtype, a->weight_dtype,
                                                   &bounds_off, &done_off, &num_done, &cap_mb);
   char* fws = static_cast<char*>(l.fused_ws);
-  int rc;
   if (plan)
     rc = moe_align_block_size_planned(l.topk_ids, MOE_ID_I32, numel, a->E, l.block, l.sorted, l.sorted_cap, l.experts,
                                       l.expert_cap, l.npp, l.align_ws, l.align_bytes, a->stream,
                                       reinterpret_cast<int32_t*>(fws + bounds_off), reinterpret_cast<int32_t*>(fws + done_off),
                                       num_done, cap_mb);
-  else
+  else if (!routed)
     rc = moe_align_block_size(l.topk_ids, MOE_ID_I32, numel, a->E, l.block, l.sorted, l.sorted_cap, l.experts, l.expert_cap,
                               l.npp, l.align_ws, l.align_bytes, a->stream);
   if (rc) return rc;

@@ -426,6 +426,22 @@ def test_streaming_kernel_finds_its_tile(moe, oracle, dev, H, I, monkeypatch):
     _close(out, oracle.fused_experts_ref(x, w13, w2, tw, ids))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("E,T", [(32, 1), (32, 8), (32, 9), (32, 64), (32, 65), (64, 32), (64, 33), (128, 1), (128, 2),
+                                 (128, 3), (128, 16), (128, 17), (256, 8), (256, 9)])
+def test_routing_and_alignment_in_one_launch(moe, dev, E, T, dtype):
+    """The layer call of a small batch (up to 2048 logits: one launch in front of the experts) against the two
+    separate calls, bit for bit, with ties, top-1 to more winners than fit the router's registers."""
+    x, w13, w2, logits = _layer(E, 64, 32, T, 1, 7 * E + T, torch.bfloat16)
+    logits = logits.to(dtype)
+    logits[0, E // 2:] = logits[0, :E // 2]
+    d = [t.to(dev) for t in (x, logits, w13, w2)]
+    for K, renorm in ((1, False), (4, True), (15, True), (16, False), (17, True)):
+        tw, ids, _ = moe.fused_topk(d[0], d[1], K, renorm)
+        want = moe.fused_experts(d[0], d[2], d[3], None, None, tw, ids)
+        assert torch.equal(moe.fused_topk_experts(*d, K, renorm), want), (K, renorm)
+
+
 def test_fp8_layered_prefill_batch_every_row(moe, oracle, dev):
     """Config 5: the 8192+256 batch with e4m3 weights and per-token e4m3
     activations, against the fp32 dequantised oracle and the one that rounds where the
