@@ -89,6 +89,15 @@ int moe_gate_topk_softmax(const void* x, const void* gate_weight, int dtype, flo
                           float* topk_weights, int32_t* topk_ids, int32_t* token_expert_indices,
                           int T, int H, int E, int K, int renormalize, void* stream);
 
+/* The same for batches whose tokens fill few workgroups of moe_gate_topk_softmax: the linear cut in pieces of K, whose
+ * fp32 sums meet in `workspace` (16-byte aligned, at least the bytes that moe_gate_topk_few_bytes returns: 0 for sizes
+ * and types that this way does not serve or serves slower).  E 32 to 256, a power of two; token_expert_indices may be
+ * NULL. */
+int64_t moe_gate_topk_few_bytes(int T, int H, int E, int dtype);
+int moe_gate_topk_few(const void* x, const void* gate_weight, int dtype, float* topk_weights, int32_t* topk_ids,
+                      int32_t* token_expert_indices, int T, int H, int E, int K, int renormalize, void* workspace,
+                      int64_t workspace_bytes, void* stream);
+
 /* Replaces `moe_align_block_size` (csrc/moe_align_block_size_kernels.cu:239-291,
  * bound at csrc/ops.cpp:53-60,119-126).  `sorted_token_ids` (capacity
  * sorted_cap >= numel + E*(block_size-1)) receives, per expert in ascending

@@ -27,7 +27,7 @@ EXPORTS = (
     "moe_last_error", "moe_abi_version", "moe_topk_softmax", "moe_align_workspace_bytes",
     "moe_align_block_size", "moe_silu_and_mul", "moe_swigluoai_and_mul", "moe_sum",
     "moe_fused_experts_workspace_bytes", "moe_fused_experts", "moe_preferred_block_size", "moe_layer_block_size",
-    "moe_quant_rows_e4m3", "moe_gate_topk_softmax", "moe_add_rms_norm",
+    "moe_quant_rows_e4m3", "moe_gate_topk_softmax", "moe_gate_topk_few_bytes", "moe_gate_topk_few", "moe_add_rms_norm",
     "moe_align_can_plan", "moe_align_block_size_planned", "moe_fused_experts_plan_layout",
     "moe_fused_experts_status", "moe_fused_experts_set_wait_limit", "moe_align_block_size_static",
     "moe_tile_expert_weights", "moe_tile_expert_weights_supported",
@@ -100,6 +100,10 @@ def _declare(L: ctypes.CDLL) -> None:
     L.moe_layer_workspace_bytes.argtypes = [ctypes.POINTER(MoeLayerArgs)]
     L.moe_layer.restype = i32
     L.moe_layer.argtypes = [ctypes.POINTER(MoeLayerArgs)]
+    L.moe_gate_topk_few_bytes.restype = i64
+    L.moe_gate_topk_few_bytes.argtypes = [i32, i32, i32, i32]
+    L.moe_gate_topk_few.restype = i32
+    L.moe_gate_topk_few.argtypes = [p, p, i32, p, p, p, i32, i32, i32, i32, i32, p, i64, p]
     L.moe_gate_topk_softmax.restype = i32
     L.moe_gate_topk_softmax.argtypes = [p, p, i32, p, p, p, p, i32, i32, i32, i32, i32, p]
     L.moe_align_workspace_bytes.restype = i64

@@ -262,7 +262,9 @@ PyObject* rms_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// gate_topk(x, gate_weight, top_k, renormalize) -> (weights, ids, token_expert_indices), or None.
+// gate_topk(x, gate_weight, top_k, renormalize) -> (weights, ids, token_expert_indices), or None;
+// gate_topk_few: the same for batches that moe_gate_topk_few serves.
+template <bool FEW>
 PyObject* gate_topk(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   int64_t K;
@@ -276,7 +278,14 @@ PyObject* gate_topk(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (T < 1 || g->device() != dev || g->scalar_type() != x->scalar_type() || g->size(1) != H || K < 1 || K > E ||
       T * K > INT32_MAX || T * H * 2 >= (int64_t{1} << 32))
     MOE_NONE;
-  if ((dtype != MOE_BF16 && dtype != MOE_F16) || (E != 32 && E != 64 && E != 128) || H % 64) MOE_NONE;
+  int64_t few_bytes = 0;
+  if (FEW) {
+    if (T > INT32_MAX || H > INT32_MAX || E > INT32_MAX) MOE_NONE;
+    few_bytes = moe_gate_topk_few_bytes(static_cast<int>(T), static_cast<int>(H), static_cast<int>(E), dtype);
+    if (!few_bytes) MOE_NONE;
+  } else if ((dtype != MOE_BF16 && dtype != MOE_F16) || (E != 32 && E != 64 && E != 128) || H % 64) {
+    MOE_NONE;
+  }
   if ((reinterpret_cast<uintptr_t>(x->data_ptr()) | reinterpret_cast<uintptr_t>(g->data_ptr())) & 15u) MOE_NONE;
   c10::OptionalDeviceGuard guard(dev);
   void* const stream = current_stream(dev);
@@ -284,6 +293,12 @@ PyObject* gate_topk(PyObject*, PyObject* const* a, Py_ssize_t n) {
   at::Tensor w, ids, tei;
   check(enqueue([&] {
     w = empty({T, K}, at::kFloat, dev), ids = empty({T, K}, at::kInt, dev), tei = empty({T, K}, at::kInt, dev);
+    if (FEW) {
+      const at::Tensor scratch = empty({few_bytes / 4}, at::kFloat, dev);
+      return moe_gate_topk_few(in, gate, dtype, static_cast<float*>(w.data_ptr()), static_cast<int32_t*>(ids.data_ptr()),
+                               static_cast<int32_t*>(tei.data_ptr()), static_cast<int>(T), static_cast<int>(H),
+                               static_cast<int>(E), static_cast<int>(K), renormalize, scratch.data_ptr(), few_bytes, stream);
+    }
     return moe_gate_topk_softmax(in, gate, dtype, nullptr, static_cast<float*>(w.data_ptr()),
                                  static_cast<int32_t*>(ids.data_ptr()), static_cast<int32_t*>(tei.data_ptr()),
                                  static_cast<int>(T), static_cast<int>(H), static_cast<int>(E), static_cast<int>(K),
@@ -297,7 +312,8 @@ PyMethodDef methods[] = {
     {"layer", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(layer)), METH_FASTCALL, nullptr},
     {"topk", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(topk)), METH_FASTCALL, nullptr},
     {"rms_norm", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(rms_norm)), METH_FASTCALL, nullptr},
-    {"gate_topk", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(gate_topk)), METH_FASTCALL, nullptr},
+    {"gate_topk", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(gate_topk<false>)), METH_FASTCALL, nullptr},
+    {"gate_topk_few", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(gate_topk<true>)), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_moe_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

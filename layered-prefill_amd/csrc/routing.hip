@@ -9,6 +9,8 @@
 // Any other E takes one wavefront per row: in registers up to 1024 columns, in LDS up to 16384.
 #include <stdarg.h>
 
+#include <type_traits>
+
 #include "common.h"
 #include "routing_device.h"
 
@@ -218,6 +220,104 @@ int launch_gate_e(const void* x, const void* wg, float* logits_out, float* w, in
     default: return moe_fail(MOE_ERR_UNSUPPORTED, "gate_topk_softmax: num_experts %d (32, 64 or 128)", E);
   }
   return moe_check_launch("gate_topk_softmax");
+}
+
+// ---------------------------------------------------------------------------
+// The same for up to a few hundred tokens, as two short kernels.  A workgroup of the kernel above pulls all E gate rows
+// through one CU, which a CU does at 37 bytes a nanosecond (E 128, H 2048: 512 KB, 17 us, whatever T).  Here the gate
+// linear is cut in tokens, experts and K: a workgroup takes 16 tokens by 16 experts by 512 elements of K, everything it
+// reads (32 KB) is on its way at once, its four wavefronts multiply straight out of registers (MFMA 16x16x32, gate rows as
+// the A operand; a wavefront's two units of 64 elements fill whole lines) and add up in LDS.  The sums of the K pieces
+// leave in fp32; the kernel that routes adds them, rounds the logit once, to the activation dtype, as the output of a
+// gate linear is, and goes on with the lane layout of the stand-alone router.
+// ---------------------------------------------------------------------------
+typedef __attribute__((ext_vector_type(4))) float gate_f32x4;
+template <typename El>
+__device__ __forceinline__ gate_f32x4 gate_mma16(const uint4& a, const uint4& b, gate_f32x4 c) {
+  if constexpr (std::is_same_v<El, ElemBF16>)
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gate_bf16x8, a), __builtin_bit_cast(gate_bf16x8, b), c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(gate_f16x8, a), __builtin_bit_cast(gate_f16x8, b), c, 0, 0, 0);
+}
+constexpr int kPieceUnits = 8;                     // units of 64 elements in a piece of K
+constexpr int kPieceWaves = 4, kPieceThreads = kWave * kPieceWaves;
+static int gate_pieces(int H) { return (H / 64 + kPieceUnits - 1) / kPieceUnits; }
+
+// grid: token tiles x (pieces x expert tiles), the latter fastest, so that a gate piece stays with one XCD's L2
+template <typename El>
+__global__ __launch_bounds__(kPieceThreads) void gate_piece_kernel(
+    const typename El::S* __restrict__ x, const typename El::S* __restrict__ wg, float* __restrict__ sums, int T, int H, int E,
+    int pieces) {
+  constexpr int ROW = 16 + 4;  // floats of a token in LDS, padded: the sixteen tokens of a store spread over the banks
+  __shared__ __attribute__((aligned(16))) float part[kPieceWaves][16][ROW];
+  const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int l15 = lane & 15, lq = lane >> 4;
+  const int et = E / 16, per_token_tile = pieces * et;
+  const int t0 = blockIdx.x / per_token_tile * 16, rest = blockIdx.x % per_token_tile;
+  const int piece = rest / et, e0 = rest % et * 16;
+  const int nu = H / 64;
+  const typename El::S* xr = x + static_cast<size_t>(min(t0 + l15, T - 1)) * H + lq * 8;
+  const typename El::S* wr = wg + static_cast<size_t>(e0 + l15) * H + lq * 8;
+  gate_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  uint4 xf[4], wf[4];
+#pragma unroll
+  for (int kk = 0; kk < 4; ++kk) {
+    const int u = piece * kPieceUnits + 2 * wave + (kk >> 1);  // a unit behind the end of K: zeros
+    const size_t k = static_cast<size_t>(u) * 64 + (kk & 1) * 32;
+    wf[kk] = u < nu ? *reinterpret_cast<const uint4*>(wr + k) : uint4{0, 0, 0, 0};
+    xf[kk] = u < nu ? *reinterpret_cast<const uint4*>(xr + k) : uint4{0, 0, 0, 0};
+  }
+  __builtin_amdgcn_sched_barrier(0);  // all requests first
+#pragma unroll
+  for (int kk = 0; kk < 4; ++kk) acc = gate_mma16<El>(wf[kk], xf[kk], acc);
+  // acc[i]: token l15, expert 4 lq + i
+  *reinterpret_cast<gate_f32x4*>(&part[wave][l15][4 * lq]) = acc;
+  __syncthreads();
+  const int tok = threadIdx.x / 16, col = threadIdx.x % 16;
+  if (t0 + tok < T)
+    sums[(static_cast<size_t>(piece) * T + t0 + tok) * E + e0 + col] =
+        (part[0][tok][col] + part[1][tok][col]) + (part[2][tok][col] + part[3][tok][col]);
+}
+
+template <int E, typename El>
+__global__ __launch_bounds__(kWave* kWavesPerBlock) void topk_softmax_sums_kernel(
+    const float* __restrict__ sums, float* __restrict__ topk_w, int32_t* __restrict__ topk_ids,
+    int32_t* __restrict__ tok_exp_idx, int T, int K, int renormalize, int pieces) {
+  using G = Pow2Geom<E>;
+  constexpr int VPT = G::kVpt, TPR = G::kTpr;
+  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  const int row = (blockIdx.x * kWavesPerBlock + wave) * G::kRowsPerWave + lane / TPR;
+  const bool live = row < T;
+  const int ld_row = live ? row : (T - 1);
+  float v[VPT];
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) v[i] = 0.f;
+  for (int p0 = 0; p0 < pieces; p0 += 4) {
+    float q[4][VPT];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) load_row<E>(sums + static_cast<size_t>(min(p0 + j, pieces - 1)) * T * E, ld_row, lane % TPR, q[j]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (p0 + j < pieces)
+#pragma unroll
+        for (int i = 0; i < VPT; ++i) v[i] += q[j][i];
+  }
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) v[i] = El::ld(El::st(v[i]));
+  route_row<E>(v, lane % TPR, row, live, topk_w, topk_ids, tok_exp_idx, T, K, renormalize);
+}
+
+template <int E, typename El>
+int launch_gate_pieces(const void* x, const void* wg, float* sums, float* w, int32_t* ids, int32_t* tei, int T, int H, int K,
+                       int renorm, hipStream_t s) {
+  using S = typename El::S;
+  const int pieces = gate_pieces(H);
+  hipLaunchKernelGGL(gate_piece_kernel<El>, dim3(static_cast<unsigned>((T + 15) / 16) * pieces * (E / 16)), dim3(kPieceThreads), 0, s,
+                     static_cast<const S*>(x), static_cast<const S*>(wg), sums, T, H, E, pieces);
+  constexpr int rows = kWavesPerBlock * Pow2Geom<E>::kRowsPerWave;
+  hipLaunchKernelGGL((topk_softmax_sums_kernel<E, El>), dim3((T + rows - 1) / rows), dim3(kWave * kWavesPerBlock), 0, s, sums, w,
+                     ids, tei, T, K, renorm, pieces);
+  return moe_check_launch("gate_topk_softmax (pieces of K)");
 }
 
 // One wavefront per row; lane l holds columns l, l+64, ... (up to 16 of them).
@@ -452,4 +552,46 @@ MOE_EXPORT int moe_gate_topk_softmax(const void* x, const void* gate_weight, int
     case MOE_F16: return launch_gate_e<ElemF16>(x, gate_weight, logits_out, topk_weights, topk_ids, token_expert_indices, T, H, E, K, renormalize, s);
     default: return moe_fail(MOE_ERR_UNSUPPORTED, "gate_topk_softmax: dtype code %d (bf16 or fp16)", dtype);
   }
+}
+
+// Sizes for which the kernels that cut K serve a call: up to 768 workgroups of the first one, three a CU; then what all
+// token tiles read of the gate outgrows what fewer, larger tiles would.  us, gate linear and router, against the library's
+// GEMM and the router: E 128, H 2048, top-8: 8.1 and 10.8 at 1 token, 9.6 and 11.4 at 135, 9.9 and 11.4 at 256 (512
+// workgroups), 11.7 and 11.5 at 512 (1024), 15.6 and 12.1 at 1024; E 32, H 2048: 6.7 and 9.3 at 135, 7.8 and 9.6 at 1024
+// (512); E 64, H 4096: 9.1 and 12.5 at 135 (288), 11.4 and 12.7 at 512 (1024), 15.0 and 12.8 at 1024; E 256, H 7168: 18.8
+// and 15.0 at 135 (2016).  From Python the call is one entry into native code instead of two and an operator.
+MOE_EXPORT int64_t moe_gate_topk_few_bytes(int T, int H, int E, int dtype) {
+  if (T < 1 || H < 64 || H % 64 || (E != 32 && E != 64 && E != 128 && E != 256) || (dtype != MOE_BF16 && dtype != MOE_F16)) return 0;
+  if ((static_cast<int64_t>(T) + 15) / 16 * (E / 16) * gate_pieces(H) > 768) return 0;
+  return static_cast<int64_t>(gate_pieces(H)) * T * E * static_cast<int64_t>(sizeof(float));
+}
+
+template <typename El>
+static int launch_gate_pieces_e(const void* x, const void* wg, float* sums, float* w, int32_t* ids, int32_t* tei, int T, int H,
+                                int E, int K, int renorm, hipStream_t s) {
+  switch (E) {
+    case 32: return launch_gate_pieces<32, El>(x, wg, sums, w, ids, tei, T, H, K, renorm, s);
+    case 64: return launch_gate_pieces<64, El>(x, wg, sums, w, ids, tei, T, H, K, renorm, s);
+    case 128: return launch_gate_pieces<128, El>(x, wg, sums, w, ids, tei, T, H, K, renorm, s);
+    default: return launch_gate_pieces<256, El>(x, wg, sums, w, ids, tei, T, H, K, renorm, s);
+  }
+}
+
+MOE_EXPORT int moe_gate_topk_few(const void* x, const void* gate_weight, int dtype, float* topk_weights, int32_t* topk_ids,
+                                 int32_t* token_expert_indices, int T, int H, int E, int K, int renormalize, void* workspace,
+                                 int64_t workspace_bytes, void* stream) {
+  const int64_t need = moe_gate_topk_few_bytes(T, H, E, dtype);
+  if (need == 0) return moe_fail(MOE_ERR_UNSUPPORTED, "gate_topk_few: T=%d H=%d E=%d dtype code %d", T, H, E, dtype);
+  if (K < 1 || K > E) return moe_fail(MOE_ERR_ARG, "gate_topk_few: topk %d of %d experts", K, E);
+  if (!x || !gate_weight || !topk_weights || !topk_ids) return moe_fail(MOE_ERR_ARG, "gate_topk_few: null pointer");
+  if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(gate_weight)) & 15u)
+    return moe_fail(MOE_ERR_ARG, "gate_topk_few: x and the gate weight must be 16-byte aligned");
+  if (!workspace || workspace_bytes < need || (reinterpret_cast<uintptr_t>(workspace) & 15u))
+    return moe_fail(MOE_ERR_WORKSPACE, "gate_topk_few: workspace %lld B, needs %lld B, 16-byte aligned",
+                    static_cast<long long>(workspace_bytes), static_cast<long long>(need));
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  float* sums = static_cast<float*>(workspace);
+  return dtype == MOE_BF16
+             ? launch_gate_pieces_e<ElemBF16>(x, gate_weight, sums, topk_weights, topk_ids, token_expert_indices, T, H, E, K, renormalize, s)
+             : launch_gate_pieces_e<ElemF16>(x, gate_weight, sums, topk_weights, topk_ids, token_expert_indices, T, H, E, K, renormalize, s);
 }

@@ -125,12 +125,15 @@ def fused_gate_topk(hidden_states: torch.Tensor, gate_weight: torch.Tensor, topk
     """The gate linear (nanovllm/models/qwen3_moe.py:93-104,113) and ``fused_topk``
     (nanovllm/layers/for_moe/fused_moe.py:393-419) as one kernel when the shape
     allows and the batch is large enough for it to pay (a workgroup walks all of
-    K for 32 tokens: at a few hundred tokens the library GEMM's wider
-    parallelism wins, measured 13 us against 20 us at 256 tokens, 30 us against
-    28 us at 8448), else as the two steps the reference runs.  Returns what
+    K for 32 tokens: 20 us up to 4096 tokens, 27 us at 8448), as two kernels that
+    share K out over workgroups when it is small (``moe_gate_topk_few_bytes`` draws the
+    line: 9.6 us at 135 tokens of 128 experts, where the library's GEMM and the
+    router take 11.4), else as the two steps the reference runs.  Returns what
     ``fused_topk`` returns."""
-    if hidden_states.shape[0] >= FUSED_GATE_MIN_TOKENS and hidden_states.is_cuda:
-        routed = _lib.host().gate_topk(hidden_states, gate_weight, topk, renormalize)
+    if hidden_states.is_cuda:
+        host = _lib.host()
+        route = host.gate_topk if hidden_states.shape[0] >= FUSED_GATE_MIN_TOKENS else host.gate_topk_few
+        routed = route(hidden_states, gate_weight, topk, renormalize)
         if routed is not None:
             return routed
     if hidden_states.shape[0] >= FUSED_GATE_MIN_TOKENS and \

@@ -248,6 +248,27 @@ def test_gate_topk_softmax_against_oracle(moe, oracle, dev, dtype, T, H, E, K):
         assert torch.equal(w.cpu().view(torch.int32), ow.view(torch.int32))
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("E,H", [(32, 64), (32, 2048), (64, 448), (128, 512), (128, 576), (128, 2048), (256, 1088)])
+def test_gate_of_few_tokens_is_exact_where_the_sums_are(moe, oracle, dev, E, H, dtype):
+    """The gate cut in pieces of K, up to the last batch that it serves: small whole numbers (the gate's times 2^-6)
+    add up exactly in any order, so the logits are known and the routing must be the oracle's bit for bit.  The batch
+    behind the last one goes the two steps' way."""
+    served = lambda T: moe._lib.lib().moe_gate_topk_few_bytes(T, H, E, moe._lib.DTYPE_CODE[dtype]) > 0
+    last = next(T for T in range(1, 10**6) if not served(T + 1))
+    g = torch.Generator().manual_seed(E + H)
+    wg = torch.randint(-2, 3, (E, H), generator=g).float() / 64
+    for T in sorted({1, 15, 16, 17, 33, last, last + 1}):
+        x = torch.randint(-3, 4, (T, H), generator=g).float()
+        logits = (x @ wg.t()).to(dtype).float()
+        for K in (1, min(8, E), 17):
+            w, ids, tei = moe.fused_gate_topk(x.to(dtype).to(dev), wg.to(dtype).to(dev), K, T % 2 == 1)
+            ow, oids, otei = oracle.topk_softmax(logits, K, renormalize=T % 2 == 1)
+            assert torch.equal(ids.cpu(), oids) and torch.equal(tei.cpu(), otei), (T, K)
+            assert torch.equal(w.cpu().view(torch.int32), ow.view(torch.int32)), (T, K)
+
+
 def test_fused_gate_topk_falls_back_and_block_matches_two_step(moe, oracle, dev, monkeypatch):
     g = torch.Generator().manual_seed(11)
     # unsupported expert count: the gate runs as a plain linear, then fused_topk
