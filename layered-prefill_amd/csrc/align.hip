@@ -55,38 +55,51 @@ __device__ __forceinline__ int load_id(const void* ids, int dtype, int64_t i) {
 
 // Lanes of the wavefront whose (valid) id equals this lane's id.
 __device__ __forceinline__ uint64_t same_id_lanes(int id, bool valid, int id_bits) {
-  uint64_t m = __ballot(valid);
-  for (int b = 0; b < id_bits; ++b) {
-    const bool bit = (id >> b) & 1;
+  const uint64_t m = __ballot(valid);
+  uint32_t lo = static_cast<uint32_t>(m), hi = static_cast<uint32_t>(m >> 32);
+  // four vector instructions a bit: sixteen wavefronts share the issue of four SIMDs, and that bounds the ranking
+  auto keep = [&](int b) {
+    const int bit = (id << (31 - b)) >> 31;  // 0 or -1
     const uint64_t bal = __ballot(bit);
-    m &= bit ? bal : ~bal;
+    lo &= ~(static_cast<uint32_t>(bal) ^ bit);
+    hi &= ~(static_cast<uint32_t>(bal >> 32) ^ bit);
+  };
+  int b = 0;
+#pragma unroll
+  for (; b < 8; ++b) {
+    if (b == id_bits) break;
+    keep(b);
   }
-  return m;
+  for (; b < id_bits; ++b) keep(b);
+  return static_cast<uint64_t>(hi) << 32 | lo;
 }
 
 __device__ __forceinline__ uint64_t lanes_below(int lane) { return (1ull << lane) - 1ull; }
+
+// Inclusive prefix sum over a wavefront, by lane exchanges inside the vector unit: shifts inside rows of 16 lanes, then the
+// last lane of a row to the row behind it and of the first half to the second (a shuffle through the LDS crossbar costs
+// about a hundred clocks, six of them more than a short kernel's whole scan).
+__device__ __forceinline__ int wave_inclusive_scan(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);   // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);   // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);   // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);   // row_shr:8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
+  return v;
+}
 
 // Exclusive prefix sum of one int per thread over a kScanThreads workgroup.
 // `wave_tot` is LDS scratch of kScanWaves + 1 ints; slot kScanWaves receives
 // the grand total.  Contains workgroup barriers.
 __device__ int block_exclusive_scan(int v, volatile int* wave_tot) {
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-  int inc = v;
-#pragma unroll
-  for (int d = 1; d < kWave; d *= 2) {
-    int o = __shfl_up(inc, d, kWave);
-    if (lane >= d) inc += o;
-  }
+  const int inc = wave_inclusive_scan(v);
   if (lane == kWave - 1) wave_tot[wave] = inc;
   __syncthreads();
   if (wave == 0) {
     int w = lane < kScanWaves ? wave_tot[lane] : 0;
-    int winc = w;
-#pragma unroll
-    for (int d = 1; d < kScanWaves; d *= 2) {
-      int o = __shfl_up(winc, d, kWave);
-      if (lane >= d) winc += o;
-    }
+    const int winc = wave_inclusive_scan(w);
     if (lane < kScanWaves) wave_tot[lane] = winc - w;
     if (lane == kScanWaves - 1) wave_tot[kScanWaves] = winc;
   }
@@ -205,6 +218,75 @@ __device__ void plan_from_counts(const volatile int* cum, const volatile int* to
   }
 }
 
+// The same by one wavefront on its own, without a barrier, for up to kPlanWaveExperts experts and a total cost that times
+// eight fits an int: the others of the workgroup write padding meanwhile.  `s_b` (LDS): kPlanXcds + 1 ints of its own.
+constexpr int kPlanWaveExperts = 4 * kWave;
+__device__ __forceinline__ void plan_by_wave(const int* cum, const int* tot, int E, int cap_mb, int32_t* bounds, int32_t* done,
+                                             int num_done, volatile int* s_b) {
+  const int lane = threadIdx.x % kWave;
+  for (int i = lane; i < num_done; i += kWave) done[i] = 0;
+  int w[4], nb[4], first[4], sum = 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int e = 4 * lane + i;
+    w[i] = nb[i] = first[i] = 0;
+    if (e < E) {
+      nb[i] = (cum[e + 1] - cum[e]) / kPlanBlock;
+      first[i] = cum[e] / kPlanBlock;
+      const int r = tot[e] - (nb[i] - 1) * kPlanBlock;  // real slots of the expert's last block
+      if (nb[i] > 0) w[i] = (nb[i] - 1) * 64 + (r <= 32 ? 38 : (r <= 64 ? 48 : 64));
+    }
+    sum += w[i];
+  }
+  const int inc = wave_inclusive_scan(sum), excl = inc - sum;
+  const int total = __builtin_amdgcn_readlane(inc, kWave - 1), live_mb = __builtin_amdgcn_readfirstlane(cum[E]) / kPlanBlock;
+  if (lane <= kPlanXcds) s_b[lane] = lane == 0 ? 0 : live_mb;
+#pragma unroll
+  for (int x = 1; x < kPlanXcds; ++x) {
+    // the block whose cost takes the running sum across x / 8 of the total is the last of XCD x - 1
+    const int target = (total * x + kPlanXcds - 1) / kPlanXcds;
+    if (excl < target && inc >= target) {
+      int at = excl, n = nb[0], f = first[0], reached = excl + w[0];
+#pragma unroll
+      for (int i = 1; i < 4; ++i) {
+        if (reached < target) at = reached, n = nb[i], f = first[i];
+        reached += w[i];
+      }
+      const int j = (target - at + 63) / 64;  // full blocks cost 64 each
+      s_b[x] = f + (j < n ? j : n);
+    }
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the wavefront's own LDS writes
+  if (lane == 0) {
+    int b[kPlanXcds + 1];
+#pragma unroll
+    for (int x = 0; x <= kPlanXcds; ++x) b[x] = s_b[x];
+#pragma unroll
+    for (int x = 1; x <= kPlanXcds; ++x) b[x] = max(b[x], b[x - 1]);
+#pragma unroll
+    for (int x = 1; x <= kPlanXcds; ++x) b[x] = min(b[x], b[x - 1] + cap_mb);
+    b[kPlanXcds] = live_mb;
+#pragma unroll
+    for (int x = kPlanXcds - 1; x >= 1; --x) b[x] = max(b[x], b[x + 1] - cap_mb);
+#pragma unroll
+    for (int x = 0; x <= kPlanXcds; ++x) bounds[x] = b[x];
+    bounds[kMoeStatusWord] = 0;  // expired waits of the one-launch form
+  }
+}
+
+// Slots [beg, end) of sorted_ids take `value`, by one wavefront: 16 bytes a lane where the address allows it.  (The bounds
+// are the wavefront's, in scalar registers: what is left to the vector unit is three stores.)
+__device__ __forceinline__ void fill_slots(int32_t* __restrict__ sorted_ids, int beg, int end, int value) {
+  const int lane = threadIdx.x % kWave;
+  // the first slot at a 16-byte boundary (slots are 4-byte aligned, if that)
+  const int skew = static_cast<int>((reinterpret_cast<uintptr_t>(sorted_ids) >> 2) & 3);
+  const int head = min(end, ((beg + skew + 3) & ~3) - skew), vecs = (end - head) >> 2;
+  if (beg + lane < head) sorted_ids[beg + lane] = value;
+  for (int i = lane; i < vecs; i += kWave)
+    *reinterpret_cast<int4*>(sorted_ids + head + 4 * i) = int4{value, value, value, value};
+  if (head + 4 * vecs + lane < end) sorted_ids[head + 4 * vecs + lane] = value;
+}
+
 // The single-workgroup alignment: histogram, scans and scatter in LDS (`lds`: kScanWaves * E +
 // 2 E + kScanWaves + 2 ints).  Called by all kScanThreads threads; contains barriers.
 __device__ void align_small_body(const void* __restrict__ ids, int dtype, int numel, int E, int BM, int id_bits,
@@ -281,12 +363,7 @@ __device__ __forceinline__ void align_tiny_body(
       total += c[w];
     }
     padded = (total + BM - 1) / BM * BM;
-    inc = padded;
-#pragma unroll
-    for (int d = 1; d < kWave; d *= 2) {
-      const int o = __shfl_up(inc, d, kWave);
-      if (lane >= d) inc += o;
-    }
+    inc = wave_inclusive_scan(padded);
     if (lane == kWave - 1) wave_tot[wave] = inc;
   }
   __syncthreads();
@@ -363,16 +440,20 @@ __global__ __launch_bounds__(kScanThreads) void align_small_kernel(
 // registers and needs one pass over them: the lanes of an id read the wavefront's count so far, which is the
 // rank of the first of them, and the lowest one advances it.
 // 128 experts, blocks of 256 with the plan: 5928 ids 20.7 us in align_small_kernel, which passes over its ids twice
-// and loads them in each, 13.6 us here.
+// and loads them in each, 11.9 us here.  The rest of it is the issue of one CU's four SIMDs: with ranks in half the
+// instructions, N as small as the ids allow (2048 ids left half the wavefronts idle), sums across lanes without the LDS
+// crossbar, padding in 16-byte stores and the plan by one wavefront while the others write it, 11.9 -> 10.2 us; 2048 ids
+// 8.8 -> 7.1, 1204 ids of 32 experts, blocks of 32, 5.1 -> 4.4, 67584 ids (two kernels, same ranks and sums) 17.3 -> 16.1.
 template <int N>
 __global__ __launch_bounds__(kScanThreads) void align_mid_kernel(
     const int32_t* __restrict__ ids, int numel, int E, int BM, int id_bits, int32_t* __restrict__ sorted_ids,
     int sorted_cap, int32_t* __restrict__ expert_ids, int expert_cap, int32_t* __restrict__ num_post_pad,
     int32_t* plan_bounds, int32_t* plan_done, int plan_num_done, int plan_cap_mb) {
   __shared__ int s_cnt[kScanWaves * kTinyExperts];   // [wave][expert]: counts, then the first slot of the wave's ids
-  __shared__ int s_cum[kTinyExperts + 1], s_tot[kTinyExperts], s_wave[kScanWaves + 1];
+  __shared__ int s_cum[kTinyExperts + 1], s_tot[kTinyExperts], s_wave[kScanWaves + 1], s_plan[kPlanXcds + 1];
+  static_assert(kTinyExperts <= kPlanWaveExperts, "one wavefront plans");
   volatile int* cnt = s_cnt;
-  const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
+  const int tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int beg = wave * (N * kWave) + lane;
   int id[N], rank[N];
 #pragma unroll
@@ -422,13 +503,18 @@ __global__ __launch_bounds__(kScanThreads) void align_mid_kernel(
 #pragma unroll
   for (int j = 0; j < N; ++j)
     if (id[j] >= 0) sorted_ids[s_cnt[wave * E + id[j]] + rank[j]] = beg + j * kWave;
-  for (int e = wave; e < E; e += kScanWaves) {
-    const int end = s_cum[e + 1];
-    for (int p = s_cum[e] + s_tot[e] + lane; p < end; p += kWave) sorted_ids[p] = numel;
+  if (plan_bounds && wave == 0) {
+    plan_by_wave(s_cum, s_tot, E, plan_cap_mb, plan_bounds, plan_done, plan_num_done, s_plan);
+    return;
   }
-  for (int p = all + tid; p < sorted_cap; p += kScanThreads) sorted_ids[p] = numel;
-  for (int b = all / BM + tid; b < expert_cap; b += kScanThreads) expert_ids[b] = 0;
-  if (plan_bounds) plan_from_counts(s_cum, s_tot, E, plan_cap_mb, plan_bounds, plan_done, plan_num_done, s_wave);
+  // padding, the wavefronts left taking turns: of the experts' last blocks, then behind all of them
+  const int w0 = plan_bounds ? 1 : 0;
+  for (int e = wave - w0; e < E; e += kScanWaves - w0)
+    fill_slots(sorted_ids, __builtin_amdgcn_readfirstlane(s_cum[e] + s_tot[e]), __builtin_amdgcn_readfirstlane(s_cum[e + 1]), numel);
+  constexpr int kTail = 4 * kWave;
+  for (int p = __builtin_amdgcn_readfirstlane(all) + (wave - w0) * kTail; p < sorted_cap; p += (kScanWaves - w0) * kTail)
+    fill_slots(sorted_ids, p, min(p + kTail, sorted_cap), numel);
+  for (int b = all / BM + tid - w0 * kWave; b < expert_cap; b += kScanThreads - w0 * kWave) expert_ids[b] = 0;
 }
 
 // Routing and alignment of a very small batch in one launch (such a call is a handful of short
@@ -731,7 +817,8 @@ static int align_impl(const void* topk_ids, int ids_dtype, int64_t numel, int E,
   }
   if (numel <= 8 * kScanThreads && E <= kTinyExperts && ids_dtype == MOE_ID_I32 && sorted_cap <= INT32_MAX &&
       expert_cap <= INT32_MAX) {
-    auto kern = numel <= 4 * kScanThreads ? align_mid_kernel<4> : align_mid_kernel<8>;
+    auto kern = numel <= 2 * kScanThreads ? align_mid_kernel<2> : numel <= 4 * kScanThreads ? align_mid_kernel<4>
+              : numel <= 6 * kScanThreads ? align_mid_kernel<6> : align_mid_kernel<8>;
     hipLaunchKernelGGL(kern, dim3(1), dim3(kScanThreads), 0, s, static_cast<const int32_t*>(topk_ids),
                        static_cast<int>(numel), E, block_size, id_bits, sorted_token_ids, static_cast<int>(sorted_cap),
                        expert_ids, static_cast<int>(expert_cap), num_tokens_post_pad, plan_bounds, plan_done, plan_num_done,

@@ -163,6 +163,22 @@ def test_alignment_of_a_small_batch(moe, oracle, dev, numel, E, bm):
         assert torch.equal(a.cpu(), b)
 
 
+@pytest.mark.parametrize("numel,E,bm", [(2047, 128, 256), (2048, 7, 3), (2049, 256, 32), (4095, 128, 65), (6143, 128, 256),
+                                        (6144, 256, 1), (6145, 3, 256)])
+@pytest.mark.parametrize("skew", [0, 1, 2, 3])
+def test_alignment_into_slots_at_any_address(moe, oracle, dev, numel, E, bm, skew):
+    """Both sides of the sizes up to which two, four, six and eight loads per thread serve, into outputs that begin at
+    every place of 16 bytes; what lies around them stays."""
+    ids = _skewed_ids(numel, E, numel + E + skew)
+    want = oracle.moe_align_block_size(ids, bm, E)
+    bufs = [torch.full((w.numel() + 8,), -9, dtype=torch.int32, device=dev) for w in want]
+    views = [b[skew + 1:skew + 1 + w.numel()] for b, w in zip(bufs, want)]
+    moe.ops.moe_align_block_size(ids.to(dev), E, bm, *views)
+    for b, v, w in zip(bufs, views, want):
+        assert torch.equal(v.cpu(), w.to(torch.int32).view(-1))
+        assert (b[:skew + 1] == -9).all() and (b[skew + 1 + w.numel():] == -9).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.int32, torch.int64, torch.int16, torch.uint8, torch.int8])
 def test_moe_align_block_size_id_dtypes_and_out_of_range_ids(moe, oracle, dev, dtype):
     E = 100
