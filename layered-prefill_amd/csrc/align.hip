@@ -916,8 +916,9 @@ bool moe_layer_route_align(const void* logits, int dtype, float* topk_w, int T, 
                            hipStream_t s, int* rc) {
   // One CU routes all rows: with up to half its wavefronts at work that costs less than a launch and a trip of the ids
   // through memory, with more of them the rows queue up.  Whole layer, us, against the two launches: E 128, H 2048,
-  // I 768, top-8: 28.1 and 29.2 at 1 token, 34.2 and 35.5 at 2, 54.0 and 54.8 at 9, 63.4 and 63.9 at 16, but 74.6 and
-  // 74.4 at 24, 96.6 and 95.7 at 32; E 32, I 1024, top-4: 23.8 and 25.5 at 1, 61.7 and 63.1 at 64, 75.4 and 75.4 at 128.
+  // I 768, top-8: 26.0 and 27.1 at 1 token, 52.4 and 53.0 at 9, 60.4 and 60.9 at 16, but 71.5 and 71.1 at 24, 92.6 and
+  // 91.5 at 32; E 64: 74.9 and 75.6 at 32, 97.6 and 96.7 at 64; E 32, I 1024, top-4: 23.1 and 24.0 at 1, 61.4 and 61.9 at
+  // 64, 74.7 and 74.3 at 128.
   if (static_cast<int64_t>(T) * E > 2048 || static_cast<int64_t>(T) * K > kTinyNumel || K > E || K < 1 || block_size > 64 || !logits || sorted_cap > INT32_MAX ||
       expert_cap > INT32_MAX || (dtype != MOE_BF16 && dtype != MOE_F16 && dtype != MOE_F32))
     return false;

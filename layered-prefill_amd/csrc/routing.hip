@@ -556,10 +556,10 @@ MOE_EXPORT int moe_gate_topk_softmax(const void* x, const void* gate_weight, int
 
 // Sizes for which the kernels that cut K serve a call: up to 768 workgroups of the first one, three a CU; then what all
 // token tiles read of the gate outgrows what fewer, larger tiles would.  us, gate linear and router, against the library's
-// GEMM and the router: E 128, H 2048, top-8: 8.1 and 10.8 at 1 token, 9.6 and 11.4 at 135, 9.9 and 11.4 at 256 (512
-// workgroups), 11.7 and 11.5 at 512 (1024), 15.6 and 12.1 at 1024; E 32, H 2048: 6.7 and 9.3 at 135, 7.8 and 9.6 at 1024
-// (512); E 64, H 4096: 9.1 and 12.5 at 135 (288), 11.4 and 12.7 at 512 (1024), 15.0 and 12.8 at 1024; E 256, H 7168: 18.8
-// and 15.0 at 135 (2016).  From Python the call is one entry into native code instead of two and an operator.
+// GEMM and the router: E 128, H 2048, top-8: 6.5 and 9.2 at 1 token, 7.8 and 9.3 at 135, 9.1 and 9.4 at 384 (768
+// workgroups), 10.0 and 9.3 at 512 (1024), 13.8 and 10.4 at 1024; E 32, H 2048: 6.2 and 9.0 at 135, 7.3 and 9.1 at 1024
+// (512); E 64, H 4096: 8.0 and 11.6 at 135 (288), 10.2 and 11.7 at 512 (1024), 13.9 and 11.8 at 1024; E 256, H 7168: 17.3
+// and 13.5 at 135 (2016).  From Python the call is one entry into native code instead of two and an operator.
 MOE_EXPORT int64_t moe_gate_topk_few_bytes(int T, int H, int E, int dtype) {
   if (T < 1 || H < 64 || H % 64 || (E != 32 && E != 64 && E != 128 && E != 256) || (dtype != MOE_BF16 && dtype != MOE_F16)) return 0;
   if ((static_cast<int64_t>(T) + 15) / 16 * (E / 16) * gate_pieces(H) > 768) return 0;

@@ -18,41 +18,55 @@ struct Pow2Geom {
 
 constexpr int kWavesPerBlock = 4;
 
-// Lane exchange for the order-independent reductions (max, argmax): partner at
-// distance M inside a row of TPR lanes.  Distances 1 and 2 are exact xor
-// butterflies (quad_perm); 4 and 8 use the mirror patterns of DPP, which pair
-// every lane with a lane of the other half of its 8- or 16-lane group: the same
-// thing once the lanes of each half already agree, which is why these
-// reductions run from distance 1 upwards.  DPP moves cost a few clocks; the
-// LDS-crossbar shuffle behind __shfl_xor costs ~100 and was most of a round.
-template <int M>
-__device__ __forceinline__ int lane_exchange(int v) {
-  if constexpr (M == 1) return __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xf, 0xf, true);        // quad_perm [1,0,3,2]
-  else if constexpr (M == 2) return __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xf, 0xf, true);   // quad_perm [2,3,0,1]
-  else if constexpr (M == 4) return __builtin_amdgcn_update_dpp(0, v, 0x141, 0xf, 0xf, true);  // row_half_mirror
-  else if constexpr (M == 8) return __builtin_amdgcn_update_dpp(0, v, 0x140, 0xf, 0xf, true);  // row_mirror
-  else return __shfl_xor(v, M, kWave);
+// Lane exchanges of a row of TPR lanes, by DPP moves and v_permlane16_swap: a few clocks each, where the LDS-crossbar
+// shuffle behind __shfl_xor costs ~100 and was most of a round.
+// max over the row: any order will do, so distances 4 and 8 use the mirror patterns, which pair every lane with a lane of
+// the other half of its 8- or 16-lane group: the same thing once the lanes of each half already agree.
+template <int CTRL>
+__device__ __forceinline__ float dpp_move(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
 }
-template <int M>
-__device__ __forceinline__ float lane_exchange(float v) {
-  return __builtin_bit_cast(float, lane_exchange<M>(__builtin_bit_cast(int, v)));
+// The values of the lane's row of 16 and of the row beside it (lane ^ 16), as an unordered pair.  (In assembly: given the
+// same value twice, the compiler takes the builtin's two results for one.  The wait states are those that it puts in
+// front of the instruction.)
+__device__ __forceinline__ void rows_of_16(float v, float& a, float& b) {
+  a = b = v;
+  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
 }
-
-template <int M, int TPR>
-__device__ __forceinline__ void max_level(float& mx) {
-  if constexpr (M < TPR) {
-    mx = fmaxf(mx, lane_exchange<M>(mx));
-    max_level<M * 2, TPR>(mx);
+template <int TPR>
+__device__ __forceinline__ float row_max(float v) {
+  static_assert(TPR <= 32, "a row of lanes");
+  if constexpr (TPR > 1) v = fmaxf(v, dpp_move<0xB1>(v));   // quad_perm [1,0,3,2]
+  if constexpr (TPR > 2) v = fmaxf(v, dpp_move<0x4E>(v));   // quad_perm [2,3,0,1]
+  if constexpr (TPR > 4) v = fmaxf(v, dpp_move<0x141>(v));  // row_half_mirror
+  if constexpr (TPR > 8) v = fmaxf(v, dpp_move<0x140>(v));  // row_mirror
+  if constexpr (TPR > 16) {
+    float a, b;
+    rows_of_16(v, a, b);
+    v = fmaxf(a, b);
   }
+  return v;
 }
-template <int M, int TPR>
-__device__ __forceinline__ void argmax_level(float& best, int& bidx) {
-  if constexpr (M < TPR) {
-    const float ov = lane_exchange<M>(best);
-    const int oi = lane_exchange<M>(bidx);
-    if (ov > best || (ov == best && oi < bidx)) { best = ov; bidx = oi; }
-    argmax_level<M * 2, TPR>(best, bidx);
+// The sum with the association of the xor butterfly from distance TPR / 2 down to 1.
+template <int TPR>
+__device__ __forceinline__ float row_sum(float v) {
+  static_assert(TPR <= 32, "a row of lanes");
+  if constexpr (TPR > 16) {
+    float a, b;
+    rows_of_16(v, a, b);
+    v = a + b;
   }
+  if constexpr (TPR > 8) v += dpp_move<0x128>(v);  // row_ror:8 is lane ^ 8
+  if constexpr (TPR > 8) {
+    v += dpp_move<0x124>(v);                       // row_ror:4 is lane ^ 4 where lanes eight apart agree
+  } else if constexpr (TPR > 4) {
+    // lane ^ 4: row_shl:4 into the first and third four lanes of a row of 16, row_shr:4 into the others
+    const int b = __builtin_bit_cast(int, v), up = __builtin_amdgcn_update_dpp(0, b, 0x104, 0xf, 0x5, false);
+    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(up, b, 0x114, 0xf, 0xa, false));
+  }
+  if constexpr (TPR > 2) v += dpp_move<0x4E>(v);   // quad_perm [2,3,0,1]
+  if constexpr (TPR > 1) v += dpp_move<0xB1>(v);   // quad_perm [1,0,3,2]
+  return v;
 }
 
 // The logits of row `row` as route_row wants them, widened to fp32: lane t of the row loads columns
@@ -90,7 +104,7 @@ __device__ __forceinline__ void route_row(float (&v)[Pow2Geom<E>::kVpt], int t, 
   float mx = v[0];
 #pragma unroll
   for (int i = 1; i < VPT; ++i) mx = fmaxf(mx, v[i]);
-  max_level<1, TPR>(mx);
+  mx = row_max<TPR>(mx);
 
   float sum = 0.f;
 #pragma unroll
@@ -98,8 +112,7 @@ __device__ __forceinline__ void route_row(float (&v)[Pow2Geom<E>::kVpt], int t, 
     v[i] = moe_expf(v[i] - mx);
     sum += v[i];
   }
-#pragma unroll
-  for (int m = TPR / 2; m > 0; m /= 2) sum += __shfl_xor(sum, m, kWave);
+  sum = row_sum<TPR>(sum);
   const float rinv = 1.f / sum;
 #pragma unroll
   for (int i = 0; i < VPT; ++i) v[i] = v[i] * rinv;  // subnormal probabilities are kept, as the reference keeps them
@@ -115,24 +128,39 @@ __device__ __forceinline__ void route_row(float (&v)[Pow2Geom<E>::kVpt], int t, 
   int bi[kRegK];
 #pragma unroll
   for (int k = 0; k < kRegK; ++k) { bw[k] = 0.f; bi[k] = 0; }
+  // One round: the row's largest value, then the lowest of the columns that hold it, from one ballot per value of a
+  // lane.  (Column 0 where none does: all values NaN.  A row of one lane looks for itself.)  Carrying value and column
+  // through every exchange, two of them through the LDS crossbar, was most of the kernel: 128 experts top-8, 1 token
+  // 5.4 -> 3.7 us, 256 tokens 5.9 -> 4.2, 16896 13.4 -> 12.0.
+  const int lane = threadIdx.x % kWave, row0 = lane & 31 & ~(TPR - 1);
   auto round = [&](float& best_out, int& bidx_out) {
     float best = v[0];
-    int bidx = t * EPL;
+    uint32_t col = TPR == 1 ? 0u : ~0u;
 #pragma unroll
     for (int i = 1; i < VPT; ++i) {
-      const int col = (i / EPL) * (EPL * TPR) + t * EPL + (i % EPL);
-      if (v[i] > best) { best = v[i]; bidx = col; }
+      if constexpr (TPR == 1) {
+        if (v[i] > best) best = v[i], col = i;
+      } else {
+        best = fmaxf(best, v[i]);
+      }
     }
-    argmax_level<1, TPR>(best, bidx);
+    best = row_max<TPR>(best);
+#pragma unroll
+    for (int i = 0; TPR > 1 && i < VPT; ++i) {
+      const uint64_t bal = __ballot(v[i] == best);
+      const uint32_t half = lane & 32 ? static_cast<uint32_t>(bal >> 32) : static_cast<uint32_t>(bal);
+      const uint32_t mine = TPR == 32 ? half : __builtin_amdgcn_ubfe(half, row0, TPR);
+      const uint32_t c = (i / EPL) * (EPL * TPR) + static_cast<uint32_t>(__builtin_ctz(mine)) * EPL + i % EPL;
+      col = min(col, mine ? c : ~0u);
+    }
+    const int bidx = col == ~0u ? 0 : static_cast<int>(col);
     wsum += best;
     best_out = best;
     bidx_out = bidx;
     // blank the winner in the lane that holds it
-    const int owner = (bidx / EPL) % TPR;
-    const int slot = (bidx / (EPL * TPR)) * EPL + (bidx % EPL);
 #pragma unroll
     for (int i = 0; i < VPT; ++i)
-      if (t == owner && i == slot) v[i] = -10000.f;
+      if (bidx == (i / EPL) * (EPL * TPR) + t * EPL + i % EPL) v[i] = -10000.f;
   };
   if (K <= kRegK) {
 #pragma unroll

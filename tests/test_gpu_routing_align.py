@@ -150,6 +150,22 @@ def test_moe_align_block_size_bit_exact(moe, oracle, dev, numel, E, bm):
     assert torch.equal(s.cpu(), os_)
 
 
+@pytest.mark.parametrize("E", [1, 2, 4, 8, 16, 32, 64, 128, 256])
+def test_rows_without_a_largest_value(moe, oracle, dev, E):
+    """A row of NaN (or with an infinity, which makes all its probabilities NaN) routes to experts that exist and leaves
+    the rows that share its wavefront alone; -inf beside finite logits is a probability of zero."""
+    T, K = 70, min(E, 5)
+    logits = torch.randn(T, E, generator=torch.Generator().manual_seed(E))
+    logits[3], logits[20], logits[41, 0] = float("nan"), float("-inf"), float("inf")
+    logits[50, E // 2:] = float("-inf") if E > 1 else 0.0
+    ow, oids, _ = oracle.topk_softmax(logits, K, renormalize=True)
+    w, ids, _ = moe.fused_topk(torch.empty(T, 8, device=dev), logits.to(dev), K, True)
+    good = torch.ones(T, dtype=torch.bool)
+    good[[3, 20, 41]] = False
+    assert torch.equal(ids.cpu()[good], oids[good]) and torch.equal(w.cpu()[good], ow[good])
+    assert torch.isnan(w.cpu()[~good]).all() and ids.min() >= 0 and ids.max() < E
+
+
 @pytest.mark.parametrize("bm", [1, 32, 64, 65, 256])
 @pytest.mark.parametrize("numel", [0, 1, 63, 64, 65, 1023, 1024, 1025, 4096, 4097, 8191, 8192, 8193])
 @pytest.mark.parametrize("E", [1, 3, 64, 128, 256, 257])
