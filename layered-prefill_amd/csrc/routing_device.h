@@ -18,57 +18,6 @@ struct Pow2Geom {
 
 constexpr int kWavesPerBlock = 4;
 
-// Lane exchanges of a row of TPR lanes, by DPP moves and v_permlane16_swap: a few clocks each, where the LDS-crossbar
-// shuffle behind __shfl_xor costs ~100 and was most of a round.
-// max over the row: any order will do, so distances 4 and 8 use the mirror patterns, which pair every lane with a lane of
-// the other half of its 8- or 16-lane group: the same thing once the lanes of each half already agree.
-template <int CTRL>
-__device__ __forceinline__ float dpp_move(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
-}
-// The values of the lane's row of 16 and of the row beside it (lane ^ 16), as an unordered pair.  (In assembly: given the
-// same value twice, the compiler takes the builtin's two results for one.  The wait states are those that it puts in
-// front of the instruction.)
-__device__ __forceinline__ void rows_of_16(float v, float& a, float& b) {
-  a = b = v;
-  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
-}
-template <int TPR>
-__device__ __forceinline__ float row_max(float v) {
-  static_assert(TPR <= 32, "a row of lanes");
-  if constexpr (TPR > 1) v = fmaxf(v, dpp_move<0xB1>(v));   // quad_perm [1,0,3,2]
-  if constexpr (TPR > 2) v = fmaxf(v, dpp_move<0x4E>(v));   // quad_perm [2,3,0,1]
-  if constexpr (TPR > 4) v = fmaxf(v, dpp_move<0x141>(v));  // row_half_mirror
-  if constexpr (TPR > 8) v = fmaxf(v, dpp_move<0x140>(v));  // row_mirror
-  if constexpr (TPR > 16) {
-    float a, b;
-    rows_of_16(v, a, b);
-    v = fmaxf(a, b);
-  }
-  return v;
-}
-// The sum with the association of the xor butterfly from distance TPR / 2 down to 1.
-template <int TPR>
-__device__ __forceinline__ float row_sum(float v) {
-  static_assert(TPR <= 32, "a row of lanes");
-  if constexpr (TPR > 16) {
-    float a, b;
-    rows_of_16(v, a, b);
-    v = a + b;
-  }
-  if constexpr (TPR > 8) v += dpp_move<0x128>(v);  // row_ror:8 is lane ^ 8
-  if constexpr (TPR > 8) {
-    v += dpp_move<0x124>(v);                       // row_ror:4 is lane ^ 4 where lanes eight apart agree
-  } else if constexpr (TPR > 4) {
-    // lane ^ 4: row_shl:4 into the first and third four lanes of a row of 16, row_shr:4 into the others
-    const int b = __builtin_bit_cast(int, v), up = __builtin_amdgcn_update_dpp(0, b, 0x104, 0xf, 0x5, false);
-    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(up, b, 0x114, 0xf, 0xa, false));
-  }
-  if constexpr (TPR > 2) v += dpp_move<0x4E>(v);   // quad_perm [2,3,0,1]
-  if constexpr (TPR > 1) v += dpp_move<0xB1>(v);   // quad_perm [1,0,3,2]
-  return v;
-}
-
 // The logits of row `row` as route_row wants them, widened to fp32: lane t of the row loads columns
 // (i / EPL) * EPL * TPR + t * EPL + i % EPL into v[i], EPL at a time.  A caller's rows need no more than the
 // alignment of an element, and the type says so; the load is one instruction all the same (a global load takes

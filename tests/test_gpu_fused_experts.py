@@ -250,6 +250,21 @@ def test_swigluoai_and_mul_bit_exact(moe, oracle, dev, dtype, rows, d):
                        want.view(torch.int16 if dtype != torch.float32 else torch.int32))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T,K,H", [(1, 8, 8), (3, 4, 24), (5, 8, 2048), (7, 4, 72), (2, 7, 64), (9, 9, 40), (1, 8, 4), (6, 4, 9),
+                                   (9300, 8, 2048)])
+def test_moe_sum_adds_in_order(moe, dev, T, K, H, dtype):
+    """Terms in ascending order, one fp32 addition each, bit for bit: four and eight at once, other numbers, rows that
+    are no whole vectors, and more than the caches hold."""
+    x = torch.randn(T, K, H, device=dev, dtype=torch.float32).to(dtype)
+    out = torch.empty(T, H, device=dev, dtype=dtype)
+    moe.ops.moe_sum(x, out)
+    want = torch.zeros(T, H, device=dev)
+    for k in range(K):
+        want += x[:, k].float()
+    assert torch.equal(out, want.to(dtype))
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 def test_moe_sum(moe, dev, dtype):
     x = torch.randn(33, 8, 200, generator=torch.Generator().manual_seed(3)).to(dtype)
