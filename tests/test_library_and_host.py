@@ -248,6 +248,22 @@ def test_layer_block_size_changes_once_at_its_line(moe, I, E, K, act, wgt, line)
     assert sizes == [32] * line + [256] * (300 - line)
 
 
+@pytest.mark.parametrize("E,H,I,K,weights,layout,last", [
+    (128, 2048, 768, 8, 2, 0, 263), (128, 2048, 768, 8, 1, 0, 263), (128, 2048, 768, 8, 2, 1, 255), (32, 2048, 1024, 4, 2, 0, 397),
+    (128, 2880, 1440, 4, 2, 0, 597), (32, 2048, 1024, 4, 3, 0, 701), (128, 2880, 1440, 4, 3, 0, 1194), (128, 2048, 768, 8, 3, 0, 511),
+    (128, 512, 128, 2, 2, 0, 16108), (6, 24, 40, 2, 2, 0, 287)])
+def test_layer_call_changes_its_block_once_at_its_line(moe, E, H, I, K, weights, layout, last):
+    """The last batch that streams, by the call's matrix work (and at least 16, e4m3 32, rows per expert; sizes that only
+    the register-staged kernels take keep the rule by rows): the workspace a call asks for is that of the block it will use."""
+    L, A = moe._lib.lib(), moe._lib.MoeLayerArgs
+    act = weights if weights != 3 else 2
+    need = lambda T, block: L.moe_layer_workspace_bytes(A(T=T, H=H, I=I, E=E, K=K, act_dtype=act, weight_dtype=weights,
+                                                         weight_layout=layout, block_size=block, router_logits=1))
+    for T in (1, last // 2, last, last + 1, 2 * last, 16896):
+        assert need(T, 32) != need(T, 256)
+        assert need(T, 0) == need(T, 32 if T <= last else 256), T
+
+
 def test_layer_block_size_of_fp32_is_the_old_rule(moe):
     L = moe._lib.lib()
     for m in (1, 256, 768, 2048, 8448):
