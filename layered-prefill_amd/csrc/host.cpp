@@ -6,6 +6,7 @@
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
+#include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/ops/empty.h>
 #include <c10/core/DeviceGuard.h>
 #include <torch/csrc/Exceptions.h>
@@ -263,7 +264,8 @@ PyObject* rms_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 // gate_topk(x, gate_weight, top_k, renormalize) -> (weights, ids, token_expert_indices), or None;
-// gate_topk_few: the same for batches that moe_gate_topk_few serves.
+// gate_topk_few: the same for batches that moe_gate_topk_few serves.  Plain tensors (or Parameters) outside function
+// modes only: anything else may have a linear of its own, which the caller then asks for.
 template <bool FEW>
 PyObject* gate_topk(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
@@ -272,6 +274,7 @@ PyObject* gate_topk(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (n != 4 || !int_arg(a[2], &K) || !flag_arg(a[3], &renormalize)) MOE_NONE;
   const at::Tensor *x = gpu_tensor(a[0]), *g = gpu_tensor(a[1]);
   if (!x || !g || x->dim() != 2 || g->dim() != 2 || !x->is_contiguous() || !g->is_contiguous()) MOE_NONE;
+  if (FEW && (!THPVariable_CheckExact(a[0]) || !THPVariable_CheckExact(a[1]) || at::impl::torch_function_mode_enabled())) MOE_NONE;
   const at::Device dev = x->device();
   const int dtype = dtype_code(x->scalar_type());
   const int64_t T = x->size(0), H = x->size(1), E = g->size(0);

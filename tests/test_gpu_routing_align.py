@@ -301,6 +301,46 @@ def test_gate_of_few_tokens_is_exact_where_the_sums_are(moe, oracle, dev, E, H, 
             assert torch.equal(w.cpu().view(torch.int32), ow.view(torch.int32)), (T, K)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("form", ["plain", "columns", "transposed", "odd", "parameter", "subclass", "mode"])
+def test_gate_that_the_kernels_do_not_serve_is_the_two_steps(moe, dev, dtype, form):
+    """Sizes and forms that go to the library's linear: the same bits as linear and fused_topk apart; a tensor type or
+    a function mode with a linear of its own is asked for it, at a size that the kernels serve, too."""
+    T, H, E, K = {"odd": (37, 100, 21, 3), "subclass": (37, 256, 128, 8), "mode": (37, 256, 128, 8)}.get(form, (2000, 256, 128, 8))
+    if T == 2000 and dtype != torch.float32:  # (125 token tiles by 8 expert tiles: more than the kernels are given)
+        assert moe._lib.lib().moe_gate_topk_few_bytes(T, H, E, moe._lib.DTYPE_CODE[dtype]) == 0
+    g = torch.Generator(dev).manual_seed(3)
+    x = torch.randn(T, 2 * H, device=dev, generator=g).to(dtype)
+    x = x[:, H:] if form == "columns" else x[:, :H].contiguous()
+    wg = (torch.randn(E, H, device=dev, generator=g) * 0.1).to(dtype)
+    if form == "transposed":
+        wg = wg.t().contiguous().t()
+    want = moe.fused_topk(x, torch.nn.functional.linear(x, wg), K, True)
+    asked = []
+    if form == "parameter":
+        wg = torch.nn.Parameter(wg)
+    if form == "subclass":
+        class Own(torch.Tensor):
+            @classmethod
+            def __torch_function__(cls, func, types, args=(), kwargs=None):
+                asked.append(func)
+                return super().__torch_function__(func, types, args, kwargs or {})
+        wg = wg.as_subclass(Own)
+    if form == "mode":
+        class Mode(torch.overrides.TorchFunctionMode):
+            def __torch_function__(self, func, types, args=(), kwargs=None):
+                asked.append(func)
+                return func(*args, **(kwargs or {}))
+        with Mode():
+            got = moe.fused_gate_topk(x, wg, K, True)
+    else:
+        got = moe.fused_gate_topk(x, wg, K, True)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+    assert (torch.nn.functional.linear in asked) == (form in ("subclass", "mode"))
+
+
 def test_fused_gate_topk_falls_back_and_block_matches_two_step(moe, oracle, dev, monkeypatch):
     g = torch.Generator().manual_seed(11)
     # unsupported expert count: the gate runs as a plain linear, then fused_topk
