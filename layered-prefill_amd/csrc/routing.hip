@@ -225,8 +225,8 @@ int launch_gate_e(const void* x, const void* wg, float* logits_out, float* w, in
 // ---------------------------------------------------------------------------
 // The same for up to a few hundred tokens, as two short kernels.  A workgroup of the kernel above pulls all E gate rows
 // through one CU, which a CU does at 37 bytes a nanosecond (E 128, H 2048: 512 KB, 17 us, whatever T).  Here the gate
-// linear is cut in tokens, experts and K: a workgroup takes 16 tokens by 16 experts by 512 elements of K, everything it
-// reads (32 KB) is on its way at once, its four wavefronts multiply straight out of registers (MFMA 16x16x32, gate rows as
+// linear is cut in tokens, experts and K: a workgroup takes 16 (32) tokens by 16 (32) experts by 512 elements of K,
+// everything it reads (32 or 64 KB) is on its way at once, its four wavefronts multiply straight out of registers (MFMA 16x16x32, gate rows as
 // the A operand; a wavefront's two units of 64 elements fill whole lines) and add up in LDS.  The sums of the K pieces
 // leave in fp32; the kernel that routes adds them, rounds the logit once, to the activation dtype, as the output of a
 // gate linear is, and goes on with the lane layout of the stand-alone router.
@@ -242,41 +242,59 @@ __device__ __forceinline__ gate_f32x4 gate_mma16(const uint4& a, const uint4& b,
 constexpr int kPieceUnits = 8;                     // units of 64 elements in a piece of K
 constexpr int kPieceWaves = 4, kPieceThreads = kWave * kPieceWaves;
 static int gate_pieces(int H) { return (H / 64 + kPieceUnits - 1) / kPieceUnits; }
+static int64_t gate_small_tiles(int T, int H, int E) {
+  return (static_cast<int64_t>(T) + 15) / 16 * (E / 16) * gate_pieces(H);
+}
 
-// grid: token tiles x (pieces x expert tiles), the latter fastest, so that a gate piece stays with one XCD's L2
-template <typename El>
+// grid: token tiles x (pieces x expert tiles), the latter fastest, so that a gate piece stays with one XCD's L2.  Tiles of
+// 16 M tokens by 16 N experts.
+template <typename El, int M, int N>
 __global__ __launch_bounds__(kPieceThreads) void gate_piece_kernel(
     const typename El::S* __restrict__ x, const typename El::S* __restrict__ wg, float* __restrict__ sums, int T, int H, int E,
     int pieces) {
-  constexpr int ROW = 16 + 4;  // floats of a token in LDS, padded: the sixteen tokens of a store spread over the banks
-  __shared__ __attribute__((aligned(16))) float part[kPieceWaves][16][ROW];
+  constexpr int ROW = 16 * N + 4;  // floats of a token in LDS, padded: the sixteen tokens of a store spread over the banks
+  __shared__ __attribute__((aligned(16))) float part[kPieceWaves][16 * M][ROW];
   const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int l15 = lane & 15, lq = lane >> 4;
-  const int et = E / 16, per_token_tile = pieces * et;
-  const int t0 = blockIdx.x / per_token_tile * 16, rest = blockIdx.x % per_token_tile;
-  const int piece = rest / et, e0 = rest % et * 16;
+  const int et = E / (16 * N), per_token_tile = pieces * et;
+  const int t0 = blockIdx.x / per_token_tile * (16 * M), rest = blockIdx.x % per_token_tile;
+  const int piece = rest / et, e0 = rest % et * (16 * N);
   const int nu = H / 64;
-  const typename El::S* xr = x + static_cast<size_t>(min(t0 + l15, T - 1)) * H + lq * 8;
-  const typename El::S* wr = wg + static_cast<size_t>(e0 + l15) * H + lq * 8;
-  gate_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  uint4 xf[4], wf[4];
+  const typename El::S *xr[M], *wr[N];
+#pragma unroll
+  for (int m = 0; m < M; ++m) xr[m] = x + static_cast<size_t>(min(t0 + 16 * m + l15, T - 1)) * H + lq * 8;
+#pragma unroll
+  for (int n = 0; n < N; ++n) wr[n] = wg + static_cast<size_t>(e0 + 16 * n + l15) * H + lq * 8;
+  gate_f32x4 acc[M][N];
+  uint4 xf[4][M], wf[4][N];
 #pragma unroll
   for (int kk = 0; kk < 4; ++kk) {
     const int u = piece * kPieceUnits + 2 * wave + (kk >> 1);  // a unit behind the end of K: zeros
     const size_t k = static_cast<size_t>(u) * 64 + (kk & 1) * 32;
-    wf[kk] = u < nu ? *reinterpret_cast<const uint4*>(wr + k) : uint4{0, 0, 0, 0};
-    xf[kk] = u < nu ? *reinterpret_cast<const uint4*>(xr + k) : uint4{0, 0, 0, 0};
+#pragma unroll
+    for (int n = 0; n < N; ++n) wf[kk][n] = u < nu ? *reinterpret_cast<const uint4*>(wr[n] + k) : uint4{0, 0, 0, 0};
+#pragma unroll
+    for (int m = 0; m < M; ++m) xf[kk][m] = u < nu ? *reinterpret_cast<const uint4*>(xr[m] + k) : uint4{0, 0, 0, 0};
   }
   __builtin_amdgcn_sched_barrier(0);  // all requests first
 #pragma unroll
-  for (int kk = 0; kk < 4; ++kk) acc = gate_mma16<El>(wf[kk], xf[kk], acc);
-  // acc[i]: token l15, expert 4 lq + i
-  *reinterpret_cast<gate_f32x4*>(&part[wave][l15][4 * lq]) = acc;
+  for (int m = 0; m < M; ++m)
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+      acc[m][n] = gate_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk) acc[m][n] = gate_mma16<El>(wf[kk][n], xf[kk][m], acc[m][n]);
+      // element i: token 16 m + l15, expert 16 n + 4 lq + i
+      *reinterpret_cast<gate_f32x4*>(&part[wave][16 * m + l15][16 * n + 4 * lq]) = acc[m][n];
+    }
   __syncthreads();
-  const int tok = threadIdx.x / 16, col = threadIdx.x % 16;
-  if (t0 + tok < T)
-    sums[(static_cast<size_t>(piece) * T + t0 + tok) * E + e0 + col] =
-        (part[0][tok][col] + part[1][tok][col]) + (part[2][tok][col] + part[3][tok][col]);
+#pragma unroll
+  for (int r = 0; r < M * N; ++r) {
+    const int at = r * kPieceThreads + threadIdx.x, tok = at / (16 * N), col = at % (16 * N);
+    if (t0 + tok < T)
+      sums[(static_cast<size_t>(piece) * T + t0 + tok) * E + e0 + col] =
+          (part[0][tok][col] + part[1][tok][col]) + (part[2][tok][col] + part[3][tok][col]);
+  }
 }
 
 template <int E, typename El>
@@ -312,8 +330,16 @@ int launch_gate_pieces(const void* x, const void* wg, float* sums, float* w, int
                        int renorm, hipStream_t s) {
   using S = typename El::S;
   const int pieces = gate_pieces(H);
-  hipLaunchKernelGGL(gate_piece_kernel<El>, dim3(static_cast<unsigned>((T + 15) / 16) * pieces * (E / 16)), dim3(kPieceThreads), 0, s,
-                     static_cast<const S*>(x), static_cast<const S*>(wg), sums, T, H, E, pieces);
+  auto go = [&](auto kernel, int tokens, int experts) {
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((T + tokens - 1) / tokens) * pieces * (E / experts)), dim3(kPieceThreads),
+                       0, s, static_cast<const S*>(x), static_cast<const S*>(wg), sums, T, H, E, pieces);
+  };
+  // Up to 512 small tiles, two a CU, are done sooner than an eighth as many large ones; beyond, what they read twice as
+  // often counts.  us, gate and router, tiles of 16 and of 32: E 128, H 2048: 7.8 and 8.4 at 135 tokens, 8.1 and 8.4 at 256
+  // (512 tiles of 16), 9.1 and 8.5 at 384, 10.0 and 8.7 at 512; E 32: 7.3 and 7.6 at 1024 tokens (512); E 64, H 4096: 8.3
+  // and 8.6 at 256 (512), 10.2 and 8.9 at 512.
+  if (gate_small_tiles(T, H, E) > 512) go(gate_piece_kernel<El, 2, 2>, 32, 32);
+  else go(gate_piece_kernel<El, 1, 1>, 16, 16);
   constexpr int rows = kWavesPerBlock * Pow2Geom<E>::kRowsPerWave;
   hipLaunchKernelGGL((topk_softmax_sums_kernel<E, El>), dim3((T + rows - 1) / rows), dim3(kWave * kWavesPerBlock), 0, s, sums, w,
                      ids, tei, T, K, renorm, pieces);
@@ -554,15 +580,16 @@ MOE_EXPORT int moe_gate_topk_softmax(const void* x, const void* gate_weight, int
   }
 }
 
-// Sizes for which the kernels that cut K serve a call: up to 768 workgroups of the first one, three a CU; then what all
-// token tiles read of the gate outgrows what fewer, larger tiles would.  us, gate linear and router, against the library's
-// GEMM and the router: E 128, H 2048, top-8: 6.5 and 9.2 at 1 token, 7.8 and 9.3 at 135, 9.1 and 9.4 at 384 (768
-// workgroups), 10.0 and 9.3 at 512 (1024), 13.8 and 10.4 at 1024; E 32, H 2048: 6.2 and 9.0 at 135, 7.3 and 9.1 at 1024
-// (512); E 64, H 4096: 8.0 and 11.6 at 135 (288), 10.2 and 11.7 at 512 (1024), 13.9 and 11.8 at 1024; E 256, H 7168: 17.3
-// and 13.5 at 135 (2016).  From Python the call is one entry into native code instead of two and an operator.
+// Sizes for which the kernels that cut K serve a call: up to 1024 tiles of 16 tokens by 16 experts by 512 of K (256 of the
+// large ones); then what all token tiles read of the gate outgrows what a product with fewer, larger tiles reads.  us, gate
+// linear and router, against the library's GEMM and the router: E 128, H 2048, top-8: 6.5 and 9.2 at 1 token, 7.8 and 9.4
+// at 135, 8.5 and 9.4 at 384, 8.7 and 9.4 at 512 (1024 tiles), 10.5 and 10.2 at 640, 10.9 and 10.4 at 1024; E 32, H 2048:
+// 7.3 and 9.1 at 1024, 7.9 and 9.2 at 2047 (1024); E 64, H 4096: 8.0 and 11.6 at 135, 8.9 and 11.5 at 512 (1024), 11.0 and
+// 11.9 at 1024; E 256, H 7168: 12.3 and 12.8 at 64 (896), 15.4 and 13.5 at 135 (2016).  From Python the call is one entry into
+// native code instead of two and an operator.
 MOE_EXPORT int64_t moe_gate_topk_few_bytes(int T, int H, int E, int dtype) {
   if (T < 1 || H < 64 || H % 64 || (E != 32 && E != 64 && E != 128 && E != 256) || (dtype != MOE_BF16 && dtype != MOE_F16)) return 0;
-  if ((static_cast<int64_t>(T) + 15) / 16 * (E / 16) * gate_pieces(H) > 768) return 0;
+  if (gate_small_tiles(T, H, E) > 1024) return 0;
   return static_cast<int64_t>(gate_pieces(H)) * T * E * static_cast<int64_t>(sizeof(float));
 }
 

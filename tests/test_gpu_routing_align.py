@@ -291,7 +291,8 @@ def test_gate_of_few_tokens_is_exact_where_the_sums_are(moe, oracle, dev, E, H, 
     last = next(T for T in range(1, 10**6) if not served(T + 1))
     g = torch.Generator().manual_seed(E + H)
     wg = torch.randint(-2, 3, (E, H), generator=g).float() / 64
-    for T in sorted({1, 15, 16, 17, 33, last, last + 1}):
+    wide = last // 2 // 16 * 16   # tiles of 16 tokens by 16 experts up to here, of 32 by 32 behind it
+    for T in sorted({1, 15, 16, 17, 33, wide, wide + 1, last - 15, last, last + 1} - {0}):
         x = torch.randint(-3, 4, (T, H), generator=g).float()
         logits = (x @ wg.t()).to(dtype).float()
         for K in (1, min(8, E), 17):
@@ -307,8 +308,8 @@ def test_gate_of_few_tokens_is_exact_where_the_sums_are(moe, oracle, dev, E, H, 
 def test_gate_that_the_kernels_do_not_serve_is_the_two_steps(moe, dev, dtype, form):
     """Sizes and forms that go to the library's linear: the same bits as linear and fused_topk apart; a tensor type or
     a function mode with a linear of its own is asked for it, at a size that the kernels serve, too."""
-    T, H, E, K = {"odd": (37, 100, 21, 3), "subclass": (37, 256, 128, 8), "mode": (37, 256, 128, 8)}.get(form, (2000, 256, 128, 8))
-    if T == 2000 and dtype != torch.float32:  # (125 token tiles by 8 expert tiles: more than the kernels are given)
+    T, H, E, K = {"odd": (37, 100, 21, 3), "subclass": (37, 256, 128, 8), "mode": (37, 256, 128, 8)}.get(form, (2000, 1024, 128, 8))
+    if T == 2000 and dtype != torch.float32:  # (125 by 8 tiles by 2 pieces of K: more than the kernels are given)
         assert moe._lib.lib().moe_gate_topk_few_bytes(T, H, E, moe._lib.DTYPE_CODE[dtype]) == 0
     g = torch.Generator(dev).manual_seed(3)
     x = torch.randn(T, 2 * H, device=dev, generator=g).to(dtype)
