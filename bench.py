@@ -96,19 +96,27 @@ class Layer:
                 self.w2_run = moe.ops.tile_expert_weights(self.w2, False)
         self.dev = dev
         s = self.shape
-        self.bm = moe.try_get_optimal_moe_config(self.w13.shape, self.w2.shape, s.top_k, None,
-                                                 self.T)["BLOCK_SIZE_M"]
-        ws = moe.fused_moe.fused_experts_workspace_bytes(self.T, s.hidden, s.intermediate,
-                                                         s.experts, s.top_k, self.bm, x.dtype)
-        self.workspace = torch.empty(ws, dtype=torch.uint8, device=dev)
         self.out = torch.empty_like(self.x)
+        self._place()
+
+    def _place(self):
+        """Block size and scratch of the steps that ``step_instrumented`` enqueues one by one: those of the call
+        that ``step`` makes with this layout, its rounding of the gated product included (passes bit 64)."""
+        moe, s = self.moe, self.shape
+        self.bm = moe.try_get_optimal_moe_config(self.w13.shape, self.w2.shape, s.top_k, None, self.T,
+                                                 act_dtype=self.x.dtype, weight_layout=self.layout)["BLOCK_SIZE_M"]
+        code = moe._lib.DTYPE_CODE[self.x.dtype]
+        self.once = 64 if self.bm < moe._lib.lib().moe_preferred_block_size(self.T, s.experts, s.top_k, code, code) else 0
+        ws = moe.fused_moe.fused_experts_workspace_bytes(self.T, s.hidden, s.intermediate,
+                                                         s.experts, s.top_k, self.bm, self.x.dtype)
+        self.workspace = torch.empty(ws, dtype=torch.uint8, device=self.dev)
 
     def experts(self, x, tw, ids):
         """``fused_experts`` on this layer's weights in the layout it runs with."""
         return self.moe.fused_experts(x, self.w13_run, self.w2_run, None, None, tw, ids, weight_layout=self.layout)
 
     def with_layout(self, layout: str) -> "Layer":
-        """The same inputs, weights and scratch run with the other weight layout."""
+        """The same inputs, weights and scratch run with the other weight layout, its block size and scratch its own."""
         other = Layer.__new__(Layer)
         other.__dict__.update(self.__dict__)
         other.layout = layout
@@ -117,6 +125,7 @@ class Layer:
         elif self.layout != "tiled":
             other.w13_run = self.moe.ops.tile_expert_weights(self.w13, True)
             other.w2_run = self.moe.ops.tile_expert_weights(self.w2, False)
+        other._place()
         return other
 
     def step(self):
@@ -140,12 +149,12 @@ class Layer:
         for i, mask in enumerate((1, 2, 4)):
             fm.launch_fused_experts(self.x, self.out, self.w13_run, self.w2_run, None, None, None, None, tw,
                                     sorted_ids, expert_ids, npp, self.bm, workspace=self.workspace,
-                                    passes=mask, weight_layout=self.layout)
+                                    passes=mask | self.once, weight_layout=self.layout)
             ev[3 + i].record()
         ev[6].record()
         fm.launch_fused_experts(self.x, self.out, self.w13_run, self.w2_run, None, None, None, None, tw,
-                                sorted_ids, expert_ids, npp, self.bm, workspace=self.workspace, passes=3,
-                                weight_layout=self.layout)
+                                sorted_ids, expert_ids, npp, self.bm, workspace=self.workspace,
+                                passes=3 | self.once, weight_layout=self.layout)
         ev[7].record()
         return ids
 

@@ -240,7 +240,7 @@ typedef struct MoeFusedExpertsArgs {
      result is the same, bit for bit.  Bit 64: with SiLU and blocks of 32 slots the
      gated product is rounded once, as with blocks of 256 (rows of x must be whole
      multiples of 128 bytes; no effect elsewhere).  A caller that takes its block size
-     from moe_layer_block_size sets it when that is smaller than
+     from moe_call_block_size or moe_layer_block_size sets it when that is smaller than
      moe_preferred_block_size, so that the choice does not decide the precision. */
   int32_t passes;
   int32_t weight_layout;     /* MoeWeightLayout of w13 and w2 (both): 0 = plain                   */
@@ -309,8 +309,11 @@ int moe_fused_experts_plan_layout(int T, int H, int I, int E, int K, int block_s
  * tokens; plays the role of config["BLOCK_SIZE_M"] chosen by
  * try_get_optimal_moe_config (nanovllm/layers/for_moe/fused_moe.py:354-390). */
 int moe_preferred_block_size(int M, int E, int K, int act_dtype, int weight_dtype);
-/* The same for a layer of intermediate size I (0: not known; below 768 the same as 768): a layer of few experts leaves the large
- * tiles too few workgroups for the chip and keeps the small blocks longer. */
+/* The same for a call whose sizes and weight layout (MoeWeightLayout) are known: what moe_layer takes where block_size is 0,
+ * and what a caller that enqueues the steps itself should take to run on the same kernels. */
+int moe_call_block_size(int M, int H, int I, int E, int K, int act_dtype, int weight_dtype, int weight_layout);
+/* The same for a layer of intermediate size I (0: not known; below 768 the same as 768) of which H and the layout are not
+ * known: a layer of few experts leaves the large tiles too few workgroups for the chip and keeps the small blocks longer. */
 int moe_layer_block_size(int M, int I, int E, int K, int act_dtype, int weight_dtype);
 
 /* One-time re-ordering of expert weights for the DMA kernels (no counterpart in the reference, whose

@@ -27,6 +27,7 @@ EXPORTS = (
     "moe_last_error", "moe_abi_version", "moe_topk_softmax", "moe_align_workspace_bytes",
     "moe_align_block_size", "moe_silu_and_mul", "moe_swigluoai_and_mul", "moe_sum",
     "moe_fused_experts_workspace_bytes", "moe_fused_experts", "moe_preferred_block_size", "moe_layer_block_size",
+    "moe_call_block_size",
     "moe_quant_rows_e4m3", "moe_gate_topk_softmax", "moe_gate_topk_few_bytes", "moe_gate_topk_few", "moe_add_rms_norm",
     "moe_align_can_plan", "moe_align_block_size_planned", "moe_fused_experts_plan_layout",
     "moe_fused_experts_status", "moe_fused_experts_set_wait_limit", "moe_align_block_size_static",
@@ -137,6 +138,8 @@ def _declare(L: ctypes.CDLL) -> None:
     L.moe_preferred_block_size.argtypes = [i32] * 5
     L.moe_layer_block_size.restype = i32
     L.moe_layer_block_size.argtypes = [i32] * 6
+    L.moe_call_block_size.restype = i32
+    L.moe_call_block_size.argtypes = [i32] * 8
     L.moe_quant_rows_e4m3.restype = i32
     L.moe_quant_rows_e4m3.argtypes = [p, i32, i64, i32, p, p, p]
     L.moe_route_align_supported.restype = i32

@@ -140,7 +140,7 @@ struct GemmParams {
   int mul_weight;    // multiply by topk_w[tok] in the epilogue
   int activation;    // MoeActivation (gated pass only)
   // Streaming kernel with SiLU, rows of whole units: the product is rounded once.  Those are the calls that
-  // moe_layer_block_size takes from the large-tile kernel, which forms silu(gate) * up on its fp32
+  // moe_call_block_size takes from the large-tile kernel, which forms silu(gate) * up on its fp32
   // accumulators: which of the two runs must not decide the precision.  Error of the whole layer against
   // float64, 32 experts, H 2048, I 1024, 256 tokens top-4: bf16 2.88e-3 on both kernels, 4.26e-3 with
   // gate, up and silu rounded as well; fp16 3.61e-4 and 5.27e-4.

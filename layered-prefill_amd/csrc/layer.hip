@@ -25,36 +25,6 @@ struct Layout {
   int32_t *topk_ids, *sorted, *experts, *npp;
   void *align_ws, *fused_ws;
 };
-// Block size of a call that does not name one: 256 (large-tile kernel) or 32 (streaming kernel, with the large tile's
-// roundings where that would do as well: passes bit 64 of moe_fused_experts).  The streaming kernel reads the weights
-// again for every 32 rows of an expert; the large tile leaves CUs idle where there are few tiles, and its blocks half empty
-// where experts have few rows.  What decides between them is the call's matrix work, T * K * H * I, with 40000 beside H * I
-// for what a routed row costs outside its products (rows of narrow layers).  Measured over 1233 points, whole layer, Zipf
-// routing: 1 to 128 experts, H 128 to 4096, I 128 to 1440, 16 to 4000 routed rows per expert.  Mean and worst excess over the
-// faster of the two, by this rule and by rows and tiles (moe_layer_block_size):
-//   16 bit, plain weights, line 3.4e9: 0.5 % and 15 %; 8.3 % and 118 %
-//   16 bit, tiled weights, line 3.2e9: 0.5 % and 16 %; 3.1 % and 51 %
-//   16 bit, I 1440, line 1e10: 1.1 % and 22 %; 12.9 % and 68 %
-//   e4m3, line 6e9: 0.7 % and 23 %; 8.4 % and 86 %.  e4m3, I 1440, line 2e10: 0.7 % and 19 %; 16 % and 67 %
-// (H or I that is no whole number of the large tile's K units, as 1440 is not: that pass runs on the register-staged
-// kernel at blocks of 256, and the line lies where it lies with that.)  For instance, us with blocks of 256 and of 32: 128
-// experts, H 1024, I 512, 640 tokens top-4: 70.8 and 54.8; 128, H 2880, I 1440, 640 tokens: 489 and 407; 128, H 2048, I 768,
-// 256 tokens top-8: plain 171 and 161, tiled 152 and 156; 16, H 2048, I 768, 384 tokens top-4: 1.25 times.  Fewer than 16
-// (e4m3: 32) rows per expert always stream, as under the older rules.
-int layer_block(const MoeLayerArgs* a) {
-  const bool e4m3 = a->weight_dtype == MOE_E4M3;
-  const int es = e4m3 ? 1 : 2;
-  // rows that are no whole 32-byte steps run on the register-staged kernels with either block: the older rule stands
-  if (a->act_dtype == MOE_F32 || a->weight_dtype == MOE_F32 || a->H * static_cast<int64_t>(es) % 32 || a->I * static_cast<int64_t>(es) % 32)
-    return moe_layer_block_size(a->T, a->I, a->E, a->K, a->act_dtype, a->weight_dtype);
-  const int64_t numel = static_cast<int64_t>(a->T) * a->K;
-  if (numel / a->E < (e4m3 ? 32 : 16)) return 32;
-  const int unit = e4m3 ? 128 : 64;  // elements of a K unit of the large tile
-  const bool whole = a->H % unit == 0 && a->I % unit == 0;
-  const double line = e4m3 ? (whole ? 6e9 : 2e10) : !whole ? 1e10 : a->weight_layout == MOE_WEIGHTS_TILED ? 3.2e9 : 3.4e9;
-  return static_cast<double>(numel) * (static_cast<double>(a->H) * a->I + 40000.) >= line ? 256 : 32;
-}
-
 Layout layout_of(const MoeLayerArgs* a) {
   Layout l{};
   Carver c{static_cast<char*>(a->workspace)};
@@ -66,7 +36,8 @@ Layout layout_of(const MoeLayerArgs* a) {
     l.topk_w = a->topk_weights;
     l.topk_ids = a->topk_ids;
   }
-  l.block = a->block_size ? a->block_size : layer_block(a);
+  l.block = a->block_size ? a->block_size
+                          : moe_call_block_size(a->T, a->H, a->I, a->E, a->K, a->act_dtype, a->weight_dtype, a->weight_layout);
   l.sorted_cap = numel + static_cast<int64_t>(a->E) * (l.block - 1);
   l.expert_cap = (l.sorted_cap + l.block - 1) / l.block;
   l.align_bytes = moe_align_workspace_bytes(numel, a->E);
@@ -91,7 +62,40 @@ int check_layer_args(const MoeLayerArgs* a) {
 
 }  // namespace
 
-// The rule for callers that know neither H nor the weights' layout (moe_layer does, and has a better one: layer_block).
+// Block size of a call that does not name one: 256 (large-tile kernel) or 32 (streaming kernel, with the large tile's
+// roundings where that would do as well: passes bit 64 of moe_fused_experts).  The streaming kernel reads the weights
+// again for every 32 rows of an expert; the large tile leaves CUs idle where there are few tiles, and its blocks half empty
+// where experts have few rows.  What decides between them is the call's matrix work, T * K * H * I, with 40000 beside H * I
+// for what a routed row costs outside its products (rows of narrow layers).  Measured over 1233 points, whole layer, Zipf
+// routing: 1 to 128 experts, H 128 to 4096, I 128 to 1440, 16 to 4000 routed rows per expert.  Mean and worst excess over the
+// faster of the two, by this rule and by rows and tiles (moe_layer_block_size):
+//   16 bit, plain weights, line 3.4e9: 0.5 % and 15 %; 8.3 % and 118 %
+//   16 bit, tiled weights, line 3.2e9: 0.5 % and 16 %; 3.1 % and 51 %
+//   16 bit, I 1440, line 1e10: 1.1 % and 22 %; 12.9 % and 68 %
+//   e4m3, line 6e9: 0.7 % and 23 %; 8.4 % and 86 %.  e4m3, I 1440, line 2e10: 0.7 % and 19 %; 16 % and 67 %
+// (H or I that is no whole number of the large tile's K units, as 1440 is not: that pass runs on the register-staged
+// kernel at blocks of 256, and the line lies where it lies with that.)  For instance, us with blocks of 256 and of 32: 128
+// experts, H 1024, I 512, 640 tokens top-4: 70.8 and 54.8; 128, H 2880, I 1440, 640 tokens: 489 and 407; 128, H 2048, I 768,
+// 256 tokens top-8: plain 171 and 161, tiled 152 and 156; 16, H 2048, I 768, 384 tokens top-4: 1.25 times.  Fewer than 16
+// (e4m3: 32) rows per expert always stream, as under the older rules.
+// Every caller that enqueues a call's steps asks here, so that a call runs on the same kernels whichever way it is entered.
+MOE_EXPORT int moe_call_block_size(int M, int H, int I, int E, int K, int act_dtype, int weight_dtype, int weight_layout) {
+  const bool e4m3 = weight_dtype == MOE_E4M3;
+  const int es = e4m3 ? 1 : 2;
+  // rows that are no whole 32-byte steps run on the register-staged kernels with either block: the rule by rows and tiles
+  if (E < 1 || H < 1 || I < 1 || act_dtype == MOE_F32 || weight_dtype == MOE_F32 || H * static_cast<int64_t>(es) % 32 ||
+      I * static_cast<int64_t>(es) % 32)
+    return moe_layer_block_size(M, I, E, K, act_dtype, weight_dtype);
+  const int64_t numel = static_cast<int64_t>(M) * K;
+  if (numel / E < (e4m3 ? 32 : 16)) return 32;
+  const int unit = e4m3 ? 128 : 64;  // elements of a K unit of the large tile
+  const bool whole = H % unit == 0 && I % unit == 0;
+  const double line = e4m3 ? (whole ? 6e9 : 2e10) : !whole ? 1e10 : weight_layout == MOE_WEIGHTS_TILED ? 3.2e9 : 3.4e9;
+  return static_cast<double>(numel) * (static_cast<double>(H) * I + 40000.) >= line ? 256 : 32;
+}
+
+// The rule for callers that know neither H nor the weights' layout; moe_call_block_size is the better one and the one that
+// calls of this library take.
 // Blocks of 256 slots (large-tile kernel) or of 32 (streaming kernel, with the large tile's roundings from its old
 // line on: passes bit 64 of moe_fused_experts).  What the large tile costs below its crossover
 // is idle CUs: an expert's weights are walked by I / 128 + H / 256 workgroups, each a serial chain of K tiles, and with

@@ -66,19 +66,24 @@ def _plan_in_workspace(workspace: torch.Tensor, T: int, H: int, I: int, E: int, 
 def try_get_optimal_moe_config(w1_shape, w2_shape, top_k: int, dtype: Optional[str], M: int,
                                is_marlin: bool = False,
                                block_shape: Optional[list] = None,
-                               act_dtype: torch.dtype = torch.bfloat16) -> dict:
+                               act_dtype: torch.dtype = torch.bfloat16,
+                               weight_layout: str = "plain") -> dict:
     """Role of nanovllm/layers/for_moe/fused_moe.py:354-390.  The reference looks
     up Triton tile tables per device name; the HIP kernels own their tiling, so
     the only entry that still matters to callers is BLOCK_SIZE_M, the block size
     handed to moe_align_block_size.  ``act_dtype`` (not in the reference, whose
     ``dtype`` string only names quantised forms) is the activation dtype: fp32
-    runs on other kernels than the 16-bit dtypes and has its own rule."""
+    runs on other kernels than the 16-bit dtypes and has its own rule.
+    ``weight_layout`` (likewise) is that of the weights: with it the block size is the
+    one that the native layer call takes for the same call."""
     E = w2_shape[0]
     act_code = _lib.DTYPE_CODE[act_dtype]
     weight_code = _lib.E4M3_CODE if dtype == "fp8_w8a8" else act_code
     if w1_shape[1] == 0:   # the layer's width is not known
         return {"BLOCK_SIZE_M": lib().moe_preferred_block_size(M, E, top_k, act_code, weight_code)}
-    bm = lib().moe_layer_block_size(M, w1_shape[1] // 2, E, top_k, act_code, weight_code)
+    H = w1_shape[2] if len(w1_shape) > 2 else 0   # 0: not known
+    bm = lib().moe_call_block_size(M, H, w1_shape[1] // 2, E, top_k, act_code, weight_code,
+                                   _lib.WEIGHT_LAYOUT_CODE[weight_layout])
     return {"BLOCK_SIZE_M": bm}
 
 
@@ -390,8 +395,10 @@ def fused_experts_impl(hidden_states: torch.Tensor,
     CHUNK_SIZE: int = 64 * 1024
     M = min(num_tokens, CHUNK_SIZE)
     config_dtype = "fp8_w8a8" if fp8 else None
-    config = try_get_optimal_moe_config(w1.size(), w2.size(), top_k_num, config_dtype, M,
-                                        act_dtype=hidden_states.dtype)
+    config_args = dict(act_dtype=hidden_states.dtype)
+    if try_get_optimal_moe_config is _LIBRARY_CONFIG:   # (a caller's own need not know of layouts)
+        config_args["weight_layout"] = weight_layout
+    config = try_get_optimal_moe_config(w1.size(), w2.size(), top_k_num, config_dtype, M, **config_args)
 
     out_hidden_states = hidden_states if inplace else torch.empty_like(hidden_states)
     if topk_weights.dtype != torch.float32:
@@ -411,7 +418,7 @@ def fused_experts_impl(hidden_states: torch.Tensor,
             break
         if tokens_in_chunk < CHUNK_SIZE and chunk > 0:
             config = try_get_optimal_moe_config(w1.size(), w2.size(), top_k_num, config_dtype,
-                                                tokens_in_chunk, act_dtype=hidden_states.dtype)
+                                                tokens_in_chunk, **config_args)
         bm = config["BLOCK_SIZE_M"]
         curr_ids = topk_ids[begin:end]
         curr_w = topk_weights[begin:end]

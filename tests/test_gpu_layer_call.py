@@ -71,6 +71,27 @@ def test_one_call_is_its_steps(moe, dev, monkeypatch, T, activation, on_input):
     assert (one.float() - steps.float()).norm() <= 2e-3 * steps.float().norm()
 
 
+@pytest.mark.parametrize("E,H,I,K,T,layout", [(16, 4096, 1024, 2, 500, "plain"), (128, 256, 128, 2, 2048, "plain"),
+                                              (128, 256, 128, 2, 2048, "tiled")])
+def test_checked_hand_off_runs_the_kernels_of_the_call(moe, dev, monkeypatch, E, H, I, K, T, layout):
+    """With the hand-off check on, the call is enqueued step by step: on the same kernels, with the same bits, where the
+    rule by rows and tiles would take the other block size."""
+    print(f"hand-off check E={E} H={H} I={I} T={T} {layout}", flush=True)
+    g = torch.Generator(dev).manual_seed(T)
+    normal = lambda *shape: torch.empty(shape, dtype=torch.bfloat16, device=dev).normal_(generator=g)
+    x, logits, w13, w2 = normal(T, H), normal(T, E), normal(E, 2 * I, H) * 0.05, normal(E, H, I) * 0.05
+    if layout == "tiled":
+        w13, w2 = moe.ops.tile_expert_weights(w13, True), moe.ops.tile_expert_weights(w2, False)
+    one = moe.fused_topk_experts(x, logits, w13, w2, K, True, weight_layout=layout)
+    blocks, launch = [], moe.fused_moe.launch_fused_experts
+    monkeypatch.setattr(moe.fused_moe, "launch_fused_experts",
+                        lambda *a, **k: (blocks.append(a[12]), launch(*a, **k))[1])
+    monkeypatch.setattr(moe.fused_moe, "_CHECK_HANDOFF", True)
+    checked = moe.fused_topk_experts(x, logits, w13, w2, K, True, weight_layout=layout)
+    assert blocks == [256 if E == 16 else 32]
+    assert torch.equal(checked, one)
+
+
 def test_arguments_are_converted_or_refused_as_python_does(moe, dev):
     """What is no plain int, bool or float takes the Python path: what converts, converts; what does not is that
     path's error, in front of any launch."""

@@ -264,6 +264,26 @@ def test_layer_call_changes_its_block_once_at_its_line(moe, E, H, I, K, weights,
         assert need(T, 0) == need(T, 32 if T <= last else 256), T
 
 
+@pytest.mark.parametrize("E,H,I,K,weights,tokens", [
+    (128, 2048, 768, 8, 2, (64, 255, 256, 260, 263, 264, 8448)), (16, 4096, 1024, 2, 1, (401, 402, 600, 767, 768)),
+    (128, 256, 128, 2, 2, (2048,)), (128, 2880, 1440, 4, 2, (500, 597, 598)), (32, 2048, 1024, 4, 3, (300, 701, 702)),
+    (6, 24, 40, 2, 2, (287, 288)), (8, 256, 128, 2, 0, (5, 100, 500))])
+def test_a_call_has_the_same_block_size_whichever_way_it_is_entered(moe, E, H, I, K, weights, tokens):
+    """The steps enqueued from Python take their block size from ``try_get_optimal_moe_config``, the native call from its
+    own arguments: a call of more tokens than the native one takes, or one whose hand-off is checked, must run on the
+    kernels of the others.  (The native block shows in the workspace that the call asks for.)"""
+    L, A = moe._lib.lib(), moe._lib.MoeLayerArgs
+    act = weights if weights != 3 else 2
+    dtype = {0: torch.float32, 1: torch.float16, 2: torch.bfloat16}[act]
+    for T in tokens:
+        for layout, code in moe._lib.WEIGHT_LAYOUT_CODE.items():
+            need = lambda block: L.moe_layer_workspace_bytes(A(T=T, H=H, I=I, E=E, K=K, act_dtype=act, weight_dtype=weights,
+                                                               weight_layout=code, block_size=block, router_logits=1))
+            block = moe.fused_moe.try_get_optimal_moe_config((E, 2 * I, H), (E, H, I), K, "fp8_w8a8" if weights == 3 else None,
+                                                             T, act_dtype=dtype, weight_layout=layout)["BLOCK_SIZE_M"]
+            assert need(block) == need(0), (T, layout, block)
+
+
 def test_layer_block_size_of_fp32_is_the_old_rule(moe):
     L = moe._lib.lib()
     for m in (1, 256, 768, 2048, 8448):
