@@ -7,8 +7,10 @@
 #include <Python.h>
 
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/autocast_mode.h>
 #include <ATen/ops/empty.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -263,9 +265,20 @@ PyObject* rms_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// False when a linear of these two is anything but the library's product of their bytes, so that it has to be asked for:
+// tensor subclasses and wrappers, negated or zero tensors, function and dispatch modes (a flop counter, a tracer),
+// transforms, and autocast to another type.
+bool linear_is_plain(PyObject* px, const at::Tensor& x, PyObject* pg, const at::Tensor& g) {
+  if (!THPVariable_CheckExact(px) || !THPVariable_CheckExact(pg) || at::impl::torch_function_mode_enabled()) return false;
+  constexpr c10::DispatchKeySet dense({c10::DispatchKey::CUDA, c10::DispatchKey::AutogradCUDA, c10::DispatchKey::ADInplaceOrView,
+                                       c10::DispatchKey::AutocastCUDA});
+  const uint64_t included = c10::impl::tls_local_dispatch_key_set().included_.raw_repr();
+  if (((x.key_set() | g.key_set()).raw_repr() & ~dense.raw_repr()) | (included & ~c10::default_included_set.raw_repr())) return false;
+  return !at::autocast::is_autocast_enabled(at::kCUDA) || at::autocast::get_autocast_dtype(at::kCUDA) == x.scalar_type();
+}
+
 // gate_topk(x, gate_weight, top_k, renormalize) -> (weights, ids, token_expert_indices), or None;
-// gate_topk_few: the same for batches that moe_gate_topk_few serves.  Plain tensors (or Parameters) outside function
-// modes only: anything else may have a linear of its own, which the caller then asks for.
+// gate_topk_few: the same for batches that moe_gate_topk_few serves, where a linear would be no other.
 template <bool FEW>
 PyObject* gate_topk(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
@@ -274,7 +287,7 @@ PyObject* gate_topk(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (n != 4 || !int_arg(a[2], &K) || !flag_arg(a[3], &renormalize)) MOE_NONE;
   const at::Tensor *x = gpu_tensor(a[0]), *g = gpu_tensor(a[1]);
   if (!x || !g || x->dim() != 2 || g->dim() != 2 || !x->is_contiguous() || !g->is_contiguous()) MOE_NONE;
-  if (FEW && (!THPVariable_CheckExact(a[0]) || !THPVariable_CheckExact(a[1]) || at::impl::torch_function_mode_enabled())) MOE_NONE;
+  if (FEW && !linear_is_plain(a[0], *x, a[1], *g)) MOE_NONE;
   const at::Device dev = x->device();
   const int dtype = dtype_code(x->scalar_type());
   const int64_t T = x->size(0), H = x->size(1), E = g->size(0);

@@ -1,7 +1,10 @@
 """GPU parity, bit-exact: router softmax/top-k and expert-sorted alignment
 through the C ABI (via the Python ops) against the CPU oracle."""
+import contextlib
+
 import pytest
 import torch
+from torch.utils._python_dispatch import TorchDispatchMode
 
 pytestmark = pytest.mark.gpu
 
@@ -340,6 +343,44 @@ def test_gate_that_the_kernels_do_not_serve_is_the_two_steps(moe, dev, dtype, fo
     for a, b in zip(got, want):
         assert torch.equal(a, b)
     assert (torch.nn.functional.linear in asked) == (form in ("subclass", "mode"))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", ["dispatch mode", "autocast", "negated", "autocast to the same type", "parameter", "inference"])
+def test_gate_of_few_tokens_asks_whoever_has_a_say_in_its_linear(moe, dev, monkeypatch, form):
+    """Where a mode, a cast or the tensor itself takes part in a linear, it is asked for one, with the bits of the two
+    steps; where none does, the kernels serve the call."""
+    T, H, E, K = 37, 256, 128, 8
+    g = torch.Generator(dev).manual_seed(4)
+    dtype = torch.float16 if form == "autocast" else torch.bfloat16
+    x = torch.randn(T, H, device=dev, generator=g).to(dtype)
+    wg = (torch.randn(E, H, device=dev, generator=g) * 0.1).to(dtype)
+    ops, linears, linear = [], [], torch.nn.functional.linear
+    monkeypatch.setattr(torch.nn.functional, "linear", lambda *a, **k: (linears.append(1), linear(*a, **k))[1])
+
+    class Counter(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            ops.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    if form == "negated":
+        x = torch._neg_view(x)
+    if form == "parameter":
+        wg = torch.nn.Parameter(wg)
+    inside = {"dispatch mode": Counter, "autocast": lambda: torch.autocast("cuda", torch.bfloat16), "inference": torch.inference_mode,
+              "autocast to the same type": lambda: torch.autocast("cuda", torch.bfloat16)}.get(form, contextlib.nullcontext)
+    with inside():
+        got = moe.fused_gate_topk(x, wg, K, True)
+    asked = form in ("dispatch mode", "autocast", "negated")
+    assert bool(linears) == asked
+    assert (form != "dispatch mode") or any("mm" in op for op in ops), ops
+    with inside():
+        want = moe.fused_topk(x, linear(x, wg), K, True)
+    if asked:
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+    else:   # sums in another order: a logit below 8 may take the neighbouring value, 2^-5 away, which moves a weight w
+            # by at most 2 * 2^-5 * w (1 - w)
+        assert (got[0] - want[0]).abs().max() <= 2.0 ** -6
 
 
 def test_fused_gate_topk_falls_back_and_block_matches_two_step(moe, oracle, dev, monkeypatch):
