@@ -26,11 +26,11 @@ constexpr int kMaxExperts = 1024;
 // Rows the routing + alignment workgroup takes.  One workgroup routes 32 rows of 128 experts side by
 // side in about 6 us (one CU's instruction throughput: a row is ~750 instructions), and every further
 // 32 rows cost as much again, while the stand-alone router spreads its rows over the whole chip:
-// measured on the Qwen3-30B-A3B router (128 experts, top-8), launches included, 14.8 us against
-// 17.7 us for the router and align_small_kernel at 32 rows, 21.0 against 17.6 at 64, 59.7 against 17.2 at 256.
-// What it saves is a launch from Python, not GPU time: 14.4 us against 5.9 + 4.3 us of the router and
-// align_tiny_kernel, which the layer's call enqueues from native code (they follow each other within about a
-// microsecond).  Spreading the
+// measured on the Qwen3-30B-A3B router (128 experts, top-8) when the router and align_small_kernel took 17.7 us,
+// launches included, 14.8 us at 32 rows, 21.0 against 17.6 at 64, 59.7 against 17.2 at 256.
+// What it saves is a launch from Python, not GPU time: at 32 rows 13.6 us against 21.9 called from Python, 13.7 against
+// 8.6 replayed from a graph, where the router and align_tiny_kernel follow each other within about a microsecond, as they
+// do in the layer's call.  Spreading the
 // routing over several workgroups and letting the last one to finish align (release fence, arrival
 // counter, acquire fence) cost 4.5 us more than the two kernels from 64 to 256 rows.
 constexpr int kRouteAlignMaxTokens = 32;

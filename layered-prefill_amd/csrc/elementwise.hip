@@ -253,7 +253,9 @@ int launch_sum(void* out, const void* in, int64_t T, int K, int H, hipStream_t s
   if (H % V == 0 && aligned16(out) && aligned16(in)) {
     // All terms at once pays while they come out of the caches (the expert pass has just written them): 8 terms of 2048
     // elements, bf16, us, this way and term by term: 1 row 2.3 and 3.0, 64 rows 2.5 and 3.4, 741 rows 3.5 and 3.8, 8448
-    // rows (277 MB) 47.4 and 49.4, but 10000 rows 69.5 and 68.9, 16896 rows 124.8 and 118.7.
+    // rows (277 MB) 47.4 and 49.4, but 10000 rows 69.5 and 68.9, 16896 rows 124.8 and 118.7.  4 and 8 terms have an
+    // instance.  2 would gain next to nothing by one (64 rows 2.13 and 2.24, 8448 rows 16.5 and 16.4); 6 would gain half a
+    // microsecond where rows are few (64 rows 2.23 and 2.80, 741 rows 3.01 and 3.36, 8448 rows 36.2 and 36.0).
     const bool cached = T * K * static_cast<int64_t>(H) * static_cast<int64_t>(sizeof(S)) <= (int64_t{288} << 20);
     auto kern = cached && K == 8 ? moe_sum_kernel<El, V, 8> : cached && K == 4 ? moe_sum_kernel<El, V, 4> : moe_sum_kernel<El, V, 0>;
     hipLaunchKernelGGL(kern, dim3(grid_for(T * (H / V))), dim3(kThreads), 0, s, static_cast<S*>(out), static_cast<const S*>(in), T,

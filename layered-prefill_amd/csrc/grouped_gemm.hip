@@ -1431,8 +1431,9 @@ __global__ __launch_bounds__(kThreads, 1) void big_fused_kernel(const GemmParams
 // with equal estimated work instead of equal counts.  A block of an expert that
 // received at most 32 (64) rows is weight streaming only and costs about 0.60
 // (0.75) of a full one, a partly filled one as much as a full one (its six gate-up
-// and eight down tiles: 334 / 424 / 568 / 561 us of CU time at 8448 tokens); with
-// equal counts the XCDs finished up to 25 % apart.
+// and eight down tiles: 334 / 424 / 568 / 561 us of CU time at 8448 tokens when the
+// weights were set, 324 / 344 / 480 / 529 since the tiles have their present loops);
+// with equal counts the XCDs finished up to 25 % apart.
 // Ranges stay contiguous so that the blocks of one expert keep sharing its
 // weights through one L2.  No range is longer than cap_mb blocks (the grid has
 // that many slots per XCD).  One workgroup; bounds[0..8] in m-blocks.
@@ -1578,8 +1579,8 @@ constexpr int kStDmaPerUnit = 3;                               // requests per w
 // choice in the epilogue it cost e4m3 calls of 100 tokens 0.9 %.
 // The arguments in front of the structure are what the start-up needs first: the compiler puts leading scalar arguments
 // into registers that are filled with the workgroup's start (the build's -amdgpu-kernarg-preload-count), everything in a
-// structure is fetched from memory, and a workgroup's first fetch depends on it.  1 token 23.2 -> 22.2 us (both passes
-// and the combine), 64 tokens 100.7 -> 99.4, 128 131.7 -> 130.3, e4m3 100 72.1 -> 71.0.
+// structure is fetched from memory, and a workgroup's first fetch depends on it.  Both passes and the combine, without
+// preloading and with it, us: 1 token 20.8 and 20.2, 64 tokens 101.1 and 99.8, 128 130.7 and 129.2, e4m3 100 70.4 and 68.3.
 template <typename Mma, bool GATED, bool TAIL, bool ONCE = false>
 __global__ __launch_bounds__(kThreads, 3) void stream_gemm_kernel(
     const int32_t* __restrict__ num_post_pad, const int32_t* __restrict__ expert_ids,
@@ -2053,6 +2054,8 @@ MOE_EXPORT int moe_preferred_block_size(int M, int E, int K, int act_dtype, int 
   // at 512; at 192 tokens the streaming kernel still leads, 0.171 against 0.189 ms).
   // e4m3 weights quantise the intermediate between the passes (two launches): from 32
   // rows per expert on (0.181 against 0.193 ms at 512 tokens; 0.172 against 0.166 at 384).
+  // (These lines know only rows per expert and were drawn before the streaming kernel reached its present speed:
+  // moe_call_block_size is the rule for calls whose sizes are known.)
   if (avg >= (weight_dtype == MOE_E4M3 ? 32 : 16)) return 256;
   return 32;
 }

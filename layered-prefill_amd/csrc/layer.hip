@@ -101,19 +101,13 @@ MOE_EXPORT int moe_call_block_size(int M, int H, int I, int E, int K, int act_dt
 // is idle CUs: an expert's weights are walked by I / 128 + H / 256 workgroups, each a serial chain of K tiles, and with
 // `tiles` = E * ceil(I / 128) gate-up tiles for the 256 CUs a layer of few experts leaves the chip half empty, however
 // many rows an expert has.  What the streaming kernel costs above it is re-reading the weights for every 32 rows.
-// The crossover measured, in routed rows per expert, both GEMM passes and the combine, MI355X, Zipf routing:
+// The crossover as measured when the line was drawn, in routed rows per expert, both GEMM passes and the combine, Zipf
+// routing:
 //   bf16 tiles 768 (E 128, I 768): 24; 384 (E 64): 44; 256 (E 32, I 1024): 64; 96 (E 16, I 768; E 32, I 384): 97 and 115;
 //   64 (E 16, I 512): beyond 128.  e4m3 tiles 768: 34; 256: 84; 64: beyond 96.  The 16-bit line lies lower than these
-//   because tiled weights favour the large tile: at 768 tiles it leads from 16 rows on (183.4 us against 187.0 for the
-//   whole call of 256 tokens).
-// The rule knows neither the layout nor H, so plain weights are given to the large tile too early in places (us, large
-// tile against streaming): E 128 at 16 rows 188.4 against 177.6; E 64 at 32 rows 161.8 against 145.2; E 32, I 1024 at 48
-// rows 126.9 against 117.2; and because an expert counts as six tiles at least and 96 rows are always enough, E 32, I 384
-// at 64 and 96 rows 110.5 against 86.1 and 117.2 against 108.2, E 16, I 512 at 96 rows 56.2 against 32.9 (e4m3, H 4096:
-// 88.3 against 69.6).  None of these is slower than under the plain lines of moe_preferred_block_size.
-// For instance E 32, H 2048, I 1024, 256 tokens top-4: 101.5 us against 122.2; 768 tokens: 169.6 against 139.8.
-// E 16, H 1024, I 512, 256 tokens top-4: 25.8 against 55.9.  Layers of more tiles keep the lines of
-// moe_preferred_block_size (16 and 32 rows).
+//   because tiled weights favour the large tile.
+// On the present kernels it gives calls to the large tile too early where weights are plain or the layer is narrow, by 3 to
+// 16 % in the mean and up to 118 % (the figures at moe_call_block_size).
 MOE_EXPORT int moe_layer_block_size(int M, int I, int E, int K, int act_dtype, int weight_dtype) {
   if (act_dtype == MOE_F32 || E < 1 || I < 0) return moe_preferred_block_size(M, E, K, act_dtype, weight_dtype);
   // An expert counts as six tiles at least: a caller that passes 0 for a size it does not know gets the line of I = 768.

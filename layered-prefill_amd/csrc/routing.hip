@@ -585,8 +585,10 @@ MOE_EXPORT int moe_gate_topk_softmax(const void* x, const void* gate_weight, int
 // linear and router, against the library's GEMM and the router: E 128, H 2048, top-8: 6.5 and 9.2 at 1 token, 7.8 and 9.4
 // at 135, 8.5 and 9.4 at 384, 8.7 and 9.4 at 512 (1024 tiles), 10.5 and 10.2 at 640, 10.9 and 10.4 at 1024; E 32, H 2048:
 // 7.3 and 9.1 at 1024, 7.9 and 9.2 at 2047 (1024); E 64, H 4096: 8.0 and 11.6 at 135, 8.9 and 11.5 at 512 (1024), 11.0 and
-// 11.9 at 1024; E 256, H 7168: 12.3 and 12.8 at 64 (896), 15.4 and 13.5 at 135 (2016).  From Python the call is one entry into
-// native code instead of two and an operator.
+// 11.9 at 1024; E 256, H 7168: 12.3 and 12.8 at 64 (896), 15.4 and 13.5 at 135 (2016).  The line follows the GPU's time, as
+// a replayed graph sees it.  Called from Python these sizes are bound by the host, for which this way is one entry into
+// native code and the other two and an operator: norm and router, us, E 128: 15.5 and 30.9 at 640 tokens, 17.9 and 30.8 at
+// 1024, 23.9 and 30.7 at 2047; E 256, H 7168, 135 tokens: 23.2 and 30.9.  16 experts (33 us from Python) have no instance.
 MOE_EXPORT int64_t moe_gate_topk_few_bytes(int T, int H, int E, int dtype) {
   if (T < 1 || H < 64 || H % 64 || (E != 32 && E != 64 && E != 128 && E != 256) || (dtype != MOE_BF16 && dtype != MOE_F16)) return 0;
   if (gate_small_tiles(T, H, E) > 1024) return 0;
