@@ -106,7 +106,9 @@ class Layer:
         self.bm = moe.try_get_optimal_moe_config(self.w13.shape, self.w2.shape, s.top_k, None, self.T,
                                                  act_dtype=self.x.dtype, weight_layout=self.layout)["BLOCK_SIZE_M"]
         code = moe._lib.DTYPE_CODE[self.x.dtype]
-        self.once = 64 if self.bm < moe._lib.lib().moe_preferred_block_size(self.T, s.experts, s.top_k, code, code) else 0
+        own = moe.try_get_optimal_moe_config is moe.fused_moe._LIBRARY_CONFIG   # (not --block-size-m)
+        least = moe._lib.lib().moe_preferred_block_size(self.T, s.experts, s.top_k, code, code)
+        self.once = 64 if own and self.bm < least else 0
         ws = moe.fused_moe.fused_experts_workspace_bytes(self.T, s.hidden, s.intermediate,
                                                          s.experts, s.top_k, self.bm, self.x.dtype)
         self.workspace = torch.empty(ws, dtype=torch.uint8, device=self.dev)
