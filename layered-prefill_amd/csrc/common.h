@@ -35,6 +35,10 @@ bool moe_layer_route_align(const void* logits, int dtype, float* topk_w, int T, 
                            int32_t* sorted_ids, int64_t sorted_cap, int32_t* expert_ids, int64_t expert_cap, int32_t* npp,
                            hipStream_t s, int* rc);
 
+// A layer call of a few tokens in two launches, where it is one that they serve (few.hip); false, and nothing enqueued,
+// elsewhere.  `experts` holds E + 1 ids, `inter` T * K rows.  `rc` is the launches' status.
+bool moe_layer_few(const MoeLayerArgs* a, float* topk_w, int32_t* topk_ids, int32_t* experts, void* inter, int* rc);
+
 // int32 index, inside the 256-byte table of per-XCD ranges at the end of a moe_fused_experts
 // workspace, of the count of expired waits of the one-launch form (cleared with the plan).
 constexpr int kMoeStatusWord = 16;

@@ -139,6 +139,7 @@ MOE_EXPORT int moe_layer(const MoeLayerArgs* a) {
     return moe_fail(MOE_ERR_WORKSPACE, "layer: workspace must be 256-byte aligned");
   const int64_t numel = static_cast<int64_t>(a->T) * a->K;
   int rc = MOE_OK;
+  if (moe_layer_few(a, l.topk_w, l.topk_ids, l.sorted, l.fused_ws, &rc)) return rc;
   const bool routed = a->router_logits &&
                       moe_layer_route_align(a->router_logits, a->logits_dtype, l.topk_w, a->T, a->E, a->K, a->renormalize, l.block,
                                             l.sorted, l.sorted_cap, l.experts, l.expert_cap, l.npp,
