@@ -16,6 +16,7 @@
 // the caller's workspace; three launches (count / scan / scatter) when the
 // tables of the second launch would not fit in LDS.
 #include "common.h"
+#include "quant_device.h"
 #include "routing_device.h"
 
 #include <type_traits>
@@ -402,16 +403,25 @@ __global__ __launch_bounds__(kScanThreads) void align_tiny_kernel(
 }
 
 // Routing in front of it, for the layer call: the ids stay in LDS.  The one workgroup routes its rows with the lane
-// layout, reduction order and results of topk_softmax_pow2_kernel, sixteen wavefronts side by side.
-template <int E, typename El>
+// layout, reduction order and results of topk_softmax_pow2_kernel, sixteen wavefronts side by side.  NV: with e4m3
+// weights further workgroups quantise x meanwhile, rows of up to NV * 512 columns a wavefront each.
+template <int E, typename El, int NV = 0>
 __global__ __launch_bounds__(kScanThreads) void route_align_tiny_kernel(
     const typename El::S* __restrict__ gating, float* __restrict__ topk_w, int32_t* __restrict__ sorted_ids,
     int32_t* __restrict__ expert_ids, int32_t* __restrict__ num_post_pad, int T, int K, int renormalize, int BM, int id_bits,
-    int sorted_cap, int expert_cap) {
+    int sorted_cap, int expert_cap, const typename El::S* __restrict__ x, int H, uint8_t* __restrict__ codes,
+    float* __restrict__ scales) {
   using G = Pow2Geom<E>;
   constexpr int VPT = G::kVpt, TPR = G::kTpr, RPW = G::kRowsPerWave;
   __shared__ int cnt[kScanWaves * kTinyExperts], s_ids[kTinyNumel];
   const int tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  if constexpr (NV > 0) {
+    if (blockIdx.x > 0) {
+      const int64_t row = static_cast<int64_t>(blockIdx.x - 1) * kScanWaves + wave;
+      if (row < T) quant_row<El, NV, kWave>(x + row * H, lane, H, codes + row * H, scales + row);
+      return;
+    }
+  }
   for (int r0 = wave * RPW; r0 < T; r0 += kScanWaves * RPW) {  // (whole wavefronts take part in a row's exchanges)
     const int row = r0 + lane / TPR;
     float v[VPT];
@@ -901,19 +911,26 @@ MOE_EXPORT int moe_align_block_size_planned(const void* topk_ids, int ids_dtype,
 template <int E>
 static int launch_route_align_tiny(const void* logits, int dtype, float* topk_w, int T, int K, int renormalize, int block_size,
                                    int32_t* sorted_ids, int sorted_cap, int32_t* expert_ids, int expert_cap, int32_t* npp,
-                                   hipStream_t s) {
+                                   const MoeXCodes* xc, hipStream_t s) {
   auto go = [&](auto kernel, auto* gating) {
-    hipLaunchKernelGGL(kernel, dim3(1), dim3(kScanThreads), 0, s, gating, topk_w, sorted_ids, expert_ids, npp, T, K, renormalize,
-                       block_size, bits_for(E), sorted_cap, expert_cap);
+    using S = std::remove_reference_t<decltype(*gating)>;
+    const int quant_blocks = xc ? (T + kScanWaves - 1) / kScanWaves : 0;
+    hipLaunchKernelGGL(kernel, dim3(1 + quant_blocks), dim3(kScanThreads), 0, s, gating, topk_w, sorted_ids, expert_ids, npp, T, K,
+                       renormalize, block_size, bits_for(E), sorted_cap, expert_cap, xc ? static_cast<S*>(xc->x) : nullptr,
+                       xc ? xc->H : 0, xc ? xc->codes : nullptr, xc ? xc->scales : nullptr);
   };
-  if (dtype == MOE_BF16) go(route_align_tiny_kernel<E, ElemBF16>, static_cast<const ElemBF16::S*>(logits));
+  if (xc) {
+    const bool wide = xc->H > 2048;
+    if (dtype == MOE_BF16) go(wide ? route_align_tiny_kernel<E, ElemBF16, 8> : route_align_tiny_kernel<E, ElemBF16, 4>, static_cast<const ElemBF16::S*>(logits));
+    else go(wide ? route_align_tiny_kernel<E, ElemF16, 8> : route_align_tiny_kernel<E, ElemF16, 4>, static_cast<const ElemF16::S*>(logits));
+  } else if (dtype == MOE_BF16) go(route_align_tiny_kernel<E, ElemBF16>, static_cast<const ElemBF16::S*>(logits));
   else if (dtype == MOE_F16) go(route_align_tiny_kernel<E, ElemF16>, static_cast<const ElemF16::S*>(logits));
   else go(route_align_tiny_kernel<E, ElemF32>, static_cast<const ElemF32::S*>(logits));
   return moe_check_launch("layer (routing and alignment)");
 }
 bool moe_layer_route_align(const void* logits, int dtype, float* topk_w, int T, int E, int K, int renormalize, int block_size,
                            int32_t* sorted_ids, int64_t sorted_cap, int32_t* expert_ids, int64_t expert_cap, int32_t* npp,
-                           hipStream_t s, int* rc) {
+                           const MoeXCodes* xc, hipStream_t s, int* rc) {
   // One CU routes all rows: with up to half its wavefronts at work that costs less than a launch and a trip of the ids
   // through memory, with more of them the rows queue up.  Whole layer, us, against the two launches: E 128, H 2048,
   // I 768, top-8: 26.0 and 27.1 at 1 token, 52.4 and 53.0 at 9, 60.4 and 60.9 at 16, but 71.5 and 71.1 at 24, 92.6 and
@@ -925,7 +942,7 @@ bool moe_layer_route_align(const void* logits, int dtype, float* topk_w, int T, 
   auto go = [&](auto tag) {
     *rc = launch_route_align_tiny<decltype(tag)::value>(logits, dtype, topk_w, T, K, renormalize, block_size, sorted_ids,
                                                         static_cast<int>(sorted_cap), expert_ids, static_cast<int>(expert_cap),
-                                                        npp, s);
+                                                        npp, xc, s);
     return true;
   };
   switch (E) {

@@ -29,11 +29,33 @@ struct MoeLdsOptIn {
 };
 int moe_opt_in_lds(MoeLdsOptIn& flags, const void* kernel, int lds_bytes, const char* what);
 
+// The e4m3 codes of a layer call's x, which wait for nothing and so may be made beside the routing: where x is and where
+// they and their row scales go.  moe_x_codes_ok: rows that the routing kernels quantise.
+struct MoeXCodes {
+  const void* x;
+  int H;
+  uint8_t* codes;
+  float* scales;
+};
+static inline bool moe_x_codes_ok(const MoeXCodes& c) {
+  return c.H % 8 == 0 && c.H <= 4096 && (reinterpret_cast<uintptr_t>(c.x) & 15u) == 0 && (reinterpret_cast<uintptr_t>(c.codes) & 7u) == 0;
+}
+
 // Router and alignment of a layer call in one launch, for the batches and layers where that is the faster way (align.hip);
-// false, and nothing enqueued, elsewhere.  `rc` is the launch's status.
+// false, and nothing enqueued, elsewhere.  With `xc` it makes those codes, too.  `rc` is the launch's status.
 bool moe_layer_route_align(const void* logits, int dtype, float* topk_w, int T, int E, int K, int renormalize, int block_size,
                            int32_t* sorted_ids, int64_t sorted_cap, int32_t* expert_ids, int64_t expert_cap, int32_t* npp,
-                           hipStream_t s, int* rc);
+                           const MoeXCodes* xc, hipStream_t s, int* rc);
+
+// Router and e4m3 codes of x, which wait for nothing of each other, in one launch; false, and nothing enqueued, where no
+// instance serves the call.
+bool moe_layer_route_quant(const void* logits, int dtype, float* topk_w, int32_t* topk_ids, int T, int E, int K, int renormalize,
+                           const MoeXCodes& xc, hipStream_t s, int* rc);
+
+// Where a moe_fused_experts call of e4m3 weights keeps the codes and scales of x in its workspace, and that call with them
+// there already.
+void moe_experts_x_codes(const MoeFusedExpertsArgs* a, uint8_t** codes, float** scales);
+int moe_fused_experts_of_codes(const MoeFusedExpertsArgs* a, bool x_coded);
 
 // A layer call of a few tokens in two launches, where it is one that they serve (few.hip); false, and nothing enqueued,
 // elsewhere.  `experts` holds E + 1 ids, `inter` T * K rows.  `rc` is the launches' status.

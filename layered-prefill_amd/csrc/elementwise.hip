@@ -3,6 +3,7 @@
 // combine (nanovllm/layers/for_moe/moe_easy_kernel.py:26-31) and fp8 row
 // quantisation.  16-byte vector accesses, grid-stride loops.
 #include "common.h"
+#include "quant_device.h"
 
 namespace {
 
@@ -106,18 +107,6 @@ __device__ __forceinline__ uint8_t f32_to_e4m3(float v) {
   return static_cast<uint8_t>(__builtin_amdgcn_cvt_pk_fp8_f32(v, v, 0, false) & 0xff);
 }
 
-// Two values at once: bits 0-7 the code of a, bits 8-15 the code of b.
-__device__ __forceinline__ uint32_t f32x2_to_e4m3(float a, float b) {
-  a = __builtin_amdgcn_fmed3f(a, -448.f, 448.f);
-  b = __builtin_amdgcn_fmed3f(b, -448.f, 448.f);
-  return static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false)) & 0xffffu;
-}
-
-// Smallest row scale: a row whose largest magnitude is tiny but not zero would get
-// a scale whose reciprocal overflows (amax below about 1.3e-36); from 2^-100 down
-// the scale stays 2^-100 and the row's codes are simply small.
-constexpr float kMinScale = 7.888609052210118e-31f;  // 2^-100
-
 // One wavefront per row: s = max(amax|row| / 448, 2^-100) (1 for an all-zero row),
 // q = e4m3(row * (1 / s)): one correctly rounded division per row, then one
 // multiplication per element (a division per element made the kernel
@@ -153,39 +142,7 @@ __global__ __launch_bounds__(kThreads) void quant_rows_e4m3_vec_kernel(
   const int64_t row = blockIdx.x * static_cast<int64_t>(kThreads / LPR) + threadIdx.x / LPR;
   if (row >= rows) return;
   if (row_ids && (row >= id_count || row_ids[row] >= numel)) return;  // a padding slot: nobody reads it
-  const uint4* src = reinterpret_cast<const uint4*>(w + row * cols);
-  const int nvec = cols / 8;
-  uint4 v[NV];
-  float amax = 0.f;
-#pragma unroll
-  for (int i = 0; i < NV; ++i) {
-    const int c = lane + i * LPR;
-    v[i] = c < nvec ? src[c] : uint4{0, 0, 0, 0};
-    const uint32_t wds[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      amax = fmaxf(amax, fabsf(El::ld(static_cast<uint16_t>(wds[j]))));
-      amax = fmaxf(amax, fabsf(El::ld(static_cast<uint16_t>(wds[j] >> 16))));
-    }
-  }
-  amax = row_max<LPR>(amax);
-  const float s = amax > 0.f ? fmaxf(amax / 448.f, kMinScale) : 1.f;
-  if (lane == 0) scales[row] = s;
-  const float inv = 1.0f / s;
-  uint2* dst = reinterpret_cast<uint2*>(q + row * cols);
-#pragma unroll
-  for (int i = 0; i < NV; ++i) {
-    const int c = lane + i * LPR;
-    if (c >= nvec) continue;
-    const uint32_t wds[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
-    uint32_t o[2] = {0, 0};
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      o[j >> 1] |= f32x2_to_e4m3(El::ld(static_cast<uint16_t>(wds[j])) * inv,
-                                 El::ld(static_cast<uint16_t>(wds[j] >> 16)) * inv)
-                   << (16 * (j & 1));
-    dst[c] = uint2{o[0], o[1]};
-  }
+  quant_row<El, NV, LPR>(w + row * cols, lane, cols, q + row * cols, scales + row);
 }
 
 template <typename El>

@@ -2128,7 +2128,16 @@ MOE_EXPORT int moe_fused_experts_status(const MoeFusedExpertsArgs* a) {
   return MOE_OK;
 }
 
-MOE_EXPORT int moe_fused_experts(const MoeFusedExpertsArgs* a) {
+void moe_experts_x_codes(const MoeFusedExpertsArgs* a, uint8_t** codes, float** scales) {
+  const int64_t es = elem_size(a->act_dtype), numel = static_cast<int64_t>(a->T) * a->K;
+  const int64_t rows = moe_align_up(numel + static_cast<int64_t>(a->E) * (a->block_size - 1), a->block_size);
+  *codes = static_cast<uint8_t*>(a->workspace) + moe_align_up(rows * a->I * es, 256) + moe_align_up(numel * a->H * es, 256);
+  *scales = reinterpret_cast<float*>(*codes + moe_align_up(static_cast<int64_t>(a->T) * a->H, 256));
+}
+
+MOE_EXPORT int moe_fused_experts(const MoeFusedExpertsArgs* a) { return moe_fused_experts_of_codes(a, false); }
+
+int moe_fused_experts_of_codes(const MoeFusedExpertsArgs* a, bool x_coded) {
   int64_t cap = 0, need_ws = 0;
   if (int rc0 = check_fused_args(a, &cap, &need_ws)) return rc0;
   if (a->T == 0) return MOE_OK;
@@ -2140,8 +2149,9 @@ MOE_EXPORT int moe_fused_experts(const MoeFusedExpertsArgs* a) {
   const int64_t rows = moe_align_up(cap, a->block_size);
   char* inter = static_cast<char*>(a->workspace);
   char* c3 = inter + moe_align_up(rows * a->I * es, 256);
-  char* xq = c3 + moe_align_up(numel * a->H * es, 256);                        // fp8 only from here on
-  float* xs = reinterpret_cast<float*>(xq + moe_align_up(static_cast<int64_t>(a->T) * a->H, 256));
+  uint8_t* xq;                                                                 // fp8 only from here on
+  float* xs;
+  moe_experts_x_codes(a, &xq, &xs);
   char* iq = reinterpret_cast<char*>(xs) + moe_align_up(static_cast<int64_t>(a->T) * 4, 256);
   float* is = reinterpret_cast<float*>(iq + moe_align_up(rows * a->I, 256));
 
@@ -2209,7 +2219,7 @@ MOE_EXPORT int moe_fused_experts(const MoeFusedExpertsArgs* a) {
   }
   if (fp8 && (passes & 1)) {
     // dynamic per-token e4m3 activations: s[t] = amax|x[t]| / 448
-    rc = moe_quant_rows_e4m3(a->x, a->act_dtype, a->T, a->H, reinterpret_cast<uint8_t*>(xq), xs, a->stream);
+    if (!x_coded) rc = moe_quant_rows_e4m3(a->x, a->act_dtype, a->T, a->H, xq, xs, a->stream);
     if (rc) return rc;
     p.a = xq; p.a_scale = xs; p.w_scale = a->w13_scale; p.w_scale_stride_e = 2LL * a->I;
     rc = a->act_dtype == MOE_BF16 ? launch_bm<MmaE4M3<ElemBF16>, true>(p, a->block_size, cap, s)

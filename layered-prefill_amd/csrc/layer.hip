@@ -140,12 +140,25 @@ MOE_EXPORT int moe_layer(const MoeLayerArgs* a) {
   const int64_t numel = static_cast<int64_t>(a->T) * a->K;
   int rc = MOE_OK;
   if (moe_layer_few(a, l.topk_w, l.topk_ids, l.sorted, l.fused_ws, &rc)) return rc;
+  // what the expert passes will be given: the routing of an e4m3 call leaves the codes of x in their workspace
+  MoeFusedExpertsArgs f{};
+  f.workspace = l.fused_ws; f.workspace_bytes = l.fused_bytes;
+  f.T = a->T; f.H = a->H; f.I = a->I; f.E = a->E; f.K = a->K;
+  f.block_size = l.block; f.act_dtype = a->act_dtype; f.weight_dtype = a->weight_dtype;
+  MoeXCodes xc{a->x, a->H, nullptr, nullptr};
+  moe_experts_x_codes(&f, &xc.codes, &xc.scales);
+  const bool code_x = a->router_logits && a->weight_dtype == MOE_E4M3 && a->logits_dtype == a->act_dtype && moe_x_codes_ok(xc);
   const bool routed = a->router_logits &&
                       moe_layer_route_align(a->router_logits, a->logits_dtype, l.topk_w, a->T, a->E, a->K, a->renormalize, l.block,
-                                            l.sorted, l.sorted_cap, l.experts, l.expert_cap, l.npp,
+                                            l.sorted, l.sorted_cap, l.experts, l.expert_cap, l.npp, code_x ? &xc : nullptr,
                                             static_cast<hipStream_t>(a->stream), &rc);
   if (rc) return rc;
-  if (a->router_logits && !routed) {
+  bool x_coded = routed && code_x;
+  if (code_x && !routed)
+    x_coded = moe_layer_route_quant(a->router_logits, a->logits_dtype, l.topk_w, l.topk_ids, a->T, a->E, a->K, a->renormalize, xc,
+                                    static_cast<hipStream_t>(a->stream), &rc);
+  if (rc) return rc;
+  if (a->router_logits && !routed && !x_coded) {
     if (int rc = moe_topk_softmax_typed(a->router_logits, a->logits_dtype, l.topk_w, l.topk_ids, nullptr, a->T, a->E, a->K,
                                         a->renormalize, a->stream))
       return rc;
@@ -166,17 +179,14 @@ MOE_EXPORT int moe_layer(const MoeLayerArgs* a) {
     rc = moe_align_block_size(l.topk_ids, MOE_ID_I32, numel, a->E, l.block, l.sorted, l.sorted_cap, l.experts, l.expert_cap,
                               l.npp, l.align_ws, l.align_bytes, a->stream);
   if (rc) return rc;
-  MoeFusedExpertsArgs f{};
   f.x = a->x; f.out = a->out; f.w13 = a->w13; f.w2 = a->w2;
   f.w13_bias = a->w13_bias; f.w2_bias = a->w2_bias; f.w13_scale = a->w13_scale; f.w2_scale = a->w2_scale;
   f.topk_weights = l.topk_w;
   f.sorted_token_ids = l.sorted; f.expert_ids = l.experts; f.num_tokens_post_pad = l.npp;
-  f.workspace = l.fused_ws; f.workspace_bytes = l.fused_bytes;
   f.w13_stride_e = a->w13_stride_e; f.w13_stride_n = a->w13_stride_n;
   f.w2_stride_e = a->w2_stride_e; f.w2_stride_n = a->w2_stride_n;
-  f.T = a->T; f.H = a->H; f.I = a->I; f.E = a->E; f.K = a->K;
-  f.block_size = l.block; f.sorted_cap = l.sorted_cap;
-  f.act_dtype = a->act_dtype; f.weight_dtype = a->weight_dtype; f.activation = a->activation;
+  f.sorted_cap = l.sorted_cap;
+  f.activation = a->activation;
   f.apply_router_weight_on_input = a->apply_router_weight_on_input;
   f.swiglu_alpha = a->swiglu_alpha; f.swiglu_limit = a->swiglu_limit;
   f.passes = plan ? 16 : 0;
@@ -184,5 +194,5 @@ MOE_EXPORT int moe_layer(const MoeLayerArgs* a) {
   if (!a->block_size && l.block < moe_preferred_block_size(a->T, a->E, a->K, a->act_dtype, a->weight_dtype)) f.passes |= 64;
   f.weight_layout = a->weight_layout;
   f.stream = a->stream;
-  return moe_fused_experts(&f);
+  return moe_fused_experts_of_codes(&f, x_coded);
 }
