@@ -121,6 +121,7 @@ struct GemmParams {
   int w_tiled;       // weights: units [expert][n-tile][K tile] (moe_tile_expert_weights)
   int a_tiled;       // A operand of the down pass: units [m-block][K tile]
   int c_tiled;       // result of the gate-up pass written as such units
+  int chain;         // down pass of the large-tile kernel: a workgroup takes two n-tiles of a full block (big_chain)
   int ragged;        // rows are not whole 16-byte chunks (K or a stride not a multiple of 16 bytes, or a
                      // base that is not 16-byte aligned): the register-staged kernel loads element by element
 };
@@ -512,6 +513,15 @@ constexpr uint32_t dma_win_bias(int j) { return static_cast<uint32_t>(4096 - (j 
 // long as one of 256.
 constexpr int kFragStep = 2 * 32 * kBigRowBytes;
 
+// Two n-tiles of a full block one behind the other (big_chain): the second one's A(0) and W(0) go to ring slots
+// kChainUnit and kChainUnit + 1 while the first one's results are parked and written, kChainRows rows of a wavefront at a
+// time, in front of them.
+constexpr int kChainUnit = 3, kChainRows = 64;
+constexpr int kChainEpiBytes = kChainRows * kEpiRowBytes;
+constexpr int kChainSide = 4 * kChainEpiBytes;
+static_assert(kChainSide + kBigSideBytes <= kChainUnit * kBigUnitBytes, "the epilogue stays in front of the next operands");
+constexpr int kChainStores = 32;   // of a wavefront and n-tile
+
 // Main loop for a wavefront that has FMC live token fragments (0..4).
 // Unit j of the stream  A(0) W(0) A(1) W(1) ...  lives in ring slot j % 5.
 // The caller has requested W(0) and the first half of W(1) (when nk > 1) before
@@ -531,9 +541,9 @@ constexpr int kFragStep = 2 * 32 * kBigRowBytes;
 // instances of the tile body instead of tests around every request, an LDS read
 // is one instruction (lane base + slot in one addition per operand and step,
 // everything else in the offset field), a DMA request three.
-template <typename Mma, int FMC, bool GATED>
+template <typename Mma, int FMC, bool GATED, bool CHAIN = false>
 __device__ __forceinline__ void big_mainloop(const BigCtx& c, const char* smem, int nk,
-                                             f32x16 (&acc)[4][4]) {
+                                             f32x16 (&acc)[4][4], bool second = false) {
   constexpr int CH = Mma::kBigChunks, STEPS = 4 / CH;
   constexpr int PER = 12 / (STEPS - 1);  // requests carried by each of the first STEPS-1 steps
   constexpr int XF = FMC > 0 ? FMC : 1;
@@ -591,6 +601,7 @@ __device__ __forceinline__ void big_mainloop(const BigCtx& c, const char* smem, 
   // A(kt+2) to fw
   auto next_slot = [](int s) { return s + 2 * kBigUnitBytes >= kBigUnits * kBigUnitBytes ? s + (2 - kBigUnits) * kBigUnitBytes : s + 2 * kBigUnitBytes; };
   int sa = 0, sw = kBigUnitBytes, fa = 3 * kBigUnitBytes, fw = 4 * kBigUnitBytes;
+  if (CHAIN && second) sa = kChainUnit * kBigUnitBytes, sw = (kChainUnit + 1) * kBigUnitBytes, fa = kBigUnitBytes, fw = 2 * kBigUnitBytes;
   const char* a2 = c.a_base + 2 * c.a_step;  // rows of A(kt+2)
   const char* w1 = c.w_base + c.w_step;      // rows of W(kt+1)
 
@@ -639,6 +650,18 @@ __device__ __forceinline__ void big_mainloop(const BigCtx& c, const char* smem, 
 
   // fill the ring: W(0) and half of W(1) were requested by the caller as soon as it knew
   // the expert; A(0) and A(1) follow here.  Then wait for tile 0 only.
+  if (CHAIN && second) {
+    // A(0) and W(0) were requested ahead of the first n-tile's epilogue, whose stores are behind them: exactly so many
+    static_for<0, 4>([&](auto it) {
+      constexpr int i = decltype(it)::value;
+      lds_dma16_win<i, i == 0>(w1, c.w_off[i], c.dma_lds + fa);
+    });
+    static_for<0, 8>([&](auto it) {
+      constexpr int i = decltype(it)::value;
+      lds_dma16_win<i, i == 0>(c.a_base + c.a_step, c.a_off[i], c.dma_lds);
+    });
+    wait_vmcnt<12 + kChainStores>();
+  } else {
   static_for<0, 8>([&](auto it) {
     constexpr int i = decltype(it)::value;
     lds_dma16_win<i, i == 0>(c.a_base, c.a_off[i], c.dma_lds);
@@ -651,6 +674,7 @@ __device__ __forceinline__ void big_mainloop(const BigCtx& c, const char* smem, 
     wait_vmcnt<kBigDmaPerUnit>();
   } else {
     wait_vmcnt<0>();
+  }
   }
   bare_barrier();
   if constexpr (FMC > 0) {
@@ -764,7 +788,7 @@ __device__ __forceinline__ void big_light_mainloop(const BigCtx& c, const char* 
 // exp2/rcp, one rounding at the end) and only the 64 output columns are parked.
 // The other activations park gate and up rounded, as the stand-alone activation
 // kernels see them, and the flush combines them.
-template <typename El, int FMC, bool GATED, bool SCALED, bool BIAS, bool FAST_SILU>
+template <typename El, int FMC, bool GATED, bool SCALED, bool BIAS, bool FAST_SILU, int FM0 = 0, bool PIN = false>
 __device__ __forceinline__ void big_park(const GemmParams& p, int e, int n0, int wn, int wm, int lhi, int l32,
                                          const float* s_rw, const float* s_as, const float* s_ws,
                                          const float* s_bias, char* epi, f32x16 (&acc)[4][4]) {
@@ -783,7 +807,7 @@ __device__ __forceinline__ void big_park(const GemmParams& p, int e, int n0, int
     // this way, 8448 tokens 568.8 and 543.2; 32 experts, H 4096, I 1024, 2000 tokens 362.7 and 353.3.  Same bits.)
     float as[4], rw[4];
 #pragma unroll
-    for (int fm = 0; fm < FMC; ++fm) {
+    for (int fm = FM0; fm < FMC; ++fm) {
       as[fm] = s_as[(2 * fm + wm) * 32 + l32];
       rw[fm] = s_rw[(2 * fm + wm) * 32 + l32];
     }
@@ -800,13 +824,13 @@ __device__ __forceinline__ void big_park(const GemmParams& p, int e, int n0, int
           if constexpr (BIAS) bs[q][g] = *reinterpret_cast<const f32x4*>(s_bias + at);
         }
 #pragma unroll
-      for (int fm = 0; fm < FMC; ++fm) {
+      for (int fm = FM0; fm < FMC; ++fm) {
         // The accumulators stay where they are until their turn.  (The compiler copies them out of the accumulation
         // registers behind the last product of each, in front of the branches that lead here, which takes 256 more
         // registers than its main loop leaves.  The 16-bit loop leaves enough, and there the copies are as well placed.)
         asm volatile("" : "+a"(acc[fn][fm]));
         if constexpr (FAST_SILU) asm volatile("" : "+a"(acc[fn + 2][fm]));
-        char* row = epi + (fm * 32 + l32) * kEpiRowBytes;
+        char* row = epi + ((fm - FM0) * 32 + l32) * kEpiRowBytes;
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
           auto value = [&](int q, int i) {
@@ -841,10 +865,13 @@ __device__ __forceinline__ void big_park(const GemmParams& p, int e, int n0, int
     for (int i = 0; i < 4; ++i) v[i] *= rw;
   };
 #pragma unroll
-  for (int fm = 0; fm < FMC; ++fm) {
+  for (int fm = FM0; fm < FMC; ++fm) {
+    if constexpr (PIN)
+#pragma unroll
+      for (int fn = 0; fn < 4; ++fn) asm volatile("" : "+a"(acc[fn][fm]));
     const int slot = (2 * fm + wm) * 32 + l32;   // of the block
     const float rw = s_rw[slot];
-    char* row = epi + (fm * 32 + l32) * kEpiRowBytes;
+    char* row = epi + ((fm - FM0) * 32 + l32) * kEpiRowBytes;
 #pragma unroll
     for (int fn = 0; fn < (FAST_SILU ? 2 : 4); ++fn) {
 #pragma unroll
@@ -1019,7 +1046,93 @@ __device__ __forceinline__ void big_wave(const GemmParams& p, BigCtx& c, char* s
   }
 }
 
-// One output tile of the large-tile kernel: m-block mb, n-tile nt.  `wait.ready()` is called by the workgroup's first
+// kChainRows parked rows of a wavefront, of the token fragments fm0 and fm0 + 1, to global memory: a full block inside the
+// matrix, so that every wavefront makes the same number of stores.
+template <typename El>
+__device__ __forceinline__ void chain_flush(const GemmParams& p, int n0, int wn, int wm, int lane, int fm0, const int* s_tok,
+                                            const char* epi) {
+  constexpr int COLS = 128, LPR = COLS / 8, RPS = kWave / LPR, UNR = 8;
+  const int c8 = (lane % LPR) * 8, lrow = lane / LPR;
+  char* const cbase = static_cast<char*>(p.c) + static_cast<int64_t>(n0 + wn * COLS + c8) * 2;
+  const int64_t ldc_bytes = static_cast<int64_t>(p.ldc) * 2;
+#pragma unroll
+  for (int r0 = 0; r0 < kChainRows; r0 += RPS * UNR) {
+    int crow[UNR];
+    uint4 out[UNR];
+#pragma unroll
+    for (int u = 0; u < UNR; ++u) {
+      const int r = r0 + u * RPS + lrow;
+      crow[u] = s_tok[(2 * (fm0 + (r >> 5)) + wm) * 32 + (r & 31)];
+      out[u] = *reinterpret_cast<const uint4*>(epi + r * kEpiRowBytes + c8 * 2);
+    }
+#pragma unroll
+    for (int u = 0; u < UNR; ++u) *reinterpret_cast<uint4*>(cbase + crow[u] * ldc_bytes) = out[u];
+  }
+}
+
+// Two n-tiles of a full block of the down pass, whose K is short (12 K tiles of the benchmark's layer): the second one's
+// first operands arrive while the first one's results leave, so that it has no start, which with the ring's fill is 7 of a
+// tile's 28 us.  One loop over both, not unrolled, and accumulators pinned where they are until they are parked: otherwise
+// the 16-bit kernel spills up to 42 registers (67584 rows 806 us).
+template <typename Mma>
+__device__ __forceinline__ void big_chain(const GemmParams& p, BigCtx& c, char* smem, int nk, int n0, int wn, int wm, int my_tok,
+                                          float my_rw, float my_as, float my_ws, float my_ws2) {
+  using El = typename Mma::El;
+  {
+    constexpr int CH = Mma::kBigChunks;
+    const int lane = fresh_lane(), l32 = lane & 31, lhi = lane >> 5;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      c.rd_k[q] = l32 * kBigRowBytes + (((CH * (2 * (q / CH) + lhi) + q % CH) ^ ((l32 >> 1) & 7)) << 4);
+  }
+  int* s_tok = reinterpret_cast<int*>(smem + kChainSide);
+  float* s_rw = reinterpret_cast<float*>(smem + kChainSide + kBigBM * 4);
+  char* epi = smem + (2 * wn + wm) * kChainEpiBytes;
+#pragma unroll 1
+  for (int t = 0; t < 2; ++t) {
+    f32x16 acc[4][4];
+#pragma unroll
+    for (int fn = 0; fn < 4; ++fn)
+#pragma unroll
+      for (int fm = 0; fm < 4; ++fm)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[fn][fm][r] = 0.f;
+    big_mainloop<Mma, 4, false, true>(c, smem, nk, acc, t != 0);
+    bare_barrier();  // every wavefront is done reading the ring before it is reused
+    if (t == 0) {
+      c.w_base += p.w_tiled ? static_cast<int64_t>(nk) * kBigUnitBytes : static_cast<int64_t>(kBigBNW) * p.w_stride_n * Mma::kEs;
+      static_for<0, 8>([&](auto it) {
+        constexpr int i = decltype(it)::value;
+        lds_dma16_win<i, i == 0>(c.w_base, c.w_off[i], c.dma_lds + (kChainUnit + 1) * kBigUnitBytes);
+      });
+      static_for<0, 8>([&](auto it) {
+        constexpr int i = decltype(it)::value;
+        lds_dma16_win<i, i == 0>(c.a_base, c.a_off[i], c.dma_lds + kChainUnit * kBigUnitBytes);
+      });
+    }
+    const int lane = fresh_lane(), tid = (2 * wn + wm) * kWave + lane;
+    s_tok[tid] = my_tok;
+    s_rw[tid] = my_rw;
+    if constexpr (Mma::kEs == 1) {
+      s_rw[kBigBM + tid] = my_as;
+      s_rw[2 * kBigBM + tid] = t == 0 ? my_ws : my_ws2;
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    bare_barrier();
+    big_park<El, 2, false, Mma::kEs == 1, false, false, 0, true>(p, 0, n0, wn, wm, lane >> 5, lane & 31, s_rw, s_rw + kBigBM,
+                                                           s_rw + 2 * kBigBM, nullptr, epi, acc);
+    chain_flush<El>(p, n0, wn, wm, lane, 0, s_tok, epi);
+    big_park<El, 4, false, Mma::kEs == 1, false, false, 2, true>(p, 0, n0, wn, wm, lane >> 5, lane & 31, s_rw, s_rw + kBigBM,
+                                                           s_rw + 2 * kBigBM, nullptr, epi, acc);
+    chain_flush<El>(p, n0, wn, wm, lane, 2, s_tok, epi);
+    n0 += kBigBNW;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    bare_barrier();  // the parked rows are read: the next operands may land on them
+  }
+}
+
+// One output tile of the large-tile kernel: m-block mb, n-tile nt; or, `chained`, n-tiles nt and nt + 1 of a full block.
+// `wait.ready()` is called by the workgroup's first
 // wavefront before any row of the A operand is read; it returns whether that operand is complete.  Where it is not, the
 // workgroup calls `wait.expired(p, mb, nt)` instead of multiplying.
 // The start of a tile is a chain of memory latencies with idle matrix pipes.  The expert's id and the slot ids are one
@@ -1029,7 +1142,7 @@ __device__ __forceinline__ void big_wave(const GemmParams& p, BigCtx& c, char* s
 // ids one after the other and eight divisions between the requests: 8448 tokens 766 us, 757 now, 256 tokens 166.5 and
 // 164.1, e4m3 8448 554 and 548 (both passes and the combine).
 template <typename Mma, bool GATED, typename Wait>
-__device__ __forceinline__ void big_tile(const GemmParams& p, int mb, int nt, char* smem, Wait wait) {
+__device__ __forceinline__ void big_tile(const GemmParams& p, int mb, int nt, bool chained, char* smem, Wait wait) {
   using El = typename Mma::El;
   // (uniform, and known to the compiler as such: a branch on a vector register keeps the operands of the bodies not
   // taken alive through the one that is)
@@ -1117,6 +1230,7 @@ __device__ __forceinline__ void big_tile(const GemmParams& p, int mb, int nt, ch
     if (__builtin_amdgcn_readfirstlane(s_cnt[4]) == 0) {
       wait_vmcnt<0>();  // nothing may still be landing in LDS when the workgroup ends
       wait.template expired<typename Mma::El>(p, mb, nt);
+      if (chained) wait.template expired<typename Mma::El>(p, mb, nt + 1);
       return;
     }
   }
@@ -1129,6 +1243,7 @@ __device__ __forceinline__ void big_tile(const GemmParams& p, int mb, int nt, ch
   if (p.mul_weight) my_rw = my_tok < p.numel ? p.topk_w[my_tok] : 0.f;
   if (p.a_scale && my_tok < p.numel) my_as = p.a_scale[p.a_by_slot ? my_slot : my_tok / p.top_k];
   float my_bias = 0.f;
+  [[maybe_unused]] float my_ws2 = 1.f;
   if (p.w_scale || p.bias) {
     // scale and bias of the weight row that sits at row `tid` of a weight unit
     int64_t wr;
@@ -1140,6 +1255,7 @@ __device__ __forceinline__ void big_tile(const GemmParams& p, int mb, int nt, ch
       wr = n0 + tid < p.N ? n0 + tid : p.N - 1;
     }
     if (p.w_scale) my_ws = p.w_scale[e * p.w_scale_stride_e + wr];
+    if (!GATED && p.w_scale && chained) my_ws2 = p.w_scale[e * p.w_scale_stride_e + wr + kBigBNW];
     if (p.bias) my_bias = El::ld(static_cast<const typename El::S*>(p.bias)[e * p.bias_stride_e + wr]);
   }
   if (p.a_tiled) {
@@ -1187,6 +1303,12 @@ __device__ __forceinline__ void big_tile(const GemmParams& p, int mb, int nt, ch
     big_wave<Mma, decltype(fm_tag)::value, GATED, decltype(light_tag)::value != 0>(
         p, c, smem, nk, e, n0, wn, wm, my_tok, my_rw, my_as, my_ws, my_bias, s_tok, s_rw_all, epi);
   };
+  if constexpr (!GATED) {
+    if (chained) {
+      big_chain<Mma>(p, c, smem, nk, n0, wn, wm, my_tok, my_rw, my_as, my_ws, my_ws2);
+      return;
+    }
+  }
   using Yes = IntTag<1>;
   using No = IntTag<0>;
   // The streaming-shaped loop is a workgroup-wide choice.  The compiler lays the bodies out one behind the other and
@@ -1214,6 +1336,33 @@ __device__ __forceinline__ void big_tile(const GemmParams& p, int mb, int nt, ch
   }
 }
 
+// Whether n-tile nt of m-block mb is one of two that one workgroup takes: of the first, whose workgroup takes both, or of
+// the second, whose workgroup has nothing to do.
+__device__ __forceinline__ bool chained_tile(const GemmParams& p, int mb, int nt) {
+  if (!p.chain || (nt | 1) >= p.num_n_tiles) return false;
+  const int64_t last = static_cast<int64_t>(mb) * kBigBM + kBigBM - 1;   // real slots come first in a block
+  return last < p.sorted_cap && uniform_load(p.sorted_ids + last) < p.numel;
+}
+
+// Place i of an XCD's list of tiles: block (counted from the range's first) and n-tile.  Where blocks may be chained, four
+// blocks' tiles go in two groups, all even n-tiles and all odd ones: of a chained block the workgroups of the odd ones have
+// nothing to do.  The shader engines of an XCD take its workgroups in turn, so the ones that stay have to come in whole
+// rounds of them: one of two in turn, half the CUs were idle.
+constexpr int kChainGroup = 4;
+struct TilePlace { int mb, nt; };
+__device__ __forceinline__ TilePlace tile_place(const GemmParams& p, int i) {
+  const int n = p.num_n_tiles;
+  if (!p.chain) return {i / n, i % n};
+  const int g = i / (kChainGroup * n), r = i - g * (kChainGroup * n), evens = (n + 1) >> 1, odds = n >> 1;
+  if (r < kChainGroup * evens) return {g * kChainGroup + r / evens, r % evens * 2};
+  const int q = r - kChainGroup * evens;
+  return {g * kChainGroup + q / odds, q % odds * 2 + 1};
+}
+// Blocks of an XCD's range that its list has places for.
+__host__ __device__ __forceinline__ int listed_blocks(const GemmParams& p, int cap_mb) {
+  return p.chain ? (cap_mb + kChainGroup - 1) / kChainGroup * kChainGroup : cap_mb;
+}
+
 struct NoWait {
   static constexpr bool kWaits = false;
 };
@@ -1228,8 +1377,9 @@ __global__ __launch_bounds__(kThreads, 1) void big_gemm_kernel(const GemmParams 
   if (p.xcd_bounds) {
     // ranges of equal estimated work (big_plan_kernel), m-block major inside a range
     const int lo = p.xcd_bounds[blockIdx.x % kXcds], hi = p.xcd_bounds[blockIdx.x % kXcds + 1];
-    mb = lo + xslot / p.num_n_tiles;
-    nt = xslot % p.num_n_tiles;
+    const TilePlace at = GATED ? TilePlace{xslot / p.num_n_tiles, xslot % p.num_n_tiles} : tile_place(p, xslot);
+    mb = lo + at.mb;
+    nt = at.nt;
     // the second test keeps a plan that was never written from sending a tile out of range
     if (mb >= hi || lo < 0 || mb >= p.num_m_blocks) return;
   } else {
@@ -1247,7 +1397,9 @@ __global__ __launch_bounds__(kThreads, 1) void big_gemm_kernel(const GemmParams 
     mb = logical - nt * live_mb;
   }
   }
-  big_tile<Mma, GATED>(p, mb, nt, smem, NoWait{});
+  const bool chained = !GATED && chained_tile(p, mb, nt);
+  if (chained && (nt & 1)) return;
+  big_tile<Mma, GATED>(p, mb, nt, chained, smem, NoWait{});
 }
 
 // Both passes in one launch, for the 16-bit dtypes.  Workgroup ids go to the XCDs
@@ -1318,7 +1470,7 @@ __global__ __launch_bounds__(kThreads, 1) void big_fused_kernel(const GemmParams
   if (xslot < n1) {
     const int mb = lo + xslot / p1.num_n_tiles, nt = xslot % p1.num_n_tiles;
     if (mb >= hi || lo < 0 || mb >= p1.num_m_blocks) return;  // (an unwritten plan must not send a tile out of range)
-    big_tile<Mma, true>(p1, mb, nt, smem, NoWait{});
+    big_tile<Mma, true>(p1, mb, nt, false, smem, NoWait{});
     // Every store of this workgroup is complete before the barrier.  With write-through stores
     // (whole tiles inside the matrix) that means visible device-wide; otherwise the release
     // writes the L2 back first.  Measured at 8448 tokens, both passes: 766 us with no ordering
@@ -1331,9 +1483,12 @@ __global__ __launch_bounds__(kThreads, 1) void big_fused_kernel(const GemmParams
     }
   } else {
     const int j = xslot - n1;
-    const int mb = lo + j / p2.num_n_tiles, nt = j % p2.num_n_tiles;
+    const TilePlace at = tile_place(p2, j);
+    const int mb = lo + at.mb, nt = at.nt;
     if (mb >= hi || lo < 0 || mb >= p1.num_m_blocks) return;
-    big_tile<Mma, false>(p2, mb, nt, smem, GateUpWait{done + mb, status, p1.num_n_tiles, spin_limit});
+    const bool chained = chained_tile(p2, mb, nt);
+    if (chained && (nt & 1)) return;
+    big_tile<Mma, false>(p2, mb, nt, chained, smem, GateUpWait{done + mb, status, p1.num_n_tiles, spin_limit});
   }
 }
 
@@ -1757,6 +1912,20 @@ static int big_plan_cap(int64_t sorted_cap) {
   return static_cast<int>(cap < mbs ? cap : mbs);
 }
 
+// Whether the workgroups of a down pass take two n-tiles of every full block (big_chain): from so many tiles on that whole
+// pairs still fill the CUs evenly, in routed rows times n-tiles.  Whole layer, us, a tile and a pair a workgroup:
+//   bf16, 128 experts, H 2048 (8 n-tiles), I 768, top-8: 12000 rows 301.0 and 301.7; 32000 478.2 and 476.1; 48000 623.9 and
+//   603.8; 67584 803.2 and 783.9; 135168 1471.7 and 1410.2.  32 experts, H 2048, I 1024, top-4: 4800 rows 141.2 and 147.1;
+//   20000 315.2 and 309.3; 48000 650.8 and 631.8; H 4096 (16), top-8: 8000 rows 303.5 and 303.1; 16000 498.9 and 485.9
+//   e4m3, the first layer: 32000 rows 341.0 and 342.5; 67584 558.3 and 543.7; 135168 1040.5 and 996.8
+// Four tiles a workgroup lose again (67584 rows 795 us), and so do pairs of the gate-up pass, whose start is a smaller part
+// of a tile and whose products run at the clock that the board's power leaves, bubbles or not (67584 rows 825 against 804).
+static void set_chain(GemmParams& p, int es) {
+  const int64_t line = es == 1 ? 400000 : 240000;
+  p.chain = p.xcd_bounds && !p.bias && p.N % kBigBNW == 0 && p.ldc % 8 == 0 && p.num_n_tiles > 1 &&
+            static_cast<int64_t>(p.Kd) * es >= 2 * kBigRowBytes && static_cast<int64_t>(p.numel) * p.num_n_tiles >= line;
+}
+
 template <typename Mma, bool GATED>
 int launch_big(GemmParams& p, int64_t sorted_cap, hipStream_t s) {
   constexpr int lds = kBigLdsTotal;
@@ -1767,8 +1936,9 @@ int launch_big(GemmParams& p, int64_t sorted_cap, hipStream_t s) {
   p.num_n_tiles = (p.N + (GATED ? 128 : 256) - 1) / (GATED ? 128 : 256);
   const int64_t tiles = static_cast<int64_t>(p.num_m_blocks) * p.num_n_tiles;
   int64_t grid = (tiles + kXcds - 1) / kXcds * kXcds;
+  if (!GATED) set_chain(p, Mma::kEs);
   if (p.xcd_bounds)  // work-balanced ranges: as many slots per XCD as the longest range may have blocks
-    grid = static_cast<int64_t>(big_plan_cap(sorted_cap)) * p.num_n_tiles * kXcds;
+    grid = static_cast<int64_t>(listed_blocks(p, big_plan_cap(sorted_cap))) * p.num_n_tiles * kXcds;
   if (grid > INT32_MAX) return moe_fail(MOE_ERR_ARG, "fused_experts: grid of %lld workgroups", static_cast<long long>(grid));
   hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(grid)), dim3(kThreads), lds, s, p);
   return moe_check_launch(GATED ? "fused_experts (gate-up pass)" : "fused_experts (down pass)");
@@ -1826,8 +1996,9 @@ int launch_big_fused(GemmParams& p1, GemmParams& p2, int block_size, int64_t sor
   p2.num_n_tiles = (p2.N + 255) / 256;
   // every gate-up tile inside the matrix: its flush takes the 16-byte path, which can write through
   p1.wt_stores = (p1.N % 128 == 0 && p1.ldc % 8 == 0) ? 1 : 0;
+  set_chain(p2, Mma::kEs);
   const int cap_mb = big_plan_cap(sorted_cap);
-  const int64_t grid = static_cast<int64_t>(cap_mb) * (p1.num_n_tiles + p2.num_n_tiles) * kXcds;
+  const int64_t grid = (static_cast<int64_t>(cap_mb) * p1.num_n_tiles + static_cast<int64_t>(listed_blocks(p2, cap_mb)) * p2.num_n_tiles) * kXcds;
   if (grid > INT32_MAX) return moe_fail(MOE_ERR_ARG, "fused_experts: grid of %lld workgroups", static_cast<long long>(grid));
   hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(grid)), dim3(kThreads), lds, s, p1, p2, done, cap_mb,
                      g_wait_limit.load(std::memory_order_relaxed), status, down_xcd_shift);
