@@ -69,6 +69,13 @@ static inline int64_t moe_align_up(int64_t v, int64_t a) { return (v + a - 1) / 
 
 constexpr int kWave = 64;
 
+// 16 bytes that nothing reads again: not kept in the caches on the way.  A large buffer that a kernel has just written lies
+// partly unwritten-back in the 256 MB memory-side cache, and every line taken in on the way to it has one of those evicted.
+__device__ __forceinline__ uint4 load_once(const void* p) {
+  typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
+  return __builtin_bit_cast(uint4, __builtin_nontemporal_load(static_cast<const u32x4*>(p)));
+}
+
 // ---------------------------------------------------------------------------
 // Lane exchanges of a row of TPR lanes (a power of two, up to the wavefront), by DPP moves and the swaps of 16 and 32 lanes: a few clocks each, where the LDS-crossbar
 // shuffle behind __shfl_xor costs ~100 and was most of a round.

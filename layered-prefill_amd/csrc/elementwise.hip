@@ -14,6 +14,12 @@ struct alignas(sizeof(S) * N) Vec {
   S v[N];
 };
 
+template <typename S, int N>
+__device__ __forceinline__ Vec<S, N> load_terms(const S* p) {
+  if constexpr (sizeof(Vec<S, N>) == 16) return __builtin_bit_cast(Vec<S, N>, load_once(p));
+  else return *reinterpret_cast<const Vec<S, N>*>(p);
+}
+
 // out[r, i] = T(silu(in[r, i])) * in[r, d + i]; the product is taken in T.
 template <typename El, int VEC>
 __global__ __launch_bounds__(kThreads) void silu_and_mul_kernel(typename El::S* __restrict__ out,
@@ -60,7 +66,9 @@ __global__ __launch_bounds__(kThreads) void swigluoai_and_mul_kernel(
 }
 
 // out[t, h] = sum_k in[t, k, h], ascending k, fp32 accumulation.  KK: K, where it is known here and all of a
-// result's terms are asked for at once; else 0.
+// result's terms are asked for at once; else 0.  Bound by memory.  The terms are read once, and past the caches
+// (load_once): 277 MB of them that the down pass has just written 52.0 -> 47.9 us, 554 MB 118.5 -> 93.1 (6.7 TB/s with
+// the result).
 template <typename El, int VEC, int KK>
 __global__ __launch_bounds__(kThreads) void moe_sum_kernel(typename El::S* __restrict__ out,
                                                            const typename El::S* __restrict__ in,
@@ -79,15 +87,14 @@ __global__ __launch_bounds__(kThreads) void moe_sum_kernel(typename El::S* __res
       const S* src = in + t * KK * static_cast<int64_t>(H) + c;
       Vec<S, VEC> x[KK];
 #pragma unroll
-      for (int k = 0; k < KK; ++k) x[k] = *reinterpret_cast<const Vec<S, VEC>*>(src + k * static_cast<int64_t>(H));
+      for (int k = 0; k < KK; ++k) x[k] = load_terms<S, VEC>(src + k * static_cast<int64_t>(H));
 #pragma unroll
       for (int k = 0; k < KK; ++k)
 #pragma unroll
         for (int i = 0; i < VEC; ++i) acc[i] += El::ld(x[k].v[i]);
     } else {
       for (int k = 0; k < K; ++k) {
-        const Vec<S, VEC> x =
-            *reinterpret_cast<const Vec<S, VEC>*>(in + (t * K + k) * static_cast<int64_t>(H) + c);
+        const Vec<S, VEC> x = load_terms<S, VEC>(in + (t * K + k) * static_cast<int64_t>(H) + c);
 #pragma unroll
         for (int i = 0; i < VEC; ++i) acc[i] += El::ld(x.v[i]);
       }
@@ -208,15 +215,15 @@ int launch_sum(void* out, const void* in, int64_t T, int K, int H, hipStream_t s
   using S = typename El::S;
   constexpr int V = 16 / sizeof(S);
   if (H % V == 0 && aligned16(out) && aligned16(in)) {
-    // All terms at once pays while they come out of the caches (the expert pass has just written them): 8 terms of 2048
-    // elements, bf16, us, this way and term by term: 1 row 2.3 and 3.0, 64 rows 2.5 and 3.4, 741 rows 3.5 and 3.8, 8448
-    // rows (277 MB) 47.4 and 49.4, but 10000 rows 69.5 and 68.9, 16896 rows 124.8 and 118.7.  4 and 8 terms have an
+    // All terms at once: 8 terms of 2048 elements, bf16, us, this way and term by term: 1 row 2.3 and 3.0, 64 rows 2.5
+    // and 3.4, 741 rows 3.5 and 3.8, 8448 rows (277 MB) 47.9 and 48.7, 16896 rows 93.1 and 94.8.  4 and 8 terms have an
     // instance.  2 would gain next to nothing by one (64 rows 2.13 and 2.24, 8448 rows 16.5 and 16.4); 6 would gain half a
     // microsecond where rows are few (64 rows 2.23 and 2.80, 741 rows 3.01 and 3.36, 8448 rows 36.2 and 36.0).
-    const bool cached = T * K * static_cast<int64_t>(H) * static_cast<int64_t>(sizeof(S)) <= (int64_t{288} << 20);
-    auto kern = cached && K == 8 ? moe_sum_kernel<El, V, 8> : cached && K == 4 ? moe_sum_kernel<El, V, 4> : moe_sum_kernel<El, V, 0>;
-    hipLaunchKernelGGL(kern, dim3(grid_for(T * (H / V))), dim3(kThreads), 0, s, static_cast<S*>(out), static_cast<const S*>(in), T,
-                       K, H);
+    // A workgroup for every 256 vectors (16896 rows 93.1 us; 4096 workgroups that stride on 97.6).
+    auto kern = K == 8 ? moe_sum_kernel<El, V, 8> : K == 4 ? moe_sum_kernel<El, V, 4> : moe_sum_kernel<El, V, 0>;
+    const int64_t want = (T * (H / V) + kThreads - 1) / kThreads;
+    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(want < (1 << 22) ? want : 1 << 22)), dim3(kThreads), 0, s,
+                       static_cast<S*>(out), static_cast<const S*>(in), T, K, H);
   } else {
     hipLaunchKernelGGL((moe_sum_kernel<El, 1, 0>), dim3(grid_for(T * H)), dim3(kThreads), 0, s,
                        static_cast<S*>(out), static_cast<const S*>(in), T, K, H);
