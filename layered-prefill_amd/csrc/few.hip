@@ -170,8 +170,8 @@ __global__ __launch_bounds__(kFewThreads, 1) void few_gate_kernel(const void* __
   auto ask = [&] {
 #pragma unroll
     for (int q = 0; q < UN; ++q) {
-      lds_dma16(w_at, w_off[0], ring + at_ask + q * kFewGateStep);
-      lds_dma16(w_at, w_off[1], ring + at_ask + q * kFewGateStep + 1024);
+      lds_dma16<true>(w_at, w_off[0], ring + at_ask + q * kFewGateStep);
+      lds_dma16<true>(w_at, w_off[1], ring + at_ask + q * kFewGateStep + 1024);
       w_at += w_step;
     }
     at_ask = at_ask + UN * kFewGateStep == kRing * UN * kFewGateStep ? 0 : at_ask + UN * kFewGateStep;
@@ -341,7 +341,7 @@ __global__ __launch_bounds__(NW * kWave, NW == 4 ? 2 : 1) void few_down_kernel(c
     for (int s = 0; s < UN; ++s) {
 #pragma unroll
       for (int h = 0; h < HALVES; ++h) {
-        lds_dma16(w_at[h], w_lane[h], ring + at_ask + s * kFewDownStep + h * 1024);
+        lds_dma16<true>(w_at[h], w_lane[h], ring + at_ask + s * kFewDownStep + h * 1024);
         w_at[h] += w_step;
       }
 #pragma unroll

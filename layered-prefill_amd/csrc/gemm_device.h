@@ -54,15 +54,28 @@ __device__ __forceinline__ uint32_t lds_offset_of(const char* p) {
 
 // 16 bytes per lane from global memory straight into LDS at
 // lds_wave_base + 16 * lane.  `base` and `lds_wave_base` are wavefront-uniform.
+// ONCE: nobody reads these bytes again soon, so they are not kept in the caches (the non-temporal hint).  Weights that one
+// workgroup reads arrive up to a tenth faster that way, which is most of a decode call (whole calls: stream_gemm_kernel).
+template <bool ONCE = false>
 __device__ __forceinline__ void lds_dma16(const char* base, uint32_t lane_byte_offset,
                                           uint32_t lds_wave_base) {
-  asm volatile(
-      "s_mov_b32 m0, %0\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %1, %2"
-      :
-      : "s"(lds_wave_base), "v"(lane_byte_offset), "s"(base)
-      : "memory");
+  if constexpr (ONCE) {
+    asm volatile(
+        "s_mov_b32 m0, %0\n\t"
+        "s_nop 0\n\t"
+        "global_load_lds_dwordx4 %1, %2 nt"
+        :
+        : "s"(lds_wave_base), "v"(lane_byte_offset), "s"(base)
+        : "memory");
+  } else {
+    asm volatile(
+        "s_mov_b32 m0, %0\n\t"
+        "s_nop 0\n\t"
+        "global_load_lds_dwordx4 %1, %2"
+        :
+        : "s"(lds_wave_base), "v"(lane_byte_offset), "s"(base)
+        : "memory");
+  }
 }
 
 template <int N>

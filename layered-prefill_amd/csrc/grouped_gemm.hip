@@ -1632,6 +1632,11 @@ __device__ __forceinline__ void stream_store(const GemmParams& p, const float (&
 // through the scalar cache meanwhile, as everything before them does, and what hangs on them follows the weights.  No
 // branch and no division in it.  (Slot ids and the expert once more in front of the weights, a run of branches and two
 // divisions: 64 tokens of the layer above 104.4 us, 103.1 this way, e4m3 100 tokens 73.9 and 71.8.)
+// Weights of an expert with one block are read by one workgroup and asked for as such (lds_dma16<true>); those that blocks
+// share through L2 are not: all of them that way, 301 tokens of 32 experts lose 5 %.  Whole layer with the norm, three sets
+// of weights in rotation, without the hint, on all weights and as it is, us: 2 tokens (few.hip) 37.5 and 33.7; 9 62.5 and
+// 58; 16 77 / 70 / 70; 32 100 / 92 / 93; 64 113 / 106 / 101; 128 141 / 140 / 131; 192 161 / 163 / 153; 240 (tiled) 175 /
+// 184 / 172; 32 experts, 301 tokens 116 / 122 / 116; e4m3, 100 tokens 80 / 77 / 75, 250 109 / 113 / 107.
 // e4m3 runs here too (100 tokens of that layer: gate-up 45.6 -> 40.1 us, down 40.9 -> 25.9 us
 // against the register-staged kernel, whose two stages hold 36 KB per workgroup and drain at every K tile), its scales
 // fetched ahead of the stream like the routed weights.  Rows need whole 32-byte steps, not whole units.
@@ -1683,6 +1688,7 @@ __global__ __launch_bounds__(kThreads, 3) void stream_gemm_kernel(
   const int lo = me - __builtin_clz(~(links << (31 - me) << 1)), hi = me + __builtin_ctz(~(links >> me));
   const int e = me == 0 ? eq[0] : me == 1 ? eq[1] : me == 2 ? eq[2] : eq[3];
   const int g = hi - lo + 1;
+  const bool alone = g == 1;  // nobody else here reads these weights (or hardly: a run may go on in the next four blocks)
   const int li = (me - lo) * num_n_tiles + nt;
   nt = g == 1 ? li : static_cast<int>(__umulhi(li, g == 2 ? 0x80000000u : g == 3 ? 0x55555556u : 0x40000000u));  // li / g
   mb = q0 + lo + (li - nt * g);
@@ -1763,7 +1769,11 @@ __global__ __launch_bounds__(kThreads, 3) void stream_gemm_kernel(
       if (a_live) lds_dma16(a_base + u * kStRowBytes, a, dma_a + ring);
     if constexpr ((PART & 2) != 0) {
 #pragma unroll
-      for (int j = 0; j < 2; ++j) lds_dma16(w_base + static_cast<int64_t>(u) * w_step, w[j], dma_w + ring + j * 1024);
+      for (int j = 0; j < 2; ++j) {
+        const char* const src = w_base + static_cast<int64_t>(u) * w_step;
+        if (alone) lds_dma16<true>(src, w[j], dma_w + ring + j * 1024);
+        else lds_dma16(src, w[j], dma_w + ring + j * 1024);
+      }
     }
   };
 
