@@ -480,10 +480,18 @@ __device__ __forceinline__ void static_for(F&& f) {
 // were sixteen (0.5 to 1 % of the launch at 8448 and at 256 tokens, results unchanged bit for bit).
 // M0 has to keep its value from one request of a window to the next; nothing else in the K loops
 // writes it (they are MFMAs, LDS reads, waits and these requests).
-template <int OFF, bool SET_M0>
+template <int OFF, bool SET_M0, bool ONCE = false>
 __device__ __forceinline__ void lds_dma16_rel(const char* base, uint32_t lane_byte_offset, uint32_t lds_m0) {
   static_assert(OFF >= -4096 && OFF <= 4095, "13-bit signed offset field");
-  if constexpr (SET_M0) {
+  if constexpr (SET_M0 && ONCE) {  // (ONCE: lds_dma16)
+    asm volatile(
+        "s_mov_b32 m0, %0\n\t"
+        "s_nop 0\n\t"
+        "global_load_lds_dwordx4 %1, %2 offset:%3 nt"
+        :
+        : "s"(lds_m0), "v"(lane_byte_offset), "s"(base), "n"(OFF)
+        : "memory");
+  } else if constexpr (SET_M0) {
     asm volatile(
         "s_mov_b32 m0, %0\n\t"
         "s_nop 0\n\t"
@@ -491,6 +499,8 @@ __device__ __forceinline__ void lds_dma16_rel(const char* base, uint32_t lane_by
         :
         : "s"(lds_m0), "v"(lane_byte_offset), "s"(base), "n"(OFF)
         : "memory");
+  } else if constexpr (ONCE) {
+    asm volatile("global_load_lds_dwordx4 %0, %1 offset:%2 nt" : : "v"(lane_byte_offset), "s"(base), "n"(OFF) : "memory");
   } else {
     asm volatile("global_load_lds_dwordx4 %0, %1 offset:%2" : : "v"(lane_byte_offset), "s"(base), "n"(OFF) : "memory");
   }
@@ -498,9 +508,9 @@ __device__ __forceinline__ void lds_dma16_rel(const char* base, uint32_t lane_by
 // Request J (0..7) of a wavefront's 8 KB window of a 32 KB unit; lds_mid = LDS address of the
 // window's middle.  Unit byte 8192 * wave + 1024 * J + 16 * lane, i.e. row 64 * wave + 8 * J +
 // lane / 8 of the unit, position lane % 8 of that row.
-template <int J, bool SET_M0>
+template <int J, bool SET_M0, bool ONCE = false>
 __device__ __forceinline__ void lds_dma16_win(const char* base, uint32_t lane_byte_offset, uint32_t lds_mid) {
-  lds_dma16_rel<(J - 4) * 1024, SET_M0>(base, lane_byte_offset, lds_mid);
+  lds_dma16_rel<(J - 4) * 1024, SET_M0, ONCE>(base, lane_byte_offset, lds_mid);
 }
 // What a per-lane offset of request J carries besides the data's offset from the operand's start:
 // the offset field's share taken out again, and 4096 that the base pointers are short of (so that
@@ -704,6 +714,11 @@ __device__ __forceinline__ void big_mainloop(const BigCtx& c, const char* smem, 
 // belong) and four 8 KB token units of 64 rows inside slot 4.  Three K tiles are
 // in flight while one is multiplied, twice what the general loop keeps in flight
 // for weights, and a token unit costs two requests per wavefront instead of eight.
+// The weights are read by this workgroup only (nearly: the block may be the last of several) and requested as such
+// (lds_dma16, ONCE).  Whole calls, without and with it, us: 256 tokens 171.1 and 161.9, fp16 741 241.4 and 229.7; layer
+// with the norm, 1500 tokens 311 and 304.5, e4m3 600 163.8 and 157.8; 32 experts, H 4096, I 1024, 500 tokens 239 and 232;
+// 8448 and 16896 tokens the same.  In the general loop's tiles of up to 192 rows it gains 1 to 2 % where an expert has one
+// block (256 tokens 178 and 174.5) and loses 4 % where blocks share the weights (32 experts, 400 tokens 168.5 and 175.5).
 template <typename Mma, int FMC>
 __device__ __forceinline__ void big_light_mainloop(const BigCtx& c, const char* smem, int nk,
                                                    f32x16 (&acc)[4][4]) {
@@ -720,7 +735,7 @@ __device__ __forceinline__ void big_light_mainloop(const BigCtx& c, const char* 
     const uint32_t mid = c.dma_lds + w_slot(k);
     static_for<0, 8>([&](auto it) {
       constexpr int i = decltype(it)::value;
-      lds_dma16_win<i, i == 0>(src, c.w_off[i], mid);
+      lds_dma16_win<i, i == 0, true>(src, c.w_off[i], mid);
     });
   };
   // a token unit is 64 rows: the wavefront's window is 2 KB, two requests around its middle
