@@ -10,11 +10,12 @@
 //   + (same-expert lanes below it in the current 64 ids)    -- ballot + popcount
 // which is the stable order and needs no global atomics.
 //
-// Small inputs run as ONE workgroup of 16 wavefronts (histogram, scans and
-// scatter in LDS; a decode batch in a kernel of its own, one id per thread); larger ones as two launches (count, then scan + scatter with
-// every workgroup deriving its own prefixes) with the per-segment histograms in
-// the caller's workspace; three launches (count / scan / scatter) when the
-// tables of the second launch would not fit in LDS.
+// A decode batch runs as one workgroup, one id per thread.  More int32 ids of up to 256 experts go to one workgroup for
+// every 1024 of them, each of which finds the counts it needs by itself: by counting all ids, or from per-segment
+// histograms in the caller's workspace that a first launch leaves there.  Other id types and more experts: one workgroup
+// (histogram, scans and scatter in LDS) for small inputs; two launches (count, then scan + scatter with every workgroup
+// deriving its own prefixes) for larger ones; three (count / scan / scatter) when the tables of the second launch would not
+// fit in LDS.
 #include "common.h"
 #include "quant_device.h"
 #include "routing_device.h"
@@ -445,57 +446,93 @@ __global__ __launch_bounds__(kScanThreads) void align_small_kernel(
                    plan_bounds, plan_done, plan_num_done, plan_cap_mb, lds);
 }
 
-// The same for up to N * 1024 int32 ids over up to 256 experts and any block size (a chunk of a prompt; with
-// blocks of 256 it also leaves the large-tile kernel's plan).  A wavefront holds its N * 64 consecutive ids in
-// registers and needs one pass over them: the lanes of an id read the wavefront's count so far, which is the
-// rank of the first of them, and the lowest one advances it.
-// 128 experts, blocks of 256 with the plan: 5928 ids 20.7 us in align_small_kernel, which passes over its ids twice
-// and loads them in each, 11.9 us here.  The rest of it is the issue of one CU's four SIMDs: with ranks in half the
-// instructions, N as small as the ids allow (2048 ids left half the wavefronts idle), sums across lanes without the LDS
-// crossbar, padding in 16-byte stores and the plan by one wavefront while the others write it, 11.9 -> 10.2 us; 2048 ids
-// 8.8 -> 7.1, 1204 ids of 32 experts, blocks of 32, 5.1 -> 4.4, 67584 ids (two kernels, same ranks and sums) 17.3 -> 16.1.
-template <int N>
-__global__ __launch_bounds__(kScanThreads) void align_mid_kernel(
+// The same for more int32 ids of up to 256 experts and any block size (a chunk of a prompt and more; with blocks of 256 it also
+// leaves the large-tile kernel's plan).  A workgroup places 1024 ids, a lane one of them.  What it needs of the others it
+// finds by itself, so that nothing is handed from one workgroup to another.  MOST > 0, up to MOST * 1024 ids: it counts them
+// all, one LDS addition an id, in whose upper half stand the ids in front of the workgroup's own.  MOST == 0: it adds up
+// the segments' counts that align_count_kernel has left.  One workgroup that ranked all of up to 8192 ids was bound by the
+// issue of its CU's four SIMDs, and of larger calls each wavefront placed 512 ids one step behind the other, on a few CUs.
+// 128 experts, top-8, blocks of 256 with the plan, us, before and now: 2048 ids 7.2 and 5.8, 5928 9.9 and 5.9, 8192 11.6 and
+// 6.5, 12000 22.7 and 7.7, 16384 26.7 and 8.6; with the counting kernel in front: 32776 15.6 and 9.0, 67584 16.0 and 9.6,
+// 135168 17.4 and 11.5, 262144 19.8 and 14.9.  Blocks of 32: 1204 ids of 32 experts 4.3 and 4.2, 1920 of 128 6.1 and 4.9.
+constexpr int kSpreadMost = 16;
+static_assert((kSpreadMost - 1) * kScanThreads < 1 << 15 && kSpreadMost * kScanThreads < 1 << 16, "two counts in a word");
+static_assert(kScanThreads % kSegLen == 0, "a workgroup takes whole segments");
+// With the counts from segments, every workgroup reads all of them: from 256 workgroups on that is what it takes
+// (524288 ids 25.1 us by align_place_kernel, 27.0 here).
+constexpr int64_t kSpreadTableMost = 256 * kScanThreads;
+template <int MOST>
+__global__ __launch_bounds__(kScanThreads) void align_spread_kernel(
     const int32_t* __restrict__ ids, int numel, int E, int BM, int id_bits, int32_t* __restrict__ sorted_ids,
     int sorted_cap, int32_t* __restrict__ expert_ids, int expert_cap, int32_t* __restrict__ num_post_pad,
-    int32_t* plan_bounds, int32_t* plan_done, int plan_num_done, int plan_cap_mb) {
+    int32_t* plan_bounds, int32_t* plan_done, int plan_num_done, int plan_cap_mb, const int32_t* __restrict__ seg_cnt,
+    int nseg) {
   __shared__ int s_cnt[kScanWaves * kTinyExperts];   // [wave][expert]: counts, then the first slot of the wave's ids
+  __shared__ int s_all[kTinyExperts];                // ids of an expert (MOST > 0: and in the upper half those of earlier workgroups)
+  __shared__ int s_before[kTinyExperts];             // MOST == 0: those of earlier workgroups
   __shared__ int s_cum[kTinyExperts + 1], s_tot[kTinyExperts], s_wave[kScanWaves + 1], s_plan[kPlanXcds + 1];
   static_assert(kTinyExperts <= kPlanWaveExperts, "one wavefront plans");
-  volatile int* cnt = s_cnt;
   const int tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
-  const int beg = wave * (N * kWave) + lane;
-  int id[N], rank[N];
+  const int wg = blockIdx.x, nwg = gridDim.x;
+  int id[MOST > 0 ? MOST : 1], own = -1;
+  if constexpr (MOST > 0) {
 #pragma unroll
-  for (int j = 0; j < N; ++j) id[j] = beg + j * kWave < numel ? ids[beg + j * kWave] : -1;
-  for (int i = tid; i < kScanWaves * E; i += kScanThreads) cnt[i] = 0;
-  __syncthreads();
-#pragma unroll
-  for (int j = 0; j < N; ++j) {
-    const bool valid = id[j] >= 0 && id[j] < E;
-    const uint64_t grp = same_id_lanes(id[j], valid, id_bits);
-    if (!valid) {
+    for (int j = 0; j < MOST; ++j) {
+      const int i = j * kScanThreads + tid;
       id[j] = -1;
-      continue;
+      if (j * kScanThreads < numel && i < numel) id[j] = ids[i];
     }
-    const int below = __popcll(grp & lanes_below(lane));
-    const int before = cnt[wave * E + id[j]];
-    rank[j] = before + below;
-    if (below == 0) cnt[wave * E + id[j]] = before + __popcll(grp);
+  } else {
+    const int i = wg * kScanThreads + tid;
+    if (i < numel) own = ids[i];
   }
+  for (int i = tid; i < kScanWaves * E; i += kScanThreads) s_cnt[i] = 0;
+  if (tid < E) s_all[tid] = s_before[tid] = 0;
   __syncthreads();
-  int c[kScanWaves], total = 0, padded = 0;
+  if constexpr (MOST > 0) {
+#pragma unroll
+    for (int j = 0; j < MOST; ++j) {
+      if (j * kScanThreads >= numel) break;
+      if (j == wg) own = id[j];
+      if (id[j] >= 0 && id[j] < E) atomicAdd(&s_all[id[j]], j < wg ? 1 + (1 << 16) : 1);
+    }
+  } else {
+    // thread t sums expert t % E over the segments t / E, t / E + R, .. (a wavefront reads one segment's counts side by side)
+    const int R = kScanThreads / E, e = tid % E, r = tid / E;
+    constexpr int CH = 16;
+    int sum = 0, early = 0;
+    for (int s0 = r < R ? r : nseg; s0 < nseg; s0 += CH * R) {
+      int c[CH];
+#pragma unroll
+      for (int i = 0; i < CH; ++i) c[i] = s0 + i * R < nseg ? seg_cnt[static_cast<size_t>(s0 + i * R) * E + e] : 0;
+#pragma unroll
+      for (int i = 0; i < CH; ++i) {
+        sum += c[i];
+        early += s0 + i * R < wg * (kScanThreads / kSegLen) ? c[i] : 0;
+      }
+    }
+    if (r < R) {
+      atomicAdd(&s_all[e], sum);
+      atomicAdd(&s_before[e], early);
+    }
+  }
+  const bool valid = own >= 0 && own < E;
+  const uint64_t grp = same_id_lanes(own, valid, id_bits);
+  const int below = __popcll(grp & lanes_below(lane));
+  if (valid && below == 0) s_cnt[wave * E + own] = __popcll(grp);
+  __syncthreads();
+  int c[kScanWaves], total = 0, before = 0, padded = 0;
   if (tid < E) {
 #pragma unroll
     for (int w = 0; w < kScanWaves; ++w) c[w] = s_cnt[w * E + tid];
-#pragma unroll
-    for (int w = 0; w < kScanWaves; ++w) total += c[w];
+    total = MOST > 0 ? s_all[tid] & 0xffff : s_all[tid];
+    before = MOST > 0 ? s_all[tid] >> 16 : s_before[tid];
     padded = (total + BM - 1) / BM * BM;
   }
   const int first = block_exclusive_scan(padded, s_wave);
   const int all = s_wave[kScanWaves];
   if (tid < E) {
-    int at = first;
+    int at = first + before;
 #pragma unroll
     for (int w = 0; w < kScanWaves; ++w) {
       s_cnt[w * E + tid] = at;
@@ -503,28 +540,27 @@ __global__ __launch_bounds__(kScanThreads) void align_mid_kernel(
     }
     s_cum[tid] = first;
     s_tot[tid] = total;
-    for (int b = first / BM; b < (first + padded) / BM; ++b) expert_ids[b] = tid;
+    if (tid % nwg == wg)
+      for (int b = first / BM; b < (first + padded) / BM; ++b) expert_ids[b] = tid;
   }
   if (tid == 0) {
     s_cum[E] = all;
-    *num_post_pad = all;
+    if (wg == 0) *num_post_pad = all;
   }
   __syncthreads();
-#pragma unroll
-  for (int j = 0; j < N; ++j)
-    if (id[j] >= 0) sorted_ids[s_cnt[wave * E + id[j]] + rank[j]] = beg + j * kWave;
-  if (plan_bounds && wave == 0) {
+  if (valid) sorted_ids[s_cnt[wave * E + own] + below] = wg * kScanThreads + tid;
+  // the last wavefront plans; the others take turns with the padding: of the experts' last blocks, then behind all of them
+  const int turn = wg * kScanWaves + wave, turns = nwg * kScanWaves - (plan_bounds ? 1 : 0);
+  if (turn == turns) {
     plan_by_wave(s_cum, s_tot, E, plan_cap_mb, plan_bounds, plan_done, plan_num_done, s_plan);
     return;
   }
-  // padding, the wavefronts left taking turns: of the experts' last blocks, then behind all of them
-  const int w0 = plan_bounds ? 1 : 0;
-  for (int e = wave - w0; e < E; e += kScanWaves - w0)
+  for (int e = turn; e < E; e += turns)
     fill_slots(sorted_ids, __builtin_amdgcn_readfirstlane(s_cum[e] + s_tot[e]), __builtin_amdgcn_readfirstlane(s_cum[e + 1]), numel);
   constexpr int kTail = 4 * kWave;
-  for (int p = __builtin_amdgcn_readfirstlane(all) + (wave - w0) * kTail; p < sorted_cap; p += (kScanWaves - w0) * kTail)
+  for (int p = __builtin_amdgcn_readfirstlane(all) + turn * kTail; p < sorted_cap; p += turns * kTail)
     fill_slots(sorted_ids, p, min(p + kTail, sorted_cap), numel);
-  for (int b = all / BM + tid - w0 * kWave; b < expert_cap; b += kScanThreads - w0 * kWave) expert_ids[b] = 0;
+  for (int b = all / BM + turn * kWave + lane; b < expert_cap; b += turns * kWave) expert_ids[b] = 0;
 }
 
 // Routing and alignment of a very small batch in one launch (such a call is a handful of short
@@ -825,15 +861,15 @@ static int align_impl(const void* topk_ids, int ids_dtype, int64_t numel, int E,
                        expert_ids, static_cast<int>(expert_cap), num_tokens_post_pad);
     return moe_check_launch("moe_align_block_size (single workgroup, up to 1024 ids)");
   }
-  if (numel <= 8 * kScanThreads && E <= kTinyExperts && ids_dtype == MOE_ID_I32 && sorted_cap <= INT32_MAX &&
+  if (numel <= kSpreadMost * kScanThreads && E <= kTinyExperts && ids_dtype == MOE_ID_I32 && sorted_cap <= INT32_MAX &&
       expert_cap <= INT32_MAX) {
-    auto kern = numel <= 2 * kScanThreads ? align_mid_kernel<2> : numel <= 4 * kScanThreads ? align_mid_kernel<4>
-              : numel <= 6 * kScanThreads ? align_mid_kernel<6> : align_mid_kernel<8>;
-    hipLaunchKernelGGL(kern, dim3(1), dim3(kScanThreads), 0, s, static_cast<const int32_t*>(topk_ids),
+    const int wgs = numel > kScanThreads ? static_cast<int>((numel + kScanThreads - 1) / kScanThreads) : 1;
+    auto kern = wgs <= 8 ? align_spread_kernel<8> : align_spread_kernel<kSpreadMost>;
+    hipLaunchKernelGGL(kern, dim3(wgs), dim3(kScanThreads), 0, s, static_cast<const int32_t*>(topk_ids),
                        static_cast<int>(numel), E, block_size, id_bits, sorted_token_ids, static_cast<int>(sorted_cap),
                        expert_ids, static_cast<int>(expert_cap), num_tokens_post_pad, plan_bounds, plan_done, plan_num_done,
-                       plan_cap_mb);
-    return moe_check_launch("moe_align_block_size (single workgroup, up to 8192 ids)");
+                       plan_cap_mb, static_cast<const int32_t*>(nullptr), 0);
+    return moe_check_launch("moe_align_block_size (one launch)");
   }
   if (numel <= kSmallNumel && E <= kSmallMaxExperts) {
     const size_t lds = (static_cast<size_t>(kScanWaves) * E + (E + 1) + E + kScanWaves + 1) * sizeof(int);
@@ -852,6 +888,15 @@ static int align_impl(const void* topk_ids, int ids_dtype, int64_t numel, int E,
   int32_t* cum = seg_cnt + static_cast<size_t>(nseg) * E;
   hipLaunchKernelGGL(align_count_kernel, dim3(nseg), dim3(kWave), E * sizeof(int), s, topk_ids,
                      ids_dtype, numel, E, seg_cnt);
+  if (numel <= kSpreadTableMost && E <= kTinyExperts && ids_dtype == MOE_ID_I32 && sorted_cap <= INT32_MAX &&
+      expert_cap <= INT32_MAX) {
+    hipLaunchKernelGGL(align_spread_kernel<0>, dim3(static_cast<unsigned>((numel + kScanThreads - 1) / kScanThreads)),
+                       dim3(kScanThreads), 0, s, static_cast<const int32_t*>(topk_ids), static_cast<int>(numel), E, block_size,
+                       id_bits, sorted_token_ids, static_cast<int>(sorted_cap), expert_ids, static_cast<int>(expert_cap),
+                       num_tokens_post_pad, plan_bounds, plan_done, plan_num_done, plan_cap_mb,
+                       static_cast<const int32_t*>(seg_cnt), nseg);
+    return moe_check_launch("moe_align_block_size (count + spread)");
+  }
   // scan and scatter as one launch while its LDS tables fit
   const int nwg = (nseg + kScanWaves - 1) / kScanWaves;
   const size_t place_lds = (static_cast<size_t>(nwg + kScanWaves) * E + (E + 1) + E + kScanWaves + 1) * sizeof(int);
