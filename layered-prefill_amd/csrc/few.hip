@@ -15,15 +15,18 @@ namespace {
 constexpr int kFewTokens = 16;     // columns of a 16x16 product
 constexpr int kFewFlats = 128;     // most (token, k)
 constexpr int kFewCus = 256;
-constexpr int kFewWaves = 8, kFewThreads = kFewWaves * kWave;   // of a gate-up workgroup
 constexpr int kFewRow = 128;       // bytes of a row that a step takes: 64 elements
 // Steps that a wavefront has in flight; a unit has more of them, so that its requests are at most one unit ahead.  Eight
 // wavefronts of four steps: 1, 2 and 9 tokens of the layer below 21.0, 27.0 and 48.3 us; four of eight: 20.8, 28.7 and 50.6.
+// A gate-up workgroup has twelve of them where its rings leave room for the hidden states, else eight: a CU's 8 to 12 units
+// then go side by side instead of in two rounds.  Layer with the norm, three sets of weights, eight and twelve, us: 4
+// tokens 40.1 and 40.3, 8 52.6 and 51.7, 9 57 and 56, 10 56.5 and 55.9; 32 experts, H 2048, I 1024, 12 tokens 74.0 and 72.9;
+// H 4096, 4 tokens 101.8 and 98.1.
 constexpr int kFewGateRing = 4, kFewDownRing = 4;
 constexpr int kFewGateStep = 16 * kFewRow;                // 16 weight rows
 constexpr int kFewDownStep = 2 * 16 * kFewRow;            // 16 weight rows and 16 token rows
-constexpr int kFewGateRingBytes = kFewWaves * kFewGateRing * kFewGateStep;
 constexpr int kFewXBytes = 64 * 1024;                     // most bytes of hidden states
+constexpr int kFewXMost12 = 56 * 1024;                    // the same beside the rings of twelve wavefronts
 constexpr int kFewLeastLds = 84 * 1024;                   // of which no two fit a CU
 
 struct FewParams {
@@ -73,11 +76,12 @@ __device__ __forceinline__ int nth_set(const uint64_t (&m)[W], int rank) {
 // elements an iteration (one where H is an odd number of them): two keep the chain of a wait, LDS reads, requests and
 // dependent products short (H 1536, I 512, top-2: 12.9 -> 11.1 us at 1 token).  The products, their order and every
 // rounding are the streaming kernel's.
-template <int E, typename Mma, int UN>
-__global__ __launch_bounds__(kFewThreads, 1) void few_gate_kernel(const void* __restrict__ logits, int logits_dtype, int renormalize,
+template <int E, typename Mma, int UN, int NW>
+__global__ __launch_bounds__(NW * kWave, 1) void few_gate_kernel(const void* __restrict__ logits, int logits_dtype, int renormalize,
                                                                const FewParams p) {
   using El = typename Mma::El;
   using G = Pow2Geom<E>;
+  constexpr int RING = NW * kFewGateRing * kFewGateStep;
   constexpr int TPR = G::kTpr, RPW = G::kRowsPerWave, W = (E + 63) / 64;
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   __shared__ int s_ids[kFewFlats], s_flag[E];
@@ -91,17 +95,17 @@ __global__ __launch_bounds__(kFewThreads, 1) void few_gate_kernel(const void* __
   {
     const int cells = T * nu;
     const uint32_t rcp = 65536u / T + 1;
-    for (int j = wave; j * 8 < cells; j += kFewWaves) {
+    for (int j = wave; j * 8 < cells; j += NW) {
       int i = j * 8 + (lane >> 3);
       i = i < cells ? i : cells - 1;
       const int s = static_cast<int>((static_cast<uint32_t>(i) * rcp) >> 16), t = i - s * T;
       const uint32_t off = static_cast<uint32_t>(t) * (p.H * 2) + s * kFewRow + (((lane & 7) ^ ((t >> 1) & 7)) << 4);
-      lds_dma16(static_cast<const char*>(p.x), off, __builtin_amdgcn_readfirstlane(lds0 + kFewGateRingBytes + j * 1024));
+      lds_dma16(static_cast<const char*>(p.x), off, __builtin_amdgcn_readfirstlane(lds0 + RING + j * 1024));
     }
   }
-  for (int i = tid; i < kFewTokens * E / 4; i += kFewThreads) s_kmap[i] = ~0u;
-  for (int i = tid; i < E; i += kFewThreads) s_flag[i] = 0;
-  for (int r0 = wave * RPW; r0 < T; r0 += kFewWaves * RPW) {  // (whole wavefronts take part in a row's exchanges)
+  for (int i = tid; i < kFewTokens * E / 4; i += (NW * kWave)) s_kmap[i] = ~0u;
+  for (int i = tid; i < E; i += (NW * kWave)) s_flag[i] = 0;
+  for (int r0 = wave * RPW; r0 < T; r0 += NW * RPW) {  // (whole wavefronts take part in a row's exchanges)
     const int row = r0 + lane / TPR, from = row < T ? row : T - 1;
     float v[G::kVpt];
     if (logits_dtype == MOE_BF16) load_row<E, ElemBF16>(static_cast<const uint16_t*>(logits), from, lane % TPR, v);
@@ -134,9 +138,14 @@ __global__ __launch_bounds__(kFewThreads, 1) void few_gate_kernel(const void* __
 
   const int cols8 = p.I / 8;
   const uint32_t units = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(experts)) * cols8;
-  const int first = __builtin_amdgcn_readfirstlane(static_cast<int>(units * blockIdx.x / kFewCus) + wave);
+  const int begin_u = __builtin_amdgcn_readfirstlane(static_cast<int>(units * blockIdx.x / kFewCus));
   const int last = __builtin_amdgcn_readfirstlane(static_cast<int>(units * (blockIdx.x + 1) / kFewCus));  // (one behind)
-  if (first >= last) return;
+  // no more wavefronts than share the units in as many rounds
+  const int first = begin_u + wave;
+  const int rounds = (last - begin_u + NW - 1) / NW;
+  int stride = NW;
+  while (rounds > 1 && (stride - 1) * rounds >= last - begin_u) --stride;
+  if (wave >= stride || first >= last) return;
   // the side of a unit that asks for weights
   const char* w_at = nullptr;
   uint32_t w_off[2] = {0, 0};
@@ -177,7 +186,7 @@ __global__ __launch_bounds__(kFewThreads, 1) void few_gate_kernel(const void* __
     at_ask = at_ask + UN * kFewGateStep == kRing * UN * kFewGateStep ? 0 : at_ask + UN * kFewGateStep;
     if ((k_ask += UN) == nu) {
       k_ask = 0;
-      u_ask += kFewWaves;
+      u_ask += stride;
       if (u_ask < last) begin(u_ask);
     }
   };
@@ -189,10 +198,10 @@ __global__ __launch_bounds__(kFewThreads, 1) void few_gate_kernel(const void* __
 #pragma unroll
   for (int kk = 0; kk < 2; ++kk) {
     rd_w[kk] = l15 * kFewRow + (((4 * kk + lq) ^ ((l15 >> 1) & 7)) << 4);
-    rd_x[kk] = kFewGateRingBytes + t * kFewRow + (((4 * kk + lq) ^ ((t >> 1) & 7)) << 4);
+    rd_x[kk] = RING + t * kFewRow + (((4 * kk + lq) ^ ((t >> 1) & 7)) << 4);
   }
   int at = 0;
-  for (int u = first; u < last; u += kFewWaves) {
+  for (int u = first; u < last; u += stride) {
     // what the unit's end needs
     const int k_of = reinterpret_cast<const uint8_t*>(s_kmap)[t * E + e];
     const bool mine = l15 < T && k_of != 0xff;
@@ -436,14 +445,17 @@ __global__ __launch_bounds__(NW * kWave, NW == 4 ? 2 : 1) void few_down_kernel(c
 
 template <int E, typename Mma>
 int launch_few(const void* logits, int logits_dtype, int renormalize, const FewParams& p, hipStream_t s) {
-  static MoeLdsOptIn odd, even;
-  auto gate = p.H % 128 ? few_gate_kernel<E, Mma, 1> : few_gate_kernel<E, Mma, 2>;
-  MoeLdsOptIn& opted = p.H % 128 ? odd : even;
-  const int cells = p.T * (p.H / 64);
-  const int want = kFewGateRingBytes + (cells + 7) / 8 * 1024, lds = want > kFewLeastLds ? want : kFewLeastLds;
-  if (int rc = moe_opt_in_lds(opted, reinterpret_cast<const void*>(gate), kFewGateRingBytes + kFewXBytes, "layer")) return rc;
-  hipLaunchKernelGGL(gate, dim3(kFewCus), dim3(kFewThreads), lds, s, logits, logits_dtype, renormalize, p);
-  if (int rc = moe_check_launch("layer (routing and gate-up pass)")) return rc;
+  const int x_bytes = (p.T * (p.H / 64) + 7) / 8 * 1024;
+  auto gate = [&](auto un, auto nw) {
+    constexpr int NW = decltype(nw)::value, ring = NW * kFewGateRing * kFewGateStep;
+    static MoeLdsOptIn flags;
+    auto kernel = few_gate_kernel<E, Mma, decltype(un)::value, NW>;
+    const int lds = ring + x_bytes > kFewLeastLds ? ring + x_bytes : kFewLeastLds;
+    if (int rc = moe_opt_in_lds(flags, reinterpret_cast<const void*>(kernel), ring + (NW > 8 ? kFewXMost12 : kFewXBytes), "layer"))
+      return rc;
+    hipLaunchKernelGGL(kernel, dim3(kFewCus), dim3(NW * kWave), lds, s, logits, logits_dtype, renormalize, p);
+    return moe_check_launch("layer (routing and gate-up pass)");
+  };
   auto down = [&](auto un, auto nw) {
     constexpr int UN = decltype(un)::value, NW = decltype(nw)::value, bytes = NW * kFewDownRing * kFewDownStep;
     static MoeLdsOptIn flags;
@@ -456,6 +468,10 @@ int launch_few(const void* logits, int logits_dtype, int renormalize, const FewP
   using Two = std::integral_constant<int, 2>;
   using Four = std::integral_constant<int, 4>;
   using Eight = std::integral_constant<int, 8>;
+  using Twelve = std::integral_constant<int, 12>;
+  const bool wide = x_bytes <= kFewXMost12;
+  const int rc = p.H % 128 ? (wide ? gate(One{}, Twelve{}) : gate(One{}, Eight{})) : wide ? gate(Two{}, Twelve{}) : gate(Two{}, Eight{});
+  if (rc) return rc;
   const bool many = p.H / 8 > kFewCus;
   if (p.I % 128) return many ? down(One{}, Four{}) : down(One{}, Eight{});
   return many ? down(Two{}, Four{}) : down(Two{}, Eight{});

@@ -82,3 +82,17 @@ def test_few_tokens_replay_from_a_graph(moe, dev):
         graph.replay()
         assert torch.equal(out, moe.fused_topk_experts(x, logits, w13, w2, K, True)) and not torch.equal(out, want)
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("case", [
+    (7, 256, 8, 4096, 384, _BF, "plain", "silu", False, False, _BF),      # most hidden states beside twelve wavefronts' rings
+    (16, 32, 6, 512, 1024, _BF, "plain", "silu", False, False, _BF),      # more units to a CU than those have
+    (14, 32, 6, 576, 832, _FP, "plain", "swigluoai", True, False, _BF),   # 13 of them, an odd number of steps
+], ids=lambda c: "-".join(str(v).replace("torch.", "") for v in c))
+def test_units_of_a_cu_over_twelve_wavefronts(moe, dev, monkeypatch, case):
+    print(case, flush=True)
+    x, logits, w13, w2, K, kw = _args(moe, dev, *case)
+    one = moe.fused_topk_experts(x, logits, w13, w2, K, True, **kw)
+    monkeypatch.setattr(moe.fused_moe, "_layer_call", lambda *a: None)
+    steps = moe.fused_topk_experts(x, logits, w13, w2, K, True, **kw)
+    assert bool(steps.isfinite().all()) and float(steps.float().abs().max()) > 0 and torch.equal(one, steps)
