@@ -78,19 +78,6 @@ __device__ __forceinline__ uint64_t same_id_lanes(int id, bool valid, int id_bit
 
 __device__ __forceinline__ uint64_t lanes_below(int lane) { return (1ull << lane) - 1ull; }
 
-// Inclusive prefix sum over a wavefront, by lane exchanges inside the vector unit: shifts inside rows of 16 lanes, then the
-// last lane of a row to the row behind it and of the first half to the second (a shuffle through the LDS crossbar costs
-// about a hundred clocks, six of them more than a short kernel's whole scan).
-__device__ __forceinline__ int wave_inclusive_scan(int v) {
-  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);   // row_shr:1
-  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);   // row_shr:2
-  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);   // row_shr:4
-  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);   // row_shr:8
-  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
-  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
-  return v;
-}
-
 // Exclusive prefix sum of one int per thread over a kScanThreads workgroup.
 // `wave_tot` is LDS scratch of kScanWaves + 1 ints; slot kScanWaves receives
 // the grand total.  Contains workgroup barriers.

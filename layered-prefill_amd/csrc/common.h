@@ -55,7 +55,10 @@ bool moe_layer_route_quant(const void* logits, int dtype, float* topk_w, int32_t
 // Where a moe_fused_experts call of e4m3 weights keeps the codes and scales of x in its workspace, and that call with them
 // there already.
 void moe_experts_x_codes(const MoeFusedExpertsArgs* a, uint8_t** codes, float** scales);
-int moe_fused_experts_of_codes(const MoeFusedExpertsArgs* a, bool x_coded);
+// `ids`: the call's [T, K] ids, whose alignment (sorted_token_ids, expert_ids and num_tokens_post_pad, all of them) the gate-up
+// pass makes and leaves; only where moe_experts_align says so.  Null: they are aligned already.
+int moe_fused_experts_of_codes(const MoeFusedExpertsArgs* a, bool x_coded, const int32_t* ids);
+bool moe_experts_align(const MoeFusedExpertsArgs* a);
 
 // A layer call of a few tokens in two launches, where it is one that they serve (few.hip); false, and nothing enqueued,
 // elsewhere.  `experts` holds E + 1 ids, `inter` T * K rows.  `rc` is the launches' status.
@@ -68,6 +71,19 @@ constexpr int kMoeStatusWord = 16;
 static inline int64_t moe_align_up(int64_t v, int64_t a) { return (v + a - 1) / a * a; }
 
 constexpr int kWave = 64;
+
+// Inclusive prefix sum over a wavefront, by lane exchanges inside the vector unit: shifts inside rows of 16 lanes, then the
+// last lane of a row to the row behind it and of the first half to the second (a shuffle through the LDS crossbar costs
+// about a hundred clocks, six of them more than a short kernel's whole scan).
+__device__ __forceinline__ int wave_inclusive_scan(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);   // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);   // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);   // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);   // row_shr:8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
+  return v;
+}
 
 // 16 bytes that nothing reads again: not kept in the caches on the way.  A large buffer that a kernel has just written lies
 // partly unwritten-back in the 256 MB memory-side cache, and every line taken in on the way to it has one of those evicted.

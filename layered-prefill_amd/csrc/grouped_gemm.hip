@@ -112,6 +112,8 @@ struct GemmParams {
   int interleaved;   // gate/up rows interleaved (2n, 2n+1) instead of halves (n, N+n)
   float alpha, limit;
   int64_t sorted_cap; // capacity of sorted_ids
+  const int32_t* ids; // gate-up pass of the streaming kernel: ids that it aligns itself (stream_gemm_kernel, ALIGN), or null
+  int num_experts;
   int align_bs;      // block size the alignment was made with (a multiple of the kernel's M tile)
   int m_major;       // workgroup order inside an XCD: all n-tiles of an m-block are neighbours
   const int32_t* xcd_bounds;  // large-tile kernel: m-block range [b[x], b[x+1]) of XCD x, or null
@@ -1667,10 +1669,17 @@ constexpr int kStDmaPerUnit = 3;                               // requests per w
 // into registers that are filled with the workgroup's start (the build's -amdgpu-kernarg-preload-count), everything in a
 // structure is fetched from memory, and a workgroup's first fetch depends on it.  Both passes and the combine, without
 // preloading and with it, us: 1 token 20.8 and 20.2, 64 tokens 101.1 and 99.8, 128 130.7 and 129.2, e4m3 100 70.4 and 68.3.
-template <typename Mma, bool GATED, bool TAIL, bool ONCE = false>
+// ALIGN (gate-up pass, up to kStAlignMost ids of up to 256 experts): `head` are the call's ids, and every workgroup finds its
+// block's expert and slots among them by itself, while the kernel in front of it would take a launch of its own to sort
+// them; the workgroups of n-tile 0 leave the sorted slots for the down pass.  Else `head` is the padded count of slots.
+// It costs a workgroup no more than the two round trips for the count of blocks and their experts.  Layer with the norm,
+// aligned in front and here, us: 20 tokens 78.3 and 74.7, 64 100.3 and 96.7, 128 tiled 126.5 and 123.4, e4m3 100 74.3 and
+// 72.2; 64 experts, H 1024, I 512, top-4, fp16, 100 tokens 34.9 and 31.8.
+constexpr int kStAlignMost = 4 * kThreads;
+template <typename Mma, bool GATED, bool TAIL, bool ONCE = false, bool ALIGN = false>
 __global__ __launch_bounds__(kThreads, 3) void stream_gemm_kernel(
-    const int32_t* __restrict__ num_post_pad, const int32_t* __restrict__ expert_ids,
-    const int32_t* __restrict__ sorted_ids, int num_n_tiles, uint32_t n_tiles_rcp, const GemmParams p) {
+    const int32_t* __restrict__ head, int32_t* __restrict__ expert_ids,
+    int32_t* __restrict__ sorted_ids, int num_n_tiles, uint32_t n_tiles_rcp, int numel, int num_experts, const GemmParams p) {
   using El = typename Mma::El;
   constexpr int ES = Mma::kEs;
   __shared__ __attribute__((aligned(1024))) char smem[kStUnits * kStUnitBytes];
@@ -1679,7 +1688,39 @@ __global__ __launch_bounds__(kThreads, 3) void stream_gemm_kernel(
   // blocks only: the n-tiles of a block run side by side and share its token
   // rows through one L2 (in the down pass those rows are 1.5 KB x 32 per block
   // and were re-fetched for every n-tile otherwise).
-  const int live_mb = (*num_post_pad + kStBM - 1) / kStBM;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l15 = lane & 15, lq = lane >> 4;
+  __shared__ __attribute__((aligned(16))) int s_cnt[ALIGN ? 256 : 4], s_slots[kStBM], s_part[kThreads / kWave];
+  [[maybe_unused]] int id[4], nb[4], blocks_in;   // ALIGN: ids 4 tid .., blocks of experts 4 lane .., and up to their end
+  int live_mb;
+  if constexpr (ALIGN) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) id[i] = 4 * tid + i < numel ? head[4 * tid + i] : -1;
+    s_cnt[tid] = 0;
+    if (tid < kStBM) s_slots[tid] = numel;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (id[i] >= 0 && id[i] < num_experts) atomicAdd(&s_cnt[id[i]], 1);
+    __syncthreads();
+    const int4 n = *reinterpret_cast<const int4*>(s_cnt + 4 * lane);
+    nb[0] = (n.x + kStBM - 1) / kStBM;
+    nb[1] = (n.y + kStBM - 1) / kStBM;
+    nb[2] = (n.z + kStBM - 1) / kStBM;
+    nb[3] = (n.w + kStBM - 1) / kStBM;
+    blocks_in = wave_inclusive_scan((nb[0] + nb[1]) + (nb[2] + nb[3]));
+    live_mb = __builtin_amdgcn_readlane(blocks_in, kWave - 1);
+    // the slots behind the last block, a block of them each, and the padded count
+    const int behind = live_mb + static_cast<int>(blockIdx.x);
+    if (behind < p.num_m_blocks) {
+      if (tid < kStBM && static_cast<int64_t>(behind) * kStBM + tid < p.sorted_cap) sorted_ids[behind * kStBM + tid] = numel;
+      if (tid == 0) expert_ids[behind] = 0;
+    }
+    if (blockIdx.x == 0 && tid == 0) *const_cast<int32_t*>(p.num_post_pad) = live_mb * kStBM;
+  } else {
+    live_mb = (*head + kStBM - 1) / kStBM;
+  }
   const int live = live_mb * num_n_tiles;
   const int per_xcd = (live + kXcds - 1) / kXcds;
   const int xslot = blockIdx.x / kXcds;
@@ -1693,33 +1734,56 @@ __global__ __launch_bounds__(kThreads, 3) void stream_gemm_kernel(
   // blocks from (block, n-tile) to (n-tile, block): the g workgroups that
   // read one weight tile then start back to back on one XCD and the second
   // to g-th find the lines in L2 (or already requested).
-  const int q0 = mb & ~3, me = mb & 3;
-  int eq[4];
+  int e, g;
+  [[maybe_unused]] int in_expert = 0;  // ALIGN: the block's number among its expert's
+  if constexpr (ALIGN) {
+    // the expert whose blocks hold mb: its lane, then which of the lane's four
+    const int in = (nb[0] + nb[1]) + (nb[2] + nb[3]);
+    const int at = __builtin_ctzll(__ballot(blocks_in > mb));
+    int first = __builtin_amdgcn_readlane(blocks_in - in, at), mine_nb = __builtin_amdgcn_readlane(nb[0], at);
+    e = 4 * at;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) eq[i] = uniform_load(expert_ids + (q0 + i < live_mb ? q0 + i : live_mb - 1));
-  uint32_t links = 0;  // bit i: blocks i and i + 1 of the group belong to one expert
+    for (int i = 1; i < 4; ++i) {
+      const bool on = mb >= first + mine_nb;   // (once it is not, it stays so)
+      first += on ? mine_nb : 0;
+      mine_nb = on ? __builtin_amdgcn_readlane(nb[i], at) : mine_nb;
+      e += on ? 1 : 0;
+    }
+    const int q0 = mb & ~3, lo = first > q0 ? first : q0;
+    const int end = first + mine_nb < q0 + 4 ? first + mine_nb : q0 + 4;
+    g = end - lo;
+    const int li = (mb - lo) * num_n_tiles + nt;
+    nt = g == 1 ? li : static_cast<int>(__umulhi(li, g == 2 ? 0x80000000u : g == 3 ? 0x55555556u : 0x40000000u));  // li / g
+    mb = lo + (li - nt * g);
+    in_expert = mb - first;
+  } else {
+    const int q0 = mb & ~3, me = mb & 3;
+    int eq[4];
 #pragma unroll
-  for (int i = 0; i < 3; ++i) links |= (q0 + i + 1 < live_mb && eq[i] == eq[i + 1]) ? 1u << i : 0u;
-  const int lo = me - __builtin_clz(~(links << (31 - me) << 1)), hi = me + __builtin_ctz(~(links >> me));
-  const int e = me == 0 ? eq[0] : me == 1 ? eq[1] : me == 2 ? eq[2] : eq[3];
-  const int g = hi - lo + 1;
+    for (int i = 0; i < 4; ++i) eq[i] = uniform_load(expert_ids + (q0 + i < live_mb ? q0 + i : live_mb - 1));
+    uint32_t links = 0;  // bit i: blocks i and i + 1 of the group belong to one expert
+#pragma unroll
+    for (int i = 0; i < 3; ++i) links |= (q0 + i + 1 < live_mb && eq[i] == eq[i + 1]) ? 1u << i : 0u;
+    const int lo = me - __builtin_clz(~(links << (31 - me) << 1)), hi = me + __builtin_ctz(~(links >> me));
+    e = me == 0 ? eq[0] : me == 1 ? eq[1] : me == 2 ? eq[2] : eq[3];
+    g = hi - lo + 1;
+    const int li = (me - lo) * num_n_tiles + nt;
+    nt = g == 1 ? li : static_cast<int>(__umulhi(li, g == 2 ? 0x80000000u : g == 3 ? 0x55555556u : 0x40000000u));  // li / g
+    mb = q0 + lo + (li - nt * g);
+  }
   const bool alone = g == 1;  // nobody else here reads these weights (or hardly: a run may go on in the next four blocks)
-  const int li = (me - lo) * num_n_tiles + nt;
-  nt = g == 1 ? li : static_cast<int>(__umulhi(li, g == 2 ? 0x80000000u : g == 3 ? 0x55555556u : 0x40000000u));  // li / g
-  mb = q0 + lo + (li - nt * g);
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int l15 = lane & 15, lq = lane >> 4;
   const int n0 = nt * BN_OUT;
 
   // second round trip, scalar: the block's slots and the eight whose token rows this wavefront requests.  The first
   // weights are asked for meanwhile: vector loads whose results are needed this early would wait for them, too
-  const int32_t* sid = sorted_ids + static_cast<int64_t>(mb) * kStBM;
-  int slots[kStBM], mine[8];
+  [[maybe_unused]] int slots[kStBM], mine[8];
+  if constexpr (!ALIGN) {
+    const int32_t* sid = sorted_ids + static_cast<int64_t>(mb) * kStBM;
 #pragma unroll
-  for (int i = 0; i < kStBM; ++i) slots[i] = uniform_load(sid + i);
+    for (int i = 0; i < kStBM; ++i) slots[i] = uniform_load(sid + i);
 #pragma unroll
-  for (int i = 0; i < 8; ++i) mine[i] = uniform_load(sid + 8 * wave + i);
+    for (int i = 0; i < 8; ++i) mine[i] = uniform_load(sid + 8 * wave + i);
+  }
   const char* w_base = static_cast<const char*>(p.w) + static_cast<int64_t>(e < 0 ? 0 : e) * p.w_stride_e * ES;
   // The lane's results: columns n_out and n_out + 1 (their gate and up rows), or n_out .. n_out + 3.
   const int n_out = n0 + (GATED ? 8 * wave + 2 * lq : 16 * wave + 4 * lq);
@@ -1797,18 +1861,45 @@ __global__ __launch_bounds__(kThreads, 3) void stream_gemm_kernel(
   using Both = IntTag<3>;
   issue(0, Weights{});
   if (1 < nu) issue(1, Weights{});
-  if (slots[0] >= p.numel) {  // real slots come first: the block is empty
-    wait_vmcnt<0>();          // nothing may still be landing in LDS when the workgroup ends
-    return;
-  }
-  // slots of this lane's results: tokens lane % 16 and 16 + lane % 16 of the block
-  int tok[2];
+  // slots of this lane's results, tokens lane % 16 and 16 + lane % 16 of the block, and of the row that it asks for
+  int tok[2], slot_tok;
+  if constexpr (ALIGN) {
+    int have = 0;
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    int v = slots[16 * h];
+    for (int i = 0; i < 4; ++i) have += id[i] == e ? 1 : 0;
+    const int upto = wave_inclusive_scan(have);
+    if (lane == kWave - 1) s_part[wave] = upto;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    bare_barrier();
+    int rank = upto - have - kStBM * in_expert;
 #pragma unroll
-    for (int i = 1; i < 16; ++i) v = l15 == i ? slots[16 * h + i] : v;
-    tok[h] = v;
+    for (int w = 0; w < kThreads / kWave - 1; ++w) rank += w < wave ? s_part[w] : 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (id[i] == e) {
+        if (rank >= 0 && rank < kStBM) s_slots[rank] = 4 * tid + i;
+        ++rank;
+      }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    bare_barrier();
+    tok[0] = s_slots[l15];
+    tok[1] = s_slots[16 + l15];
+    slot_tok = s_slots[8 * wave + (lane >> 3)];
+  } else {
+    if (slots[0] >= p.numel) {  // real slots come first: the block is empty
+      wait_vmcnt<0>();          // nothing may still be landing in LDS when the workgroup ends
+      return;
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      int v = slots[16 * h];
+#pragma unroll
+      for (int i = 1; i < 16; ++i) v = l15 == i ? slots[16 * h + i] : v;
+      tok[h] = v;
+    }
+    slot_tok = mine[0];
+#pragma unroll
+    for (int i = 1; i < 8; ++i) slot_tok = lane >> 3 == i ? mine[i] : slot_tok;
   }
   // What the epilogue needs per slot and per weight row is fetched now, ahead of the stream: a load
   // issued behind ~100 KB of queued DMA requests would take microseconds to return.
@@ -1831,9 +1922,6 @@ __global__ __launch_bounds__(kThreads, 3) void stream_gemm_kernel(
     const int q = lane >> 3;
     const int rr = 8 * wave + q;
     int64_t src = mb * kStBM + rr;
-    int slot_tok = mine[0];
-#pragma unroll
-    for (int i = 1; i < 8; ++i) slot_tok = q == i ? mine[i] : slot_tok;
     if (!p.a_by_slot) src = slot_tok < p.numel ? slot_tok / p.top_k : 0;
     a_live = slot_tok < p.numel || lane == 0;
     a_off = static_cast<uint32_t>(src * p.lda * ES + (((lane & 7) ^ ((rr >> 1) & 7)) << 4));
@@ -1901,6 +1989,12 @@ __global__ __launch_bounds__(kThreads, 3) void stream_gemm_kernel(
     else if (p.activation == MOE_ACT_SWIGLUOAI) stream_store<El, GATED, MOE_ACT_SWIGLUOAI>(p, v, crow, n_out);
     else stream_store<El, GATED, MOE_ACT_GELU>(p, v, crow, n_out);
   }
+  if constexpr (ALIGN) {
+    if (nt == 0) {
+      if (tid < kStBM) sorted_ids[mb * kStBM + tid] = s_slots[tid];
+      if (tid == 0) expert_ids[mb] = e;
+    }
+  }
 }
 
 template <typename Mma, bool GATED>
@@ -1913,8 +2007,17 @@ int launch_stream(GemmParams& p, int64_t sorted_cap, hipStream_t s) {
   if (grid > INT32_MAX) return moe_fail(MOE_ERR_ARG, "fused_experts: grid of %lld workgroups", static_cast<long long>(grid));
   const dim3 blocks(static_cast<unsigned>(grid)), threads(kThreads);
   auto go = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, blocks, threads, 0, s, p.num_post_pad, p.expert_ids, p.sorted_ids, p.num_n_tiles, n_tiles_rcp, p);
+    hipLaunchKernelGGL(kernel, blocks, threads, 0, s, p.ids ? p.ids : p.num_post_pad, const_cast<int32_t*>(p.expert_ids),
+                       const_cast<int32_t*>(p.sorted_ids), p.num_n_tiles, n_tiles_rcp, p.numel, p.num_experts, p);
   };
+  if constexpr (GATED) {
+    if (p.ids) {
+      if (p.Kd * Mma::kEs % kStRowBytes) go((stream_gemm_kernel<Mma, true, true, false, true>));
+      else if (!p.silu_once) go((stream_gemm_kernel<Mma, true, false, false, true>));
+      else go((stream_gemm_kernel<Mma, true, false, true, true>));
+      return moe_check_launch("fused_experts (alignment and gate-up pass)");
+    }
+  }
   if (p.Kd * Mma::kEs % kStRowBytes)
     go((stream_gemm_kernel<Mma, GATED, true>));
   else if (!GATED || !p.silu_once)  // (named in front of the once-rounding instance and so placed in front of it, as
@@ -2331,9 +2434,21 @@ void moe_experts_x_codes(const MoeFusedExpertsArgs* a, uint8_t** codes, float** 
   *scales = reinterpret_cast<float*>(*codes + moe_align_up(static_cast<int64_t>(a->T) * a->H, 256));
 }
 
-MOE_EXPORT int moe_fused_experts(const MoeFusedExpertsArgs* a) { return moe_fused_experts_of_codes(a, false); }
+MOE_EXPORT int moe_fused_experts(const MoeFusedExpertsArgs* a) { return moe_fused_experts_of_codes(a, false, nullptr); }
 
-int moe_fused_experts_of_codes(const MoeFusedExpertsArgs* a, bool x_coded) {
+// (what launch_bm asks before it takes the streaming kernel for the gate-up pass)
+bool moe_experts_align(const MoeFusedExpertsArgs* a) {
+  const int64_t numel = static_cast<int64_t>(a->T) * a->K, es = elem_size(a->weight_dtype);
+  if (a->block_size != kStBM || numel < 1 || numel > kStAlignMost || a->E > 256 || es > 2 || (a->passes & 7) || a->H * es % 32) return false;
+  if (fused_args_ragged(a)) return false;
+  GemmParams p{};
+  p.numel = static_cast<int>(numel);
+  p.top_k = a->K;
+  p.lda = a->H; p.N = a->I; p.w_stride_n = a->w13_stride_n; p.a_by_slot = 0;
+  return dma_offsets_fit(p, true, numel + static_cast<int64_t>(a->E) * (kStBM - 1), static_cast<int>(es));
+}
+
+int moe_fused_experts_of_codes(const MoeFusedExpertsArgs* a, bool x_coded, const int32_t* ids) {
   int64_t cap = 0, need_ws = 0;
   if (int rc0 = check_fused_args(a, &cap, &need_ws)) return rc0;
   if (a->T == 0) return MOE_OK;
@@ -2387,6 +2502,8 @@ int moe_fused_experts_of_codes(const MoeFusedExpertsArgs* a, bool x_coded) {
   p.bias = a->w13_bias; p.bias_stride_e = 2LL * a->I;
   p.c = inter; p.ldc = a->I; p.Kd = a->H; p.N = a->I; p.a_by_slot = 0;
   p.mul_weight = a->apply_router_weight_on_input ? 1 : 0;
+  p.ids = ids;
+  p.num_experts = a->E;
   const int passes = (a->passes & 7) ? a->passes : (a->passes | 7);
   int rc = MOE_OK;
   // When both passes run on the 16-bit large-tile kernel the intermediate lives in the workspace as
@@ -2428,6 +2545,7 @@ int moe_fused_experts_of_codes(const MoeFusedExpertsArgs* a, bool x_coded) {
   if (rc) return rc;
 
   // pass 2: inter . W2^T times the routed weight, rows written by flat token id
+  p.ids = nullptr;
   p.a = inter; p.lda = a->I; p.w = a->w2; p.w_stride_e = a->w2_stride_e; p.w_stride_n = a->w2_stride_n;
   p.bias = a->w2_bias; p.bias_stride_e = a->H;
   p.c = c3; p.ldc = a->H; p.Kd = a->I; p.N = a->H; p.a_by_slot = 1;

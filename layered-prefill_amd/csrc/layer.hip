@@ -170,15 +170,6 @@ MOE_EXPORT int moe_layer(const MoeLayerArgs* a) {
                     moe_fused_experts_plan_layout(a->T, a->H, a->I, a->E, a->K, l.block, a->act_dtype, a->weight_dtype,
                                                   &bounds_off, &done_off, &num_done, &cap_mb);
   char* fws = static_cast<char*>(l.fused_ws);
-  if (plan)
-    rc = moe_align_block_size_planned(l.topk_ids, MOE_ID_I32, numel, a->E, l.block, l.sorted, l.sorted_cap, l.experts,
-                                      l.expert_cap, l.npp, l.align_ws, l.align_bytes, a->stream,
-                                      reinterpret_cast<int32_t*>(fws + bounds_off), reinterpret_cast<int32_t*>(fws + done_off),
-                                      num_done, cap_mb);
-  else if (!routed)
-    rc = moe_align_block_size(l.topk_ids, MOE_ID_I32, numel, a->E, l.block, l.sorted, l.sorted_cap, l.experts, l.expert_cap,
-                              l.npp, l.align_ws, l.align_bytes, a->stream);
-  if (rc) return rc;
   f.x = a->x; f.out = a->out; f.w13 = a->w13; f.w2 = a->w2;
   f.w13_bias = a->w13_bias; f.w2_bias = a->w2_bias; f.w13_scale = a->w13_scale; f.w2_scale = a->w2_scale;
   f.topk_weights = l.topk_w;
@@ -194,5 +185,16 @@ MOE_EXPORT int moe_layer(const MoeLayerArgs* a) {
   if (!a->block_size && l.block < moe_preferred_block_size(a->T, a->E, a->K, a->act_dtype, a->weight_dtype)) f.passes |= 64;
   f.weight_layout = a->weight_layout;
   f.stream = a->stream;
-  return moe_fused_experts_of_codes(&f, x_coded);
+  // a few hundred ids are aligned by the gate-up pass itself
+  const bool aligns = !routed && !plan && !a->block_size && moe_experts_align(&f);
+  if (plan)
+    rc = moe_align_block_size_planned(l.topk_ids, MOE_ID_I32, numel, a->E, l.block, l.sorted, l.sorted_cap, l.experts,
+                                      l.expert_cap, l.npp, l.align_ws, l.align_bytes, a->stream,
+                                      reinterpret_cast<int32_t*>(fws + bounds_off), reinterpret_cast<int32_t*>(fws + done_off),
+                                      num_done, cap_mb);
+  else if (!routed && !aligns)
+    rc = moe_align_block_size(l.topk_ids, MOE_ID_I32, numel, a->E, l.block, l.sorted, l.sorted_cap, l.experts, l.expert_cap,
+                              l.npp, l.align_ws, l.align_bytes, a->stream);
+  if (rc) return rc;
+  return moe_fused_experts_of_codes(&f, x_coded, aligns ? l.topk_ids : nullptr);
 }
