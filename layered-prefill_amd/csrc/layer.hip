@@ -140,15 +140,32 @@ MOE_EXPORT int moe_layer(const MoeLayerArgs* a) {
   const int64_t numel = static_cast<int64_t>(a->T) * a->K;
   int rc = MOE_OK;
   if (moe_layer_few(a, l.topk_w, l.topk_ids, l.sorted, l.fused_ws, &rc)) return rc;
-  // what the expert passes will be given: the routing of an e4m3 call leaves the codes of x in their workspace
+  // what the expert passes will be given (the routing of an e4m3 call leaves the codes of x in their workspace)
   MoeFusedExpertsArgs f{};
   f.workspace = l.fused_ws; f.workspace_bytes = l.fused_bytes;
   f.T = a->T; f.H = a->H; f.I = a->I; f.E = a->E; f.K = a->K;
   f.block_size = l.block; f.act_dtype = a->act_dtype; f.weight_dtype = a->weight_dtype;
+  f.x = a->x; f.out = a->out; f.w13 = a->w13; f.w2 = a->w2;
+  f.w13_bias = a->w13_bias; f.w2_bias = a->w2_bias; f.w13_scale = a->w13_scale; f.w2_scale = a->w2_scale;
+  f.topk_weights = l.topk_w;
+  f.sorted_token_ids = l.sorted; f.expert_ids = l.experts; f.num_tokens_post_pad = l.npp;
+  f.w13_stride_e = a->w13_stride_e; f.w13_stride_n = a->w13_stride_n;
+  f.w2_stride_e = a->w2_stride_e; f.w2_stride_n = a->w2_stride_n;
+  f.sorted_cap = l.sorted_cap;
+  f.activation = a->activation;
+  f.apply_router_weight_on_input = a->apply_router_weight_on_input;
+  f.swiglu_alpha = a->swiglu_alpha; f.swiglu_limit = a->swiglu_limit;
+  f.weight_layout = a->weight_layout;
+  f.stream = a->stream;
+  // A few hundred ids are aligned by the gate-up pass itself; the launch that routes and aligns in one workgroup is for calls
+  // whose gate-up pass does not.  Layer with the norm, us, that launch and this way: 128 experts, 12 tokens 62.8 and 60.0,
+  // 14 65.2 and 62.4, e4m3 8 tokens 41.0 and 38.7, 16 49.1 and 47.0; 64 experts, 30 tokens 80.2 and 75.8; 32 experts, 60
+  // tokens 71.0 and 69.3.
+  const bool aligns = !a->block_size && moe_experts_align(&f);
   MoeXCodes xc{a->x, a->H, nullptr, nullptr};
   moe_experts_x_codes(&f, &xc.codes, &xc.scales);
   const bool code_x = a->router_logits && a->weight_dtype == MOE_E4M3 && a->logits_dtype == a->act_dtype && moe_x_codes_ok(xc);
-  const bool routed = a->router_logits &&
+  const bool routed = a->router_logits && !aligns &&
                       moe_layer_route_align(a->router_logits, a->logits_dtype, l.topk_w, a->T, a->E, a->K, a->renormalize, l.block,
                                             l.sorted, l.sorted_cap, l.experts, l.expert_cap, l.npp, code_x ? &xc : nullptr,
                                             static_cast<hipStream_t>(a->stream), &rc);
@@ -170,23 +187,9 @@ MOE_EXPORT int moe_layer(const MoeLayerArgs* a) {
                     moe_fused_experts_plan_layout(a->T, a->H, a->I, a->E, a->K, l.block, a->act_dtype, a->weight_dtype,
                                                   &bounds_off, &done_off, &num_done, &cap_mb);
   char* fws = static_cast<char*>(l.fused_ws);
-  f.x = a->x; f.out = a->out; f.w13 = a->w13; f.w2 = a->w2;
-  f.w13_bias = a->w13_bias; f.w2_bias = a->w2_bias; f.w13_scale = a->w13_scale; f.w2_scale = a->w2_scale;
-  f.topk_weights = l.topk_w;
-  f.sorted_token_ids = l.sorted; f.expert_ids = l.experts; f.num_tokens_post_pad = l.npp;
-  f.w13_stride_e = a->w13_stride_e; f.w13_stride_n = a->w13_stride_n;
-  f.w2_stride_e = a->w2_stride_e; f.w2_stride_n = a->w2_stride_n;
-  f.sorted_cap = l.sorted_cap;
-  f.activation = a->activation;
-  f.apply_router_weight_on_input = a->apply_router_weight_on_input;
-  f.swiglu_alpha = a->swiglu_alpha; f.swiglu_limit = a->swiglu_limit;
   f.passes = plan ? 16 : 0;
   // a block of 32 of the library's own choice where the large tile would also do: same roundings as that
   if (!a->block_size && l.block < moe_preferred_block_size(a->T, a->E, a->K, a->act_dtype, a->weight_dtype)) f.passes |= 64;
-  f.weight_layout = a->weight_layout;
-  f.stream = a->stream;
-  // a few hundred ids are aligned by the gate-up pass itself
-  const bool aligns = !routed && !plan && !a->block_size && moe_experts_align(&f);
   if (plan)
     rc = moe_align_block_size_planned(l.topk_ids, MOE_ID_I32, numel, a->E, l.block, l.sorted, l.sorted_cap, l.experts,
                                       l.expert_cap, l.npp, l.align_ws, l.align_bytes, a->stream,
