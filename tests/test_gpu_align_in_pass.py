@@ -49,3 +49,23 @@ def test_bits_of_the_steps(moe, dev, monkeypatch, case, given):
     monkeypatch.setattr(moe.fused_moe, "_layer_call", lambda *a: None)
     steps = call()
     assert bool(steps.isfinite().all()) and float(steps.float().abs().max()) > 0 and torch.equal(one, steps)
+
+
+@pytest.mark.parametrize("T", [100, 700])   # aligned in the pass; by a workgroup for every 1024 ids
+def test_replay_from_a_graph(moe, dev, T):
+    E, K, H, I = 64, 8, 256, 128
+    g = torch.Generator().manual_seed(T)
+    x, logits = torch.randn(T, H, generator=g).to(_BF).to(dev), torch.randn(T, E, generator=g).to(_BF).to(dev)
+    w13 = (0.1 * torch.randn(E, 2 * I, H, generator=g)).to(_BF).to(dev)
+    w2 = (0.1 * torch.randn(E, H, I, generator=g)).to(_BF).to(dev)
+    moe.fused_topk_experts(x, logits, w13, w2, K, True)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = moe.fused_topk_experts(x, logits, w13, w2, K, True)
+    for _ in range(4):
+        x.normal_()
+        logits.normal_()
+        graph.replay()
+        assert torch.equal(out, moe.fused_topk_experts(x, logits, w13, w2, K, True))
+        torch.cuda.synchronize()
