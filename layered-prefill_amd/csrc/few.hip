@@ -86,7 +86,7 @@ __global__ __launch_bounds__(NW * kWave, 1) void few_gate_kernel(const void* __r
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   __shared__ int s_ids[kFewFlats], s_flag[E];
   __shared__ float s_w[kFewFlats];
-  __shared__ uint32_t s_kmap[kFewTokens * E / 4];   // which of a token's k an expert is, a byte each
+  __shared__ uint32_t s_kmap[kFewTokens * E / 4];   // which of a token's k an expert is (ids that repeat: any of them), a byte each
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l15 = lane & 15, lq = lane >> 4;
   const int T = p.T, K = p.K, numel = T * K, nu = p.H / 64;
@@ -194,6 +194,9 @@ __global__ __launch_bounds__(NW * kWave, 1) void few_gate_kernel(const void* __r
   int e = e_ask, c = c_ask;
   for (int i = 0; i < kRing; ++i) ask();
   const int t = l15 < T ? l15 : T - 1;
+  // a row of logits without a largest one has expert 0 at every k, and its first weight is no number (without
+  // renormalisation only that one)
+  const bool repeats = s_w[t * K] != s_w[t * K];
   int rd_w[2], rd_x[2];
 #pragma unroll
   for (int kk = 0; kk < 2; ++kk) {
@@ -250,20 +253,23 @@ __global__ __launch_bounds__(NW * kWave, 1) void few_gate_kernel(const void* __r
       x_at += UN * T * kFewRow;
     }
     if (mine) {
-      const float rw = p.weight_on_input ? s_w[t * K + k_of] : 1.f;
-      float v[4];
+      // (every k of a row whose ids repeat: the down pass reads all of them)
+      for (int k = repeats ? 0 : k_of; k < (repeats ? K : k_of + 1); ++k) {
+        const float rw = p.weight_on_input ? s_w[t * K + k] : 1.f;
+        float v[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        v[i] = acc[i];
-        if (p.b13) v[i] += bias[i];
-        v[i] *= rw;
+        for (int i = 0; i < 4; ++i) {
+          v[i] = acc[i];
+          if (p.b13) v[i] += bias[i];
+          v[i] *= rw;
+        }
+        const uint32_t g = pack2<El>(v[0], v[1]), up = pack2<El>(v[2], v[3]);
+        uint32_t o;
+        if (p.activation == MOE_ACT_SILU) o = gated_pair<El, MOE_ACT_SILU>(p.alpha, p.limit, g, up);
+        else if (p.activation == MOE_ACT_SWIGLUOAI) o = gated_pair<El, MOE_ACT_SWIGLUOAI>(p.alpha, p.limit, g, up);
+        else o = gated_pair<El, MOE_ACT_GELU>(p.alpha, p.limit, g, up);
+        *reinterpret_cast<uint32_t*>(static_cast<uint16_t*>(p.inter) + static_cast<int64_t>(t * K + k) * p.I + 8 * c + 2 * lq) = o;
       }
-      const uint32_t g = pack2<El>(v[0], v[1]), up = pack2<El>(v[2], v[3]);
-      uint32_t o;
-      if (p.activation == MOE_ACT_SILU) o = gated_pair<El, MOE_ACT_SILU>(p.alpha, p.limit, g, up);
-      else if (p.activation == MOE_ACT_SWIGLUOAI) o = gated_pair<El, MOE_ACT_SWIGLUOAI>(p.alpha, p.limit, g, up);
-      else o = gated_pair<El, MOE_ACT_GELU>(p.alpha, p.limit, g, up);
-      *reinterpret_cast<uint32_t*>(static_cast<uint16_t*>(p.inter) + static_cast<int64_t>(t * K + k_of) * p.I + 8 * c + 2 * lq) = o;
     }
     e = e_ask;
     c = c_ask;

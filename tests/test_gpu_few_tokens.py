@@ -69,6 +69,28 @@ def test_all_tokens_on_the_same_experts_and_rows_that_are_no_numbers(moe, dev, m
     assert torch.equal(got[1][rows], want[rows]) and bool(got[1][~rows].isnan().all())
 
 
+@pytest.mark.parametrize("activation", ["silu", "swigluoai", "gelu"])
+@pytest.mark.parametrize("on_input", [False, True])
+@pytest.mark.parametrize("renormalize", [False, True])
+def test_rows_whose_ids_repeat_have_every_term(moe, dev, monkeypatch, activation, on_input, renormalize):
+    """Logits without a largest one go to expert 0 K times, with the weights NaN, -10000, -10000, ...: the result is that of
+    the steps, whatever an earlier call (of finite rows, twice as large) left in the workspace."""
+    print(activation, on_input, renormalize, flush=True)
+    x, logits, w13, w2, K, kw = _args(moe, dev, 12, 32, 6, 512, 384, _BF, "plain", activation, False, on_input, _BF)
+    lost = logits.clone()
+    lost[3], lost[5, 7], lost[8], lost[11, 31] = float("nan"), float("inf"), -float("inf"), float("nan")
+    got = []
+    for _ in range(4):
+        assert bool(moe.fused_topk_experts(2 * x, logits, w13, w2, K, renormalize, **kw).isfinite().all())
+        got.append(moe.fused_topk_experts(x, lost, w13, w2, K, renormalize, **kw))
+    monkeypatch.setattr(moe.fused_moe, "_layer_call", lambda *a: None)
+    want = moe.fused_topk_experts(x, lost, w13, w2, K, renormalize, **kw)
+    whole = torch.tensor([t not in (3, 5, 8, 11) for t in range(12)], device=dev)
+    assert bool(want[whole].isfinite().all())
+    for g in got:
+        assert torch.equal(g.isnan(), want.isnan()) and torch.equal(g.nan_to_num(nan=0.0), want.nan_to_num(nan=0.0))
+
+
 def test_few_tokens_replay_from_a_graph(moe, dev):
     x, logits, w13, w2, K, kw = _args(moe, dev, 5, 64, 4, 512, 384, _BF, "plain", "silu", False, False, _BF)
     want = moe.fused_topk_experts(x, logits, w13, w2, K, True)
