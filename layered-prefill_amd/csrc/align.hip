@@ -121,7 +121,7 @@ __device__ void write_blocks_and_padding(const volatile int* cum, const volatile
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   for (int e = wave; e < E; e += kScanWaves) {
     const int beg = cum[e] + tot[e], end = cum[e + 1];
-    for (int p = beg + lane; p < end; p += kWave) sorted_ids[p] = numel;
+    for (int64_t p = beg + lane; p < end; p += kWave) sorted_ids[p] = numel;
   }
   for (int64_t p = total + threadIdx.x; p < sorted_cap; p += kScanThreads) sorted_ids[p] = numel;
 }
@@ -448,6 +448,9 @@ static_assert(kScanThreads % kSegLen == 0, "a workgroup takes whole segments");
 // With the counts from segments, every workgroup reads all of them: from 256 workgroups on that is what it takes
 // (524288 ids 25.1 us by align_place_kernel, 27.0 here).
 constexpr int64_t kSpreadTableMost = 256 * kScanThreads;
+// Longest outputs of the kernels that count slots in 32 bits: a wavefront's next turn at them, up to 4096 wavefronts of 256
+// slots further on, must not wrap around.  Longer ones go to the kernels that count in 64.
+constexpr int64_t kIntCapMost = INT32_MAX - kSpreadTableMost / kWave * (4 * kWave);
 template <int MOST>
 __global__ __launch_bounds__(kScanThreads) void align_spread_kernel(
     const int32_t* __restrict__ ids, int numel, int E, int BM, int id_bits, int32_t* __restrict__ sorted_ids,
@@ -770,7 +773,7 @@ __global__ __launch_bounds__(kScanThreads) void align_place_kernel(
   }
   for (int x = blockIdx.x * kScanWaves + wave; x < E; x += nwg * kScanWaves) {
     const int beg = cum[x] + tot[x], end = cum[x + 1];
-    for (int p = beg + lane; p < end; p += kWave) sorted_ids[p] = static_cast<int32_t>(numel);
+    for (int64_t p = beg + lane; p < end; p += kWave) sorted_ids[p] = static_cast<int32_t>(numel);
   }
   for (int64_t p = total + gtid; p < sorted_cap; p += gthreads) sorted_ids[p] = static_cast<int32_t>(numel);
   if (plan_bounds && blockIdx.x == 0)
@@ -840,16 +843,15 @@ static int align_impl(const void* topk_ids, int ids_dtype, int64_t numel, int E,
     return moe_fail(MOE_ERR_ARG, "moe_align_block_size: null pointer");
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int id_bits = bits_for(E);
-  if (numel <= kTinyNumel && E <= kTinyExperts && block_size <= 64 && ids_dtype == MOE_ID_I32 && !plan_bounds &&
-      sorted_cap <= INT32_MAX && expert_cap <= INT32_MAX) {
+  const bool int_caps = sorted_cap <= kIntCapMost && expert_cap <= kIntCapMost;
+  if (numel <= kTinyNumel && E <= kTinyExperts && block_size <= 64 && ids_dtype == MOE_ID_I32 && !plan_bounds && int_caps) {
     // (longer blocks have more padding per expert than one thread should write)
     hipLaunchKernelGGL(align_tiny_kernel, dim3(1), dim3(kScanThreads), 0, s, static_cast<const int32_t*>(topk_ids),
                        static_cast<int>(numel), E, block_size, id_bits, sorted_token_ids, static_cast<int>(sorted_cap),
                        expert_ids, static_cast<int>(expert_cap), num_tokens_post_pad);
     return moe_check_launch("moe_align_block_size (single workgroup, up to 1024 ids)");
   }
-  if (numel <= kSpreadMost * kScanThreads && E <= kTinyExperts && ids_dtype == MOE_ID_I32 && sorted_cap <= INT32_MAX &&
-      expert_cap <= INT32_MAX) {
+  if (numel <= kSpreadMost * kScanThreads && E <= kTinyExperts && ids_dtype == MOE_ID_I32 && int_caps) {
     const int wgs = numel > kScanThreads ? static_cast<int>((numel + kScanThreads - 1) / kScanThreads) : 1;
     auto kern = wgs <= 8 ? align_spread_kernel<8> : align_spread_kernel<kSpreadMost>;
     hipLaunchKernelGGL(kern, dim3(wgs), dim3(kScanThreads), 0, s, static_cast<const int32_t*>(topk_ids),
@@ -875,8 +877,7 @@ static int align_impl(const void* topk_ids, int ids_dtype, int64_t numel, int E,
   int32_t* cum = seg_cnt + static_cast<size_t>(nseg) * E;
   hipLaunchKernelGGL(align_count_kernel, dim3(nseg), dim3(kWave), E * sizeof(int), s, topk_ids,
                      ids_dtype, numel, E, seg_cnt);
-  if (numel <= kSpreadTableMost && E <= kTinyExperts && ids_dtype == MOE_ID_I32 && sorted_cap <= INT32_MAX &&
-      expert_cap <= INT32_MAX) {
+  if (numel <= kSpreadTableMost && E <= kTinyExperts && ids_dtype == MOE_ID_I32 && int_caps) {
     hipLaunchKernelGGL(align_spread_kernel<0>, dim3(static_cast<unsigned>((numel + kScanThreads - 1) / kScanThreads)),
                        dim3(kScanThreads), 0, s, static_cast<const int32_t*>(topk_ids), static_cast<int>(numel), E, block_size,
                        id_bits, sorted_token_ids, static_cast<int>(sorted_cap), expert_ids, static_cast<int>(expert_cap),

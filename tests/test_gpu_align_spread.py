@@ -62,3 +62,27 @@ def test_plan_of_many_workgroups_is_that_of_the_ids(moe, dev, numel):
     # roundings of the intermediate, of each term and of the sum: 3 of 2^-9 relative, sums of 128 and 256 products in fp32
     err = (out.float() - want).norm() / want.norm()
     assert err < 3 * 2 ** -8
+
+
+@pytest.mark.parametrize("cap", [2 ** 31 - 1 - 2 ** 20, 2 ** 31 - 2 ** 20, 2 ** 31 - 1])
+@pytest.mark.parametrize("numel", [300, 1500, 20000])
+def test_longest_outputs(moe, oracle, dev, numel, cap):
+    """Output buffers up to the largest length there is, on both sides of the line behind which slots are counted in 64 bits:
+    all of them is written, and nothing in front of it."""
+    print(numel, cap, flush=True)
+    E, block, guard = 8, 32, 1024
+    ids = _ids(numel, E, "skewed")
+    want = oracle.moe_align_block_size(ids.view(-1, 1), block, E)
+    whole = torch.full((guard + cap,), -7, dtype=torch.int32, device=dev)   # 8.6 GB
+    experts = torch.full((want[1].numel() + 100,), -7, dtype=torch.int32, device=dev)
+    total = torch.empty(1, dtype=torch.int32, device=dev)
+    slots = whole[guard:]
+    moe.ops.moe_align_block_size(ids.to(dev), E, block, slots, experts, total)
+    need = want[0].numel()
+    assert torch.equal(slots[:need].cpu(), want[0]) and torch.equal(total.cpu(), want[2])
+    assert torch.equal(experts[:want[1].numel()].cpu(), want[1]) and not bool(experts[want[1].numel():].any())
+    for at in range(need, cap, 1 << 28):
+        assert bool((slots[at:at + (1 << 28)] == numel).all())
+    assert bool((whole[:guard] == -7).all())
+    del whole, slots
+    torch.cuda.empty_cache()
