@@ -530,8 +530,8 @@ __global__ __launch_bounds__(kScanThreads) void align_spread_kernel(
     }
     s_cum[tid] = first;
     s_tot[tid] = total;
-    if (tid % nwg == wg)
-      for (int b = first / BM; b < (first + padded) / BM; ++b) expert_ids[b] = tid;
+    // (an expert's blocks dealt to the workgroups: 250000 ids of 8 experts are a thousand blocks of 32 to each of them)
+    for (int b = first / BM + wg; b < (first + padded) / BM; b += nwg) expert_ids[b] = tid;
   }
   if (tid == 0) {
     s_cum[E] = all;

@@ -17,9 +17,9 @@ def _ids(numel, E, kind):
     return ids
 
 
-@pytest.mark.parametrize("numel", [1023, 1024, 1025, 2049, 8191, 8192, 8193, 16384, 16385, 17000, 67585])
+@pytest.mark.parametrize("numel", [1023, 1024, 1025, 2049, 8191, 8192, 8193, 16384, 16385, 17000, 67585, 262144])
 @pytest.mark.parametrize("E,block,kind", [(128, 256, "skewed"), (256, 32, "skewed"), (1, 64, "skewed"), (100, 16, "holes"),
-                                          (5, 256, "one")])
+                                          (5, 256, "one"), (3, 1, "skewed"), (2, 32, "holes")])
 def test_alignment_at_the_seams(moe, oracle, dev, numel, E, block, kind):
     ids = _ids(numel, E, kind)
     got = moe.moe_align_block_size(ids.view(-1, 1).to(dev), block, E)
