@@ -439,9 +439,9 @@ __global__ __launch_bounds__(kScanThreads) void align_small_kernel(
 // all, one LDS addition an id, in whose upper half stand the ids in front of the workgroup's own.  MOST == 0: it adds up
 // the segments' counts that align_count_kernel has left.  One workgroup that ranked all of up to 8192 ids was bound by the
 // issue of its CU's four SIMDs, and of larger calls each wavefront placed 512 ids one step behind the other, on a few CUs.
-// 128 experts, top-8, blocks of 256 with the plan, us, before and now: 2048 ids 7.2 and 5.8, 5928 9.9 and 5.9, 8192 11.6 and
-// 6.5, 12000 22.7 and 7.7, 16384 26.7 and 8.6; with the counting kernel in front: 32776 15.6 and 9.0, 67584 16.0 and 9.6,
-// 135168 17.4 and 11.5, 262144 19.8 and 14.9.  Blocks of 32: 1204 ids of 32 experts 4.3 and 4.2, 1920 of 128 6.1 and 4.9.
+// 128 experts, blocks of 256, alone, us, before and now: 2048 ids 6.7 and 5.1, 5928 10.4 and 5.1, 8192 12.2 and 5.1, 12000
+// 21.5 and 6.8, 16384 25.8 and 7.5; with the counting kernel in front: 67584 14.7 and 8.8, 262144 18.8 and 12.9.  8 experts,
+// blocks of 32: 2048 4.2 and 4.1, 8192 8.3 and 5.2, 262144 13.8 and 7.9.
 constexpr int kSpreadMost = 16;
 static_assert((kSpreadMost - 1) * kScanThreads < 1 << 15 && kSpreadMost * kScanThreads < 1 << 16, "two counts in a word");
 static_assert(kScanThreads % kSegLen == 0, "a workgroup takes whole segments");
@@ -451,7 +451,11 @@ constexpr int64_t kSpreadTableMost = 256 * kScanThreads;
 // Longest outputs of the kernels that count slots in 32 bits: a wavefront's next turn at them, up to 4096 wavefronts of 256
 // slots further on, must not wrap around.  Longer ones go to the kernels that count in 64.
 constexpr int64_t kIntCapMost = INT32_MAX - kSpreadTableMost / kWave * (4 * kWave);
-template <int MOST>
+// FEW: lanes that add to one word wait for each other, and with up to four experts the ranks' ballots are few, so that a
+// wavefront's lanes of an expert add once (as a run-time branch 64 experts and more lost 3 to 6 %).  Blocks of 256, us,
+// without and with it: 1 expert 2048 ids 5.1 and 4.2, 8192 10.3 and 5.4; 4 experts 1030 4.0 and 4.1, 8192 6.1 and 5.6.
+constexpr int kSpreadFew = 4;
+template <int MOST, bool FEW = false>
 __global__ __launch_bounds__(kScanThreads) void align_spread_kernel(
     const int32_t* __restrict__ ids, int numel, int E, int BM, int id_bits, int32_t* __restrict__ sorted_ids,
     int sorted_cap, int32_t* __restrict__ expert_ids, int expert_cap, int32_t* __restrict__ num_post_pad,
@@ -484,7 +488,14 @@ __global__ __launch_bounds__(kScanThreads) void align_spread_kernel(
     for (int j = 0; j < MOST; ++j) {
       if (j * kScanThreads >= numel) break;
       if (j == wg) own = id[j];
-      if (id[j] >= 0 && id[j] < E) atomicAdd(&s_all[id[j]], j < wg ? 1 + (1 << 16) : 1);
+      const bool count = id[j] >= 0 && id[j] < E;
+      if constexpr (FEW) {
+        const uint64_t same = same_id_lanes(id[j], count, id_bits);
+        const int n = __popcll(same);
+        if (count && !(same & lanes_below(lane))) atomicAdd(&s_all[id[j]], j < wg ? n + (n << 16) : n);
+      } else if (count) {
+        atomicAdd(&s_all[id[j]], j < wg ? 1 + (1 << 16) : 1);
+      }
     }
   } else {
     // thread t sums expert t % E over the segments t / E, t / E + R, .. (a wavefront reads one segment's counts side by side)
@@ -853,7 +864,8 @@ static int align_impl(const void* topk_ids, int ids_dtype, int64_t numel, int E,
   }
   if (numel <= kSpreadMost * kScanThreads && E <= kTinyExperts && ids_dtype == MOE_ID_I32 && int_caps) {
     const int wgs = numel > kScanThreads ? static_cast<int>((numel + kScanThreads - 1) / kScanThreads) : 1;
-    auto kern = wgs <= 8 ? align_spread_kernel<8> : align_spread_kernel<kSpreadMost>;
+    auto kern = E <= kSpreadFew ? (wgs <= 8 ? align_spread_kernel<8, true> : align_spread_kernel<kSpreadMost, true>)
+                                : (wgs <= 8 ? align_spread_kernel<8> : align_spread_kernel<kSpreadMost>);
     hipLaunchKernelGGL(kern, dim3(wgs), dim3(kScanThreads), 0, s, static_cast<const int32_t*>(topk_ids),
                        static_cast<int>(numel), E, block_size, id_bits, sorted_token_ids, static_cast<int>(sorted_cap),
                        expert_ids, static_cast<int>(expert_cap), num_tokens_post_pad, plan_bounds, plan_done, plan_num_done,

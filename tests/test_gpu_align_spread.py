@@ -19,7 +19,8 @@ def _ids(numel, E, kind):
 
 @pytest.mark.parametrize("numel", [1023, 1024, 1025, 2049, 8191, 8192, 8193, 16384, 16385, 17000, 67585, 262144])
 @pytest.mark.parametrize("E,block,kind", [(128, 256, "skewed"), (256, 32, "skewed"), (1, 64, "skewed"), (100, 16, "holes"),
-                                          (5, 256, "one"), (3, 1, "skewed"), (2, 32, "holes")])
+                                          (5, 256, "one"), (3, 1, "skewed"), (2, 32, "holes"), (4, 256, "holes"),
+                                          (1, 256, "one")])
 def test_alignment_at_the_seams(moe, oracle, dev, numel, E, block, kind):
     ids = _ids(numel, E, kind)
     got = moe.moe_align_block_size(ids.view(-1, 1).to(dev), block, E)
