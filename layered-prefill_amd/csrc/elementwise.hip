@@ -14,9 +14,9 @@ struct alignas(sizeof(S) * N) Vec {
   S v[N];
 };
 
-template <typename S, int N>
+template <bool ONCE, typename S, int N>
 __device__ __forceinline__ Vec<S, N> load_terms(const S* p) {
-  if constexpr (sizeof(Vec<S, N>) == 16) return __builtin_bit_cast(Vec<S, N>, load_once(p));
+  if constexpr (ONCE && sizeof(Vec<S, N>) == 16) return __builtin_bit_cast(Vec<S, N>, load_once(p));
   else return *reinterpret_cast<const Vec<S, N>*>(p);
 }
 
@@ -66,10 +66,8 @@ __global__ __launch_bounds__(kThreads) void swigluoai_and_mul_kernel(
 }
 
 // out[t, h] = sum_k in[t, k, h], ascending k, fp32 accumulation.  KK: K, where it is known here and all of a
-// result's terms are asked for at once; else 0.  Bound by memory.  The terms are read once, and past the caches
-// (load_once): 277 MB of them that the down pass has just written 52.0 -> 47.9 us, 554 MB 118.5 -> 93.1 (6.7 TB/s with
-// the result).
-template <typename El, int VEC, int KK>
+// result's terms are asked for at once; else 0.  Bound by memory.  ONCE: the terms are read past the caches (load_once).
+template <typename El, int VEC, int KK, bool ONCE>
 __global__ __launch_bounds__(kThreads) void moe_sum_kernel(typename El::S* __restrict__ out,
                                                            const typename El::S* __restrict__ in,
                                                            int64_t T, int K, int H) {
@@ -87,14 +85,14 @@ __global__ __launch_bounds__(kThreads) void moe_sum_kernel(typename El::S* __res
       const S* src = in + t * KK * static_cast<int64_t>(H) + c;
       Vec<S, VEC> x[KK];
 #pragma unroll
-      for (int k = 0; k < KK; ++k) x[k] = load_terms<S, VEC>(src + k * static_cast<int64_t>(H));
+      for (int k = 0; k < KK; ++k) x[k] = load_terms<ONCE, S, VEC>(src + k * static_cast<int64_t>(H));
 #pragma unroll
       for (int k = 0; k < KK; ++k)
 #pragma unroll
         for (int i = 0; i < VEC; ++i) acc[i] += El::ld(x[k].v[i]);
     } else {
       for (int k = 0; k < K; ++k) {
-        const Vec<S, VEC> x = load_terms<S, VEC>(in + (t * K + k) * static_cast<int64_t>(H) + c);
+        const Vec<S, VEC> x = load_terms<ONCE, S, VEC>(in + (t * K + k) * static_cast<int64_t>(H) + c);
 #pragma unroll
         for (int i = 0; i < VEC; ++i) acc[i] += El::ld(x.v[i]);
       }
@@ -219,13 +217,24 @@ int launch_sum(void* out, const void* in, int64_t T, int K, int H, hipStream_t s
     // and 3.4, 741 rows 3.5 and 3.8, 8448 rows (277 MB) 47.9 and 48.7, 16896 rows 93.1 and 94.8.  4 and 8 terms have an
     // instance.  2 would gain next to nothing by one (64 rows 2.13 and 2.24, 8448 rows 16.5 and 16.4); 6 would gain half a
     // microsecond where rows are few (64 rows 2.23 and 2.80, 741 rows 3.01 and 3.36, 8448 rows 36.2 and 36.0).
-    // A workgroup for every 256 vectors (16896 rows 93.1 us; 4096 workgroups that stride on 97.6).
-    auto kern = K == 8 ? moe_sum_kernel<El, V, 8> : K == 4 ? moe_sum_kernel<El, V, 4> : moe_sum_kernel<El, V, 0>;
+    //
+    // Past the caches, and a workgroup for every 256 vectors instead of 4096 that stride on, where the terms are more than
+    // the memory-side cache still holds of what has just been written.  Behind a kernel that writes them, us, through the
+    // caches and past them: 8 terms of 2048, 1024 rows (34 MB) 7.4 and 7.8, 4096 (134 MB) 26.3 and 23.4, 8448 (277 MB)
+    // 52.8 and 33.4, 16896 (554 MB) 116 and 94; 4 of 2048 (68 to 277 MB) 13.1 and 13.9, 26.8 and 24.0, 56.9 and 40.0; 6 of
+    // 4096, 101 MB 18.2 and 18.3.  A row that is no whole number of 128-byte lines has its ends fetched twice that way:
+    // 6 of 1000, 101 MB 19.5 and 23.2, 203 MB 32.7 and 31.0, 8 of 1000, 135 MB 24.0 and 26.6, 270 MB 51.3 and 34.3.
+    const int64_t bytes = T * K * static_cast<int64_t>(H) * static_cast<int64_t>(sizeof(S));
+    const bool once = bytes > (H * static_cast<int64_t>(sizeof(S)) % 128 ? int64_t{190} << 20 : int64_t{120} << 20);
     const int64_t want = (T * (H / V) + kThreads - 1) / kThreads;
-    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(want < (1 << 22) ? want : 1 << 22)), dim3(kThreads), 0, s,
-                       static_cast<S*>(out), static_cast<const S*>(in), T, K, H);
+    const unsigned grid = once ? static_cast<unsigned>(want < (1 << 22) ? want : 1 << 22) : grid_for(T * (H / V));
+    auto go = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3(grid), dim3(kThreads), 0, s, static_cast<S*>(out), static_cast<const S*>(in), T, K, H);
+    };
+    if (once) go(K == 8 ? moe_sum_kernel<El, V, 8, true> : K == 4 ? moe_sum_kernel<El, V, 4, true> : moe_sum_kernel<El, V, 0, true>);
+    else go(K == 8 ? moe_sum_kernel<El, V, 8, false> : K == 4 ? moe_sum_kernel<El, V, 4, false> : moe_sum_kernel<El, V, 0, false>);
   } else {
-    hipLaunchKernelGGL((moe_sum_kernel<El, 1, 0>), dim3(grid_for(T * H)), dim3(kThreads), 0, s,
+    hipLaunchKernelGGL((moe_sum_kernel<El, 1, 0, false>), dim3(grid_for(T * H)), dim3(kThreads), 0, s,
                        static_cast<S*>(out), static_cast<const S*>(in), T, K, H);
   }
   return moe_check_launch("moe_sum");

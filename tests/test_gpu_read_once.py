@@ -7,7 +7,12 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("T,K,H,dtype", [(4099, 8, 2048, torch.bfloat16), (16385, 4, 520, torch.float16),
-                                         (9001, 3, 1032, torch.bfloat16), (2100, 8, 1028, torch.float32)])
+                                         (9001, 3, 1032, torch.bfloat16), (2100, 8, 1028, torch.float32),
+                                         # on both sides of the lines from which the terms are read past the caches
+                                         (7680, 8, 1024, torch.bfloat16), (7681, 8, 1024, torch.bfloat16),
+                                         (15500, 4, 1024, torch.float16), (9001, 7, 1024, torch.bfloat16),
+                                         (12000, 8, 1000, torch.float16), (17000, 6, 1000, torch.bfloat16),
+                                         (12500, 4, 1000, torch.float32), (13100, 3, 1024, torch.float32)])
 def test_combine_of_many_rows(moe, dev, T, K, H, dtype):
     g = torch.Generator(dev).manual_seed(T)
     rows = torch.empty(T, K, H, dtype=dtype, device=dev)
