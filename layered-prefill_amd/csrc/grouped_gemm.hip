@@ -1660,6 +1660,12 @@ __device__ __forceinline__ void stream_store(const GemmParams& p, const float (&
 // of weights in rotation, without the hint, on all weights and as it is, us: 2 tokens (few.hip) 37.5 and 33.7; 9 62.5 and
 // 58; 16 77 / 70 / 70; 32 100 / 92 / 93; 64 113 / 106 / 101; 128 141 / 140 / 131; 192 161 / 163 / 153; 240 (tiled) 175 /
 // 184 / 172; 32 experts, 301 tokens 116 / 122 / 116; e4m3, 100 tokens 80 / 77 / 75, 250 109 / 113 / 107.
+// "One block" is of the whole call: with the blocks outside a group of four left out of account, the last block of a longer
+// run went past the caches, too: 16 experts, H 2880, I 1440, 600 tokens top-2 172 and 168.6; 8, H 1024, I 512, 2048 tokens
+// 54.2 and 51.5; 4, H 2048, I 768, 256 tokens 32.9 and 27.2; 32, 301 tokens with biases 112.8 and 110.4.
+// Weights that the 256 MB memory-side cache holds from call to call, one layer run again and again or a model that small, do
+// not stay there with the hint: one set of weights again and again, without and with it, 32 experts, 32 tokens 47 and 56; 16,
+// H 2048, I 768, 256 tokens top-4 50 and 57; 128 experts, 64 tokens 117 and 98.
 // e4m3 runs here too (100 tokens of that layer: gate-up 45.6 -> 40.1 us, down 40.9 -> 25.9 us
 // against the register-staged kernel, whose two stages hold 36 KB per workgroup and drain at every K tile), its scales
 // fetched ahead of the stream like the routed weights.  Rows need whole 32-byte steps, not whole units.
@@ -1741,6 +1747,7 @@ __global__ __launch_bounds__(kThreads, 3) void stream_gemm_kernel(
   // read one weight tile then start back to back on one XCD and the second
   // to g-th find the lines in L2 (or already requested).
   int e, g;
+  bool alone;  // nobody else reads these weights
   [[maybe_unused]] int in_expert = 0;  // ALIGN: the block's number among its expert's
   if constexpr (ALIGN) {
     // the expert whose blocks hold mb: its lane, then which of the lane's four
@@ -1762,11 +1769,15 @@ __global__ __launch_bounds__(kThreads, 3) void stream_gemm_kernel(
     nt = g == 1 ? li : static_cast<int>(__umulhi(li, g == 2 ? 0x80000000u : g == 3 ? 0x55555556u : 0x40000000u));  // li / g
     mb = lo + (li - nt * g);
     in_expert = mb - first;
+    alone = mine_nb == 1;
   } else {
     const int q0 = mb & ~3, me = mb & 3;
     int eq[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) eq[i] = uniform_load(expert_ids + (q0 + i < live_mb ? q0 + i : live_mb - 1));
+    // (and the blocks on either side of the four, where an expert's run may go on)
+    const int before = uniform_load(expert_ids + (q0 > 0 ? q0 - 1 : 0));
+    const int behind = uniform_load(expert_ids + (q0 + 4 < live_mb ? q0 + 4 : live_mb - 1));
     uint32_t links = 0;  // bit i: blocks i and i + 1 of the group belong to one expert
 #pragma unroll
     for (int i = 0; i < 3; ++i) links |= (q0 + i + 1 < live_mb && eq[i] == eq[i + 1]) ? 1u << i : 0u;
@@ -1776,8 +1787,8 @@ __global__ __launch_bounds__(kThreads, 3) void stream_gemm_kernel(
     const int li = (me - lo) * num_n_tiles + nt;
     nt = g == 1 ? li : static_cast<int>(__umulhi(li, g == 2 ? 0x80000000u : g == 3 ? 0x55555556u : 0x40000000u));  // li / g
     mb = q0 + lo + (li - nt * g);
+    alone = g == 1 && !(lo == 0 && q0 > 0 && before == e) && !(hi == 3 && q0 + 4 < live_mb && behind == e);
   }
-  const bool alone = g == 1;  // nobody else here reads these weights (or hardly: a run may go on in the next four blocks)
   const int n0 = nt * BN_OUT;
 
   // second round trip, scalar: the block's slots and the eight whose token rows this wavefront requests.  The first
