@@ -60,6 +60,9 @@ void moe_experts_x_codes(const MoeFusedExpertsArgs* a, uint8_t** codes, float** 
 int moe_fused_experts_of_codes(const MoeFusedExpertsArgs* a, bool x_coded, const int32_t* ids);
 bool moe_experts_align(const MoeFusedExpertsArgs* a);
 
+// moe_sum of terms that a layer's down pass has just written (`in_layer`) or of a caller's own.
+int moe_sum_terms(void* out, const void* in, int64_t T, int K, int H, int dtype, bool in_layer, void* stream);
+
 // A layer call of a few tokens in two launches, where it is one that they serve (few.hip); false, and nothing enqueued,
 // elsewhere.  `experts` holds E + 1 ids, `inter` T * K rows.  `rc` is the launches' status.
 bool moe_layer_few(const MoeLayerArgs* a, float* topk_w, int32_t* topk_ids, int32_t* experts, void* inter, int* rc);

@@ -2548,7 +2548,7 @@ int moe_fused_experts_of_codes(const MoeFusedExpertsArgs* a, bool x_coded, const
                                     : launch_big_fused<MmaF16>(p, p2, a->block_size, cap, plan_done, status, shift, s);
       if (rc) return rc;
       if (!(passes & 4)) return MOE_OK;
-      return moe_sum(a->out, c3, a->T, a->K, a->H, a->act_dtype, a->stream);
+      return moe_sum_terms(a->out, c3, a->T, a->K, a->H, a->act_dtype, true, a->stream);
     }
   }
   if (fp8 && (passes & 1)) {
@@ -2590,6 +2590,6 @@ int moe_fused_experts_of_codes(const MoeFusedExpertsArgs* a, bool x_coded, const
 
   // top-k combine (nanovllm/layers/for_moe/moe_easy_kernel.py:26-31)
   if (!(passes & 4)) return MOE_OK;
-  return moe_sum(a->out, c3, a->T, a->K, a->H, a->act_dtype, a->stream);
+  return moe_sum_terms(a->out, c3, a->T, a->K, a->H, a->act_dtype, true, a->stream);
 }
 
