@@ -40,18 +40,36 @@ def test_alignment_at_the_seams(moe, oracle, dev, numel, E, block, kind):
     assert all(torch.equal(a.cpu(), b) for a, b in zip(got, want))
 
 
-@pytest.mark.parametrize("numel", [1030, 6000, 16384, 20000, 100000])
-def test_plan_of_many_workgroups_is_that_of_the_ids(moe, dev, numel):
-    """The expert passes on a plan that the alignment left, and on the one that they make from the aligned ids."""
-    E, K, H, I = 64, 2, 256, 128
-    T = numel // K
+@pytest.mark.parametrize("E,K", [(64, 2), (200, 1), (3, 1)])
+@pytest.mark.parametrize("numel", [1030, 6000, 8194, 12000, 16384, 20000, 100000])
+def test_plan_of_many_workgroups_is_that_of_the_ids(moe, dev, numel, E, K):
+    """The expert passes on a plan that the alignment left in a workspace of other contents, and on the one that they make
+    from the aligned ids: the same ranges, the same bits."""
+    print(numel, E, K, flush=True)
+    fm = moe.fused_moe
+    H, I, T = 256, 128, numel // K
     g = torch.Generator(dev).manual_seed(numel)
     x = torch.empty(T, H, dtype=torch.bfloat16, device=dev).normal_(0, 1, generator=g)
     w13 = torch.empty(E, 2 * I, H, dtype=torch.bfloat16, device=dev).normal_(0, 0.05, generator=g)
     w2 = torch.empty(E, H, I, dtype=torch.bfloat16, device=dev).normal_(0, 0.05, generator=g)
     ids = _ids(T * K, E, "skewed").view(T, K).to(dev)
     tw = torch.rand(T, K, device=dev)
-    out = moe.fused_experts(x, w13, w2, None, None, tw, ids)
+    code = moe._lib.DTYPE_CODE[torch.bfloat16]
+    size = fm.fused_experts_workspace_bytes(T, H, I, E, K, 256, torch.bfloat16)
+    out, ranges = [], []
+    for planned in (True, False):
+        ws = torch.full((size,), 0x5a, dtype=torch.uint8, device=dev)
+        plan = fm._plan_in_workspace(ws, T, H, I, E, K, 256, code, code, T * K)
+        assert plan is not None
+        so, eo, npp = fm._align_block_size(ids, 256, E, plan if planned else None)
+        out.append(torch.full_like(x, float("nan")))
+        args = fm.launch_fused_experts(x, out[-1], w13, w2, None, None, None, None, tw, so, eo, npp, 256, workspace=ws,
+                                       passes=16 if planned else 0)
+        fm.fused_experts_status(args)
+        at = plan[0] - ws.data_ptr()
+        ranges.append(ws[at:at + 36].clone().view(torch.int32).tolist())
+    assert ranges[0] == ranges[1] and ranges[0][0] == 0 and ranges[0][8] == npp.item() // 256
+    assert bool(out[1].isfinite().all()) and torch.equal(out[0], out[1])
     want = torch.zeros(T, H, device=dev)
     for k in range(K):   # one expert at a time, fp32 from the same bf16 inputs
         for e in range(E):
@@ -61,7 +79,7 @@ def test_plan_of_many_workgroups_is_that_of_the_ids(moe, dev, numel):
                 h = (torch.nn.functional.silu(gu[:, :I]) * gu[:, I:]).bfloat16().float()
                 want[rows] += tw[rows, k, None] * (h @ w2[e].float().t())
     # roundings of the intermediate, of each term and of the sum: 3 of 2^-9 relative, sums of 128 and 256 products in fp32
-    err = (out.float() - want).norm() / want.norm()
+    err = (out[0].float() - want).norm() / want.norm()
     assert err < 3 * 2 ** -8
 
 

@@ -39,16 +39,49 @@ def test_two_tiles_a_workgroup_have_the_bits_of_one(moe, dev, T, E, K, H, I, dty
         assert torch.equal(moe.fused_experts(x, w13, w2, None, None, tw, ids, **kw), want)
 
 
-def test_e4m3_tiles_in_pairs_against_smaller_calls(moe, dev):
+@pytest.mark.parametrize("T,E,K,H,I,on_input", [
+    (26000, 4, 1, 4096, 256, False),
+    (29200, 4, 2, 1792, 256, False),   # seven n-tiles: the last of a block has no partner
+    (26000, 4, 1, 4096, 256, True),
+])
+def test_e4m3_tiles_in_pairs_against_smaller_calls(moe, dev, T, E, K, H, I, on_input):
     """e4m3 takes no biases: the same rows in calls below the line."""
-    T, E, K, H, I = 26000, 4, 1, 4096, 256
+    print(T, E, K, H, I, on_input, flush=True)
     x, w13, w2, tw, ids, _ = _args(moe, dev, T, E, K, H, I, torch.bfloat16, False, 0.2)
     q13, s13, q2, s2 = moe.quantize_expert_weights(w13, w2)
-    run = lambda a, b: moe.fused_experts(x[a:b], q13, q2, None, None, tw[a:b], ids[a:b], w1_scale=s13, w2_scale=s2)
+    run = lambda a, b: moe.fused_experts(x[a:b], q13, q2, None, None, tw[a:b], ids[a:b], w1_scale=s13, w2_scale=s2,
+                                         apply_router_weight_on_input=on_input)
     whole = run(0, T)
     assert bool(whole.isfinite().all()) and float(whole.float().abs().max()) > 0
-    parts = torch.cat([run(a, a + 6500) for a in range(0, T, 6500)])
+    part = T // 4
+    assert moe._lib.lib().moe_call_block_size(part, H, I, E, K, 2, 3, 0) == 256
+    parts = torch.cat([run(a, a + part) for a in range(0, T, part)])
     assert torch.equal(whole, parts)
+
+
+@pytest.mark.parametrize("T,E,K,H,I,dtype,tiled,skew", [_CASES[0], _CASES[1], _CASES[2]])
+@pytest.mark.parametrize("on_input", [False, True])
+def test_pairs_in_launches_of_their_own_and_across_xcds(moe, dev, T, E, K, H, I, dtype, tiled, skew, on_input):
+    """The passes as two launches, one by one, and as one whose every hand-off crosses XCDs: the bits of one tile a workgroup."""
+    print(T, E, K, H, I, dtype, tiled, on_input, flush=True)
+    fm = moe.fused_moe
+    x, w13, w2, tw, ids, kw = _args(moe, dev, T, E, K, H, I, dtype, tiled, skew)
+    b13, b2 = torch.zeros(E, 2 * I, dtype=dtype, device=dev), torch.zeros(E, H, dtype=dtype, device=dev)
+    so, eo, npp = fm.moe_align_block_size(ids, 256, E)
+
+    def run(passes, b13=None, b2=None):
+        out, ws = torch.full_like(x, float("nan")), None
+        for p in passes:
+            args = fm.launch_fused_experts(x, out, w13, w2, b13, b2, None, None, tw, so, eo, npp, 256, workspace=ws, passes=p,
+                                           apply_router_weight_on_input=on_input, **kw)
+            ws = args._keepalive[0]
+        fm.fused_experts_status(args)
+        return out
+
+    want = run([7 | 8], b13, b2)
+    assert bool(want.isfinite().all()) and float(want.float().abs().max()) > 0
+    for passes in ([0], [7 | 8], [1, 2, 4], [7 | 32], [7 | 32]):
+        assert torch.equal(run(passes), want), passes
 
 
 def test_expired_wait_of_a_pair_is_nan_or_right(moe, dev):

@@ -6,10 +6,15 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("T,E,K,H,I,dtype,logits", [
-    (1, 32, 4, 64, 64, "bfloat16", None),        # routed and aligned in one launch
-    (16, 128, 8, 2048, 128, "float16", None),    # the most logits of it, a whole workgroup of rows
-    (17, 64, 2, 2064, 64, "bfloat16", None),     # rows of more than 2048 columns
-    (17, 128, 8, 2048, 64, "bfloat16", None),    # one row too many: the router's launch
+    (1, 32, 4, 64, 64, "bfloat16", None),        # the router's launch, as wherever the gate-up pass aligns
+    (16, 128, 8, 2048, 128, "float16", None),    # the widest rows of its narrower instance
+    (17, 128, 8, 2048, 64, "bfloat16", None),
+    # beside routing and alignment in one launch: up to 2048 logits, rows that are no whole 32 bytes
+    (1, 32, 4, 2000, 64, "bfloat16", None),      # one row, up to 2048 columns
+    (16, 128, 8, 2000, 128, "float16", None),    # the most logits of it, a whole workgroup of rows
+    (17, 64, 2, 2064, 64, "bfloat16", None),     # rows of more than 2048 columns, a second workgroup of them
+    (8, 256, 8, 4080, 64, "float16", None),      # the widest rows
+    (33, 64, 2, 2000, 64, "bfloat16", None),     # one row too many: the router's launch
     (33, 16, 2, 4096, 64, "float16", None),
     (130, 256, 4, 2064, 64, "bfloat16", None),
     (700, 8, 2, 256, 128, "bfloat16", None),     # experts without an instance
