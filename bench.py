@@ -58,12 +58,15 @@ def measured_traffic(workload: str, kernel: str, grid: int):
 
 def one_launch_grid(layer) -> int:
     """Workgroups of the one-launch kernel for this layer: 8 XCDs x the longest m-block
-    range the plan may give an XCD x (gate-up + down n-tiles)."""
+    range the plan may give an XCD x (gate-up + down n-tiles); where the down pass takes
+    pairs of n-tiles its list has places for whole groups of four blocks."""
     s = layer.shape
     cap = layer.T * s.top_k + s.experts * (layer.bm - 1)
     mbs = -(-cap // 256)
     cap_mb = min(2 * -(-mbs // 8), mbs)
-    return 8 * cap_mb * (-(-s.intermediate // 128) + -(-s.hidden // 256))
+    down_tiles = -(-s.hidden // 256)
+    pairs = s.hidden % 256 == 0 and down_tiles > 1 and layer.T * s.top_k * down_tiles >= 240000
+    return 8 * (cap_mb * -(-s.intermediate // 128) + (-(-cap_mb // 4) * 4 if pairs else cap_mb) * down_tiles)
 
 
 def _events(n):

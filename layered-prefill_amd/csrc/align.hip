@@ -976,11 +976,13 @@ static int launch_route_align_tiny(const void* logits, int dtype, float* topk_w,
 bool moe_layer_route_align(const void* logits, int dtype, float* topk_w, int T, int E, int K, int renormalize, int block_size,
                            int32_t* sorted_ids, int64_t sorted_cap, int32_t* expert_ids, int64_t expert_cap, int32_t* npp,
                            const MoeXCodes* xc, hipStream_t s, int* rc) {
-  // One CU routes all rows: with up to half its wavefronts at work that costs less than a launch and a trip of the ids
-  // through memory, with more of them the rows queue up.  Whole layer, us, against the two launches: E 128, H 2048,
-  // I 768, top-8: 26.0 and 27.1 at 1 token, 52.4 and 53.0 at 9, 60.4 and 60.9 at 16, but 71.5 and 71.1 at 24, 92.6 and
-  // 91.5 at 32; E 64: 74.9 and 75.6 at 32, 97.6 and 96.7 at 64; E 32, I 1024, top-4: 23.1 and 24.0 at 1, 61.4 and 61.9 at
-  // 64, 74.7 and 74.3 at 128.
+  // Calls whose gate-up pass does not align for itself come here: a block size of the caller's own, rows that are no whole 32
+  // bytes or not 16-byte aligned, fp32.  One CU routes all rows: with up to half its wavefronts at work that costs less than
+  // a launch and a trip of the ids through memory, with more of them the rows queue up.  Whole layer with blocks of 32 of the
+  // caller's own, four sets of weights in rotation, us, against the two launches: E 128, H 2048, I 768, top-8: 26.9 and 28.1
+  // at 1 token, 54.6 and 55.3 at 9, 58.6 and 59.2 at 16; E 64: 52.1 and 53.5 at 8, 76.0 and 75.9 at 32; E 32, I 1024, top-4:
+  // 28.0 and 29.4 at 1, 66.8 and 67.9 at 64.  With the codes of x (e4m3, E 64, H 2064, I 256, top-4), against routing with the
+  // codes and alignment: 46.3 and 47.4 at 1 token, 49.4 and 50.4 at 8, 52.1 and 52.9 at 32.
   if (static_cast<int64_t>(T) * E > 2048 || static_cast<int64_t>(T) * K > kTinyNumel || K > E || K < 1 || block_size > 64 || !logits || sorted_cap > INT32_MAX ||
       expert_cap > INT32_MAX || (dtype != MOE_BF16 && dtype != MOE_F16 && dtype != MOE_F32))
     return false;

@@ -61,12 +61,15 @@ __device__ __forceinline__ int nth_set(const uint64_t (&m)[W], int rank) {
 // them go here: every workgroup of the gate-up pass routes the few rows by itself, so that neither a launch nor a trip of
 // ids through memory stands in front of the weights, and nothing is aligned; and a workgroup of the down pass has all terms
 // of its columns' sums.  The weights are cut evenly: a CU's share of a pass is within one wavefront's unit of every other's.
-// Whole layer, us, replayed from a graph, against routing with alignment, two streaming passes and the combine; one set of
-// weights again and again, and four in rotation:
-//   E 128, H 2048, I 768, top-8, tiled: 1 token 25.0 -> 20.8 and 28.2 -> 22.5; 2 31.8 -> 27.0 and 37.6 -> 30.3; 9 52.8 ->
-//   48.3 and 59.9 -> 54.4; 12 55.2 -> 51.7 and 62.7 -> 57.2; 16 59.0 -> 61.4 and 67.1 -> 63.9
-//   E 64, H 1024, I 384, top-4, tiled: 1 token 17.2 -> 10.6, 5 18.0 -> 12.1, 16 20.5 -> 18.2 (one set)
-//   E 32, H 4096, I 1024, top-8: 1 token 41.0 -> 45.0 and 54.6 -> 50.6; 4 106.4 -> 103.4 and 109.7 -> 107.2
+// Whole layer, us, replayed from a graph, against routing with alignment, two streaming passes and the combine (all of them
+// with the weights asked for once, lds_dma16<true>); one set of weights again and again, and four in rotation:
+//   E 128, H 2048, I 768, top-8, tiled: 1 token 26.3 -> 19.1 and 27.6 -> 21.5; 2 33.2 -> 25.7 and 34.3 -> 28.0; 9 50.7 ->
+//   45.4 and 53.4 -> 48.5; 12 57.8 -> 55.1 and 57.6 -> 56.0
+//   E 64, H 1024, I 384, top-4, tiled: 1 token 18.3 -> 10.9 and 18.6 -> 12.4, 16 21.8 -> 17.8 and 20.6 -> 17.5
+//   E 32, H 4096, I 1024, top-8: 1 token 46.1 -> 41.5 and 47.4 -> 44.1; 4 83.4 -> 77.4 and 85.9 -> 79.6; 12 108.5 -> 106.4
+//   and 114.5 -> 112.8
+// (Weights that stay in the memory-side cache would come faster without the hint: that layer at 1 token 40.2 with one set,
+// 54.1 with six in rotation, where it takes 42.7 and 45.2 here.)
 // The line (moe_layer_few) is T * K <= 96: beyond, experts with more than eight tokens become common, whose weights the
 // down pass goes through twice.
 //

@@ -2065,6 +2065,8 @@ static int big_plan_cap(int64_t sorted_cap) {
 //   e4m3, the first layer: 32000 rows 341.0 and 342.5; 67584 558.3 and 543.7; 135168 1040.5 and 996.8
 // Four tiles a workgroup lose again (67584 rows 795 us), and so do pairs of the gate-up pass, whose start is a smaller part
 // of a tile and whose products run at the clock that the board's power leaves, bubbles or not (67584 rows 825 against 804).
+// Calls with biases keep a tile a workgroup: a pair carries what its second tile's epilogue needs of its weight rows in a
+// register a thread, and only e4m3's scales, which come without biases, have one.
 static void set_chain(GemmParams& p, int es) {
   const int64_t line = es == 1 ? 400000 : 240000;
   p.chain = p.xcd_bounds && !p.bias && p.N % kBigBNW == 0 && p.ldc % 8 == 0 && p.num_n_tiles > 1 &&

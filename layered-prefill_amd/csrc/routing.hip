@@ -38,7 +38,7 @@ __global__ __launch_bounds__(kWave* kWavesPerBlock) void topk_softmax_pow2_kerne
 // The same with the e4m3 codes of x beside it, which wait for nothing either: the first `route_blocks` workgroups route,
 // the others quantise a row per wavefront.  One launch less, and the router, a chain of latencies, hides behind a copy's
 // traffic.  Whole layer, us, 128 experts, H 2048, I 768, top-8, with the codes in a launch of their own and here: 1 token
-// 25.3 and 23.2 (beside routing and alignment, align.hip), 20 46.4 and 43.6, 100 72.6 and 69.5, 8448 543 and 536.
+// 24.6 and 22.7, 16 40.3 and 38.2, 100 69.7 and 67.5, 741 155.5 and 152.4, 8448 539 and 528.
 template <int E, typename El, int NV>
 __global__ __launch_bounds__(kWave* kWavesPerBlock) void topk_softmax_quant_kernel(
     const typename El::S* __restrict__ gating, float* __restrict__ topk_w, int32_t* __restrict__ topk_ids, int T, int K,
