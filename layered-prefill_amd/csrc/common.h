@@ -214,11 +214,10 @@ struct ElemF16 {
 // so that no other operation is fused.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ float moe_expf(float x) {
-  if (x != x) return x;
-  if (x > 88.0f) return __builtin_inff();
-  if (x < -104.0f) return 0.0f;
-  float n = __builtin_rintf(x * 1.44269504088896341f);
-  float r = __builtin_fmaf(n, -0.693359375f, x);
+  // (no branches: the ends of the range are put in at the end)
+  const float in = __builtin_fminf(__builtin_fmaxf(x, -104.0f), 88.0f);
+  float n = __builtin_rintf(in * 1.44269504088896341f);
+  float r = __builtin_fmaf(n, -0.693359375f, in);
   r = __builtin_fmaf(n, 2.12194440e-4f, r);
   float p = 1.9875691500e-4f;
   p = __builtin_fmaf(p, r, 1.3981999507e-3f);
@@ -229,12 +228,13 @@ __device__ __forceinline__ float moe_expf(float x) {
   float r2 = r * r;
   p = __builtin_fmaf(p, r2, r);
   p = p + 1.0f;
-  int32_t ni = static_cast<int32_t>(n);
-  if (ni < -125) {
-    const float t = __uint_as_float(__float_as_uint(p) + (static_cast<uint32_t>(ni + 64) << 23));
-    return t * 5.42101086242752217e-20f;  // 2^-64
-  }
-  return __uint_as_float(__float_as_uint(p) + (static_cast<uint32_t>(ni) << 23));
+  const int32_t ni = static_cast<int32_t>(n);
+  const bool small = ni < -125;
+  const float y = __uint_as_float(__float_as_uint(p) + (static_cast<uint32_t>(small ? ni + 64 : ni) << 23));
+  float e = small ? y * 5.42101086242752217e-20f : y;  // 2^-64
+  e = x < -104.0f ? 0.0f : e;
+  e = x > 88.0f ? __builtin_inff() : e;
+  return x != x ? x : e;
 }
 
 __device__ __forceinline__ float moe_silu(float x) { return x / (1.0f + moe_expf(-x)); }
