@@ -19,6 +19,7 @@
 
 #include "common.h"
 #include "gemm_device.h"
+#include "quant_device.h"
 
 
 namespace {
@@ -2014,6 +2015,218 @@ __global__ __launch_bounds__(kThreads, 3) void stream_gemm_kernel(
   }
 }
 
+// Down pass of a streaming e4m3 call that makes its tokens' codes itself: the intermediate comes in the activation dtype, and
+// neither a launch in front that quantises it nor its codes' and scales' way through memory is left.  Rows are short (NU units
+// of 128 codes), so that the codes of a block of 32 slots stay in LDS and a wavefront streams weight rows, sixteen at a time, on
+// its own: no barrier but one per block.  One workgroup to a CU takes an equal share of the (block, sixteen rows) groups, NW
+// wavefronts of it a group each (as many as make 96 KB of rings); a wavefront's next group is asked for, unit by unit, as the
+// present one is multiplied, so that only a share's start waits for memory.  Products, their order and every rounding are
+// stream_gemm_kernel's and the quantiser's.  It is bound by the weights, those of an expert with several blocks once a block:
+// 100 tokens of 128 experts, H 2048, I 768, top-8: 22 us and 5 of quantisation in front, 24 this way.  (With a workgroup for 64
+// rows of a block, as in stream_gemm_kernel, all its weights asked for at once, 33: the start of a workgroup, 7 us, once every
+// 48 KB.)  Whole layer with the norm, quantised in front and here, us: 24 tokens of that layer 47.6 and 46.1, 64 60.7 and 59.2,
+// 100 69.4 and 68.4, 300 105.1 and 102.8; 64 experts, H 1024, I 384, top-6: 120 tokens 31.7 and 29.4; 16 experts, 2200 94.8 and
+// 81.1; 32 experts, H 4096, I 512, top-4, 300 tokens 74.0 and 70.8; 16, H 2880, I 512, 1400 top-2 87.1 and 84.5.
+constexpr int kCdCus = 256;
+template <typename Mma, int NU, int NW>
+__global__ __launch_bounds__(NW * kWave, 1) void stream_codes_kernel(
+    const int32_t* __restrict__ head, const int32_t* __restrict__ expert_ids, const int32_t* __restrict__ sorted_ids,
+    int groups_per_block, uint32_t groups_rcp, int numel, const GemmParams p) {
+  using El = typename Mma::El;
+  constexpr int kTokUnit = kStBM * kStRowBytes, kCodes = NU * kTokUnit, kStep = 16 * kStRowBytes, kRing = NU * kStep;
+  constexpr int kPairs = (16 + NW - 1) / NW, kVecs = NU / 2 + NU % 2;   // pairs of rows a wavefront quantises; 32 lanes a row
+  extern __shared__ __attribute__((aligned(1024))) char smem[];         // codes of two blocks, then the wavefronts' rings
+  __shared__ float s_as[2][kStBM], s_rw[2][kStBM];
+  __shared__ int s_tok[2][kStBM];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l15 = lane & 15, lq = lane >> 4;
+  const int live_mb = (uniform_load(head) + kStBM - 1) / kStBM;
+  // (neighbouring shares on one XCD)
+  const int64_t groups = static_cast<int64_t>(live_mb) * groups_per_block;
+  const int share = (blockIdx.x % kXcds) * (kCdCus / kXcds) + blockIdx.x / kXcds;
+  const int begin = __builtin_amdgcn_readfirstlane(static_cast<int>(groups * share / kCdCus));
+  const int end = __builtin_amdgcn_readfirstlane(static_cast<int>(groups * (share + 1) / kCdCus));
+  if (begin >= end) return;
+  auto block_of = [&](int g) {
+    int mb = __umulhi(g, groups_rcp);   // g / groups_per_block, or one more
+    if (mb * groups_per_block > g) mb -= 1;
+    return mb;
+  };
+  // the side that asks for weights
+  const char* w_at = nullptr;
+  bool alone = false;   // nobody else reads these weights
+  uint32_t w_off[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int r = 8 * j + (lane >> 3);
+    w_off[j] = static_cast<uint32_t>(r * p.w_stride_n + (((lane & 7) ^ ((r >> 1) & 7)) << 4));
+  }
+  const uint32_t ring = __builtin_amdgcn_readfirstlane(lds_offset_of(smem) + 2 * kCodes + wave * kRing);
+  auto aim = [&](int g) {
+    const int mb = block_of(g);
+    const int e = uniform_load(expert_ids + mb), before = uniform_load(expert_ids + (mb > 0 ? mb - 1 : 0)),
+              behind = uniform_load(expert_ids + (mb + 1 < live_mb ? mb + 1 : mb));
+    alone = !(mb > 0 && before == e) && !(mb + 1 < live_mb && behind == e);
+    w_at = static_cast<const char*>(p.w) + static_cast<int64_t>(e < 0 ? 0 : e) * p.w_stride_e +
+           static_cast<int64_t>(16 * (g - mb * groups_per_block)) * p.w_stride_n;
+  };
+  auto ask = [&](int u) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      if (alone) lds_dma16<true>(w_at + u * kStRowBytes, w_off[j], ring + u * kStep + j * 1024);
+      else lds_dma16(w_at + u * kStRowBytes, w_off[j], ring + u * kStep + j * 1024);
+    }
+  };
+  int g = begin + wave;
+  const bool works = g < end;   // (a wavefront without a group takes part in the quantisation)
+  // codes and scales of block mb, and what the epilogue needs of its slots; `meanwhile` asks for more weights
+  typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
+  const int l31 = lane & 31, vecs = p.Kd / 8;
+  auto code = [&](int mb, int buf, auto older, auto&& meanwhile) {
+    constexpr int kYounger = decltype(older)::value;
+    const int32_t* sid = sorted_ids + static_cast<int64_t>(mb) * kStBM;
+    u32x4 v[kPairs][kVecs];
+    int lo[kPairs], hi[kPairs];   // the rows' slots
+#pragma unroll
+    for (int r = 0; r < kPairs; ++r) {
+      const int pair = (wave + r * NW) & 15;
+      lo[r] = uniform_load(sid + 2 * pair);
+      hi[r] = uniform_load(sid + 2 * pair + 1);
+      const bool used = lane < 32 ? lo[r] < numel : hi[r] < numel;
+      const int64_t row = mb * kStBM + (used ? 2 * pair + (lane >> 5) : 0);   // (of the others nothing is stored)
+      const char* const src = static_cast<const char*>(p.a) + row * p.lda * 2;
+#pragma unroll
+      for (int i = 0; i < kVecs; ++i) {
+        const int c = l31 + 32 * i < vecs ? l31 + 32 * i : 0;
+        asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(v[r][i]) : "v"(src + 16 * c) : "memory");
+      }
+    }
+    meanwhile();
+    float rw_lo[kPairs], rw_hi[kPairs];
+#pragma unroll
+    for (int r = 0; r < kPairs; ++r) {
+      const int32_t* const weights = reinterpret_cast<const int32_t*>(p.topk_w);
+      rw_lo[r] = p.mul_weight && lo[r] < numel ? __builtin_bit_cast(float, uniform_load(weights + lo[r])) : 1.f;
+      rw_hi[r] = p.mul_weight && hi[r] < numel ? __builtin_bit_cast(float, uniform_load(weights + hi[r])) : 1.f;
+    }
+#pragma unroll
+    for (int r = 0; r < kPairs; ++r)
+#pragma unroll
+      for (int i = 0; i < kVecs; ++i)
+        asm volatile("s_waitcnt vmcnt(%1)" : "+v"(v[r][i]) : "n"(kYounger) : "memory");
+#pragma unroll
+    for (int r = 0; r < kPairs; ++r) {
+      const int rr = 2 * ((wave + r * NW) & 15) + (lane >> 5);
+      uint4 q[kVecs];
+#pragma unroll
+      for (int i = 0; i < kVecs; ++i) {
+        q[i] = __builtin_bit_cast(uint4, v[r][i]);
+        if (l31 + 32 * i >= vecs) q[i] = uint4{0, 0, 0, 0};
+      }
+      uint2 codes[kVecs];
+      const float scale = quant_vecs<El, kVecs, 32>(q, codes);
+      if (l31 == 0) {
+        s_as[buf][rr] = scale;
+        s_tok[buf][rr] = lane < 32 ? lo[r] : hi[r];
+        s_rw[buf][rr] = lane < 32 ? rw_lo[r] : rw_hi[r];
+      }
+#pragma unroll
+      for (int i = 0; i < kVecs; ++i) {
+        const int c = l31 + 32 * i;   // the row's eight codes c: half a chunk
+        if (c < vecs)
+          *reinterpret_cast<uint2*>(smem + buf * kCodes + (c >> 4) * kTokUnit + rr * kStRowBytes +
+                                    ((((c >> 1) & 7) ^ ((rr >> 1) & 7)) << 4) + 8 * (c & 1)) = codes[i];
+      }
+    }
+  };
+  int mb = block_of(begin);
+  const int mb0 = mb, mb_end = block_of(end - 1);
+  if (works) {
+    aim(g);
+    ask(0);
+    ask(1);
+  }
+  code(mb, 0, IntTag<2 * (NU - 2)>{}, [&] {
+    if (works)
+#pragma unroll
+      for (int u = 2; u < NU; ++u) ask(u);
+    else wait_vmcnt<0>();
+  });
+  int rd[2];
+#pragma unroll
+  for (int kk = 0; kk < 2; ++kk) rd[kk] = l15 * kStRowBytes + (((4 * kk + lq) ^ ((l15 >> 1) & 7)) << 4);
+  const char* const ring_p = smem + 2 * kCodes + wave * kRing;
+  for (;;) {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    bare_barrier();
+    const int buf = (mb - mb0) & 1;
+    const char* const codes = smem + buf * kCodes;
+    const int stop = end < (mb + 1) * groups_per_block ? end : (mb + 1) * groups_per_block;
+    while (g < stop) {
+      const int next = g + NW;
+      const int n0 = 16 * (g - mb * groups_per_block);
+      const float* const scales = p.w_scale + static_cast<int64_t>(uniform_load(expert_ids + mb)) * p.w_scale_stride_e + n0;
+      const bool more = next < end;
+      if (more) aim(next);
+      f32x4 acc[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[h][r] = 0.f;
+#pragma unroll
+      for (int u = 0; u < NU; ++u) {
+        if (more) wait_vmcnt<2 * (NU - 1)>();
+        else wait_vmcnt<0>();
+        uint4 w[2], x[2][2];
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+          w[kk] = *reinterpret_cast<const uint4*>(ring_p + u * kStep + rd[kk]);
+#pragma unroll
+          for (int h = 0; h < 2; ++h) x[kk][h] = *reinterpret_cast<const uint4*>(codes + u * kTokUnit + h * 16 * kStRowBytes + rd[kk]);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the place is read, the next request may land there
+        if (more) ask(u);
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+          for (int h = 0; h < 2; ++h) acc[h] = Mma::mma16(w[kk], x[kk][h], acc[h]);
+      }
+      // scales of the lane's four rows, through the scalar cache: a vector load would wait for all weights asked for
+      float ws[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        int s[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          s[q] = uniform_load(reinterpret_cast<const int32_t*>(scales) + 4 * q + i);
+          asm volatile("" : "+s"(s[q]));   // (a value to choose, not an address to choose)
+        }
+        const int even = lq & 2 ? s[2] : s[0], odd = lq & 2 ? s[3] : s[1];
+        ws[i] = __builtin_bit_cast(float, lq & 1 ? odd : even);
+      }
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int tok = s_tok[buf][16 * h + l15];
+        if (tok >= numel) continue;
+        const float as = s_as[buf][16 * h + l15], rw = s_rw[buf][16 * h + l15];
+        float o[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          o[i] = acc[h][i];
+          o[i] *= as * ws[i];   // the accumulators back to the units of x . w
+          o[i] *= rw;
+        }
+        stream_store<El, false, MOE_ACT_SILU>(p, o, tok, n0 + 4 * lq);
+      }
+      g = next;
+    }
+    if (mb == mb_end) break;
+    ++mb;
+    code(mb, (mb - mb0) & 1, IntTag<0>{}, [] {});
+  }
+}
+
 template <typename Mma, bool GATED>
 int launch_stream(GemmParams& p, int64_t sorted_cap, hipStream_t s) {
   p.num_m_blocks = static_cast<int>((sorted_cap + kStBM - 1) / kStBM);
@@ -2043,6 +2256,35 @@ int launch_stream(GemmParams& p, int64_t sorted_cap, hipStream_t s) {
   else
     go((stream_gemm_kernel<Mma, GATED, false, GATED>));
   return moe_check_launch(GATED ? "fused_experts (gate-up pass)" : "fused_experts (down pass)");
+}
+
+// Whether the down pass of an e4m3 call codes the intermediate itself (stream_codes_kernel): row lengths that have an instance
+// (the ring of a wavefront is a row long; beyond 768 the codes of two blocks and the rings no longer fit a CU).  With fewer
+// than 128 ids a CU's share is a handful of rows, all asked for at once either way, and the quantisation stands in front of
+// their products: 1 token of 128 experts 25.5 us in front and 25.8 here, 8 tokens 39.6 and 39.6, 16 (128 ids) 44.3 and 44.2.
+constexpr int kCdLeast = 128;
+static bool codes_in_pass(const MoeFusedExpertsArgs* a, int64_t sorted_cap) {
+  return a->block_size == kStBM && static_cast<int64_t>(a->T) * a->K >= kCdLeast && !a->w2_bias && (a->I == 384 || a->I == 512 || a->I == 768) && a->H % 16 == 0 &&
+         (sorted_cap / kStBM + 1) * (a->H / 16) < INT32_MAX / 2 && static_cast<int64_t>(a->H) * a->w2_stride_n < (1LL << 32) - 16384;
+}
+
+template <typename Mma>
+int launch_stream_codes(const GemmParams& p, hipStream_t s) {
+  const int per_block = p.N / 16;
+  const uint32_t rcp = static_cast<uint32_t>((1LL << 32) / per_block + 1);
+  auto go = [&](auto units, auto waves) {
+    constexpr int NU = decltype(units)::value, NW = decltype(waves)::value;
+    constexpr int lds = 2 * NU * kStBM * kStRowBytes + NW * NU * 16 * kStRowBytes;
+    static MoeLdsOptIn flags;
+    auto kernel = stream_codes_kernel<Mma, NU, NW>;
+    if (int rc = moe_opt_in_lds(flags, reinterpret_cast<const void*>(kernel), lds, "fused_experts")) return rc;
+    hipLaunchKernelGGL(kernel, dim3(kCdCus), dim3(NW * kWave), lds, s, p.num_post_pad, p.expert_ids, p.sorted_ids, per_block, rcp,
+                       p.numel, p);
+    return moe_check_launch("fused_experts (quantisation and down pass)");
+  };
+  if (p.Kd == 384) return go(IntTag<3>{}, IntTag<16>{});
+  if (p.Kd == 512) return go(IntTag<4>{}, IntTag<12>{});
+  return go(IntTag<6>{}, IntTag<8>{});
 }
 
 // Polls a down tile of the one-launch form waits for its m-block's gate-up tiles (about a
@@ -2575,7 +2817,10 @@ int moe_fused_experts_of_codes(const MoeFusedExpertsArgs* a, bool x_coded, const
   p.mul_weight = a->apply_router_weight_on_input ? 0 : 1;
   p.xcd_bounds = plan_bounds;
   p.c_tiled = 0; p.a_tiled = inter_tiled ? 1 : 0;
-  if (fp8 && (passes & 2)) {
+  if (fp8 && (passes & 2) && codes_in_pass(a, cap)) {
+    p.w_scale = a->w2_scale; p.w_scale_stride_e = a->H;
+    rc = a->act_dtype == MOE_BF16 ? launch_stream_codes<MmaE4M3<ElemBF16>>(p, s) : launch_stream_codes<MmaE4M3<ElemF16>>(p, s);
+  } else if (fp8 && (passes & 2)) {
     // the activated intermediate is quantised per slot row the same way
     rc = moe_quant_slot_rows_e4m3(inter, a->act_dtype, rows, a->I, reinterpret_cast<uint8_t*>(iq), is,
                                   a->sorted_token_ids, cap, static_cast<int>(numel), a->stream);

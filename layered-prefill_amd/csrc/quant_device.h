@@ -18,19 +18,13 @@ __device__ __forceinline__ uint32_t f32x2_to_e4m3(float a, float b) {
 // the scale stays 2^-100 and the row's codes are simply small.
 constexpr float kMinScale = 7.888609052210118e-31f;  // 2^-100
 
-// A row of up to NV * LPR * 8 columns by LPR lanes of a wavefront: it stays in registers between the amax pass and the
-// conversion, 16 bytes in and 8 bytes out per lane and step.
+// The codes of a row that LPR lanes of a wavefront hold, NV vectors of eight values each (zeros behind its end), and its
+// scale.
 template <typename El, int NV, int LPR>
-__device__ __forceinline__ void quant_row(const typename El::S* __restrict__ row, int lane, int cols, uint8_t* __restrict__ q,
-                                          float* __restrict__ scale) {
-  const uint4* src = reinterpret_cast<const uint4*>(row);
-  const int nvec = cols / 8;
-  uint4 v[NV];
+__device__ __forceinline__ float quant_vecs(const uint4 (&v)[NV], uint2 (&codes)[NV]) {
   float amax = 0.f;
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
-    const int c = lane + i * LPR;
-    v[i] = c < nvec ? src[c] : uint4{0, 0, 0, 0};
     const uint32_t wds[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -40,13 +34,9 @@ __device__ __forceinline__ void quant_row(const typename El::S* __restrict__ row
   }
   amax = row_max<LPR>(amax);
   const float s = amax > 0.f ? fmaxf(amax / 448.f, kMinScale) : 1.f;
-  if (lane == 0) *scale = s;
   const float inv = 1.0f / s;
-  uint2* dst = reinterpret_cast<uint2*>(q);
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
-    const int c = lane + i * LPR;
-    if (c >= nvec) continue;
     const uint32_t wds[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
     uint32_t o[2] = {0, 0};
 #pragma unroll
@@ -54,7 +44,32 @@ __device__ __forceinline__ void quant_row(const typename El::S* __restrict__ row
       o[j >> 1] |= f32x2_to_e4m3(El::ld(static_cast<uint16_t>(wds[j])) * inv,
                                  El::ld(static_cast<uint16_t>(wds[j] >> 16)) * inv)
                    << (16 * (j & 1));
-    dst[c] = uint2{o[0], o[1]};
+    codes[i] = uint2{o[0], o[1]};
+  }
+  return s;
+}
+
+// A row of up to NV * LPR * 8 columns by LPR lanes of a wavefront: it stays in registers between the amax pass and the
+// conversion, 16 bytes in and 8 bytes out per lane and step.
+template <typename El, int NV, int LPR>
+__device__ __forceinline__ void quant_row(const typename El::S* __restrict__ row, int lane, int cols, uint8_t* __restrict__ q,
+                                          float* __restrict__ scale) {
+  const uint4* src = reinterpret_cast<const uint4*>(row);
+  const int nvec = cols / 8;
+  uint4 v[NV];
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int c = lane + i * LPR;
+    v[i] = c < nvec ? src[c] : uint4{0, 0, 0, 0};
+  }
+  uint2 codes[NV];
+  const float s = quant_vecs<El, NV, LPR>(v, codes);
+  if (lane == 0) *scale = s;
+  uint2* dst = reinterpret_cast<uint2*>(q);
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int c = lane + i * LPR;
+    if (c < nvec) dst[c] = codes[i];
   }
 }
 

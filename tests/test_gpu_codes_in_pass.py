@@ -1,0 +1,41 @@
+"""e4m3 down pass that quantises its tokens itself: the bits of the quantisation in a launch of its own, which calls with a
+bias (here of zero) keep, at every row length it serves, few and many blocks a share, blocks that are full and hardly filled."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("T,E,K,H,I,dtype,on_input", [
+    (64, 4, 2, 64, 384, "bfloat16", False),      # the fewest ids; four groups of rows a block, fewer than there are shares
+    (16, 16, 8, 160, 512, "float16", False),     # ten groups a block: wavefronts without one
+    (43, 32, 3, 2048, 768, "bfloat16", False),   # just beyond the line; shares that cross blocks
+    (100, 128, 8, 2048, 768, "bfloat16", True),
+    (300, 8, 2, 1024, 384, "float16", True),     # experts of several blocks
+    (3000, 5, 2, 96, 512, "bfloat16", False),    # many blocks a share, six groups each
+    (2500, 3, 1, 288, 768, "float16", False),
+    (1200, 16, 4, 64, 384, "bfloat16", False),
+])
+def test_codes_made_in_the_down_pass_have_the_bits_of_the_launch(moe, dev, T, E, K, H, I, dtype, on_input):
+    print(T, E, K, H, I, dtype, on_input, flush=True)
+    fm = moe.fused_moe
+    dt = getattr(torch, dtype)
+    g = torch.Generator(dev).manual_seed(T + E + H)
+    draw = lambda *shape, std=1.0: torch.empty(shape, device=dev).normal_(0.0, std, generator=g).to(dt)
+    x = draw(T, H)
+    x[T // 2] = 0   # rows of the intermediate whose scale is 1
+    q13, s13, q2, s2 = moe.quantize_expert_weights(draw(E, 2 * I, H, std=0.05), draw(E, H, I, std=0.05))
+    logits = torch.randn(T, E, generator=g, device=dev) + 2.0 * torch.rand(E, generator=g, device=dev)
+    tw, ids, _ = moe.fused_topk(x, logits, K, True)
+    so, eo, npp = fm.moe_align_block_size(ids, 32, E)
+
+    def run(b2):
+        out = torch.full_like(x, float("nan"))
+        fm.launch_fused_experts(x, out, q13, q2, None, b2, s13, s2, tw, so, eo, npp, 32, "silu", on_input,
+                                weight_code=moe._lib.E4M3_CODE)
+        return out
+
+    want = run(torch.zeros(E, H, dtype=dt, device=dev))
+    assert bool(want.isfinite().all()) and float(want.float().abs().max()) > 0
+    for _ in range(2):
+        assert torch.equal(run(None), want)
