@@ -134,6 +134,26 @@ __device__ __forceinline__ float row_max(float v) {
   }
   return v;
 }
+// The same of integers: an exchange and the comparison are one instruction, as a float's cannot be, whose NaN has to be
+// made quiet in between.
+template <int CTRL>
+__device__ __forceinline__ int dpp_move_bits(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
+}
+template <int TPR>
+__device__ __forceinline__ int row_max_bits(int v) {
+  if constexpr (TPR > 1) v = max(v, dpp_move_bits<0xB1>(v));
+  if constexpr (TPR > 2) v = max(v, dpp_move_bits<0x4E>(v));
+  if constexpr (TPR > 4) v = max(v, dpp_move_bits<0x141>(v));
+  if constexpr (TPR > 8) v = max(v, dpp_move_bits<0x140>(v));
+  if constexpr (TPR > 16) {
+    float a, b;
+    rows_of_16(__builtin_bit_cast(float, v), a, b);
+    v = max(__builtin_bit_cast(int, a), __builtin_bit_cast(int, b));
+  }
+  static_assert(TPR <= 32, "rows of half a wavefront at most");
+  return v;
+}
 // The sum with the association of the xor butterfly from distance TPR / 2 down to 1.
 template <int TPR>
 __device__ __forceinline__ float row_sum(float v) {

@@ -67,54 +67,18 @@ __device__ __forceinline__ void route_row(float (&v)[Pow2Geom<E>::kVpt], int t, 
   for (int i = 0; i < VPT; ++i) v[i] = v[i] * rinv;  // subnormal probabilities are kept, as the reference keeps them
 
   float wsum = 0.f;
-  // One round: the row's largest value, then the lowest of the columns that hold it, from one ballot per value of a
-  // lane.  (Column 0 where none does: all values NaN.  A row of one lane looks for itself.)  Carrying value and column
-  // through every exchange, two of them through the LDS crossbar, was most of the kernel: 128 experts top-8, 1 token
-  // 5.4 -> 3.7 us, 256 tokens 5.9 -> 4.2, 16896 13.4 -> 12.0.
   const int lane = threadIdx.x % kWave, row0 = lane & 31 & ~(TPR - 1);
-  auto round = [&](float& best_out, int& bidx_out) {
-    float best = v[0];
-    uint32_t col = TPR == 1 ? 0u : ~0u;
-#pragma unroll
-    for (int i = 1; i < VPT; ++i) {
-      if constexpr (TPR == 1) {
-        if (v[i] > best) best = v[i], col = i;
-      } else {
-        best = fmaxf(best, v[i]);
-      }
-    }
-    best = row_max<TPR>(best);
-#pragma unroll
-    for (int i = 0; TPR > 1 && i < VPT; ++i) {
-      const uint64_t bal = __ballot(v[i] == best);
-      const uint32_t half = lane & 32 ? static_cast<uint32_t>(bal >> 32) : static_cast<uint32_t>(bal);
-      const uint32_t mine = TPR == 32 ? half : __builtin_amdgcn_ubfe(half, row0, TPR);
-      const uint32_t c = (i / EPL) * (EPL * TPR) + static_cast<uint32_t>(__builtin_ctz(mine)) * EPL + i % EPL;
-      col = min(col, mine ? c : ~0u);
-    }
-    const int bidx = col == ~0u ? 0 : static_cast<int>(col);
-    wsum += best;
-    best_out = best;
-    bidx_out = bidx;
-    // blank the winner in the lane that holds it
-#pragma unroll
-    for (int i = 0; i < VPT; ++i)
-      if (bidx == (i / EPL) * (EPL * TPR) + t * EPL + i % EPL) v[i] = -10000.f;
-  };
   // The rounds are one rolled loop: a kernel that runs through its code once waits for its instructions, too, and sixteen
   // rounds in a row were three quarters of the router's code (128 experts: 10.6 KB and, rolled, 2.6; few_gate_kernel 18.8
-  // and 10.2).  Norm and layer, us, unrolled and rolled, with the exp's range checks as branches and as selects: 1 token
+  // and 10.2 then).  Norm and layer, us, unrolled and rolled, with the exp's range checks as branches and as selects: 1 token
   // 24.4 and 24.0, 9 49.5 and 49.2; 64 and more the same.
   // Lane k of the row keeps winner k (every lane knows it after the round), so that the renormalised weights leave as short
   // coalesced stores; a row of fewer lanes than K writes round by round.
   const bool by_lane = K <= TPR;
   float my_w = 0.f;
   int my_i = 0;
-#pragma unroll 1
-  for (int k = 0; k < K; ++k) {
-    float best;
-    int bidx;
-    round(best, bidx);
+  auto keep = [&](int k, float best, int bidx) {
+    wsum += best;
     if (by_lane) {
       my_w = t == k ? best : my_w;
       my_i = t == k ? bidx : my_i;
@@ -123,6 +87,75 @@ __device__ __forceinline__ void route_row(float (&v)[Pow2Geom<E>::kVpt], int t, 
       topk_w[o] = best;
       topk_ids[o] = bidx;
       if (tok_exp_idx) tok_exp_idx[o] = k * T + row;
+    }
+  };
+  // The bits that a ballot has for this lane's row of lanes.
+  auto row_bits = [&](uint64_t bal) {
+    const uint32_t half = lane & 32 ? static_cast<uint32_t>(bal >> 32) : static_cast<uint32_t>(bal);
+    return TPR == 32 ? half : __builtin_amdgcn_ubfe(half, row0, TPR);
+  };
+  constexpr bool kHeads = VPT == 4 && TPR > 1;   // a lane's columns are four in a row, so that lanes are in their order
+  if (kHeads && !__ballot(v[0] != v[0])) {
+    // Probabilities are not negative, so that their bits compare as they do.  A lane sorts its four, the lower column first
+    // where two are equal, and a round looks at the lanes' largest only: one exchange, the first lane that holds the row's
+    // largest wins and goes on to its next.  A round is a chain of dependent instructions, 0.28 us of it when each looked at
+    // all four values of a lane, and stands in front of everything in a call of few tokens.  Norm and layer, us, that way
+    // and this: 1 token 22.9 and 22.2, 9 48.2 and 47.5, 64 87.8 and 87.4, 128 116.7 and 116.3.
+    int h[4], which[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) h[i] = __builtin_bit_cast(int, v[kHeads ? i : 0]), which[i] = i;
+#pragma unroll
+    for (int pass = 0; pass < 4; ++pass)
+#pragma unroll
+      for (int i = pass & 1; i + 1 < 4; i += 2) {   // (neighbours only, and never equal ones: the order of equals stays)
+        const bool swap = h[i] < h[i + 1];
+        const int hi = swap ? h[i + 1] : h[i], lo = swap ? h[i] : h[i + 1];
+        const int wi = swap ? which[i + 1] : which[i], wl = swap ? which[i] : which[i + 1];
+        h[i] = hi, h[i + 1] = lo, which[i] = wi, which[i + 1] = wl;
+      }
+    uint32_t order = which[0] | which[1] << 2 | which[2] << 4 | which[3] << 6;
+#pragma unroll 1
+    for (int k = 0; k < K; ++k) {
+      const int best = row_max_bits<TPR>(h[0]);
+      const uint32_t at = __builtin_ctz(row_bits(__ballot(h[0] == best)));
+      const uint32_t low = __builtin_amdgcn_ubfe(row_bits(__ballot((order & 1) != 0)), at, 1);
+      const uint32_t high = __builtin_amdgcn_ubfe(row_bits(__ballot((order & 2) != 0)), at, 1);
+      keep(k, __builtin_bit_cast(float, best), static_cast<int>(4 * at + 2 * high + low));
+      const bool won = t == static_cast<int>(at);
+      h[0] = won ? h[1] : h[0];
+      h[1] = won ? h[2] : h[1];
+      h[2] = won ? h[3] : h[2];
+      h[3] = won ? -1 : h[3];
+      order = won ? order >> 2 : order;
+    }
+  } else {
+    // One round: the row's largest value, then the lowest of the columns that hold it, from one ballot per value of a
+    // lane.  (Column 0 where none does: all values NaN.  A row of one lane looks for itself.)
+#pragma unroll 1
+    for (int k = 0; k < K; ++k) {
+      float best = v[0];
+      uint32_t col = TPR == 1 ? 0u : ~0u;
+#pragma unroll
+      for (int i = 1; i < VPT; ++i) {
+        if constexpr (TPR == 1) {
+          if (v[i] > best) best = v[i], col = i;
+        } else {
+          best = fmaxf(best, v[i]);
+        }
+      }
+      best = row_max<TPR>(best);
+#pragma unroll
+      for (int i = 0; TPR > 1 && i < VPT; ++i) {
+        const uint32_t mine = row_bits(__ballot(v[i] == best));
+        const uint32_t c = (i / EPL) * (EPL * TPR) + static_cast<uint32_t>(__builtin_ctz(mine)) * EPL + i % EPL;
+        col = min(col, mine ? c : ~0u);
+      }
+      const int bidx = col == ~0u ? 0 : static_cast<int>(col);
+      keep(k, best, bidx);
+      // blank the winner in the lane that holds it
+#pragma unroll
+      for (int i = 0; i < VPT; ++i)
+        if (bidx == (i / EPL) * (EPL * TPR) + t * EPL + i % EPL) v[i] = -10000.f;
     }
   }
   if (by_lane) {
