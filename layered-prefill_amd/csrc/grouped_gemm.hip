@@ -1669,7 +1669,8 @@ __device__ __forceinline__ void stream_store(const GemmParams& p, const float (&
 // H 2048, I 768, 256 tokens top-4 50 and 57; 128 experts, 64 tokens 117 and 98.
 // e4m3 runs here too (100 tokens of that layer: gate-up 45.6 -> 40.1 us, down 40.9 -> 25.9 us
 // against the register-staged kernel, whose two stages hold 36 KB per workgroup and drain at every K tile), its scales
-// fetched ahead of the stream like the routed weights.  Rows need whole 32-byte steps, not whole units.
+// fetched ahead of the stream like the routed weights; its down pass only where stream_codes_kernel has no instance.  Rows
+// need whole 32-byte steps, not whole units.
 // ---------------------------------------------------------------------------
 constexpr int kStRowBytes = 128, kStRows = 64, kStUnits = 4, kStBM = 32;
 constexpr int kStWBytes = kStRows * kStRowBytes;               // 8 KB of weights per unit
