@@ -39,3 +39,24 @@ def test_codes_made_in_the_down_pass_have_the_bits_of_the_launch(moe, dev, T, E,
     assert bool(want.isfinite().all()) and float(want.float().abs().max()) > 0
     for _ in range(2):
         assert torch.equal(run(None), want)
+
+
+def test_codes_made_in_the_down_pass_inside_a_hip_graph(moe, dev):
+    g = torch.Generator(dev).manual_seed(9)
+    T, E, K, H, I = 100, 64, 4, 1024, 768
+    draw = lambda *shape, std=1.0: torch.empty(shape, device=dev).normal_(0.0, std, generator=g).bfloat16()
+    q13, s13, q2, s2 = moe.quantize_expert_weights(draw(E, 2 * I, H, std=0.05), draw(E, H, I, std=0.05))
+    x, logits = draw(T, H), draw(T, E)
+    run = lambda: moe.fused_topk_experts(x, logits, q13, q2, K, True, w1_scale=s13, w2_scale=s2)
+    run()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = run()
+    for seed in range(4):
+        x.copy_(draw(T, H))
+        logits.copy_(draw(T, E))
+        captured.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(captured, run())
