@@ -17,6 +17,7 @@
 // consecutive output columns of one token and stores them as one 8-byte word.
 #include <stdlib.h>
 
+#include "block_groups.h"
 #include "common.h"
 #include "gemm_device.h"
 #include "quant_device.h"
@@ -2049,11 +2050,7 @@ __global__ __launch_bounds__(NW * kWave, 1) void stream_codes_kernel(
   const int begin = __builtin_amdgcn_readfirstlane(static_cast<int>(groups * share / kCdCus));
   const int end = __builtin_amdgcn_readfirstlane(static_cast<int>(groups * (share + 1) / kCdCus));
   if (begin >= end) return;
-  auto block_of = [&](int g) {
-    int mb = __umulhi(g, groups_rcp);   // g / groups_per_block, or one more
-    if (mb * groups_per_block > g) mb -= 1;
-    return mb;
-  };
+  auto block_of = [&](int g) { return block_of_group(g, groups_per_block, groups_rcp); };
   // the side that asks for weights
   const char* w_at = nullptr;
   bool alone = false;   // nobody else reads these weights
@@ -2272,7 +2269,7 @@ static bool codes_in_pass(const MoeFusedExpertsArgs* a, int64_t sorted_cap) {
 template <typename Mma>
 int launch_stream_codes(const GemmParams& p, hipStream_t s) {
   const int per_block = p.N / 16;
-  const uint32_t rcp = static_cast<uint32_t>((1LL << 32) / per_block + 1);
+  const uint32_t rcp = block_groups_rcp(per_block);
   auto go = [&](auto units, auto waves) {
     constexpr int NU = decltype(units)::value, NW = decltype(waves)::value;
     constexpr int lds = 2 * NU * kStBM * kStRowBytes + NW * NU * 16 * kStRowBytes;

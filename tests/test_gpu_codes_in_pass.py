@@ -7,6 +7,10 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("T,E,K,H,I,dtype,on_input", [
+    (300, 4, 2, 16, 384, "bfloat16", False),     # one group a block, more blocks than experts
+    (2000, 8, 4, 16, 768, "float16", False),
+    (300, 8, 2, 32, 512, "bfloat16", True),      # two groups, three
+    (500, 8, 2, 48, 768, "bfloat16", False),
     (64, 4, 2, 64, 384, "bfloat16", False),      # the fewest ids; four groups of rows a block, fewer than there are shares
     (16, 16, 8, 160, 512, "float16", False),     # ten groups a block: wavefronts without one
     (43, 32, 3, 2048, 768, "bfloat16", False),   # just beyond the line; shares that cross blocks
