@@ -15,3 +15,9 @@ constexpr int block_of_group(int g, int per_block, uint32_t rcp) {
   const int mb = static_cast<int>(static_cast<uint64_t>(static_cast<uint32_t>(g)) * rcp >> 32);  // the quotient, or one more
   return mb * per_block > g ? mb - 1 : mb;
 }
+
+// Elements from expert 0's first row to row `row` of expert e.  A block that a caller's alignment gives to no expert (-1) holds
+// no slots; what is read on its account and never used comes out of expert 0.
+constexpr int64_t expert_row(int e, int row, int64_t stride_e, int64_t stride_row) {
+  return (e < 0 ? 0 : e) * stride_e + row * stride_row;
+}

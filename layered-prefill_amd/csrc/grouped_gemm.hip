@@ -2066,8 +2066,7 @@ __global__ __launch_bounds__(NW * kWave, 1) void stream_codes_kernel(
     const int e = uniform_load(expert_ids + mb), before = uniform_load(expert_ids + (mb > 0 ? mb - 1 : 0)),
               behind = uniform_load(expert_ids + (mb + 1 < live_mb ? mb + 1 : mb));
     alone = !(mb > 0 && before == e) && !(mb + 1 < live_mb && behind == e);
-    w_at = static_cast<const char*>(p.w) + static_cast<int64_t>(e < 0 ? 0 : e) * p.w_stride_e +
-           static_cast<int64_t>(16 * (g - mb * groups_per_block)) * p.w_stride_n;
+    w_at = static_cast<const char*>(p.w) + expert_row(e, 16 * (g - mb * groups_per_block), p.w_stride_e, p.w_stride_n);
   };
   auto ask = [&](int u) {
 #pragma unroll
@@ -2164,7 +2163,7 @@ __global__ __launch_bounds__(NW * kWave, 1) void stream_codes_kernel(
     while (g < stop) {
       const int next = g + NW;
       const int n0 = 16 * (g - mb * groups_per_block);
-      const float* const scales = p.w_scale + static_cast<int64_t>(uniform_load(expert_ids + mb)) * p.w_scale_stride_e + n0;
+      const float* const scales = p.w_scale + expert_row(uniform_load(expert_ids + mb), n0, p.w_scale_stride_e, 1);
       const bool more = next < end;
       if (more) aim(next);
       f32x4 acc[2];

@@ -1,4 +1,5 @@
-"""Host build of what the e4m3 down pass works out of a group's number (csrc/block_groups.h): the block it belongs to."""
+"""Host build of what the e4m3 down pass works out of a group's number (csrc/block_groups.h): the block it belongs to
+and where its weight rows and scales lie."""
 import os
 import subprocess
 
@@ -27,6 +28,21 @@ int main() {
 }
 """
 
+# Prints the rows that lie in front of the tensor or elsewhere than their expert's.
+_ROWS = r"""
+#include <cstdio>
+#include "block_groups.h"
+int main() {
+  const int64_t strides[][2] = {{2048 * 768, 768}, {2048, 1}, {16LL * (1 << 28), 1 << 28}};
+  for (const auto& s : strides)
+    for (int e = -1; e < 4; ++e)
+      for (int row = 0; row < 16; row += 15) {
+        const int64_t want = (e == -1 ? 0 : e * s[0]) + row * s[1], got = expert_row(e, row, s[0], s[1]);
+        if (got != want) std::printf("expert %d row %d: %lld\n", e, row, static_cast<long long>(got));
+      }
+}
+"""
+
 
 def _run(tmp_path, source):
     (tmp_path / "main.cpp").write_text(source)
@@ -36,3 +52,7 @@ def _run(tmp_path, source):
 
 def test_every_group_has_its_block(tmp_path):
     assert _run(tmp_path, _BLOCKS) == ""
+
+
+def test_rows_of_a_block_without_an_expert_are_inside_the_tensor(tmp_path):
+    assert _run(tmp_path, _ROWS) == ""

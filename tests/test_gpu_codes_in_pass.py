@@ -45,6 +45,34 @@ def test_codes_made_in_the_down_pass_have_the_bits_of_the_launch(moe, dev, T, E,
         assert torch.equal(run(None), want)
 
 
+def test_blocks_of_no_expert_in_a_callers_alignment(moe, dev):
+    """Blocks without slots that name no expert (-1), in front of, between and behind the experts' own, change nothing."""
+    g = torch.Generator(dev).manual_seed(3)
+    T, E, H, I = 128, 4, 64, 512
+    draw = lambda *shape, std=1.0: torch.empty(shape, device=dev).normal_(0.0, std, generator=g).bfloat16()
+    x = draw(T, H)
+    q13, s13, q2, s2 = moe.quantize_expert_weights(draw(E, 2 * I, H, std=0.05), draw(E, H, I, std=0.05))
+    tw = torch.rand(T, 1, generator=g, device=dev)
+    slots = [[t for t in range(T) if t % E == e] for e in range(E)]   # a block an expert, all of it slots
+
+    def run(blocks):
+        so = torch.full((T + E * 31,), T, dtype=torch.int32)
+        for i, e in enumerate(blocks):
+            if e >= 0:
+                so[32 * i: 32 * i + 32] = torch.tensor(slots[e], dtype=torch.int32)
+        eo = torch.full((-(-so.numel() // 32),), -1, dtype=torch.int32)
+        eo[: len(blocks)] = torch.tensor(blocks, dtype=torch.int32)
+        npp = torch.tensor([32 * len(blocks)], dtype=torch.int32)
+        out = torch.full_like(x, float("nan"))
+        moe.fused_moe.launch_fused_experts(x, out, q13, q2, None, None, s13, s2, tw, so.to(dev), eo.to(dev), npp.to(dev), 32,
+                                           weight_code=moe._lib.E4M3_CODE)
+        return out
+
+    want = run([0, 1, 2, 3])
+    assert bool(want.isfinite().all())
+    assert torch.equal(run([-1, 0, 1, -1, 2, 3, -1]), want)
+
+
 def test_codes_made_in_the_down_pass_inside_a_hip_graph(moe, dev):
     g = torch.Generator(dev).manual_seed(9)
     T, E, K, H, I = 100, 64, 4, 1024, 768
