@@ -72,21 +72,32 @@ __device__ __forceinline__ void route_row(float (&v)[Pow2Geom<E>::kVpt], int t, 
   // rounds in a row were three quarters of the router's code (128 experts: 10.6 KB and, rolled, 2.6; few_gate_kernel 18.8
   // and 10.2 then).  Norm and layer, us, unrolled and rolled, with the exp's range checks as branches and as selects: 1 token
   // 24.4 and 24.0, 9 49.5 and 49.2; 64 and more the same.
-  // Lane k of the row keeps winner k (every lane knows it after the round), so that the renormalised weights leave as short
-  // coalesced stores; a row of fewer lanes than K writes round by round.
-  const bool by_lane = K <= TPR;
-  float my_w = 0.f;
-  int my_i = 0;
-  auto keep = [&](int k, float best, int bidx) {
-    wsum += best;
-    if (by_lane) {
-      my_w = t == k ? best : my_w;
-      my_i = t == k ? bidx : my_i;
-    } else if (live && t == 0) {
-      const size_t o = static_cast<size_t>(row) * K + k;
-      topk_w[o] = best;
-      topk_ids[o] = bidx;
-      if (tok_exp_idx) tok_exp_idx[o] = k * T + row;
+  // Winner k stays in lane k % TPR of the row (every lane knows it after the round), the TPR latest in a lane's first pair of
+  // registers and those before them one pair on: a lane has as many pairs as columns, so that all K of a row find a place,
+  // nothing is stored before the sum is known and the renormalised weights leave as short coalesced stores.  With K beyond
+  // the lanes stored round by round, read back, divided and stored again by one lane, and this way, router alone, us: 16
+  // experts top-6, 1 token 3.8 and 2.8, 135 4.3 and 3.0, 16896 5.0 and 3.7; top-8, 135 5.0 and 3.2; 8 top-8, 135 4.8 and 3.7;
+  // 32 top-16, 135 7.6 and 4.0; 64 top-24, 4096 11.7 and 5.1.  The loop without those stores is the shorter one for fewer
+  // winners, too: 128 top-8, 1 token 3.3 and 2.9, 16896 10.2 and 9.3.  Layer, 16 experts, H 1024, I 384, top-6, 16 tokens
+  // 19.9 and 19.0; 128, H 2048, I 768, top-8, 128 tokens 117.3 and 116.3.
+  float my_w[VPT];
+  int my_i[VPT];
+#pragma unroll
+  for (int j = 0; j < VPT; ++j) my_w[j] = 0.f, my_i[j] = 0;
+  // K rounds; a round says its winner to `keep`.
+  auto rounds = [&](auto&& round) {
+#pragma unroll 1
+    for (int base = 0; base < K; base += TPR) {
+#pragma unroll
+      for (int j = VPT - 1; j > 0; --j) my_w[j] = my_w[j - 1], my_i[j] = my_i[j - 1];
+      const int n = K - base < TPR ? K - base : TPR;
+#pragma unroll 1
+      for (int k = 0; k < n; ++k)
+        round([&](float best, int bidx) {
+          wsum += best;
+          my_w[0] = t == k ? best : my_w[0];
+          my_i[0] = t == k ? bidx : my_i[0];
+        });
     }
   };
   // The bits that a ballot has for this lane's row of lanes.
@@ -114,25 +125,23 @@ __device__ __forceinline__ void route_row(float (&v)[Pow2Geom<E>::kVpt], int t, 
         h[i] = hi, h[i + 1] = lo, which[i] = wi, which[i + 1] = wl;
       }
     uint32_t order = which[0] | which[1] << 2 | which[2] << 4 | which[3] << 6;
-#pragma unroll 1
-    for (int k = 0; k < K; ++k) {
+    rounds([&](auto&& keep) {
       const int best = row_max_bits<TPR>(h[0]);
       const uint32_t at = __builtin_ctz(row_bits(__ballot(h[0] == best)));
       const uint32_t low = __builtin_amdgcn_ubfe(row_bits(__ballot((order & 1) != 0)), at, 1);
       const uint32_t high = __builtin_amdgcn_ubfe(row_bits(__ballot((order & 2) != 0)), at, 1);
-      keep(k, __builtin_bit_cast(float, best), static_cast<int>(4 * at + 2 * high + low));
+      keep(__builtin_bit_cast(float, best), static_cast<int>(4 * at + 2 * high + low));
       const bool won = t == static_cast<int>(at);
       h[0] = won ? h[1] : h[0];
       h[1] = won ? h[2] : h[1];
       h[2] = won ? h[3] : h[2];
       h[3] = won ? -1 : h[3];
       order = won ? order >> 2 : order;
-    }
+    });
   } else {
     // One round: the row's largest value, then the lowest of the columns that hold it, from one ballot per value of a
     // lane.  (Column 0 where none does: all values NaN.  A row of one lane looks for itself.)
-#pragma unroll 1
-    for (int k = 0; k < K; ++k) {
+    rounds([&](auto&& keep) {
       float best = v[0];
       uint32_t col = TPR == 1 ? 0u : ~0u;
 #pragma unroll
@@ -151,24 +160,23 @@ __device__ __forceinline__ void route_row(float (&v)[Pow2Geom<E>::kVpt], int t, 
         col = min(col, mine ? c : ~0u);
       }
       const int bidx = col == ~0u ? 0 : static_cast<int>(col);
-      keep(k, best, bidx);
+      keep(best, bidx);
       // blank the winner in the lane that holds it
 #pragma unroll
       for (int i = 0; i < VPT; ++i)
         if (bidx == (i / EPL) * (EPL * TPR) + t * EPL + i % EPL) v[i] = -10000.f;
-    }
+    });
   }
-  if (by_lane) {
-    if (live && t < K) {
-      const size_t o = static_cast<size_t>(row) * K + t;
-      topk_w[o] = renormalize ? my_w / wsum : my_w;
-      topk_ids[o] = my_i;
-      if (tok_exp_idx) tok_exp_idx[o] = t * T + row;
-    }
-  } else if (renormalize && live && t == 0) {
-    for (int k = 0; k < K; ++k) {
+  const int last = (K - 1) / TPR;   // pair j of a lane holds winner (last - j) * TPR + t
+#pragma unroll
+  for (int j = 0; j < VPT; ++j) {
+    if (j > last) break;
+    const int k = (last - j) * TPR + t;
+    if (live && k < K) {
       const size_t o = static_cast<size_t>(row) * K + k;
-      topk_w[o] = topk_w[o] / wsum;
+      topk_w[o] = renormalize ? my_w[j] / wsum : my_w[j];
+      topk_ids[o] = my_i[j];
+      if (tok_exp_idx) tok_exp_idx[o] = k * T + row;
     }
   }
 }
