@@ -2255,22 +2255,34 @@ int launch_stream(GemmParams& p, int64_t sorted_cap, hipStream_t s) {
   return moe_check_launch(GATED ? "fused_experts (gate-up pass)" : "fused_experts (down pass)");
 }
 
+// Wavefronts of a workgroup of stream_codes_kernel for rows of so many units: as many as make 96 KB of rings, sixteen at most.
+constexpr int cd_waves(int units) { return units < 3 ? 16 : 48 / units / 4 * 4; }
+
 // Whether the down pass of an e4m3 call codes the intermediate itself (stream_codes_kernel): row lengths that have an instance
-// (the ring of a wavefront is a row long; beyond 768 the codes of two blocks and the rings no longer fit a CU).  With fewer
-// than 128 ids a CU's share is a handful of rows, all asked for at once either way, and the quantisation stands in front of
-// their products: 1 token of 128 experts 25.5 us in front and 25.8 here, 8 tokens 39.6 and 39.6, 16 (128 ids) 44.3 and 44.2.
-constexpr int kCdLeast = 128;
+// (beyond 768 the codes of two blocks and the rings no longer fit a CU).  With fewer than 128 ids a CU's share is a handful of
+// rows, all asked for at once either way, and the quantisation stands in front of their products: 1 token of 128 experts
+// 25.5 us in front and 25.8 here, 8 tokens 39.6 and 39.6, 16 (128 ids) 44.3 and 44.2.
+// Up to three units a wavefront codes one pair of a block's rows and the pass is the faster way from there on (layers of 8 to 128
+// experts, H 512 to 4096, 128 to 2800 ids: by 2 to 9 %).  Longer rows have fewer wavefronts, each of which codes two pairs one
+// behind the other, and want a share that is worth it, twelve groups to a CU by blocks that are full and an expert in four that
+// has one more (a skewed routing has as many).  H 1024, quantised in front and here, us, and groups to a CU: I 512, 16 experts
+// top-4, 64 tokens 20.3 and 20.8 (5), 250 24.3 and 24.8 (10), 64 experts, 300 37.4 and 36.4 (18); I 768 21.8 and 22.6, 30.2 and
+// 31.6, 44.7 and 44.1.  H 2048, I 768, 16 experts, 120 tokens (12) 33.8 and 33.9.
+constexpr int kCdLeast = 128, kCdLeastGroups = 12;
 static bool codes_in_pass(const MoeFusedExpertsArgs* a, int64_t sorted_cap) {
-  return a->block_size == kStBM && static_cast<int64_t>(a->T) * a->K >= kCdLeast && !a->w2_bias && (a->I == 384 || a->I == 512 || a->I == 768) && a->H % 16 == 0 &&
-         (sorted_cap / kStBM + 1) * (a->H / 16) < INT32_MAX / 2 && static_cast<int64_t>(a->H) * a->w2_stride_n < (1LL << 32) - 16384;
+  const int64_t ids = static_cast<int64_t>(a->T) * a->K, rows16 = a->H / 16;
+  const int units = a->I / kStRowBytes;
+  if (a->block_size != kStBM || ids < kCdLeast || a->w2_bias || (a->I != 384 && a->I != 512 && a->I != 768) || a->H % 16) return false;
+  if (cd_waves(units) < 16 && (ids / kStBM + (ids < a->E ? ids : a->E) / 4) * rows16 < kCdLeastGroups * kCdCus) return false;
+  return (sorted_cap / kStBM + 1) * rows16 < INT32_MAX / 2 && static_cast<int64_t>(a->H) * a->w2_stride_n < (1LL << 32) - 16384;
 }
 
 template <typename Mma>
 int launch_stream_codes(const GemmParams& p, hipStream_t s) {
   const int per_block = p.N / 16;
   const uint32_t rcp = block_groups_rcp(per_block);
-  auto go = [&](auto units, auto waves) {
-    constexpr int NU = decltype(units)::value, NW = decltype(waves)::value;
+  auto go = [&](auto units) {
+    constexpr int NU = decltype(units)::value, NW = cd_waves(NU);
     constexpr int lds = 2 * NU * kStBM * kStRowBytes + NW * NU * 16 * kStRowBytes;
     static MoeLdsOptIn flags;
     auto kernel = stream_codes_kernel<Mma, NU, NW>;
@@ -2279,9 +2291,9 @@ int launch_stream_codes(const GemmParams& p, hipStream_t s) {
                        p.numel, p);
     return moe_check_launch("fused_experts (quantisation and down pass)");
   };
-  if (p.Kd == 384) return go(IntTag<3>{}, IntTag<16>{});
-  if (p.Kd == 512) return go(IntTag<4>{}, IntTag<12>{});
-  return go(IntTag<6>{}, IntTag<8>{});
+  if (p.Kd == 384) return go(IntTag<3>{});
+  if (p.Kd == 512) return go(IntTag<4>{});
+  return go(IntTag<6>{});
 }
 
 // Polls a down tile of the one-launch form waits for its m-block's gate-up tiles (about a
