@@ -25,9 +25,9 @@ def _workspace(moe, x, E, K, I):
 @pytest.mark.parametrize("T,E,K,H,I,dtype,on_input,in_pass", [
     (300, 4, 2, 16, 384, "bfloat16", False, True),   # one group a block, more blocks than experts
     (2000, 8, 4, 16, 768, "float16", False, False),
-    (300, 8, 2, 32, 512, "bfloat16", True, False)),   # two groups, three
+    (300, 8, 2, 32, 512, "bfloat16", True, False),   # two groups, three
     (500, 8, 2, 48, 768, "bfloat16", False, False),
-    (64, 4, 2, 64, 384, "bfloat16", False, True)),   # the fewest ids; four groups of rows a block, fewer than there are shares
+    (64, 4, 2, 64, 384, "bfloat16", False, True),   # the fewest ids; four groups of rows a block, fewer than there are shares
     (16, 16, 8, 160, 512, "float16", False, False),   # ten groups a block: wavefronts without one
     (43, 32, 3, 2048, 768, "bfloat16", False, False),   # (a small share of long rows: codes of a launch)
     (100, 128, 8, 2048, 768, "bfloat16", True, True),
