@@ -2142,9 +2142,9 @@ __global__ __launch_bounds__(NW * kWave, 1) void stream_codes_kernel(
   if (works) {
     aim(g);
     ask(0);
-    ask(1);
+    if constexpr (NU > 1) ask(1);
   }
-  code(mb, 0, IntTag<2 * (NU - 2)>{}, [&] {
+  code(mb, 0, IntTag<(NU > 2 ? 2 * (NU - 2) : 0)>{}, [&] {
     if (works)
 #pragma unroll
       for (int u = 2; u < NU; ++u) ask(u);
@@ -2255,24 +2255,25 @@ int launch_stream(GemmParams& p, int64_t sorted_cap, hipStream_t s) {
   return moe_check_launch(GATED ? "fused_experts (gate-up pass)" : "fused_experts (down pass)");
 }
 
-// Wavefronts of a workgroup of stream_codes_kernel for rows of so many units: as many as make 96 KB of rings, sixteen at most.
+// Wavefronts of a workgroup of stream_codes_kernel for rows of so many units: as many as make 96 KB of rings, sixteen at most,
+// and as many on each SIMD (five units, with nine: layer of 128 experts, H 2048, I 640, top-8, 24 tokens 39.7 us, with eight 38.8).
 constexpr int cd_waves(int units) { return units < 3 ? 16 : 48 / units / 4 * 4; }
 
-// Whether the down pass of an e4m3 call codes the intermediate itself (stream_codes_kernel): row lengths that have an instance
-// (beyond 768 the codes of two blocks and the rings no longer fit a CU).  With fewer than 128 ids a CU's share is a handful of
-// rows, all asked for at once either way, and the quantisation stands in front of their products: 1 token of 128 experts
-// 25.5 us in front and 25.8 here, 8 tokens 39.6 and 39.6, 16 (128 ids) 44.3 and 44.2.
+// Whether the down pass of an e4m3 call codes the intermediate itself (stream_codes_kernel): rows of whole units, of which the
+// codes of two blocks and the rings fit a CU (up to six).  With fewer than 128 ids a CU's share is a handful of rows, all asked
+// for at once either way, and the quantisation stands in front of their products: 1 token of 128 experts 25.5 us in front and
+// 25.8 here, 8 tokens 39.6 and 39.6, 16 (128 ids) 44.3 and 44.2.
 // Up to three units a wavefront codes one pair of a block's rows and the pass is the faster way from there on (layers of 8 to 128
-// experts, H 512 to 4096, 128 to 2800 ids: by 2 to 9 %).  Longer rows have fewer wavefronts, each of which codes two pairs one
+// experts, H 512 to 4096, 128 to 2800 ids: by 2 to 14 %).  Longer rows have fewer wavefronts, each of which codes two pairs one
 // behind the other, and want a share that is worth it, twelve groups to a CU by blocks that are full and an expert in four that
 // has one more (a skewed routing has as many).  H 1024, quantised in front and here, us, and groups to a CU: I 512, 16 experts
 // top-4, 64 tokens 20.3 and 20.8 (5), 250 24.3 and 24.8 (10), 64 experts, 300 37.4 and 36.4 (18); I 768 21.8 and 22.6, 30.2 and
-// 31.6, 44.7 and 44.1.  H 2048, I 768, 16 experts, 120 tokens (12) 33.8 and 33.9.
+// 31.6, 44.7 and 44.1; I 640 21.1 and 21.7, 27.9 and 29.0, 40.7 and 39.9.  H 2048, I 768, 16 experts, 120 tokens (12) 33.8 and 33.9.
 constexpr int kCdLeast = 128, kCdLeastGroups = 12;
 static bool codes_in_pass(const MoeFusedExpertsArgs* a, int64_t sorted_cap) {
   const int64_t ids = static_cast<int64_t>(a->T) * a->K, rows16 = a->H / 16;
   const int units = a->I / kStRowBytes;
-  if (a->block_size != kStBM || ids < kCdLeast || a->w2_bias || (a->I != 384 && a->I != 512 && a->I != 768) || a->H % 16) return false;
+  if (a->block_size != kStBM || ids < kCdLeast || a->w2_bias || a->I % kStRowBytes || units > 6 || a->H % 16) return false;
   if (cd_waves(units) < 16 && (ids / kStBM + (ids < a->E ? ids : a->E) / 4) * rows16 < kCdLeastGroups * kCdCus) return false;
   return (sorted_cap / kStBM + 1) * rows16 < INT32_MAX / 2 && static_cast<int64_t>(a->H) * a->w2_stride_n < (1LL << 32) - 16384;
 }
@@ -2291,9 +2292,14 @@ int launch_stream_codes(const GemmParams& p, hipStream_t s) {
                        p.numel, p);
     return moe_check_launch("fused_experts (quantisation and down pass)");
   };
-  if (p.Kd == 384) return go(IntTag<3>{});
-  if (p.Kd == 512) return go(IntTag<4>{});
-  return go(IntTag<6>{});
+  switch (p.Kd / kStRowBytes) {
+    case 1: return go(IntTag<1>{});
+    case 2: return go(IntTag<2>{});
+    case 3: return go(IntTag<3>{});
+    case 4: return go(IntTag<4>{});
+    case 5: return go(IntTag<5>{});
+    default: return go(IntTag<6>{});
+  }
 }
 
 // Polls a down tile of the one-launch form waits for its m-block's gate-up tiles (about a

@@ -35,6 +35,12 @@ def _workspace(moe, x, E, K, I):
     (3000, 5, 2, 96, 512, "bfloat16", False, False),    # many blocks a share, six groups each
     (2500, 3, 1, 288, 768, "float16", False, False),
     (1200, 16, 4, 64, 384, "bfloat16", False, True),
+    (64, 4, 2, 64, 128, "float16", False, True),   # rows of one unit: a ring of one place
+    (900, 8, 2, 272, 128, "bfloat16", True, True),
+    (100, 64, 4, 1024, 256, "bfloat16", False, True),
+    (1100, 6, 2, 48, 256, "float16", False, True),
+    (300, 64, 4, 1024, 640, "float16", False, True),   # an odd number of units
+    (2500, 8, 4, 160, 640, "bfloat16", True, True),
     (2750, 3, 2, 288, 512, "float16", False, True),    # rows that two pairs a wavefront code, in many blocks of few groups
     (8250, 8, 4, 48, 768, "bfloat16", False, True),
     (25000, 8, 4, 16, 512, "bfloat16", False, True),   # and of one
@@ -68,9 +74,9 @@ def test_codes_made_in_the_down_pass_have_the_bits_of_the_launch(moe, dev, T, E,
 
 
 @pytest.mark.parametrize("T,E,H,I,in_pass", [
-    (127, 4, 64, 384, False), (128, 4, 64, 384, True), (128, 4, 64, 64, False), (128, 4, 64, 192, False),
-    (128, 4, 64, 512, False), (511, 32, 2048, 512, False), (512, 32, 2048, 512, True), (512, 32, 2048, 768, True),
-    (512, 32, 2032, 768, False), (2048, 32, 2048, 896, False)])
+    (127, 4, 64, 256, False), (128, 4, 64, 256, True), (128, 4, 64, 384, True), (128, 4, 64, 64, False), (128, 4, 64, 192, False),
+    (128, 4, 64, 512, False), (511, 32, 2048, 512, False), (512, 32, 2048, 512, True), (512, 32, 2048, 640, True),
+    (512, 32, 2048, 768, True), (512, 32, 2032, 768, False), (2048, 32, 2048, 896, False)])
 def test_which_calls_make_their_codes_in_the_down_pass(moe, dev, T, E, H, I, in_pass):
     print(T, E, H, I, flush=True)
     g = torch.Generator(dev).manual_seed(T + I)
