@@ -1,6 +1,7 @@
-"""Results of the native host calls are made past the dispatcher only where nobody listens to it."""
+"""Results of the native host calls are made past the dispatcher only where it would make the same ones."""
 import pytest
 import torch
+from torch.profiler import ProfilerActivity, profile
 from torch.utils._python_dispatch import TorchDispatchMode
 
 pytestmark = pytest.mark.gpu
@@ -14,6 +15,13 @@ class _Seen(TorchDispatchMode):
     def __torch_dispatch__(self, func, types, args=(), kwargs=None):
         self.empties += func in (torch.ops.aten.empty.memory_format,)
         return func(*args, **(kwargs or {}))
+
+
+def _profiled(run):
+    """What it returns, and how many tensors the dispatcher was asked for."""
+    with profile(activities=[ProfilerActivity.CPU]) as p:
+        got = run()
+    return got, sum(e.name == "aten::empty" for e in p.events())
 
 
 @pytest.mark.parametrize("form", ["plain", "mode", "inference", "deterministic"])
@@ -31,17 +39,19 @@ def test_results_are_what_empty_makes(moe, dev, form):
             got = run()
     elif form == "inference":
         with torch.inference_mode():
-            got = run()
+            got, through = _profiled(run)
     elif form == "deterministic":
+        before = torch.are_deterministic_algorithms_enabled(), torch.is_deterministic_algorithms_warn_only_enabled()
         torch.use_deterministic_algorithms(True)
         try:
-            got = run()
+            got, through = _profiled(run)
         finally:
-            torch.use_deterministic_algorithms(False)
+            torch.use_deterministic_algorithms(before[0], warn_only=before[1])
     else:
-        got = run()
+        got, through = _profiled(run)
     if seen is not None:
-        assert seen.empties == 4
+        through = seen.empties
+    assert through == (4 if form in ("mode", "deterministic") else 0)
     for a, b in zip(got, want):
         assert torch.equal(a, b) and a.device == x.device and a.is_contiguous() and not a.requires_grad
         assert a.is_inference() == (form == "inference") and a.dtype == b.dtype
