@@ -21,3 +21,28 @@ constexpr int block_of_group(int g, int per_block, uint32_t rcp) {
 constexpr int64_t expert_row(int e, int row, int64_t stride_e, int64_t stride_row) {
   return (e < 0 ? 0 : e) * stride_e + row * stride_row;
 }
+
+// A share of the groups, [begin, end), none of them empty.  One of a block and more is walked from the first block that starts
+// in it, and its groups in front of that block come last: workgroups whose blocks are one expert's then read the same weight
+// rows at about the same time, wherever their shares were cut.  (Shares shorter than a block don't all hold a block's start.)
+// Places of the walk are 0 .. count - 1.
+struct BlockShare {
+  int begin, count, lead, per_block, lead_block, end_block;   // `lead` groups, all of lead_block, come last
+
+  static constexpr BlockShare of(int begin, int end, int per_block, uint32_t rcp) {
+    const int mb = block_of_group(begin, per_block, rcp), behind = (mb + 1) * per_block - begin;
+    const bool turned = behind < per_block && end - begin >= per_block;
+    return {begin, end - begin, turned ? behind : 0, per_block, mb, block_of_group(end - 1, per_block, rcp)};
+  }
+  // The group at a place.
+  constexpr int group(int place) const { return begin + place + (place < count - lead ? lead : lead - count); }
+  constexpr int first_block() const { return lead ? lead_block + 1 : lead_block; }
+  constexpr bool last(int mb) const { return mb == (lead ? lead_block : end_block); }
+  // The block behind one that is not the last.
+  constexpr int next(int mb) const { return mb == end_block ? lead_block : mb + 1; }
+  // The first place behind a block's, and how far the places of a block's groups lie in front of their numbers in it.
+  constexpr int stop(int mb) const {
+    return last(mb) ? count : mb == end_block ? count - lead : (mb + 1) * per_block - begin - lead;
+  }
+  constexpr int shift(int mb) const { return begin + lead - (lead && mb == lead_block ? count : 0) - mb * per_block; }
+};

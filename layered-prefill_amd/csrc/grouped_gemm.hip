@@ -2022,7 +2022,11 @@ __global__ __launch_bounds__(kThreads, 3) void stream_gemm_kernel(
 // of 128 codes), so that the codes of a block of 32 slots stay in LDS and a wavefront streams weight rows, sixteen at a time, on
 // its own: no barrier but one per block.  One workgroup to a CU takes an equal share of the (block, sixteen rows) groups, NW
 // wavefronts of it a group each (as many as make 96 KB of rings); a wavefront's next group is asked for, unit by unit, as the
-// present one is multiplied, so that only a share's start waits for memory.  Products, their order and every rounding are
+// present one is multiplied, so that only a share's start waits for memory.  Where a share is a block and more its walk starts
+// with a block (BlockShare): with an expert in several blocks the workgroups would read its weights at places as far apart as
+// their shares were cut, past what the L2 holds.  Both passes in blocks of 32, 128 experts, H 2048, I 768, top-8, balanced, us,
+// quantised in front, walked in order and this way: 1200 tokens 230, 249 and 229; 4200 585, 631 and 569; 8448 1077, 1162 and
+// 1031; routed unevenly, 8448 1078, 1004 and 1001.  Products, their order and every rounding are
 // stream_gemm_kernel's and the quantiser's.  It is bound by the weights, those of an expert with several blocks once a block:
 // 100 tokens of 128 experts, H 2048, I 768, top-8: 22 us and 5 of quantisation in front, 24 this way.  (With a workgroup for 64
 // rows of a block, as in stream_gemm_kernel, all its weights asked for at once, 33: the start of a workgroup, 7 us, once every
@@ -2075,8 +2079,9 @@ __global__ __launch_bounds__(NW * kWave, 1) void stream_codes_kernel(
       else lds_dma16(w_at + u * kStRowBytes, w_off[j], ring + u * kStep + j * 1024);
     }
   };
-  int g = begin + wave;
-  const bool works = g < end;   // (a wavefront without a group takes part in the quantisation)
+  const BlockShare walk = BlockShare::of(begin, end, groups_per_block, groups_rcp);
+  int place = wave;   // of every NW a wavefront has one
+  const bool works = place < walk.count;   // (a wavefront without a group takes part in the quantisation)
   // codes and scales of block mb, and what the epilogue needs of its slots; `meanwhile` asks for more weights
   typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
   const int l31 = lane & 31, vecs = p.Kd / 8;
@@ -2137,10 +2142,9 @@ __global__ __launch_bounds__(NW * kWave, 1) void stream_codes_kernel(
       }
     }
   };
-  int mb = block_of(begin);
-  const int mb0 = mb, mb_end = block_of(end - 1);
+  int mb = walk.first_block(), buf = 0;
   if (works) {
-    aim(g);
+    aim(walk.group(place));
     ask(0);
     if constexpr (NU > 1) ask(1);
   }
@@ -2157,15 +2161,14 @@ __global__ __launch_bounds__(NW * kWave, 1) void stream_codes_kernel(
   for (;;) {
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     bare_barrier();
-    const int buf = (mb - mb0) & 1;
     const char* const codes = smem + buf * kCodes;
-    const int stop = end < (mb + 1) * groups_per_block ? end : (mb + 1) * groups_per_block;
-    while (g < stop) {
-      const int next = g + NW;
-      const int n0 = 16 * (g - mb * groups_per_block);
+    const int stop = walk.stop(mb), shift = walk.shift(mb);
+    while (place < stop) {
+      const int next = place + NW;
+      const int n0 = 16 * (place + shift);
       const float* const scales = p.w_scale + expert_row(uniform_load(expert_ids + mb), n0, p.w_scale_stride_e, 1);
-      const bool more = next < end;
-      if (more) aim(next);
+      const bool more = next < walk.count;
+      if (more) aim(walk.group(next));
       f32x4 acc[2];
 #pragma unroll
       for (int h = 0; h < 2; ++h)
@@ -2216,11 +2219,12 @@ __global__ __launch_bounds__(NW * kWave, 1) void stream_codes_kernel(
         }
         stream_store<El, false, MOE_ACT_SILU>(p, o, tok, n0 + 4 * lq);
       }
-      g = next;
+      place = next;
     }
-    if (mb == mb_end) break;
-    ++mb;
-    code(mb, (mb - mb0) & 1, IntTag<0>{}, [] {});
+    if (walk.last(mb)) break;
+    mb = walk.next(mb);
+    buf ^= 1;
+    code(mb, buf, IntTag<0>{}, [] {});
   }
 }
 

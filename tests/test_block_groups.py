@@ -1,5 +1,5 @@
-"""Host build of what the e4m3 down pass works out of a group's number (csrc/block_groups.h): the block it belongs to
-and where its weight rows and scales lie."""
+"""Host build of what the e4m3 down pass works out of a group's number (csrc/block_groups.h): the block it belongs to,
+where its weight rows and scales lie, and in which order a share of groups is walked."""
 import os
 import subprocess
 
@@ -43,6 +43,40 @@ int main() {
 }
 """
 
+# Prints the shares that are not walked as they should be: every group once, block by block in the order that the kernel
+# changes blocks, and from a block's first row on where the share is a block long.
+_WALKS = r"""
+#include <cstdio>
+#include <vector>
+#include "block_groups.h"
+int main() {
+  for (int per : {1, 2, 3, 6, 10, 64, 128, 180, 256})
+    for (int blocks : {1, 2, 5, 37, 128, 370, 1120, 2168}) {
+      const uint32_t rcp = block_groups_rcp(per);
+      const int64_t groups = static_cast<int64_t>(blocks) * per;
+      std::vector<int> seen(groups, 0);
+      for (int share = 0; share < 256; ++share) {
+        const int begin = groups * share / 256, end = groups * (share + 1) / 256;
+        if (begin >= end) continue;
+        const BlockShare walk = BlockShare::of(begin, end, per, rcp);
+        bool bad = end - begin >= per && walk.group(0) % per;
+        int place = 0, mb = walk.first_block(), turns = 0;
+        for (;; mb = walk.next(mb)) {
+          for (; place < walk.stop(mb) && !bad; ++place) {
+            const int g = walk.group(place);
+            if (g < begin || g >= end || g / per != mb || g - mb * per != place + walk.shift(mb) || seen[g]++) bad = true;
+            else if (place && g != walk.group(place - 1) + 1 && g != begin) bad = true;
+          }
+          if (bad || walk.last(mb) || ++turns > blocks) break;
+        }
+        if (bad || place != end - begin) std::printf("groups per block %d, blocks %d, share %d: place %d of block %d\n", per, blocks, share, place, mb);
+      }
+      for (int64_t g = 0; g < groups; ++g)
+        if (seen[g] != 1) std::printf("groups per block %d, blocks %d: group %lld walked %d times\n", per, blocks, static_cast<long long>(g), seen[g]);
+    }
+}
+"""
+
 
 def _run(tmp_path, source):
     (tmp_path / "main.cpp").write_text(source)
@@ -56,3 +90,7 @@ def test_every_group_has_its_block(tmp_path):
 
 def test_rows_of_a_block_without_an_expert_are_inside_the_tensor(tmp_path):
     assert _run(tmp_path, _ROWS) == ""
+
+
+def test_shares_are_walked_from_a_blocks_first_row(tmp_path):
+    assert _run(tmp_path, _WALKS) == ""
