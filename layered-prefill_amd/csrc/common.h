@@ -232,22 +232,43 @@ struct ElemF16 {
 // 2^-64, which rounds once.  gfx950 code objects keep fp32 subnormals (denormal
 // mode 3).  Translation units that use it are compiled with -ffp-contract=off
 // so that no other operation is fused.
+// The ends of the range leave by branches, which a wavefront whose values are all inside passes by at once; with ENDS_SELECTED
+// they are put in by selects.  Kernels of many values are bound by how many instructions a value takes: silu_and_mul, bf16, us,
+// with selects, with a branch for each end only, and this way: 67584 x 768 82, 76.4 and 71.1, 16896 x 4096 105, 98.5 and 91,
+// 8 x 768 3.1, 3.3 and 2.9 (gates of standard deviation 50, an end in nearly every wavefront, 83, 77 and 78).  A router of few
+// rows waits for one chain of instructions and is better without a branch: 128 experts, 1 token 2.5, 2.9 and 2.6.
 // ---------------------------------------------------------------------------
+template <bool ENDS_SELECTED = false>
 __device__ __forceinline__ float moe_expf(float x) {
-  // (no branches: the ends of the range are put in at the end)
-  const float in = __builtin_fminf(__builtin_fmaxf(x, -104.0f), 88.0f);
-  float n = __builtin_rintf(in * 1.44269504088896341f);
-  float r = __builtin_fmaf(n, -0.693359375f, in);
-  r = __builtin_fmaf(n, 2.12194440e-4f, r);
-  float p = 1.9875691500e-4f;
-  p = __builtin_fmaf(p, r, 1.3981999507e-3f);
-  p = __builtin_fmaf(p, r, 8.3334519073e-3f);
-  p = __builtin_fmaf(p, r, 4.1665795894e-2f);
-  p = __builtin_fmaf(p, r, 1.6666665459e-1f);
-  p = __builtin_fmaf(p, r, 5.0000001201e-1f);
-  float r2 = r * r;
-  p = __builtin_fmaf(p, r2, r);
-  p = p + 1.0f;
+  auto mantissa = [](float in, float& n) {
+    n = __builtin_rintf(in * 1.44269504088896341f);
+    float r = __builtin_fmaf(n, -0.693359375f, in);
+    r = __builtin_fmaf(n, 2.12194440e-4f, r);
+    float p = 1.9875691500e-4f;
+    p = __builtin_fmaf(p, r, 1.3981999507e-3f);
+    p = __builtin_fmaf(p, r, 8.3334519073e-3f);
+    p = __builtin_fmaf(p, r, 4.1665795894e-2f);
+    p = __builtin_fmaf(p, r, 1.6666665459e-1f);
+    p = __builtin_fmaf(p, r, 5.0000001201e-1f);
+    float r2 = r * r;
+    p = __builtin_fmaf(p, r2, r);
+    return p + 1.0f;
+  };
+  float n;
+  if constexpr (!ENDS_SELECTED) {
+    if (__builtin_expect(!__ballot(!(__builtin_fabsf(x) <= 86.0f)), 1)) {   // (n from -124 to 124; NaN is outside)
+      const float p = mantissa(x, n);
+      return __uint_as_float(__float_as_uint(p) + (static_cast<uint32_t>(static_cast<int32_t>(n)) << 23));
+    }
+    if (x != x) return x;
+    if (x > 88.0f) return __builtin_inff();
+    if (x < -104.0f) return 0.0f;
+    const float p = mantissa(x, n);
+    const int32_t ni = static_cast<int32_t>(n);
+    if (ni < -125) return __uint_as_float(__float_as_uint(p) + (static_cast<uint32_t>(ni + 64) << 23)) * 5.42101086242752217e-20f;
+    return __uint_as_float(__float_as_uint(p) + (static_cast<uint32_t>(ni) << 23));
+  }
+  const float p = mantissa(__builtin_fminf(__builtin_fmaxf(x, -104.0f), 88.0f), n);
   const int32_t ni = static_cast<int32_t>(n);
   const bool small = ni < -125;
   const float y = __uint_as_float(__float_as_uint(p) + (static_cast<uint32_t>(small ? ni + 64 : ni) << 23));

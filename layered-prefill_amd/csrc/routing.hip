@@ -399,7 +399,7 @@ __global__ __launch_bounds__(kWave* kWavesPerBlock) void topk_softmax_generic_ke
   for (int j = 0; j < kGenericMaxPerLane; ++j) {
     const int c = lane + j * kWave;
     if (c < E) {
-      v[j] = moe_expf(v[j] - mx);
+      v[j] = moe_expf<true>(v[j] - mx);
       sum += v[j];
     }
   }
@@ -468,7 +468,7 @@ __global__ __launch_bounds__(kWave) void topk_softmax_wide_kernel(
   for (int m = 32; m > 0; m /= 2) mx = fmaxf(mx, __shfl_xor(mx, m, kWave));
   float sum = 0.f;
   for (int c = lane; c < E; c += kWave) {
-    const float e = moe_expf(El::ld(src[c]) - mx);
+    const float e = moe_expf<true>(El::ld(src[c]) - mx);
     prob[c] = e;
     sum += e;
   }

@@ -58,7 +58,7 @@ __device__ __forceinline__ void route_row(float (&v)[Pow2Geom<E>::kVpt], int t, 
   float sum = 0.f;
 #pragma unroll
   for (int i = 0; i < VPT; ++i) {
-    v[i] = moe_expf(v[i] - mx);
+    v[i] = moe_expf<true>(v[i] - mx);
     sum += v[i];
   }
   sum = row_sum<TPR>(sum);
@@ -70,8 +70,9 @@ __device__ __forceinline__ void route_row(float (&v)[Pow2Geom<E>::kVpt], int t, 
   const int lane = threadIdx.x % kWave, row0 = lane & 31 & ~(TPR - 1);
   // The rounds are one rolled loop: a kernel that runs through its code once waits for its instructions, too, and sixteen
   // rounds in a row were three quarters of the router's code (128 experts: 10.6 KB and, rolled, 2.6; few_gate_kernel 18.8
-  // and 10.2 then).  Norm and layer, us, unrolled and rolled, with the exp's range checks as branches and as selects: 1 token
-  // 24.4 and 24.0, 9 49.5 and 49.2; 64 and more the same.
+  // and 10.2 then).  Router alone, 128 experts top-8, us, with them unrolled and as all of this function is now: 1 token 3.5
+  // and 2.6, 128 3.8 and 2.8, 16896 11.7 and 8.6; norm and layer 1 token 23.4 and 22.3, 9 49.9 and 48.7, 64 88.4 and 87.5,
+  // 128 114.6 and 113.7.
   // Winner k stays in lane k % TPR of the row (every lane knows it after the round), the TPR latest in a lane's first pair of
   // registers and those before them one pair on: a lane has as many pairs as columns, so that all K of a row find a place,
   // nothing is stored before the sum is known and the renormalised weights leave as short coalesced stores.  With K beyond
@@ -110,8 +111,8 @@ __device__ __forceinline__ void route_row(float (&v)[Pow2Geom<E>::kVpt], int t, 
     // Probabilities are not negative, so that their bits compare as they do.  A lane sorts its four, the lower column first
     // where two are equal, and a round looks at the lanes' largest only: one exchange, the first lane that holds the row's
     // largest wins and goes on to its next.  A round is a chain of dependent instructions, 0.28 us of it when each looked at
-    // all four values of a lane, and stands in front of everything in a call of few tokens.  Norm and layer, us, that way
-    // and this: 1 token 22.9 and 22.2, 9 48.2 and 47.5, 64 87.8 and 87.4, 128 116.7 and 116.3.
+    // all four values of a lane, and stands in front of everything in a call of few tokens.  Router alone, 128 experts top-8,
+    // us, that way and this: 1 token 3.1 and 2.6, 128 3.4 and 2.8, 16896 11.3 and 8.6; 16 top-6, 135 2.9 and 2.6.
     int h[4], which[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) h[i] = __builtin_bit_cast(int, v[kHeads ? i : 0]), which[i] = i;
