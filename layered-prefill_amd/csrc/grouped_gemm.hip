@@ -1523,8 +1523,10 @@ __global__ __launch_bounds__(kThreads, 1) void big_fused_kernel(const GemmParams
 // received at most 32 (64) rows is weight streaming only and costs about 0.60
 // (0.75) of a full one, a partly filled one as much as a full one (its six gate-up
 // and eight down tiles: 334 / 424 / 568 / 561 us of CU time at 8448 tokens when the
-// weights were set, 324 / 344 / 480 / 529 since the tiles have their present loops);
-// with equal counts the XCDs finished up to 25 % apart.
+// weights were set; with the tiles' present loops, and pairs of n-tiles in the down pass
+// of full blocks, 313 / 348 / 462 / 482, as 41.5 / 46 / 61 / 64).  With equal counts the
+// XCDs finished up to 25 % apart; with these weights an XCD's busy time is within 6 % of the
+// mean at 8448 and 16896 tokens, within 17 % at 256 and 741, where a range is a few blocks.
 // Ranges stay contiguous so that the blocks of one expert keep sharing its
 // weights through one L2.  No range is longer than cap_mb blocks (the grid has
 // that many slots per XCD).  One workgroup; bounds[0..8] in m-blocks.
@@ -1670,7 +1672,7 @@ __device__ __forceinline__ void stream_store(const GemmParams& p, const float (&
 // H 2048, I 768, 256 tokens top-4 50 and 57; 128 experts, 64 tokens 117 and 98.
 // e4m3 runs here too (100 tokens of that layer: gate-up 45.6 -> 40.1 us, down 40.9 -> 25.9 us
 // against the register-staged kernel, whose two stages hold 36 KB per workgroup and drain at every K tile), its scales
-// fetched ahead of the stream like the routed weights; its down pass only where stream_codes_kernel has no instance.  Rows
+// fetched ahead of the stream like the routed weights; its down pass only where stream_codes_kernel does not take it.  Rows
 // need whole 32-byte steps, not whole units.
 // ---------------------------------------------------------------------------
 constexpr int kStRowBytes = 128, kStRows = 64, kStUnits = 4, kStBM = 32;
@@ -2026,13 +2028,14 @@ __global__ __launch_bounds__(kThreads, 3) void stream_gemm_kernel(
 // with a block (BlockShare): with an expert in several blocks the workgroups would read its weights at places as far apart as
 // their shares were cut, past what the L2 holds.  Both passes in blocks of 32, 128 experts, H 2048, I 768, top-8, balanced, us,
 // quantised in front, walked in order and this way: 1200 tokens 230, 249 and 229; 4200 585, 631 and 569; 8448 1077, 1162 and
-// 1031; routed unevenly, 8448 1078, 1004 and 1001.  Products, their order and every rounding are
-// stream_gemm_kernel's and the quantiser's.  It is bound by the weights, those of an expert with several blocks once a block:
-// 100 tokens of 128 experts, H 2048, I 768, top-8: 22 us and 5 of quantisation in front, 24 this way.  (With a workgroup for 64
-// rows of a block, as in stream_gemm_kernel, all its weights asked for at once, 33: the start of a workgroup, 7 us, once every
-// 48 KB.)  Whole layer with the norm, quantised in front and here, us: 24 tokens of that layer 47.6 and 46.1, 64 60.7 and 59.2,
-// 100 69.4 and 68.4, 300 105.1 and 102.8; 64 experts, H 1024, I 384, top-6: 120 tokens 31.7 and 29.4; 16 experts, 2200 94.8 and
-// 81.1; 32 experts, H 4096, I 512, top-4, 300 tokens 74.0 and 70.8; 16, H 2880, I 512, 1400 top-2 87.1 and 84.5.
+// 1031 (this pass fetches 3.43 and 2.08 GB); routed unevenly, 8448 1078, 1004 and 1001.
+// Products, their order and every rounding are stream_gemm_kernel's and the quantiser's.  It is bound by the weights, which it
+// asks for once a block: 100 tokens of 128 experts, H 2048, I 768, top-8: 115 MB asked for, 96 of them distinct, 103 fetched;
+// 22 us and 5 of quantisation in front, 24 this way.  (With a workgroup for 64 rows of a block, as in stream_gemm_kernel, all
+// its weights asked for at once, 33: the start of a workgroup, 7 us, once every 48 KB.)  Whole layer with the norm, quantised
+// in front and here, us: 24 tokens of that layer 47.6 and 46.1, 64 60.7 and 59.2, 100 66.9 and 64.8, 300 105.1 and 102.8; 64
+// experts, H 1024, I 384, top-6: 120 tokens 31.7 and 29.4; 16 experts, 2200 94.8 and 81.1; 32 experts, H 4096, I 512, top-4,
+// 300 tokens 74.0 and 70.8; 16, H 2880, I 512, 1400 top-2 87.1 and 84.5.
 constexpr int kCdCus = 256;
 template <typename Mma, int NU, int NW>
 __global__ __launch_bounds__(NW * kWave, 1) void stream_codes_kernel(
